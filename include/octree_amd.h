@@ -221,8 +221,8 @@ int oct_knn_checksum(oct_ctx *ctx, const int32_t *idx_dev, const float *d2_dev, 
 
 /* ---- tuning (no counterpart in the reference: its per-query loop has no tile shape to choose).
  * OCT_TUNE_RADIUS_GROUP: queries per wave of the count-mode radius kernel (16, 32 or 64 queries
- * share one wave's traversal, 64 / G lanes serve each query), or 0 for the one-lane-per-query
- * kernel; -1 restores "autotuned, else 32". OCT_TUNE_RADIUS_MFMA: the point tests run on the vector
+ * share one wave's traversal, 64 / G lanes serve each query), or 0 for the kernel in which 8 lanes
+ * walk each query's own traversal; -1 restores "autotuned, else 32". OCT_TUNE_RADIUS_MFMA: the point tests run on the vector
  * ALUs (a matrix-core form measured slower on every workload and is not built): 0 and -1 are
  * accepted, 1 fails with OCT_ERR_UNSUPPORTED.
  * oct_autotune_radius: times each candidate (G = 0, 16, 32, 64) on sample_nq queries taken from the

@@ -294,8 +294,8 @@ int oct_batch_build(oct_batch *b) {
     if (nodes >= 0xffffffffull) return bfail(b, OCT_ERR_ARG, "batch beyond 2^32 nodes");
     // the forest
     oct_ctx *f = b->forest;
-    BCHK(f->p64.reserve(pts + 1), "alloc forest points");
-    BCHK(f->p32.reserve(pts + 1), "alloc forest points");
+    BCHK(f->p64.reserve(pts + kPointPad), "alloc forest points");
+    BCHK(f->p32.reserve(pts + kPointPad), "alloc forest points");
     BCHK(f->keys[0].reserve(pts + 1), "alloc forest keys");
     BCHK(f->vals[0].reserve(pts + 1), "alloc forest keys");
     BCHK(f->nodes.reserve(nodes + 8), "alloc forest nodes");
@@ -406,8 +406,8 @@ static int device_setup(oct_batch *b) {
         BCHK(f->keys[1].reserve(n + 1), "alloc keys");
         BCHK(f->vals[0].reserve(n + 1), "alloc keys");
         BCHK(f->vals[1].reserve(n + 1), "alloc keys");
-        BCHK(f->p64.reserve(n + 1), "alloc points");
-        BCHK(f->p32.reserve(n + 1), "alloc points");
+        BCHK(f->p64.reserve(n + kPointPad), "alloc points");
+        BCHK(f->p32.reserve(n + kPointPad), "alloc points");
         b->dev_ready = true;
     }
     const size_t cap = b->cap;

@@ -352,7 +352,7 @@ hipError_t launch_build(oct_ctx *ctx, uint32_t M, std::string &err) {
     uint32_t *total_dev = ctx->misc.p + 8;
 
     // leaf-recentred FP32 cloud and the children tables, sized for the capacity
-    if ((e = ctx->p32.reserve(ctx->n)) != hipSuccess) return e;
+    if ((e = ctx->p32.reserve(ctx->n + kPointPad)) != hipSuccess) return e;
     stage_begin(ctx, ST_BUILD);
     const size_t cap = std::min<size_t>(ctx->nodes.cap, ctx->child.cap - 1);
     if (cap < (1ull << 30)) {

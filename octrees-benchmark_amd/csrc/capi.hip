@@ -311,7 +311,7 @@ static int set_sorted_impl(oct_ctx *ctx, size_t n, const uint64_t *codes, int en
     int r = upload();
     if (r) return r;
     HCHK(ctx->keys[0].reserve(n), "alloc keys");
-    HCHK(ctx->p64.reserve(n), "alloc points");
+    HCHK(ctx->p64.reserve(n + kPointPad), "alloc points");
     if (n) {
         HCHK(hipMemcpyAsync(ctx->keys[0].p, codes, n * 8, hipMemcpyHostToDevice, ctx->stream), "copy codes");
         unsigned nb = (unsigned)std::min<size_t>((n + 255) / 256, 8192);

@@ -37,6 +37,10 @@ struct alignas(64) NodeExt {
 };
 static_assert(sizeof(NodeExt) == 192, "NodeExt is three 64-byte lines");
 
+// Points allocated past the end of the sorted clouds (p64, p32): the group kernels read a leaf's points
+// in steps of 16 and ignore what lies past it.
+constexpr size_t kPointPad = 16;
+
 // Device buffer that only grows.
 template <class T>
 struct DevBuf {
@@ -192,7 +196,7 @@ hipError_t launch_build(oct_ctx *ctx, uint32_t max_points_leaf, std::string &err
 // centre is qxyz[id] if given, else the sorted point qidx[id] (or id); outputs are indexed by id.
 struct RadiusLaunch {
     int kernel = 1, algo = 3, precision = 0, mode = 0;
-    int group = 16;  // count mode: queries per wave (16, 32, 64), or 0 for the one-lane-per-query kernel
+    int group = 16;  // count mode: queries per wave (16, 32, 64), or 0 for the group kernel (8 lanes per query)
     bool remap = true;  // count mode, vector point tests: compact the queries of sparsely wanted leaves
     uint32_t approx_level = ~0u;  // OCT_ALGO_APPROX: neighborsApprox depth cutoff and bound mode
     bool approx_upper = false;

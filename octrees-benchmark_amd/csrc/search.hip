@@ -1,319 +1,361 @@
 // H5: radius searches (neighbors / neighborsPrune / neighborsStruct x sphere / circle / cube /
 // square) on gfx950.
 //
-// Work decomposition: one wave64 = 64 consecutive query slots (SFC-ordered queries are spatially
-// coherent). The wave walks the union of its lanes' traversals with one wave-uniform DFS stack in
-// LDS; each stack entry carries the mask of lanes for which the node is OVERLAP. Per child, every
-// lane in the mask classifies the node for its own query with the reference's FP64 expressions, so
-// each lane makes exactly the reference's decisions, and - because the union DFS restricted to one
-// lane is that lane's own DFS (same child order, same LIFO stack discipline as singleTraversal,
-// linear_octree.hpp:653-686) - each lane emits its neighbours in the reference's order.
-// Node records and leaf points are wave-uniform loads (one fetch serves all 64 lanes).
+// Two kernels, both making exactly the reference's decisions for every query:
+//  - k_group: a group of 8 lanes per query, each group with its own traversal (result lists, and counts
+//    of queries that are far apart or few);
+//  - k_count: 16 - 64 consecutive queries per wave that share one traversal (counts of many queries that
+//    lie together, the all-points searches).
 //
 // Per-point tests:
 //  - FP64: the reference's isInside expression (kernel_3d.hpp:127-138, 232-242; kernel_2d.hpp:53-63,
 //    153-162), evaluated as written (no contraction).
-//  - FP32_RECHECK (sphere, circle), list kernel k_radius: leaf-recentred FP32 coordinates a
-//    (w = |a|^2 precomputed) and b = fl32(q - c_leaf); M = fl32(R - |b|^2);
-//    u = fma(ax, -2bx, fma(ay, -2by, fma(az, -2bz, w - M))) (circle: fma(ax, ax - 2bx,
-//    fma(ay, ay - 2by, -M))) approximates |p - q|^2 - R. Every rounding of this evaluation and of
-//    the reference's FP64 one is bounded by hw = 2^-20 (amax + |b|^2 + R)(1 + 2^-10) + |M - thr|,
-//    amax = max |a|^2 over the leaf (u32 = 2^-24: |error| <= u32 (13.01 amax + 12.01 |b|^2 + 4 R)
-//    + |M - thr| + O(u64)), so u < -hw is inside, u > hw outside, and points with |u| <= hw are
-//    re-evaluated with the FP64 expression. In count mode a lane re-counts a whole leaf in FP64 if
-//    any point fell in the band.
-//  - FP32_RECHECK, count kernel k_count: the same u with the band folded in, t = u + hw, from an
-//    FP32 set-up and a wider band hw = 2^-18 (amax + |b|^2 + R) that covers the FP32 set-up's
-//    roundings as well (its bound: see the leaf's tests in k_count); counts come from sign bits.
+//  - FP32_RECHECK (sphere, circle): leaf-recentred FP32 coordinates a (w = |a|^2 precomputed) and
+//    b = fl32(q - c_leaf); t = fma(ax, -2bx, fma(ay, -2by, fma(az, -2bz, w + C))) (circle: fma(ax,
+//    ax - 2bx, fma(ay, ay - 2by, C))) approximates |p - q|^2 - R + hw with a band hw = 2^-18 (amax +
+//    |b|^2 + R), amax = max |a|^2 over the leaf, that covers every rounding of this evaluation and of the
+//    reference's FP64 one (its bound: see the leaf's tests in k_count). A set sign bit is inside, t > 2 hw
+//    outside, and what lies between is decided by the FP64 expression.
 //  - A leaf/query pair whose FP32 terms could overflow, or a leaf holding a non-finite FP32 point
 //    (then amax = inf), is decided in FP64 throughout.
 //  - Cube/square tests are comparisons only and run on the FP64 coordinates in both modes.
+#include <algorithm>
 #include <type_traits>
 
 #include "search_common.hpp"
 
 namespace oct {
 
-// Per-lane output sink. MODE 0: neighbour counts only; 1: counts + list-entry counts; 2: fill lists.
-template <int ALGO, int MODE>
-struct Sink {
-    uint32_t cnt = 0;   // neighbour points
-    uint32_t ecnt = 0;  // list entries (indices, or ranges for Struct)
-    uint64_t base = 0;  // fill offset
-    uint32_t *entries = nullptr;
+// ------------------------------------------------------------------ group kernel: one query per 8 lanes
+// Result lists, and counts of queries that lie far apart. A group of 8 lanes walks its own query's
+// traversal; a wave serves 8 queries, each with its own position in the tree:
+//  - a popped node's 8 children are judged one per lane with the reference's FP64 expressions, 8 nodes
+//    (one per group) per step. The children still to be visited are one bit per (level, lane): lane c's
+//    `pend` has bit L set while child c at level L waits, `lvl` has bit L set while any does. Taking the
+//    highest waiting octant of the deepest level is the reference's LIFO order (singleTraversal,
+//    linear_octree.hpp:653-686), so lists come out in the reference's emission order;
+//  - the OVERLAP leaves (and, when lists are filled, the INSIDE ranges) of a popped node go to the
+//    group's queue in octant order, with the leaf's FP32 terms formed by the lane that judged it. When
+//    no group can go on (queue full or traversal done), every group tests its queued points, 16 per
+//    step, and writes its hits side by side: 8 lanes' hits of a step are consecutive list entries.
+// What bounds it: vector issue (4.2 k vector instructions per wave of 8 queries at 84 neighbours each)
+// and, for few queries, the chain of dependent loads of one traversal. Against a wave of 64 queries that
+// shares one traversal, each lane writing its own list and reading the points one by one: 10 000 random
+// centres of a 1 M-point box, r = 2.5 (both list passes) 14.6 -> 0.45 ms; 1 M consecutive points of a
+// 5 M-point tile, r = 1, index lists 2.91 -> 2.14 ms; 2 M of 20 M, r = 2.5, ranges 17.2 -> 12.1 ms.
+constexpr int kGroupLanes = 8;
+constexpr int kGroupsPerWave = 64 / kGroupLanes;
+constexpr int kGroupQueue = 16;  // queued items per group; a pop adds at most 8
+constexpr int kGroupMaxLevels = (int)kMaxDepth;  // levels that can hold internal nodes (0 .. 20)
 
-    __device__ inline void range(uint32_t first, uint32_t last) {  // INSIDE node
-        if (ALGO == OCT_ALGO_STRUCT || ALGO == OCT_ALGO_APPROX) {  // NeighborSet::addRange keeps empty ranges
-            if (MODE == 2) {
-                entries[2 * (base + ecnt)] = first;
-                entries[2 * (base + ecnt) + 1] = last;
-            }
-            ecnt++;
-            cnt += last - first;
-        } else {
-            if (MODE == 2)
-                for (uint32_t i = first; i < last; i++) entries[base + ecnt + (i - first)] = i;
-            ecnt += last - first;
-            cnt += last - first;
-        }
-    }
-    __device__ inline void point(uint32_t i) {  // Prune / neighbors leaf hit
-        if (MODE == 2) entries[base + ecnt] = i;
-        ecnt++;
-        cnt++;
-    }
-    __device__ inline void run(uint32_t first, uint32_t last) {  // Struct leaf run (non-empty)
-        if (MODE == 2) {
-            entries[2 * (base + ecnt)] = first;
-            entries[2 * (base + ecnt) + 1] = last;
-        }
-        ecnt++;
-        cnt += last - first;
-    }
+// A queued item, [slot * 8 + group]: the point range (bit 31 of last: an INSIDE range) and, for an FP32
+// leaf, its terms. One slot more than can be filled: groups that are done read it while others go on.
+template <bool FP32>
+struct GroupItems {
+    uint2 range[(kGroupQueue + 1) * kGroupsPerWave];
+};
+template <>
+struct GroupItems<true> {
+    uint4 range_xy[(kGroupQueue + 1) * kGroupsPerWave];  // first, last, -2bx, -2by (bits)
+    uint4 z_c_lim[(kGroupQueue + 1) * kGroupsPerWave];   // -2bz, C, lim (bits)
 };
 
+// boxIntersect / boxOverlap of one node without branches: in = INSIDE, ov = OVERLAP (neither: OUTSIDE).
+// The comparisons and sums are classify64's and overlap64's, in the same order.
+template <int KERNEL, int ALGO>
+__device__ inline void judge_node(const Query &q, const NodeRec &n, double rx, double ry, double rz, bool &in, bool &ov) {
+    constexpr bool is3d = KERNEL == OCT_KERNEL_SPHERE || KERNEL == OCT_KERNEL_CUBE;
+    if (ALGO == OCT_ALGO_NEIGHBORS || KERNEL == OCT_KERNEL_CUBE || KERNEL == OCT_KERNEL_SQUARE) {
+        const double hx = n.cx + rx, lx = n.cx - rx, hy = n.cy + ry, ly = n.cy - ry, hz = n.cz + rz, lz = n.cz - rz;
+        bool out = (hx < q.lox) | (hy < q.loy) | (lx > q.hix) | (ly > q.hiy);
+        if (is3d) out |= (hz < q.loz) | (lz > q.hiz);
+        bool inside = false;
+        if (ALGO != OCT_ALGO_NEIGHBORS) {
+            inside = (hx <= q.hix) & (hy <= q.hiy) & (lx >= q.lox) & (ly >= q.loy);
+            if (is3d) inside &= (hz <= q.hiz) & (lz >= q.loz);
+        }
+        in = !out & inside;
+        ov = !out & !inside;
+    } else {
+        const double dx = fabs(q.x - n.cx), dy = fabs(q.y - n.cy), dz = is3d ? fabs(q.z - n.cz) : 0.0;
+        bool out = (dx > q.r + rx) | (dy > q.r + ry);
+        if (is3d) out |= dz > q.r + rz;
+        const double ex = dx + rx, ey = dy + ry;
+        const double fx = dmax0(dx - rx), fy = dmax0(dy - ry);
+        double smax = ex * ex + ey * ey, smin = fx * fx + fy * fy;
+        const bool nx = dx < rx, ny = dy < ry;
+        bool two = nx & ny;  // at least two axes within the node's slab (the two of a 2-D kernel)
+        if (is3d) {
+            const double ez = dz + rz, fz = dmax0(dz - rz);
+            smax = smax + ez * ez, smin = smin + fz * fz;
+            two |= (dz < rz) & (nx | ny);
+        }
+        const bool inside = smax <= q.R;
+        in = !out & inside;
+        ov = !out & !inside & (two | (smin <= q.R));
+    }
+}
+
+// MODE 0: neighbour counts; 1: counts and list-entry counts; 2: fill the lists at their offsets.
 template <int KERNEL, int ALGO, int PREC, int MODE>
-__global__ __launch_bounds__(kSearchBlock) void k_radius(const SearchArgs a) {
-    __shared__ uint32_t s_node[kWaves][kStack];
-    __shared__ uint64_t s_mask[kWaves][kStack];
-    __shared__ uint8_t s_depth[kWaves][kStack];
+__global__ __launch_bounds__(kSearchBlock) void k_group(const SearchArgs a) {
+    constexpr bool kFp32 = PREC == OCT_PREC_FP32_RECHECK && (KERNEL == OCT_KERNEL_SPHERE || KERNEL == OCT_KERNEL_CIRCLE);
+    constexpr bool kRanges = ALGO == OCT_ALGO_STRUCT || ALGO == OCT_ALGO_APPROX;  // lists of [first, last) ranges
+    constexpr uint32_t kInside = 0x80000000u;
+    constexpr uint64_t kBit0 = 0x0101010101010101ull;  // the first lane of every group
+    __shared__ GroupItems<kFp32> s_items[kWaves];
+    __shared__ double s_rad[3 * (kMaxDepth + 1)];
+    extern __shared__ uint32_t s_gc_all[];  // per wave, per level: each lane's child's first child
+    for (uint32_t i = threadIdx.x; i < 3 * (kMaxDepth + 1); i += kSearchBlock) s_rad[i] = a.radtab[i];
+    __syncthreads();
 
-    const uint32_t w = threadIdx.x >> 6;
-    const uint32_t lane = threadIdx.x & 63;
-    const uint64_t lanebit = 1ull << lane;
+    const uint32_t w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const uint32_t grp = lane >> 3, c = lane & 7u, gshift = lane & 56u;
+    const uint32_t below = (1u << c) - 1u;
+    uint32_t *s_gc = s_gc_all + (size_t)w * a.levels * 64;
+    GroupItems<kFp32> &Q = s_items[w];
     const uint32_t tile = blockIdx.x * kWaves + w;
-    const uint32_t slot = tile * 64 + lane;
+    if (uniform_u32(tile * kGroupsPerWave) >= a.nq) return;
+    const uint32_t slot = tile * kGroupsPerWave + grp;
     const bool valid = slot < a.nq;
-    if (uniform_u32(tile * 64) >= a.nq) return;
+    auto wsync = [&]() {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
+    auto group_bits = [&](bool p) -> uint32_t { return (uint32_t)(ballot64(p) >> gshift) & 255u; };
 
-    // ---- per-lane query
     Query q;
     uint32_t qid = 0;
-    {
-        q.x = q.y = q.z = 0.0;
-        q.r = 0.0;
-        if (valid) {
-            qid = a.order ? a.order[slot] : slot;
-            if (a.qxyz) {
-                q.x = a.qxyz[3 * (size_t)qid], q.y = a.qxyz[3 * (size_t)qid + 1], q.z = a.qxyz[3 * (size_t)qid + 2];
-            } else {
-                uint32_t pi = a.qidx ? a.qidx[qid] : qid;
-                double4 p = a.p64[pi];
-                q.x = p.x, q.y = p.y, q.z = p.z;
-            }
-            q.r = a.qrad ? a.qrad[qid] : a.radius;
+    q.x = q.y = q.z = 0.0;
+    q.r = 0.0;
+    if (valid) {
+        qid = a.order ? a.order[slot] : slot;
+        if (a.qxyz) {
+            q.x = a.qxyz[3 * (size_t)qid], q.y = a.qxyz[3 * (size_t)qid + 1], q.z = a.qxyz[3 * (size_t)qid + 2];
+        } else {
+            const double4 p = a.p64[a.qidx ? a.qidx[qid] : qid];
+            q.x = p.x, q.y = p.y, q.z = p.z;
         }
-        q.R = q.r * q.r;
-        q.lox = q.x - q.r, q.loy = q.y - q.r, q.loz = q.z - q.r;
-        q.hix = q.x + q.r, q.hiy = q.y + q.r, q.hiz = q.z + q.r;
-        if (KERNEL == OCT_KERNEL_CUBE || KERNEL == OCT_KERNEL_SQUARE) box_radii(a, valid, qid, q);
+        q.r = a.qrad ? a.qrad[qid] : a.radius;
     }
-    Sink<ALGO, MODE> sink;
-    if (MODE == 2 && valid) {
-        sink.base = a.offsets[qid];
-        sink.entries = a.entries;
-    }
-    uint64_t n_class = 0, n_test = 0, n_recheck = 0, n_cslots = 0, n_tslots = 0;
+    q.R = q.r * q.r;
+    q.lox = q.x - q.r, q.loy = q.y - q.r, q.loz = q.z - q.r;
+    q.hix = q.x + q.r, q.hiy = q.y + q.r, q.hiz = q.z + q.r;
+    if (KERNEL == OCT_KERNEL_CUBE || KERNEL == OCT_KERNEL_SQUARE) box_radii(a, valid, qid, q);
+    const float qRf = (float)q.R;
+    uint32_t *out = nullptr;  // MODE 2: the query's list
+    if (MODE == 2 && valid) out = a.entries + a.offsets[qid] * (kRanges ? 2u : 1u);
 
-    // ---- classification helper: returns the lane's judgement for node c at depth d
-    auto judge = [&](uint64_t m, const NodeRec &nr, uint32_t d) -> int {
-        if (!(m & lanebit)) return -1;
-        // neighborsApprox beyond its precision level: the node's range whole, or nothing
-        // (linear_octree.hpp:987-994)
-        if (ALGO == OCT_ALGO_APPROX && d > a.approx_level) return a.approx_upper ? J_INSIDE : J_OUTSIDE;
-        if (ALGO == OCT_ALGO_NEIGHBORS)
-            return overlap64<KERNEL>(q, nr.cx, nr.cy, nr.cz, a.rad[d][0], a.rad[d][1], a.rad[d][2]) ? J_OVERLAP : J_OUTSIDE;
-        return classify64<KERNEL>(q, nr.cx, nr.cy, nr.cz, a.rad[d][0], a.rad[d][1], a.rad[d][2]);
+    uint32_t cnt = 0, ecnt = 0;  // MODE 0, 1: this lane's share of the query's counts
+    uint32_t off = 0;            // MODE 2: entries written so far (the same in the group's lanes)
+    uint32_t n_class = 0, n_recheck = 0, n_csteps = 0, n_tsteps = 0;
+    uint64_t n_test = 0;
+    uint32_t qn = 0;             // queued items
+    uint32_t lvl = 0, pend = 0;  // levels with waiting children; levels at which this lane's child waits
+    bool overflow = false;
+
+    // a judged child of the query's traversal is counted, queued, made to wait or dropped. Called by all
+    // lanes of a group at once (act = false: no child in this lane); L is the child's level.
+    auto take = [&](const bool act, const NodeRec &nr, const uint32_t gc, const float am, const uint32_t L) {
+        bool in, ov;
+        judge_node<KERNEL, ALGO>(q, nr, s_rad[3 * L], s_rad[3 * L + 1], s_rad[3 * L + 2], in, ov);
+        // neighborsApprox beyond its precision level: the node's range whole, or nothing (linear_octree.hpp:987-994)
+        if (ALGO == OCT_ALGO_APPROX && L > a.approx_level) in = a.approx_upper != 0, ov = false;
+        in &= act, ov &= act;
+        n_class += act ? 1u : 0u;
+        const bool some = nr.last > nr.first;
+        const bool leaf = ov & (gc == 0) & some;  // an empty leaf adds nothing
+        if (MODE != 2 && in) {
+            cnt += nr.last - nr.first;
+            if (kRanges) ecnt++;  // NeighborSet::addRange keeps empty ranges (neighbor_set.hpp:84-89)
+        }
+        const bool item = leaf | (MODE == 2 && in && (kRanges || some));
+        const uint32_t im = group_bits(item);
+        if (item) {
+            const uint32_t s = (qn + (uint32_t)__popc(im & below)) * kGroupsPerWave + grp;
+            const uint32_t last = nr.last | (MODE == 2 && in ? kInside : 0u);
+            if (leaf) n_test += nr.last - nr.first;
+            if constexpr (kFp32) {
+                // the leaf's FP32 form with the band folded in: t = w + C - 2 a.b (circle: its two axes)
+                // approximates |p - q|^2 - R + hw; its bound stands at the count kernel's leaf tests. Sign
+                // bit set: inside; bits above lim: outside; else (or lim = ~0, where the FP32 terms could
+                // overflow) the FP64 test decides.
+                const float bx = (float)(q.x - nr.cx), by = (float)(q.y - nr.cy), bz = (float)(q.z - nr.cz);
+                const float b2 = KERNEL == OCT_KERNEL_SPHERE ? __builtin_fmaf(bx, bx, __builtin_fmaf(by, by, bz * bz))
+                                                             : __builtin_fmaf(bx, bx, by * by);
+                const float sum = (am + b2) + qRf;
+                const float hw = 3.814697265625e-06f * sum;  // 2^-18
+                Q.range_xy[s] = make_uint4(nr.first, last, __float_as_uint(-2.0f * bx), __float_as_uint(-2.0f * by));
+                Q.z_c_lim[s] = make_uint4(__float_as_uint(-2.0f * bz), __float_as_uint((hw - qRf) + b2),
+                                          sum < 1e30f ? __float_as_uint(2.0f * hw) : 0xffffffffu, 0u);
+            } else {
+                Q.range[s] = make_uint2(nr.first, last);
+            }
+        }
+        qn += (uint32_t)__popc(im);
+        const bool wait = ov & (gc != 0);
+        const uint64_t wm = ballot64(wait);
+        if (wm) {
+            if (wait) s_gc[L * 64 + lane] = gc, pend |= 1u << L;
+            if ((wm >> gshift) & 255u) lvl |= 1u << L;
+        }
     };
 
-    // ---- leaf: lanes in m test the leaf's points (endpointAction, linear_octree.hpp:716-732, 771-780, 804-813)
-    auto leaf = [&](uint64_t m, uint32_t c, const NodeRec &nr) {
-        const bool act = (m & lanebit) != 0;
-        const uint32_t first = uniform_u32(nr.first), last = uniform_u32(nr.last);
-        n_test += (uint64_t)__popcll(m) * (last - first);
-        n_tslots += 64ull * (last - first);
-        constexpr bool kFp32 = PREC == OCT_PREC_FP32_RECHECK && (KERNEL == OCT_KERNEL_SPHERE || KERNEL == OCT_KERNEL_CIRCLE);
-        // FP32 band setup (per lane, per leaf). u = w - 2 a.b - M approximates |p - q|^2 - R with
-        // |error| <= hw (see the file header), so u < -hw is inside, u > hw outside, else recheck.
-        float M = 0.f, hw = 0.f, ux = 0.f, uy = 0.f, uz = 0.f;
-        bool force = false;  // FP32 terms could overflow: every point of the leaf is decided in FP64
-        if (kFp32) {
-            const float bx = (float)(q.x - nr.cx), by = (float)(q.y - nr.cy), bz = (float)(q.z - nr.cz);
-            double b2 = (double)bx * (double)bx + (double)by * (double)by;
-            if (KERNEL == OCT_KERNEL_SPHERE) b2 += (double)bz * (double)bz;
-            const double am = (double)a.amax[c];
-            const double thr = q.R - b2;
-            M = (float)thr;
-            const double delta = 9.5367431640625e-07 * (am + b2 + q.R) * 1.0009765625 + 1e-30;  // 2^-20 (..)(1 + 2^-10)
-            hw = __double2float_ru(delta + fabs((double)M - thr));
-            force = !(2.0 * am + 3.0 * b2 + 2.0 * q.R < 1e38);
-            ux = -2.0f * bx, uy = -2.0f * by, uz = -2.0f * bz;
-        }
-        auto u32f = [&](const float4 &p) -> float {
-            if (KERNEL == OCT_KERNEL_SPHERE) return __builtin_fmaf(p.x, ux, __builtin_fmaf(p.y, uy, __builtin_fmaf(p.z, uz, p.w - M)));
-            return __builtin_fmaf(p.x, p.x + ux, __builtin_fmaf(p.y, p.y + uy, -M));
-        };
-        if (MODE == 0) {
-            // count only: no per-point control flow. cin counts t < L; mn tracks min |t - mid| over
-            // the leaf, so a lane has a point inside the band [L, H] iff mn <= hw.
-            uint32_t cin = 0;
-            if (kFp32) {
-                const float nhw = -hw;
-                float mn = __builtin_huge_valf();
-                uint32_t c0 = 0, c1 = 0, c2 = 0, c3 = 0;  // one counter per unroll slot: compare + carry-add
-                uint32_t i = first;
-                for (; i + 4 <= last; i += 4) {
-                    const float4 p0 = a.p32[i], p1 = a.p32[i + 1], p2 = a.p32[i + 2], p3 = a.p32[i + 3];
-                    const float u0 = u32f(p0), u1 = u32f(p1), u2 = u32f(p2), u3 = u32f(p3);
-                    c0 += (u0 < nhw) ? 1u : 0u;
-                    c1 += (u1 < nhw) ? 1u : 0u;
-                    c2 += (u2 < nhw) ? 1u : 0u;
-                    c3 += (u3 < nhw) ? 1u : 0u;
-                    mn = fminf(mn, fminf(fabsf(u0), fabsf(u1)));
-                    mn = fminf(mn, fminf(fabsf(u2), fabsf(u3)));
-                }
-                for (; i < last; i++) {
-                    const float u = u32f(a.p32[i]);
-                    c0 += (u < nhw) ? 1u : 0u;
-                    mn = fminf(mn, fabsf(u));
-                }
-                cin = (c0 + c1) + (c2 + c3);
-                const bool unc = act && (!(mn > hw) || force);
-                if (ballot64(unc)) {  // rare: re-count this leaf exactly for the lanes with a band hit
-                    if (unc) {
-                        n_recheck += last - first;
-                        cin = 0;
-                        for (uint32_t j = first; j < last; j++) {
-                            const double4 pd = a.p64[j];
-                            cin += inside64<KERNEL>(q, pd.x, pd.y, pd.z);
+    // tests the queued points of every group, 16 per step, in queue order
+    auto flush = [&]() {
+        wsync();
+        uint32_t it = 0, i = 0;
+        bool fresh = true;     // step starts a new item
+        uint64_t carry = 0;    // range lists: groups (bit 8g) whose current run reaches the step's first point
+        while (ballot64(it < qn)) {
+            n_tsteps++;
+            const uint32_t s = it * kGroupsPerWave + grp;
+            uint32_t first, last, lim = 0;
+            float ux = 0.f, uy = 0.f, uz = 0.f, C = 0.f;
+            if constexpr (kFp32) {
+                const uint4 A = Q.range_xy[s], B = Q.z_c_lim[s];
+                first = A.x, last = A.y, ux = __uint_as_float(A.z), uy = __uint_as_float(A.w);
+                uz = __uint_as_float(B.x), C = __uint_as_float(B.y), lim = B.z;
+            } else {
+                const uint2 A = Q.range[s];
+                first = A.x, last = A.y;
+            }
+            const bool ins = MODE == 2 && (last & kInside) != 0;
+            const uint32_t e = MODE == 2 ? last & ~kInside : last;
+            if (fresh) i = first;
+            const uint32_t rem = it < qn ? e - i : 0u;
+            const uint32_t i0 = i + c, i1 = i0 + 8;
+            const bool v0 = c < rem, v1 = c + 8 < rem;
+            bool in0 = false, in1 = false;
+            if (v0 & !ins) {  // reads up to 15 points past the range: the sorted clouds are padded (kPointPad)
+                if constexpr (kFp32) {
+                    const float4 p0 = a.p32[i0], p1 = a.p32[i1];
+                    float t0, t1;
+                    if (KERNEL == OCT_KERNEL_SPHERE) {
+                        t0 = __builtin_fmaf(p0.x, ux, __builtin_fmaf(p0.y, uy, __builtin_fmaf(p0.z, uz, p0.w + C)));
+                        t1 = __builtin_fmaf(p1.x, ux, __builtin_fmaf(p1.y, uy, __builtin_fmaf(p1.z, uz, p1.w + C)));
+                    } else {
+                        t0 = __builtin_fmaf(p0.x, p0.x + ux, __builtin_fmaf(p0.y, p0.y + uy, C));
+                        t1 = __builtin_fmaf(p1.x, p1.x + ux, __builtin_fmaf(p1.y, p1.y + uy, C));
+                    }
+                    const uint32_t d0 = __float_as_uint(t0), d1 = __float_as_uint(t1);
+                    in0 = (int32_t)d0 < 0, in1 = v1 & ((int32_t)d1 < 0);
+                    const bool k0 = d0 <= lim, k1 = v1 & (d1 <= lim);
+                    if (k0 | k1) {
+                        if (k0) {
+                            const double4 pd = a.p64[i0];
+                            in0 = inside64<KERNEL>(q, pd.x, pd.y, pd.z);
+                            n_recheck++;
+                        }
+                        if (k1) {
+                            const double4 pd = a.p64[i1];
+                            in1 = inside64<KERNEL>(q, pd.x, pd.y, pd.z);
+                            n_recheck++;
                         }
                     }
-                }
-            } else {
-                uint32_t i = first;
-                for (; i + 4 <= last; i += 4) {
-                    const double4 p0 = a.p64[i], p1 = a.p64[i + 1], p2 = a.p64[i + 2], p3 = a.p64[i + 3];
-                    cin += inside64<KERNEL>(q, p0.x, p0.y, p0.z);
-                    cin += inside64<KERNEL>(q, p1.x, p1.y, p1.z);
-                    cin += inside64<KERNEL>(q, p2.x, p2.y, p2.z);
-                    cin += inside64<KERNEL>(q, p3.x, p3.y, p3.z);
-                }
-                for (; i < last; i++) {
-                    const double4 p = a.p64[i];
-                    cin += inside64<KERNEL>(q, p.x, p.y, p.z);
+                } else {
+                    const double4 p0 = a.p64[i0], p1 = a.p64[i1];
+                    in0 = inside64<KERNEL>(q, p0.x, p0.y, p0.z);
+                    in1 = v1 & inside64<KERNEL>(q, p1.x, p1.y, p1.z);
                 }
             }
-            if (act) sink.cnt += cin;
-            return;
+            if (MODE == 2 && ins) in0 = v0, in1 = v1;
+            const bool next = rem <= 16;  // the item ends with this step
+            if (MODE != 2) cnt += in0 ? 1u : 0u, cnt += in1 ? 1u : 0u;
+            if constexpr (kRanges && MODE != 0) {
+                // runs as lane masks: a hit starts one when the point before it is none, a miss ends one
+                const bool one = MODE == 2 && ins;  // an INSIDE range is one entry, written below
+                const uint64_t m0 = ballot64(in0 & !one), m1 = ballot64(in1 & !one);
+                const uint64_t pr0 = ((m0 << 1) & ~kBit0) | carry, pr1 = ((m1 << 1) & ~kBit0) | ((m0 >> 7) & kBit0);
+                const uint64_t st0 = m0 & ~pr0, st1 = m1 & ~pr1;
+                if (MODE == 1) {
+                    ecnt += __builtin_amdgcn_inverse_ballot_w64(st0) ? 1u : 0u;
+                    ecnt += __builtin_amdgcn_inverse_ballot_w64(st1) ? 1u : 0u;
+                } else {
+                    const uint32_t sb = ((uint32_t)(st0 >> gshift) & 255u) | (((uint32_t)(st1 >> gshift) & 255u) << 8);
+                    const uint32_t r0 = off + (uint32_t)__popc(sb & below), r1 = off + (uint32_t)__popc(sb & ((1u << (c + 8)) - 1u));
+                    off += (uint32_t)__popc(sb);
+                    if (__builtin_amdgcn_inverse_ballot_w64(st0)) out[2 * (size_t)r0] = i0;
+                    if (__builtin_amdgcn_inverse_ballot_w64(st1)) out[2 * (size_t)r1] = i1;
+                    if (__builtin_amdgcn_inverse_ballot_w64(~m0 & pr0)) out[2 * (size_t)r0 - 1] = i0;
+                    if (__builtin_amdgcn_inverse_ballot_w64(~m1 & pr1)) out[2 * (size_t)r1 - 1] = i1;
+                    // the leaf ends with the step's last point and that is a hit
+                    if (in1 & !one & (c == 7) & (rem == 16)) out[2 * (size_t)off - 1] = e;
+                    if (one && it < qn) {
+                        if (c == 0) out[2 * (size_t)off] = first, out[2 * (size_t)off + 1] = e;
+                        off++;
+                    }
+                }
+                carry = (m1 >> 7) & kBit0 & ~ballot64(next);
+            } else if constexpr (MODE == 2) {
+                const uint32_t m = group_bits(in0) | (group_bits(in1) << 8);
+                if (in0) out[off + (uint32_t)__popc(m & below)] = i0;
+                if (in1) out[off + (uint32_t)__popc(m & ((1u << (c + 8)) - 1u))] = i1;
+                off += (uint32_t)__popc(m);
+            }
+            const bool done = next | (kRanges && ins);
+            fresh = done;
+            i += 16;
+            if (it < qn && done) it++;
         }
-        // list modes: per-point decisions in the reference's order
-        uint32_t rs = first;  // Struct run start
-        for (uint32_t i = first; i < last; i++) {
-            bool in;
-            if (kFp32) {
-                const float u = u32f(a.p32[i]);
-                in = !force && u < -hw;
-                if (__builtin_expect(act && !in && (u <= hw || force), 0)) {
-                    const double4 pd = a.p64[i];
-                    in = inside64<KERNEL>(q, pd.x, pd.y, pd.z);
-                    n_recheck++;
-                }
-            } else {
-                const double4 p = a.p64[i];
-                in = inside64<KERNEL>(q, p.x, p.y, p.z);
-            }
-            in = in && act;
-            if (ALGO == OCT_ALGO_STRUCT || ALGO == OCT_ALGO_APPROX) {
-                if (act && !in) {
-                    if (rs < i) sink.run(rs, i);
-                    rs = i + 1;
-                }
-            } else if (in) {
-                sink.point(i);
-            }
-        }
-        if ((ALGO == OCT_ALGO_STRUCT || ALGO == OCT_ALGO_APPROX) && act && rs < last) sink.run(rs, last);
+        wsync();  // the queue is rewritten next
+        qn = 0;
     };
 
-    // ---- root (singleTraversal, linear_octree.hpp:655-662)
-    uint32_t sp = 0;
-    bool overflow = false;  // wave-uniform: a push found the stack full (cannot happen within 21 levels)
-    {
-        const NodeRec nr = a.nodes[0];
-        const uint64_t m0 = ballot64(valid);
-        n_class += __popcll(m0);
-        n_cslots += 64;
-        const int j = judge(m0, nr, 0);
-        if (j == J_INSIDE) sink.range(nr.first, nr.last);
-        const uint64_t ov = ballot64(j == J_OVERLAP);
-        if (ov) {
-            if (a.child[0] == 0) {
-                leaf(ov, 0, nr);
-            } else {
-                s_node[w][0] = 0, s_mask[w][0] = ov, s_depth[w][0] = 0;
-                sp = 1;
+    // root (singleTraversal, linear_octree.hpp:655-662): judged by the group's first lane
+    take(valid && c == 0, a.nodes[0], a.child[0], a.amax[0], 0);
+    for (;;) {
+        for (;;) {
+            const bool go = lvl != 0 && qn <= (uint32_t)(kGroupQueue - 8);
+            if (!ballot64(go)) break;
+            n_csteps++;
+            if (go) {
+                wsync();
+                const uint32_t L = 31u - (uint32_t)__clz(lvl);  // the deepest level with waiting children
+                const uint32_t wm = group_bits((pend >> L) & 1u);
+                const uint32_t oct = 31u - (uint32_t)__clz(wm);  // the last one made to wait
+                const uint32_t fc = s_gc[L * 64 + gshift + oct];
+                if (c == oct) pend &= ~(1u << L);
+                if ((wm & (wm - 1u)) == 0) lvl &= ~(1u << L);
+                const uint32_t node = fc + c;
+                const NodeRec nr = a.nodes[node];
+                const uint32_t gc = a.child[node];
+                const float am = kFp32 ? a.amax[node] : 0.0f;  // (an internal node's value is not used)
+                const bool fits = L + 1 < a.levels || gc == 0;
+                overflow |= !fits;  // an internal node below the tree's last level: cannot happen
+                take(fits, nr, gc, am, L + 1);
             }
         }
-    }
-    // ---- DFS: pop, classify the 8 children, emit INSIDE ranges and OVERLAP leaves in octant order,
-    //      push OVERLAP internal children (they are popped last-pushed-first, as the reference does)
-    while (sp > 0) {
-        sp--;
-        const uint32_t node = uniform_u32(s_node[w][sp]);
-        const uint64_t m = uniform_u64(s_mask[w][sp]);
-        const uint32_t d = uniform_u32(s_depth[w][sp]) + 1;
-        const uint32_t first_child = uniform_u32(a.child[node]);
-        for (uint32_t oct = 0; oct < 8; oct++) {
-            const uint32_t c = first_child + oct;
-            const NodeRec nr = a.nodes[c];
-            // An empty child cannot change counts or index lists whatever its class; only Struct
-            // range lists keep empty INSIDE ranges (neighbor_set.hpp:84-89). It still counts as
-            // classified: the reference's traversal evaluates its criterion.
-            n_class += __popcll(m);
-            if (!((ALGO == OCT_ALGO_STRUCT || ALGO == OCT_ALGO_APPROX) && MODE != 0) && uniform_u32(nr.first) == uniform_u32(nr.last))
-                continue;
-            n_cslots += 64;
-            const int j = judge(m, nr, d);
-            if (j == J_INSIDE) sink.range(nr.first, nr.last);
-            const uint64_t ov = ballot64(j == J_OVERLAP);
-            if (ov) {
-                const uint32_t cc = uniform_u32(a.child[c]);
-                if (cc == 0) {
-                    leaf(ov, c, nr);
-                } else if (sp < kStack) {
-                    s_node[w][sp] = c, s_mask[w][sp] = ov, s_depth[w][sp] = (uint8_t)d;
-                    sp++;
-                } else {
-                    overflow = true;
-                }
-            }
-        }
+        if (!ballot64(qn != 0)) break;  // nothing queued: every traversal is done
+        flush();
     }
 
-    if (overflow && lane == 0) atomicOr(a.err, kErrStack);
-    if (valid) {
-        if (MODE != 2) {
-            if (a.counts) a.counts[qid] = sink.cnt;
-            if (MODE == 1 && a.ecounts) a.ecounts[qid] = sink.ecnt;
-            if (MODE == 1 && a.ecounts64) a.ecounts64[qid] = sink.ecnt;
+    if (ballot64(overflow) && lane == 0) atomicOr(a.err, kErrStack);
+    if (MODE != 2) {
+        cnt += lane_xor<1>(cnt), cnt += lane_xor<2>(cnt), cnt += lane_xor<4>(cnt);
+        if (MODE == 1 && kRanges) ecnt += lane_xor<1>(ecnt), ecnt += lane_xor<2>(ecnt), ecnt += lane_xor<4>(ecnt);
+        if (MODE == 1 && !kRanges) ecnt = cnt;  // index lists: one entry per neighbour
+        if (valid && c == 0) {
+            if (a.counts) a.counts[qid] = cnt;
+            if (MODE == 1 && a.ecounts) a.ecounts[qid] = ecnt;
+            if (MODE == 1 && a.ecounts64) a.ecounts64[qid] = ecnt;
         }
     }
-    if (a.stats && lane == 0) {
-        atomicAdd(&a.stats[0], (unsigned long long)n_class);
-        atomicAdd(&a.stats[1], (unsigned long long)n_test);
-        atomicAdd(&a.stats[4], (unsigned long long)n_cslots);
-        atomicAdd(&a.stats[5], (unsigned long long)n_tslots);
-    }
-    if (a.stats && PREC == OCT_PREC_FP32_RECHECK) {
-        // n_recheck is per lane
-        uint64_t s = n_recheck;
-        for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
-        if (lane == 0 && s) atomicAdd(&a.stats[2], (unsigned long long)s);
-    }
     if (a.stats) {
-        uint64_t s = valid ? sink.cnt : 0;
-        for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
-        if (lane == 0) atomicAdd(&a.stats[3], (unsigned long long)s);
+        uint64_t nb = (valid && c == 0) ? cnt : 0, nc = n_class, nr = n_recheck;
+        for (int o = 32; o > 0; o >>= 1) {
+            nc += __shfl_xor(nc, o), n_test += __shfl_xor(n_test, o);
+            nr += __shfl_xor(nr, o), nb += __shfl_xor(nb, o);
+        }
+        if (lane == 0) {
+            atomicAdd(&a.stats[0], (unsigned long long)nc);
+            atomicAdd(&a.stats[1], (unsigned long long)n_test);
+            if (nr) atomicAdd(&a.stats[2], (unsigned long long)nr);
+            atomicAdd(&a.stats[3], (unsigned long long)nb);
+            atomicAdd(&a.stats[4], 64ull * n_csteps);
+            atomicAdd(&a.stats[5], 128ull * n_tsteps);
+        }
     }
 }
 
@@ -872,35 +914,39 @@ static void launch_count(const SearchArgs &a, int G, hipStream_t s) {
 }
 
 template <int KERNEL, int ALGO, int PREC>
-static void launch_k(const SearchArgs &a, int mode, int G, unsigned nb, hipStream_t s) {
-    if (mode == 0 && G > 0)
+static void launch_k(const SearchArgs &a, int mode, int G, hipStream_t s) {
+    if (mode == 0 && G > 0) {
         launch_count<KERNEL, ALGO, PREC>(a, G, s);
-    else if (mode == 0)
-        k_radius<KERNEL, ALGO, PREC, 0><<<nb, kSearchBlock, 0, s>>>(a);
+        return;
+    }
+    const unsigned nb = (unsigned)(((size_t)a.nq + kGroupsPerWave * kWaves - 1) / (kGroupsPerWave * kWaves));
+    const size_t lds = (size_t)kWaves * a.levels * 64 * sizeof(uint32_t);
+    if (mode == 0)
+        k_group<KERNEL, ALGO, PREC, 0><<<nb, kSearchBlock, lds, s>>>(a);
     else if (mode == 1)
-        k_radius<KERNEL, ALGO, PREC, 1><<<nb, kSearchBlock, 0, s>>>(a);
+        k_group<KERNEL, ALGO, PREC, 1><<<nb, kSearchBlock, lds, s>>>(a);
     else
-        k_radius<KERNEL, ALGO, PREC, 2><<<nb, kSearchBlock, 0, s>>>(a);
+        k_group<KERNEL, ALGO, PREC, 2><<<nb, kSearchBlock, lds, s>>>(a);
 }
 
 template <int KERNEL, int ALGO>
-static void launch_p(const SearchArgs &a, int prec, int mode, int G, unsigned nb, hipStream_t s) {
+static void launch_p(const SearchArgs &a, int prec, int mode, int G, hipStream_t s) {
     if (prec == OCT_PREC_FP32_RECHECK)
-        launch_k<KERNEL, ALGO, OCT_PREC_FP32_RECHECK>(a, mode, G, nb, s);
+        launch_k<KERNEL, ALGO, OCT_PREC_FP32_RECHECK>(a, mode, G, s);
     else
-        launch_k<KERNEL, ALGO, OCT_PREC_FP64>(a, mode, G, nb, s);
+        launch_k<KERNEL, ALGO, OCT_PREC_FP64>(a, mode, G, s);
 }
 
 template <int KERNEL>
-static void launch_a(const SearchArgs &a, int algo, int prec, int mode, int G, unsigned nb, hipStream_t s) {
+static void launch_a(const SearchArgs &a, int algo, int prec, int mode, int G, hipStream_t s) {
     if (algo == OCT_ALGO_NEIGHBORS)
-        launch_p<KERNEL, OCT_ALGO_NEIGHBORS>(a, prec, mode, G, nb, s);
+        launch_p<KERNEL, OCT_ALGO_NEIGHBORS>(a, prec, mode, G, s);
     else if (algo == OCT_ALGO_PRUNE)
-        launch_p<KERNEL, OCT_ALGO_PRUNE>(a, prec, mode, G, nb, s);
+        launch_p<KERNEL, OCT_ALGO_PRUNE>(a, prec, mode, G, s);
     else if (algo == OCT_ALGO_STRUCT)
-        launch_p<KERNEL, OCT_ALGO_STRUCT>(a, prec, mode, G, nb, s);
+        launch_p<KERNEL, OCT_ALGO_STRUCT>(a, prec, mode, G, s);
     else
-        launch_p<KERNEL, OCT_ALGO_APPROX>(a, prec, mode, G, nb, s);
+        launch_p<KERNEL, OCT_ALGO_APPROX>(a, prec, mode, G, s);
 }
 
 hipError_t launch_radius(oct_ctx *ctx, const RadiusLaunch &L) {
@@ -936,17 +982,15 @@ hipError_t launch_radius(oct_ctx *ctx, const RadiusLaunch &L) {
     a.entries = L.entries;
     a.stats = L.stats;
     a.err = ctx->derr.p;
-    for (int l = 0; l < 22; l++)
-        for (int k = 0; k < 3; k++) a.rad[l][k] = ctx->level_radii[l][k];
-    const size_t tiles = (L.nq + 63) / 64;
-    const unsigned nb = (unsigned)((tiles + kWaves - 1) / kWaves);
+    // levels that hold internal nodes: every level but the deepest
+    a.levels = ctx->n_levels > 1 ? std::min<uint32_t>(ctx->n_levels - 1, (uint32_t)kGroupMaxLevels) : 1u;
     stage_begin(ctx, ST_SEARCH);
     const int G = L.group;
     switch (L.kernel) {
-    case OCT_KERNEL_SPHERE: launch_a<OCT_KERNEL_SPHERE>(a, L.algo, L.precision, L.mode, G, nb, ctx->stream); break;
-    case OCT_KERNEL_CIRCLE: launch_a<OCT_KERNEL_CIRCLE>(a, L.algo, L.precision, L.mode, G, nb, ctx->stream); break;
-    case OCT_KERNEL_CUBE: launch_a<OCT_KERNEL_CUBE>(a, L.algo, L.precision, L.mode, G, nb, ctx->stream); break;
-    default: launch_a<OCT_KERNEL_SQUARE>(a, L.algo, L.precision, L.mode, G, nb, ctx->stream); break;
+    case OCT_KERNEL_SPHERE: launch_a<OCT_KERNEL_SPHERE>(a, L.algo, L.precision, L.mode, G, ctx->stream); break;
+    case OCT_KERNEL_CIRCLE: launch_a<OCT_KERNEL_CIRCLE>(a, L.algo, L.precision, L.mode, G, ctx->stream); break;
+    case OCT_KERNEL_CUBE: launch_a<OCT_KERNEL_CUBE>(a, L.algo, L.precision, L.mode, G, ctx->stream); break;
+    default: launch_a<OCT_KERNEL_SQUARE>(a, L.algo, L.precision, L.mode, G, ctx->stream); break;
     }
     stage_end(ctx, ST_SEARCH);
     return hipGetLastError();

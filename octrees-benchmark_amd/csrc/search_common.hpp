@@ -50,7 +50,7 @@ struct SearchArgs {
     uint32_t *__restrict__ entries;
     unsigned long long *__restrict__ stats;
     uint32_t *__restrict__ err;  // device error word: kErrStack when a traversal stack was full
-    double rad[22][3];
+    uint32_t levels;  // group kernel: levels that hold internal nodes (its LDS holds one row per level)
 };
 
 struct Query {

@@ -694,7 +694,7 @@ hipError_t sort_partition(oct_ctx *ctx, uint32_t *counters, uint32_t *errflag, u
     hipError_t e;
     if ((e = ctx->msd.reserve(words)) != hipSuccess) return e;
     if ((e = ctx->lookback.reserve(2 * tiles * 256 + 1)) != hipSuccess) return e;
-    if ((e = ctx->p64.reserve(n)) != hipSuccess) return e;
+    if ((e = ctx->p64.reserve(n + kPointPad)) != hipSuccess) return e;
     if ((e = ctx->keys_p.reserve(n)) != hipSuccess) return e;
     if ((e = ctx->vals_p.reserve(n)) != hipSuccess) return e;
     uint32_t *M = ctx->msd.p;
@@ -935,7 +935,7 @@ hipError_t launch_gather_raw(hipStream_t s, const double *xyz, const uint32_t *p
 
 hipError_t launch_gather(oct_ctx *ctx) {
     hipError_t e;
-    if ((e = ctx->p64.reserve(ctx->n)) != hipSuccess) return e;
+    if ((e = ctx->p64.reserve(ctx->n + kPointPad)) != hipSuccess) return e;
     stage_begin(ctx, ST_GATHER);
     if (ctx->n && !ctx->p64_sorted) {  // the partition sort writes the sorted cloud itself
         const unsigned nb = (unsigned)((ctx->n + 255) / 256);  // one point per thread (launch_gather_raw)

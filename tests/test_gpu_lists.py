@@ -1,0 +1,63 @@
+"""Result lists and group-kernel counts against the oracle where the kernels change shape: query counts around
+a wave's 8 and 64 queries, leaves around the 16-point steps and 64-point chunks of the point tests, empty and
+single-leaf trees, radii from nothing to the whole cloud. Every comparison is exact (lists entry for entry, in
+the reference's emission order)."""
+import numpy as np
+import pytest
+
+import octree_amd as A
+import pyoracle as O
+
+pytestmark = pytest.mark.gpu
+
+KERNELS = [A.K_SPHERE, A.K_CIRCLE, A.K_CUBE, A.K_SQUARE]
+ALGOS = [A.A_NEIGHBORS, A.A_PRUNE, A.A_STRUCT]
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = A.Octree(0)
+    yield c
+    c.close()
+
+
+def clouds():
+    rng = np.random.default_rng(11)
+    flat = rng.uniform(0, 10, (3000, 3)) * [1.0, 1.0, 0.02]
+    clump = np.concatenate([rng.normal(0, 0.01, (400, 3)) + [3, 3, 3], rng.uniform(0, 8, (600, 3))])
+    return {
+        "one": np.array([[1.0, 2.0, 3.0]]),
+        "root_leaf_17": rng.uniform(0, 1, (17, 3)),
+        "root_leaf_130": rng.uniform(0, 1, (130, 3)),
+        "flat": flat,
+        "clump": clump,  # leaves of every size, many empty children, deep levels
+    }
+
+
+@pytest.mark.parametrize("name,leaf", [("one", 4), ("root_leaf_17", 17), ("root_leaf_130", 130), ("flat", 1), ("flat", 15),
+                                       ("flat", 33), ("flat", 129), ("clump", 3), ("clump", 16), ("clump", 65)])
+def test_lists_equal_the_oracle(ctx, name, leaf):
+    xyz = clouds()[name]
+    ctx.set_points(xyz)
+    c, r, perm, keys = ctx.sort_points(A.ENC_HILBERT)
+    ctx.build(leaf)
+    sx, okeys, operm, oc, orad = O.sort_points(O.ENC_HILBERT, xyz)
+    tree = O.Tree(okeys, leaf, O.ENC_HILBERT, oc, orad)
+    n = len(sx)
+    rng = np.random.default_rng(5)
+    for nq in (1, 9, 65, 200):
+        nq = min(nq, n)
+        idx = np.sort(rng.choice(n, nq, replace=False)).astype(np.uint32)
+        for radius in (0.0, 0.6, 50.0):
+            for kernel in KERNELS:
+                for algo in ALGOS:
+                    ref, sizes = O.radius(tree, sx, kernel, algo, sx[idx.astype(np.int64)], radius)
+                    for prec in (A.PREC_FP64, A.PREC_FP32):
+                        tag = (name, leaf, nq, radius, kernel, algo, prec)
+                        counts, lists, _ = ctx.radius(kernel, algo, prec, idx=idx, radius=radius, lists=True)
+                        assert np.array_equal(counts, sizes), tag
+                        assert all(np.array_equal(x, y) for x, y in zip(lists, ref)), tag
+                        ctx.set_group(0)  # counts by the same traversal
+                        counts, _ = ctx.radius(kernel, algo, prec, idx=idx, radius=radius)
+                        ctx.set_group(-1)
+                        assert np.array_equal(counts, sizes), tag
