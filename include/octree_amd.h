@@ -222,14 +222,15 @@ int oct_knn_checksum(oct_ctx *ctx, const int32_t *idx_dev, const float *d2_dev, 
 /* ---- tuning (no counterpart in the reference: its per-query loop has no tile shape to choose).
  * OCT_TUNE_RADIUS_GROUP: queries per wave of the count-mode radius kernel (16, 32 or 64 queries
  * share one wave's traversal, 64 / G lanes serve each query), or 0 for the kernel in which 8 lanes
- * walk each query's own traversal; -1 restores "autotuned, else 32". OCT_TUNE_RADIUS_MFMA: the point tests run on the vector
+ * walk each query's own traversal; -1 restores the library's choice (0 for few or scattered
+ * queries, else the autotuned number, else 64). OCT_TUNE_RADIUS_MFMA: the point tests run on the vector
  * ALUs (a matrix-core form measured slower on every workload and is not built): 0 and -1 are
  * accepted, 1 fails with OCT_ERR_UNSUPPORTED.
  * oct_autotune_radius: times each candidate (G = 0, 16, 32, 64) on sample_nq queries taken from the
  * sorted cloud (16 equal strided chunks of consecutive SFC points; sample_nq >= n uses every point),
  * stores the fastest for (kernel, algo, precision), returns its G in *best and the milliseconds per G
  * in ms_out[0..3].
- * oct_tuned_radius: the G a count-mode search would use now (*mfma, if given, is always 0).
+ * oct_tuned_radius: the G a count-mode search of many consecutive points would use now (*mfma, if given, is always 0).
  * OCT_TUNE_RADIUS_REMAP: 1 (default, also -1) lets the count-mode vector point tests move the
  * queries of a leaf that at most half of a wave's queries want onto all 64 lanes; 0 keeps every
  * query on its own lanes.

@@ -44,12 +44,13 @@ int hfail(oct_ctx *ctx, hipError_t e, const char *where, const std::string &extr
 
 bool valid_encoder(int e) { return e == OCT_ENC_MORTON3D || e == OCT_ENC_HILBERT3D; }
 
-// Reads the device error word after the stream's work so far (synchronises); a set bit fails the
-// call with OCT_ERR_STATE and the word is cleared for the next call.
+// Waits for the stream's work so far and reads the device error word; a set bit fails the call with
+// OCT_ERR_STATE and the word is cleared for the next call. Small results come back through the context's
+// pinned page (ctx->mail), so their copies queue up behind the kernels and one wait serves them all.
 int check_device_error(oct_ctx *ctx) {
-    uint32_t w = 0;
-    HCHK(hipMemcpyAsync(&w, ctx->derr.p, 4, hipMemcpyDeviceToHost, ctx->stream), "copy error word");
-    HCHK(hipStreamSynchronize(ctx->stream), "copy error word");
+    HCHK(hipMemcpyAsync(&ctx->mail->err, ctx->derr.p, 4, hipMemcpyDeviceToHost, ctx->stream), "copy error word");
+    HCHK(hipStreamSynchronize(ctx->stream), "wait for the stream");
+    const uint32_t w = ctx->mail->err;
     if (!w) return OCT_OK;
     HCHK(hipMemsetAsync(ctx->derr.p, 0, 4, ctx->stream), "clear error word");
     HCHK(hipStreamSynchronize(ctx->stream), "clear error word");
@@ -278,14 +279,19 @@ double stage_ms(const oct_ctx *ctx, Stage s) {
     return (double)ms;
 }
 
-// Slot order that visits queries in SFC order (coherent waves): indices into the sorted cloud are
-// already SFC positions; explicit centres are keyed with the cloud's encoder and box.
+// Slot order that visits queries in SFC order (waves of queries that share a traversal); empty: the
+// given order is already that. Indices into the sorted cloud are SFC positions; explicit centres are
+// keyed with the cloud's encoder and box.
 void query_order(oct_ctx *ctx, const double *centers, const uint32_t *idx, size_t nq, std::vector<uint32_t> &order) {
-    order.resize(nq);
-    std::iota(order.begin(), order.end(), 0u);
+    order.clear();
     if (idx) {
+        if (std::is_sorted(idx, idx + nq)) return;
+        order.resize(nq);
+        std::iota(order.begin(), order.end(), 0u);
         std::stable_sort(order.begin(), order.end(), [&](uint32_t a, uint32_t b) { return idx[a] < idx[b]; });
     } else if (centers) {
+        order.resize(nq);
+        std::iota(order.begin(), order.end(), 0u);
         std::vector<uint64_t> k(nq);
         for (size_t i = 0; i < nq; i++) {
             uint32_t x = quantize_axis(centers[3 * i], ctx->center[0], ctx->radii[0]);
@@ -295,6 +301,17 @@ void query_order(oct_ctx *ctx, const double *centers, const uint32_t *idx, size_
         }
         std::stable_sort(order.begin(), order.end(), [&](uint32_t a, uint32_t b) { return k[a] < k[b]; });
     }
+}
+
+// Queries per point of the sorted cloud where the queries lie: nq over the span of the indices, else over
+// the whole cloud.
+double query_density(const oct_ctx *ctx, const double *centers, const uint32_t *idx, size_t nq) {
+    if (!nq) return 1.0;
+    if (idx) {
+        const auto mm = std::minmax_element(idx, idx + nq);
+        return (double)nq / ((double)*mm.second - (double)*mm.first + 1.0);
+    }
+    return centers ? (double)nq / (double)(ctx->n ? ctx->n : 1) : 1.0;
 }
 
 }  // namespace
@@ -363,8 +380,13 @@ int oct_create(oct_ctx **out, int device) {
         delete ctx;
         return OCT_ERR_HIP;
     }
+    if (hipHostMalloc((void **)&ctx->mail, sizeof(*ctx->mail), hipHostMallocDefault) != hipSuccess) {
+        delete ctx;
+        return OCT_ERR_HIP;
+    }
     if (ctx->derr.reserve(4) != hipSuccess || hipMemset(ctx->derr.p, 0, 4 * sizeof(uint32_t)) != hipSuccess) {
         ctx->derr.release();
+        (void)hipHostFree(ctx->mail);
         delete ctx;
         return OCT_ERR_HIP;
     }
@@ -392,6 +414,7 @@ int oct_destroy(oct_ctx *ctx) {
         if (ctx->ev0[s]) (void)hipEventDestroy(ctx->ev0[s]);
         if (ctx->ev1[s]) (void)hipEventDestroy(ctx->ev1[s]);
     }
+    (void)hipHostFree(ctx->mail);
     (void)hipStreamDestroy(ctx->stream);
     delete ctx;
     return OCT_OK;
@@ -617,17 +640,28 @@ static int check_search_args(oct_ctx *ctx, int kernel, int algo, int precision, 
     return OCT_OK;
 }
 
-// Queries per wave for the count-mode kernel: explicit override, else autotuned, else 32.
-static int radius_group(const oct_ctx *ctx, int kernel, int algo, int precision) {
+// Queries per wave for a count-mode search of nq queries, about one every 1 / density points of the sorted
+// cloud: an explicit override; 0 (the group kernel, 8 lanes per query) for few or scattered queries; else
+// the autotuned number, else 64. A wave of 64 queries shares the judgements and staged points of one
+// traversal, but 2^17 queries are only two such waves per SIMD, and far-apart queries share little.
+// Sphere counts, ns per query, group kernel / 64 per wave: 5 M tile, every point of a run, r = 1: 131 k
+// queries 0.96 / 1.61, 2 M 0.90 / 0.35; one point in 64, r = 2.5: 78 k queries 4.1 / 15; 40 M tile, one in 8:
+// 524 k 3.8 / 3.2; one in 32: 524 k 4.8 / 4.8; 40 M box, one in 8: 2.8 / 2.6, one in 32: 3.2 / 4.7.
+constexpr size_t kUnionMinQueries = 1u << 17;
+constexpr double kUnionMinDensity = 1.0 / 16;
+static int radius_group(const oct_ctx *ctx, int kernel, int algo, int precision, size_t nq, double density) {
     if (ctx->group_override >= 0) return ctx->group_override;
-    int t = ctx->group_tuned[kernel & 3][algo & 3][precision & 1];
-    return t >= 0 ? t : 32;
+    if (nq <= kUnionMinQueries || density < kUnionMinDensity) return 0;
+    const int t = ctx->group_tuned[kernel & 3][algo & 3][precision & 1];
+    return t >= 0 ? t : 64;
 }
 
-static int read_stats(oct_ctx *ctx, oct_search_stats *stats, double ms) {
-    unsigned long long h[6];
-    HCHK(hipMemcpyAsync(h, ctx->stats.p, sizeof(h), hipMemcpyDeviceToHost, ctx->stream), "copy stats");
-    HCHK(hipStreamSynchronize(ctx->stream), "stats");
+// enqueues the copy of the search counters (ctx->mail; valid after the next wait) / hands them out
+static hipError_t copy_stats(oct_ctx *ctx) {
+    return hipMemcpyAsync(ctx->mail->stats, ctx->stats.p, sizeof(ctx->mail->stats), hipMemcpyDeviceToHost, ctx->stream);
+}
+static void put_stats(const oct_ctx *ctx, oct_search_stats *stats, double ms) {
+    const unsigned long long *h = ctx->mail->stats;
     stats->nodes_classified = h[0];
     stats->points_tested = h[1];
     stats->rechecked = h[2];
@@ -635,7 +669,6 @@ static int read_stats(oct_ctx *ctx, oct_search_stats *stats, double ms) {
     stats->kernel_ms = ms;
     stats->class_slots = h[4];
     stats->test_slots = h[5];
-    return OCT_OK;
 }
 
 static int radius_impl(oct_ctx *ctx, int kernel, int algo, int precision, const double *centers,
@@ -650,11 +683,13 @@ static int radius_impl(oct_ctx *ctx, int kernel, int algo, int precision, const 
         for (size_t i = 0; i < nq; i++)
             if (center_idx[i] >= ctx->n) return fail(ctx, OCT_ERR_ARG, "center index out of range");
     HCHK(hipSetDevice(ctx->device), "set device");
+    const int group = want_lists ? 0 : radius_group(ctx, kernel, algo, precision, nq, query_density(ctx, centers, center_idx, nq));
+    // the group kernel takes queries in any order: sorting them costs the host more than their locality gives
     std::vector<uint32_t> order;
-    query_order(ctx, centers, center_idx, nq, order);
+    if (group) query_order(ctx, centers, center_idx, nq, order);
     HCHK(ctx->qidx.reserve(2 * nq + 1), "alloc queries");
     uint32_t *d_order = ctx->qidx.p, *d_idx = ctx->qidx.p + nq;
-    if (nq) HCHK(hipMemcpyAsync(d_order, order.data(), nq * 4, hipMemcpyHostToDevice, ctx->stream), "copy order");
+    if (!order.empty()) HCHK(hipMemcpyAsync(d_order, order.data(), nq * 4, hipMemcpyHostToDevice, ctx->stream), "copy order");
     if (center_idx && nq) HCHK(hipMemcpyAsync(d_idx, center_idx, nq * 4, hipMemcpyHostToDevice, ctx->stream), "copy idx");
     if (centers) {
         HCHK(ctx->qxyz.reserve(3 * nq + 1), "alloc centres");
@@ -669,14 +704,16 @@ static int radius_impl(oct_ctx *ctx, int kernel, int algo, int precision, const 
         if (nq) HCHK(hipMemcpyAsync(ctx->qrad3.p, radii3, nq * 24, hipMemcpyHostToDevice, ctx->stream), "copy radii");
     }
     HCHK(ctx->counts.reserve(2 * nq + 1), "alloc counts");
-    HCHK(ctx->stats.reserve(8), "alloc stats");
-    HCHK(hipMemsetAsync(ctx->stats.p, 0, 8 * sizeof(unsigned long long), ctx->stream), "clear stats");
+    if (stats) {
+        HCHK(ctx->stats.reserve(8), "alloc stats");
+        HCHK(hipMemsetAsync(ctx->stats.p, 0, 8 * sizeof(unsigned long long), ctx->stream), "clear stats");
+    }
     RadiusLaunch L;
     L.kernel = kernel, L.algo = algo, L.precision = precision, L.mode = want_lists ? 1 : 0;
-    L.group = radius_group(ctx, kernel, algo, precision);
+    L.group = group;
     L.remap = ctx->remap_override != 0;
     L.approx_level = approx_level, L.approx_upper = approx_upper;
-    L.order = d_order;
+    L.order = order.empty() ? nullptr : d_order;
     L.qidx = center_idx ? d_idx : nullptr;
     L.qxyz = centers ? ctx->qxyz.p : nullptr;
     L.qrad = radii ? ctx->qrad.p : nullptr;
@@ -690,35 +727,32 @@ static int radius_impl(oct_ctx *ctx, int kernel, int algo, int precision, const 
     L.nq = nq;
     L.counts = ctx->counts.p;
     L.ecounts = ctx->counts.p + nq;
-    L.stats = ctx->stats.p;
+    L.stats = stats ? ctx->stats.p : nullptr;
     HCHK(launch_radius(ctx, L), "radius count");
-    double ms = 0.0;
-    HCHK(hipStreamSynchronize(ctx->stream), "radius count");
-    ms += stage_ms(ctx, ST_SEARCH);
+    if (counts_out && nq) HCHK(hipMemcpyAsync(counts_out, ctx->counts.p, nq * 4, hipMemcpyDeviceToHost, ctx->stream), "copy counts");
+    if (stats) HCHK(copy_stats(ctx), "copy stats");
     ctx->has_lists = false;
+    double ms = 0.0;
     if (want_lists) {
         HCHK(ctx->qoff.reserve(nq + 1), "alloc offsets");
         HCHK(exclusive_scan_u32_to_u64(ctx, ctx->counts.p + nq, ctx->qoff.p, nq), "scan");
-        uint64_t total = 0;
-        HCHK(hipMemcpyAsync(&total, ctx->qoff.p + nq, 8, hipMemcpyDeviceToHost, ctx->stream), "copy total");
-        HCHK(hipStreamSynchronize(ctx->stream), "scan");
-        const size_t words = (size_t)total * (algo == OCT_ALGO_STRUCT || algo == OCT_ALGO_APPROX ? 2 : 1);
+        HCHK(hipMemcpyAsync(&ctx->mail->total, ctx->qoff.p + nq, 8, hipMemcpyDeviceToHost, ctx->stream), "copy total");
+        if ((s = check_device_error(ctx))) return s;
+        ms += stage_ms(ctx, ST_SEARCH);
+        const size_t words = (size_t)ctx->mail->total * (algo == OCT_ALGO_STRUCT || algo == OCT_ALGO_APPROX ? 2 : 1);
         HCHK(ctx->entries.reserve(words + 1), "alloc lists");
         L.mode = 2;
         L.offsets = ctx->qoff.p;
         L.entries = ctx->entries.p;
         L.stats = nullptr;
         HCHK(launch_radius(ctx, L), "radius fill");
-        HCHK(hipStreamSynchronize(ctx->stream), "radius fill");
-        ms += stage_ms(ctx, ST_SEARCH);
-        ctx->has_lists = true;
     }
     ctx->last_nq = nq;
     ctx->last_algo = algo;
-    if (counts_out && nq) HCHK(hipMemcpyAsync(counts_out, ctx->counts.p, nq * 4, hipMemcpyDeviceToHost, ctx->stream), "copy counts");
-    HCHK(hipStreamSynchronize(ctx->stream), "radius");
     if ((s = check_device_error(ctx))) return s;
-    if (stats) return read_stats(ctx, stats, ms);
+    ctx->has_lists = want_lists != 0;
+    ms += stage_ms(ctx, ST_SEARCH);
+    if (stats) put_stats(ctx, stats, ms);
     return OCT_OK;
 }
 
@@ -765,10 +799,9 @@ int oct_radius_lists_noalloc(oct_ctx *ctx, int kernel, int algo, int precision, 
         k_na_zero<<<1, 1, 0, ctx->stream>>>(offsets_dev);
     }
     HCHK(hipGetLastError(), "offsets");
-    uint64_t total = 0;
-    HCHK(hipMemcpyAsync(&total, offsets_dev + nq, 8, hipMemcpyDeviceToHost, ctx->stream), "copy total");
-    HCHK(hipStreamSynchronize(ctx->stream), "radius sizes");
+    HCHK(hipMemcpyAsync(&ctx->mail->total, offsets_dev + nq, 8, hipMemcpyDeviceToHost, ctx->stream), "copy total");
     if ((s = check_device_error(ctx))) return s;
+    const uint64_t total = ctx->mail->total;
     *total_out = total;
     const size_t words = (size_t)total * (algo == OCT_ALGO_STRUCT ? 2 : 1);
     if (words > entries_capacity)
@@ -782,7 +815,6 @@ int oct_radius_lists_noalloc(oct_ctx *ctx, int kernel, int algo, int precision, 
     L.offsets = offsets_dev;
     L.entries = entries_dev;
     if (words) HCHK(launch_radius(ctx, L), "radius fill");
-    HCHK(hipStreamSynchronize(ctx->stream), "radius fill");
     ctx->has_lists = false;
     return check_device_error(ctx);
 }
@@ -867,7 +899,7 @@ int oct_radius_dev(oct_ctx *ctx, int kernel, int algo, int precision, const uint
     }
     RadiusLaunch L;
     L.kernel = kernel, L.algo = algo, L.precision = precision, L.mode = 0;
-    L.group = radius_group(ctx, kernel, algo, precision);
+    L.group = radius_group(ctx, kernel, algo, precision, nq, 1.0);  // the indices' spread is not known here
     L.remap = ctx->remap_override != 0;
     L.qidx = center_idx_dev;
     L.radius = radius;
@@ -881,9 +913,9 @@ int oct_radius_dev(oct_ctx *ctx, int kernel, int algo, int precision, const uint
     HCHK(launch_radius(ctx, L), "radius");
     ctx->has_lists = false;
     if (stats) {
-        HCHK(hipStreamSynchronize(ctx->stream), "radius");
+        HCHK(copy_stats(ctx), "copy stats");
         if ((s = check_device_error(ctx))) return s;
-        return read_stats(ctx, stats, stage_ms(ctx, ST_SEARCH));
+        put_stats(ctx, stats, stage_ms(ctx, ST_SEARCH));
     }
     return OCT_OK;
 }
@@ -918,6 +950,8 @@ int oct_set_tuning(oct_ctx *ctx, int knob, int value) {
     ctx->group_override = value;
     return OCT_OK;
 }
+
+constexpr double kResidentWaves = 256.0 * 4 * 7;  // of the count kernel: 7 per SIMD
 
 int oct_autotune_radius(oct_ctx *ctx, int kernel, int algo, int precision, double radius, size_t sample_nq, int *best,
                         double ms_out[4]) {
@@ -956,6 +990,13 @@ int oct_autotune_radius(oct_ctx *ctx, int kernel, int algo, int precision, doubl
             if (rep) t = std::min(t, stage_ms(ctx, ST_SEARCH));
         }
         if (ms_out) ms_out[ci] = t;
+        // half a round of resident waves idles at the end of a launch, which weighs more in a short sample
+        // than in the search it stands for (2^20 queries of the 50 M tile: 32 per wave 1.70 ms, 64 per wave
+        // 1.78; all 50 M: 57 and 39.8 ms)
+        if (cand[ci] && nq < ctx->n) {
+            const double rounds = (double)nq / cand[ci] / kResidentWaves;
+            t *= rounds / (rounds + 0.5);
+        }
         if (t < bestms) bestms = t, bestg = cand[ci];
     }
     ctx->group_tuned[kernel & 3][algo & 3][precision & 1] = bestg;
@@ -968,7 +1009,7 @@ int oct_tuned_radius(oct_ctx *ctx, int kernel, int algo, int precision, int *gro
     if (!ctx) return OCT_ERR_ARG;
     if (kernel < 0 || kernel > 3 || algo < 1 || algo > 3 || (precision != 0 && precision != 1))
         return fail(ctx, OCT_ERR_ARG, "unknown kernel, algorithm or precision");
-    if (group) *group = radius_group(ctx, kernel, algo, precision);
+    if (group) *group = radius_group(ctx, kernel, algo, precision, std::max(ctx->n, kUnionMinQueries + 1), 1.0);
     if (mfma) *mfma = 0;  // point tests on the vector ALUs
     return OCT_OK;
 }
@@ -1001,7 +1042,7 @@ int oct_knn(oct_ctx *ctx, int precision, const double *centers, const uint32_t *
     query_order(ctx, centers, center_idx, nq, order);
     HCHK(ctx->qidx.reserve(2 * nq + 1), "alloc queries");
     uint32_t *d_order = ctx->qidx.p, *d_idx = ctx->qidx.p + nq;
-    if (nq) HCHK(hipMemcpyAsync(d_order, order.data(), nq * 4, hipMemcpyHostToDevice, ctx->stream), "copy order");
+    if (!order.empty()) HCHK(hipMemcpyAsync(d_order, order.data(), nq * 4, hipMemcpyHostToDevice, ctx->stream), "copy order");
     if (center_idx && nq) HCHK(hipMemcpyAsync(d_idx, center_idx, nq * 4, hipMemcpyHostToDevice, ctx->stream), "copy idx");
     if (centers) {
         HCHK(ctx->qxyz.reserve(3 * nq + 1), "alloc centres");
@@ -1009,25 +1050,27 @@ int oct_knn(oct_ctx *ctx, int precision, const double *centers, const uint32_t *
     }
     HCHK(ctx->kidx.reserve((size_t)nq * k + 1), "alloc knn");
     HCHK(ctx->kd2.reserve((size_t)nq * k + 1), "alloc knn");
-    HCHK(ctx->stats.reserve(8), "alloc stats");
-    HCHK(hipMemsetAsync(ctx->stats.p, 0, 8 * sizeof(unsigned long long), ctx->stream), "clear stats");
+    if (stats) {
+        HCHK(ctx->stats.reserve(8), "alloc stats");
+        HCHK(hipMemsetAsync(ctx->stats.p, 0, 8 * sizeof(unsigned long long), ctx->stream), "clear stats");
+    }
     KnnLaunch L;
     L.precision = precision;
-    L.order = d_order;
+    L.order = order.empty() ? nullptr : d_order;
     L.qidx = center_idx ? d_idx : nullptr;
     L.qxyz = centers ? ctx->qxyz.p : nullptr;
     L.nq = nq, L.k = k;
     L.idx = ctx->kidx.p, L.d2 = ctx->kd2.p;
-    L.stats = ctx->stats.p;
+    L.stats = stats ? ctx->stats.p : nullptr;
     L.lanes = knn_lanes(ctx, precision, k);
     std::string err;
     hipError_t e = launch_knn(ctx, L, err);
     if (e != hipSuccess) return err.empty() ? hfail(ctx, e, "knn") : fail(ctx, OCT_ERR_ARG, err);
     if (idx_out && nq) HCHK(hipMemcpyAsync(idx_out, ctx->kidx.p, nq * k * 4, hipMemcpyDeviceToHost, ctx->stream), "copy idx");
     if (d2_out && nq) HCHK(hipMemcpyAsync(d2_out, ctx->kd2.p, nq * k * 8, hipMemcpyDeviceToHost, ctx->stream), "copy d2");
-    HCHK(hipStreamSynchronize(ctx->stream), "knn");
+    if (stats) HCHK(copy_stats(ctx), "copy stats");
     if (int de = check_device_error(ctx)) return de;
-    if (stats) return read_stats(ctx, stats, stage_ms(ctx, ST_KNN));
+    if (stats) put_stats(ctx, stats, stage_ms(ctx, ST_KNN));
     return OCT_OK;
 }
 
@@ -1065,9 +1108,9 @@ int oct_knn_dev(oct_ctx *ctx, int precision, const uint32_t *center_idx_dev, siz
     if (e != hipSuccess) return err.empty() ? hfail(ctx, e, "knn") : fail(ctx, OCT_ERR_ARG, err);
     if (keep) ctx->knn_nq = nq, ctx->knn_k = k;
     if (stats) {
-        HCHK(hipStreamSynchronize(ctx->stream), "knn");
+        HCHK(copy_stats(ctx), "copy stats");
         if (int de = check_device_error(ctx)) return de;
-        return read_stats(ctx, stats, stage_ms(ctx, ST_KNN));
+        put_stats(ctx, stats, stage_ms(ctx, ST_KNN));
     }
     return OCT_OK;
 }
@@ -1079,7 +1122,6 @@ int oct_knn_fetch(oct_ctx *ctx, size_t q0, size_t nq, int32_t *idx_out, float *d
     const size_t k = ctx->knn_k, off = q0 * k, cnt = nq * k;
     if (idx_out && cnt) HCHK(hipMemcpyAsync(idx_out, ctx->kidx.p + off, cnt * 4, hipMemcpyDeviceToHost, ctx->stream), "copy idx");
     if (d2_out && cnt) HCHK(hipMemcpyAsync(d2_out, ctx->kd2f.p + off, cnt * 4, hipMemcpyDeviceToHost, ctx->stream), "copy d2");
-    HCHK(hipStreamSynchronize(ctx->stream), "knn fetch");
     return check_device_error(ctx);
 }
 

@@ -172,6 +172,12 @@ struct oct_ctx {
     int knn_lanes_override = -1;    // OCT_TUNE_KNN_LANES (-1: tuned / default)
     int knn_lanes_tuned[2][8];      // autotuned lanes per query per (precision, size class), -1 = not tuned
 
+    // small results on their way to the host: a pinned page, written by copies on the stream
+    struct Mail {
+        unsigned long long stats[8];
+        uint64_t total;
+        uint32_t err;
+    } *mail = nullptr;
     oct::DevBuf<uint32_t> derr;     // device error word (kErr* bits), zero when no kernel failed
 
     hipEvent_t ev0[oct::ST_N] = {}, ev1[oct::ST_N] = {};
