@@ -210,6 +210,24 @@ __device__ inline uint32_t lane_xor(uint32_t v) {
 __device__ inline uint32_t lane_xor32(uint32_t v) {
     return (uint32_t)__builtin_amdgcn_ds_bpermute((int)((lane_id() ^ 32u) << 2), (int)v);
 }
+// Reduction over aligned groups of S lanes (a power of two, 8 to 64), every lane of the wave active: the
+// result in every lane of its group. Within 16 lanes by DPP (quad swaps, then the half rows and rows
+// mirrored, which pairs each lane with one of the other half).
+template <int CTRL>
+__device__ inline uint32_t dpp_u32(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, CTRL, 0xf, 0xf, true);
+}
+template <int S, class Op>
+__device__ inline uint32_t group_reduce(uint32_t v, Op op) {
+    static_assert(S == 8 || S == 16 || S == 32 || S == 64, "8 to 64 lanes");
+    v = op(v, dpp_u32<0xB1>(v));   // quad_perm 1,0,3,2
+    v = op(v, dpp_u32<0x4E>(v));   // quad_perm 2,3,0,1
+    v = op(v, dpp_u32<0x141>(v));  // row_half_mirror
+    if (S >= 16) v = op(v, dpp_u32<0x140>(v));  // row_mirror
+    if (S >= 32) v = op(v, lane_xor<16>(v));
+    if (S >= 64) v = op(v, lane_xor32(v));
+    return v;
+}
 __device__ inline uint32_t uniform_u32(uint32_t v) { return __builtin_amdgcn_readfirstlane(v); }
 __device__ inline uint32_t readlane_u32(uint32_t v, int lane) { return __builtin_amdgcn_readlane(v, lane); }
 __device__ inline double readlane_f64(double v, int lane) {

@@ -38,8 +38,8 @@ struct alignas(64) NodeExt {
 static_assert(sizeof(NodeExt) == 192, "NodeExt is three 64-byte lines");
 
 // Points allocated past the end of the sorted clouds (p64, p32): the group kernels read a leaf's points
-// in steps of 16 and ignore what lies past it.
-constexpr size_t kPointPad = 16;
+// in steps of up to 64 and ignore what lies past it.
+constexpr size_t kPointPad = 64;
 
 // Device buffer that only grows.
 template <class T>
@@ -267,6 +267,8 @@ struct KnnLaunch {
 hipError_t launch_knn(oct_ctx *ctx, const KnnLaunch &L, std::string &err);
 // lanes-per-query shapes offered for k (default first); returns how many
 int knn_lane_options(uint32_t k, int out[3]);
+// the shape that runs a requested number of lanes per query for k, 0: refused
+int knn_shape_lanes(uint32_t k, int lanes);
 // Batches: stable sort of every cloud's (key, value) range at once (8 passes; keys0 / vals0 in and
 // out, the values of the first pass are the global positions); lookback (8 x ntiles x 256) and
 // counters (8) must be zero.

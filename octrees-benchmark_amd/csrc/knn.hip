@@ -5,29 +5,22 @@
 // dx*dx + dy*dy + dz*dz, no contraction), ordered by (distance, sorted index). The reference's
 // heap returns the same distances; only the order inside a tie class is unspecified there.
 //
-// One wave serves G = 64 / S queries that are consecutive in SFC order (S lanes per query) and
-// walks the tree once for all of them, depth first, children pushed so that the octant of the
-// wave's middle query comes off the stack first. A child is skipped for a query when a lower
-// bound of its box distance exceeds the query's current k-th distance; the bound widens every box
-// by 2^-40 of the cloud's magnitude, which covers the FP64 rounding of node centres and of points
-// on cell faces, and compares with a relative margin, so pruning never drops a true neighbour.
-// Leaf points are staged in LDS once per wave. Each query keeps an LDS buffer of 2 KC entries that
-// starts with its best entries so far, sorted, and appends every point that beats its current k-th
-// entry. When a buffer could overflow, the wave selects (S lanes per query) and keeps each query's
-// k best, which sets the new k-th distance. By merge: the sorted entries own the first KC slots and
-// points are appended to the second KC; a selection sorts the second half descending (bitonic) and
-// merges it with the first (one bitonic merge of 2 KC). By full sort: points are appended right
-// after the kept entries and a selection sorts the whole buffer, as many network stages as a merge
-// for KC = 16 but less often when every k of the wave is below KC. Merge serves every KC >= 32 and
-// the KC = 16 waves whose largest k is 16 (4 M queries, 8 lanes each, by full sorts vs by merge:
-// k = 13 17.7 vs 20.1 ms, k = 14 19.1 vs 20.7, k = 15 20.9 vs 21.2, k = 16 24.0 vs 21.8; one stage per
-// round trip, k = 32: 31.3 vs 23.5). The networks run two stages per LDS round
-// trip (k = 10: 16.4 -> 15.4 ms FP32; k = 250, 64 lanes: 28.8 -> 24.8 ms for 0.5 M queries), three
-// for KC >= 512, where LDS already bounds the occupancy (k = 1000: 37.6 -> 35.0 ms for 0.1 M queries;
-// for smaller KC three stages cost a wave per SIMD and run slower).
-// FP32_RECHECK filters the points with the leaf-recentred FP32 form
-// e = w - 2 a.b + |b|^2 (the count kernel's representation), whose error is below
-// hw / 2 = 2^-19 (amax + |b|^2); only points with e <= k-th + hw get their exact FP64 distance.
+// A group of S lanes serves one query (64 / S queries per wave), each with its own traversal:
+//  - a node's 8 children are judged one per lane; a child waits with a lower bound of its box distance,
+//    rounded down to 16 bits. The nearest waiting child of the deepest level comes next (a min over the
+//    group's lanes), and a level whose nearest child is beyond the current k-th distance is dropped. The
+//    bound widens every box by 2^-40 of the cloud's magnitude, which covers the FP64 rounding of node
+//    centres and of points on cell faces, so pruning never drops a true neighbour;
+//  - groups go down independently until each holds a leaf; then all test their leaves' points, S (or 2 S)
+//    at a time, and append those not beyond the current bound to the query's buffer in LDS;
+//  - a selection finds, by counting, a bound T on the distance's upper 32 bits with k to kw entries at or
+//    below it (a few interpolated guesses: the count grows about linearly with the squared distance),
+//    keeps those and drops the rest; T bounds the k-th distance from above. No entry is sorted until the
+//    end, when the k best of the remaining few are ordered exactly. More than kw entries can share T's
+//    upper bits (ties): where they would fill the buffer, an exact selection keeps the k best.
+// FP32_RECHECK filters the points with the leaf-recentred FP32 form e = w - 2 a.b + |b|^2 (the count
+// kernel's representation), whose error is below hw / 2 = 2^-19 (amax + |b|^2); only points with
+// e <= bound + hw get their exact FP64 distance.
 #include <cfloat>
 
 #include "device.hpp"
@@ -35,18 +28,11 @@
 
 namespace oct {
 
-constexpr int kKnnStack = 8 * 22 + 8;  // depth first: at most 7 entries per level + 8 live
-constexpr int kKnnChunk = 128;         // leaf points staged per round
-constexpr int kKnnMergeMinKC = 32;     // buffer size classes that always select by sort-and-merge
-constexpr uint32_t kKnnMergeMinK = 16; // smaller classes: by merge when the wave's largest k reaches this
-constexpr int kKnnTripleMinKC = 512;   // buffer size classes whose networks run 3 stages per LDS round trip
-
 struct KnnArgs {
     const double4 *__restrict__ p64;
     const float4 *__restrict__ p32;
     const float *__restrict__ amax;
     const NodeRec *__restrict__ nodes;
-    const NodeExt *__restrict__ next;
     const uint32_t *__restrict__ child;
     const uint32_t *__restrict__ order;
     const uint32_t *__restrict__ qidx;
@@ -70,9 +56,12 @@ struct KnnArgs {
     // work-queue form: device-resident wave-tile count and the zeroed counter waves take tiles from
     const uint32_t *__restrict__ queue_tiles;
     uint32_t *__restrict__ queue_next;
+    uint32_t levels;  // rows of waiting children in LDS: the tree's levels
 };
 
-__device__ inline bool knn_less(double da, uint32_t ia, double db, uint32_t ib) { return da < db || (da == db && ia < ib); }
+// Order of the results: squared distances are sums of squares (never -0), so their bit patterns order as
+// the values do (a NaN after every number); ties by index.
+__device__ inline bool knn_less(uint64_t da, uint32_t ia, uint64_t db, uint32_t ib) { return da < db || (da == db && ia < ib); }
 
 // Lower bound of the squared distance from q to any point of the box c +- r, each axis widened by
 // dl; the caller compares it against tau (1 + 2^-40), which covers the rounding of this sum.
@@ -81,26 +70,35 @@ __device__ inline double gap2(double q, double c, double r, double dl) {
     return gap > 0.0 ? gap * gap : 0.0;
 }
 
+// Buffer entries per query for the size class KC (k <= KC): three times KC where KC is small, so that a
+// selection is seldom needed, else twice.
+constexpr int knn_cap(int kc) { return kc <= 32 ? 3 * kc : 2 * kc; }
+constexpr uint32_t kKnnLeafBit = 0x80000000u;
+
+// LDS of one wave: per level and group lane, the waiting child's bound (upper half of its float) and its
+// first child, or its own index with kKnnLeafBit set for a leaf.
+struct KnnLevels {
+    uint32_t *node;
+    uint16_t *key;
+};
+
 // One wave tile (64 / S queries) of a kNN search, run by one wave (a 64-thread block).
 template <int S, int KC, int PREC>
-__device__ __attribute__((always_inline)) inline void knn_tile(const KnnArgs &a, const uint32_t tile) {
-    constexpr int G = 64 / S;                           // queries per wave
-    constexpr int CAP = 2 * KC;                         // buffer entries per query
-    constexpr int U = S >= 16 ? 1 : 16 / S;             // points per lane per step
-    constexpr int STEP = S * U;                         // points per query per step
+__device__ __attribute__((always_inline)) inline void knn_tile(const KnnArgs &a, const uint32_t tile, const KnnLevels lev) {
+    constexpr int G = 64 / S;                // queries per wave
+    constexpr int CAP = knn_cap(KC);         // buffer entries per query
+    constexpr int U = S <= 16 ? 2 : 1;       // points per lane per step
+    constexpr int STEP = S * U;              // points per query per step
+    constexpr int ROWS = (CAP + S - 1) / S;  // buffer entries per lane
     constexpr bool F32 = PREC == OCT_PREC_FP32_RECHECK;
-    constexpr int STG = kKnnChunk + STEP;               // staged slots incl. the last step's tail
-    static_assert(STEP <= KC, "a step must fit after a selection");
-    __shared__ double s_bd[G * CAP];
+    constexpr bool kRank = KC <= 32;         // final order by counting ranks, else by a bitonic sort in LDS
+    static_assert(CAP - STEP >= KC, "a step must fit after a selection");
+    __shared__ uint64_t s_bd[G * CAP];
     __shared__ uint32_t s_bi[G * CAP];
-    __shared__ uint32_t s_node[kKnnStack];
-    __shared__ uint8_t s_lev[kKnnStack];
-    __shared__ __attribute__((aligned(16))) unsigned char s_stage[STG * (F32 ? 16 : 32)];
-    float4 *s32 = reinterpret_cast<float4 *>(s_stage);
-    double4 *s64 = reinterpret_cast<double4 *>(s_stage);
+    __shared__ double s_rad[66];
 
     const uint32_t lane = threadIdx.x;
-    const uint32_t qs = lane / S, g = lane % S;
+    const uint32_t qs = lane / S, c = lane % S, gshift = lane & ~(uint32_t)(S - 1);
     const uint32_t slot0 = tile * G;
     const uint32_t slot = slot0 + qs;
     uint32_t cloud = 0, nvt = G, root = 0;
@@ -109,21 +107,20 @@ __device__ __attribute__((always_inline)) inline void knn_tile(const KnnArgs &a,
         cloud = ti & 0xfffffu, nvt = ti >> 20;
         root = uniform_u32(a.roots[cloud]);
     }
-    ConstDouble *radp = const_doubles(a.radtab) + 66 * cloud;  // level radii: radp[3 * level + axis]
     ConstDouble *magp = const_doubles(a.magtab) + 3 * cloud;
-    const bool valid = slot < a.nq && qs < nvt;
-    const uint64_t segmask = (S == 64 ? ~0ull : ((1ull << S) - 1ull)) << (qs * S);
-    const uint32_t kw = a.k;  // output row width
-    double *bd = s_bd + qs * CAP;
-    uint32_t *bi = s_bi + qs * CAP;
-
     auto wsync = [&]() {
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     };
+    wsync();
+    for (uint32_t i = lane; i < 66; i += 64) s_rad[i] = a.radtab[66 * (size_t)cloud + i];
+    const bool valid = slot < a.nq && qs < nvt;
+    const uint32_t kw_out = a.k;  // output row width
+    uint64_t *bd = s_bd + qs * CAP;
+    uint32_t *bi = s_bi + qs * CAP;
 
-    uint32_t qid = 0, k = kw;
+    uint32_t qid = 0, k = kw_out;
     double qx = 0.0, qy = 0.0, qz = 0.0;
     if (valid) {
         qid = a.order ? a.order[slot] : slot;
@@ -139,303 +136,330 @@ __device__ __attribute__((always_inline)) inline void knn_tile(const KnnArgs &a,
     const double dlx = 0x1p-40 * (magp[0] + fabs(qx)), dly = 0x1p-40 * (magp[1] + fabs(qy));
     const double dlz = 0x1p-40 * (magp[2] + fabs(qz));
 
-    // select by sort-and-merge (else by full sorts); the same in every lane (a ballot)
-    const bool merge = KC >= kKnnMergeMinKC || ballot64(valid && k >= kKnnMergeMinK) != 0;
-    for (uint32_t t = g; t < (uint32_t)CAP; t += S) bd[t] = __builtin_huge_val(), bi[t] = 0xffffffffu;
-    uint32_t cnt = 0;        // kept entries of this query, sorted, at [0, cnt) (same in its S lanes)
-    uint32_t fresh = 0;      // appended entries, unsorted, at [KC or cnt, + fresh) (merge or full sort)
-    bool full = false;       // k entries seen: tau is the k-th
-    double tau = __builtin_huge_val(), tau_pr = __builtin_huge_val();
-    uint32_t tau_i = 0xffffffffu;
-    float tau32 = __builtin_huge_valf();  // tau rounded up to FP32
-    uint64_t n_nodes = 0, n_test = 0, n_recheck = 0, n_select = 0, n_steps = 0;
-
-    // compare-exchange in registers: afterwards (da, ia) <= (db, ib) when up, >= when not
-    auto cx = [](double &da, uint32_t &ia, double &db, uint32_t &ib, const bool up) {
-        const bool sw = up ? knn_less(db, ib, da, ia) : knn_less(da, ia, db, ib);
-        const double lo = sw ? db : da, hi = sw ? da : db;
-        const uint32_t li = sw ? ib : ia, hj = sw ? ia : ib;
-        da = lo, db = hi, ia = li, ib = hj;
+    // lanes of the own group set in a ballot; those below this lane
+    auto gmask = [&](uint64_t m) -> uint64_t { return S == 64 ? m : (m >> gshift) & ((1ull << (S & 63)) - 1ull); };
+    auto gcount = [&](uint64_t m) -> uint32_t {
+        return S == 64 ? (uint32_t)__popcll(m) : (uint32_t)__popc((uint32_t)gmask(m));
     };
-    // bitonic stages with strides `stride`, stride / 2, ..., 1 over the n entries at (sd, si), in
-    // blocks of `size` entries alternately ascending and descending (descending first when desc).
-    // Two stages per LDS round trip: a lane loads the 4 entries that strides s and s / 2 connect
-    // (b, b + s / 2, b + s, b + 3 s / 2), applies both stages in registers and stores them back.
-    auto stages = [&](double *sd, uint32_t *si, const uint32_t n, const uint32_t size, uint32_t stride,
-                      const bool desc) {
-        if constexpr (KC >= kKnnTripleMinKC) {
-            // three stages per round trip: the 8 entries that strides s, s / 2 and s / 4 connect
+    auto gbelow = [&](uint64_t m) -> uint32_t {
+        if (S == 64) return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+        return (uint32_t)__popc((uint32_t)gmask(m) & ((1u << (c & 31)) - 1u));
+    };
+    auto hi32 = [](uint64_t b) -> uint32_t { return (uint32_t)(b >> 32); };
+    auto dbits = [](double d) -> uint64_t { return (uint64_t)__double_as_longlong(d); };
+    auto key_value = [](uint32_t key) -> double { return __longlong_as_double((long long)((uint64_t)key << 32)); };
+
+    const uint32_t kw = k + (k >> 2) + 2 < (uint32_t)(CAP - STEP) ? k + (k >> 2) + 2 : (uint32_t)(CAP - STEP);
+    constexpr uint32_t kFresh = KC / 2 > 8 ? KC / 2 : 8;  // appended entries that are worth a new bound
+    uint32_t cnt = 0, kept = 0;   // entries in the buffer; of them, after the last selection
+    uint32_t T = 0xffffffffu;     // entries have upper distance bits <= T; ~0: fewer than k seen
+    double tau = __builtin_huge_val();      // FP64 upper bound of the k-th distance with the pruning margin
+    float tauf = __builtin_huge_valf();     // the same rounded up to FP32
+    uint32_t n_nodes = 0, n_test = 0, n_recheck = 0, n_select = 0, n_steps = 0;
+
+    // rank of entry (d, i) among the group's cnt entries, for every row of the buffer; entries of rank
+    // below `keep` move to their rank. Afterwards the first `keep` entries are sorted.
+    auto rank_sort = [&](const uint32_t keep) {
+        wsync();
+        uint64_t d[ROWS];
+        uint32_t ix[ROWS], rk[ROWS];
+#pragma unroll
+        for (int j = 0; j < ROWS; j++) {
+            const uint32_t t = j * S + c;
+            d[j] = t < cnt ? bd[t] : ~0ull, ix[j] = t < cnt ? bi[t] : 0xffffffffu, rk[j] = 0;
+        }
+        for (uint32_t t = 0; ballot64(t < cnt); t++) {
+            const bool in = t < cnt;
+            const uint64_t dt = in ? bd[t] : ~0ull;
+            const uint32_t it = in ? bi[t] : 0xffffffffu;
+#pragma unroll
+            for (int j = 0; j < ROWS; j++) rk[j] += knn_less(dt, it, d[j], ix[j]) ? 1u : 0u;
+        }
+        wsync();
+#pragma unroll
+        for (int j = 0; j < ROWS; j++)
+            if ((uint32_t)(j * S) + c < cnt && rk[j] < keep) bd[rk[j]] = d[j], bi[rk[j]] = ix[j];
+        wsync();
+    };
+    // bitonic sort of the buffer's first n entries (n a power of two) by (distance, index)
+    auto bitonic = [&](const uint32_t n) {
+        for (uint32_t t = cnt + c; t < n; t += S) bd[t] = ~0ull, bi[t] = 0xffffffffu;
+        wsync();
 #pragma unroll 1
-            for (; stride >= 4; stride >>= 3) {
-                const uint32_t h = stride >> 1, q = stride >> 2;
+        for (uint32_t size = 2; size <= n; size <<= 1) {
 #pragma unroll 1
-                for (uint32_t t = g; t < n / 8; t += S) {
-                    const uint32_t e0 = ((t & ~(q - 1)) << 3) | (t & (q - 1));
-                    const bool up = ((e0 & size) == 0) != desc;
-                    const uint32_t o[8] = {0, q, h, h + q, stride, stride + q, stride + h, stride + h + q};
-                    double d[8];
-                    uint32_t ix[8];
-#pragma unroll
-                    for (int u = 0; u < 8; u++) d[u] = sd[e0 + o[u]], ix[u] = si[e0 + o[u]];
-#pragma unroll
-                    for (int u = 0; u < 4; u++) cx(d[u], ix[u], d[u + 4], ix[u + 4], up);
-#pragma unroll
-                    for (int u = 0; u < 8; u += 4) {
-                        cx(d[u], ix[u], d[u + 2], ix[u + 2], up);
-                        cx(d[u + 1], ix[u + 1], d[u + 3], ix[u + 3], up);
-                    }
-#pragma unroll
-                    for (int u = 0; u < 8; u += 2) cx(d[u], ix[u], d[u + 1], ix[u + 1], up);
-#pragma unroll
-                    for (int u = 0; u < 8; u++) sd[e0 + o[u]] = d[u], si[e0 + o[u]] = ix[u];
+            for (uint32_t stride = size >> 1; stride > 0; stride >>= 1) {
+#pragma unroll 1
+                for (uint32_t t = c; t < n / 2; t += S) {
+                    const uint32_t e0 = ((t & ~(stride - 1)) << 1) | (t & (stride - 1)), e1 = e0 + stride;
+                    const uint64_t d0 = bd[e0], d1 = bd[e1];
+                    const uint32_t i0 = bi[e0], i1 = bi[e1];
+                    const bool up = (e0 & size) == 0;
+                    if (up ? knn_less(d1, i1, d0, i0) : knn_less(d0, i0, d1, i1))
+                        bd[e0] = d1, bi[e0] = i1, bd[e1] = d0, bi[e1] = i0;
                 }
                 wsync();
             }
         }
-#pragma unroll 1
-        for (; stride >= 2; stride >>= 2) {
-            const uint32_t h = stride >> 1;
-#pragma unroll 1
-            for (uint32_t t = g; t < n / 4; t += S) {
-                const uint32_t e0 = ((t & ~(h - 1)) << 2) | (t & (h - 1));
-                const uint32_t e1 = e0 + h, e2 = e0 + stride, e3 = e2 + h;
-                const bool up = ((e0 & size) == 0) != desc;
-                double d0 = sd[e0], d1 = sd[e1], d2 = sd[e2], d3 = sd[e3];
-                uint32_t i0 = si[e0], i1 = si[e1], i2 = si[e2], i3 = si[e3];
-                cx(d0, i0, d2, i2, up);
-                cx(d1, i1, d3, i3, up);
-                cx(d0, i0, d1, i1, up);
-                cx(d2, i2, d3, i3, up);
-                sd[e0] = d0, sd[e1] = d1, sd[e2] = d2, sd[e3] = d3;
-                si[e0] = i0, si[e1] = i1, si[e2] = i2, si[e3] = i3;
-            }
-            wsync();
-        }
-        if (stride == 1) {  // an odd number of stages: the last one alone
-#pragma unroll 1
-            for (uint32_t t = g; t < n / 2; t += S) {
-                const uint32_t e0 = t << 1;
-                const bool up = ((e0 & size) == 0) != desc;
-                double d0 = sd[e0], d1 = sd[e0 + 1];
-                uint32_t i0 = si[e0], i1 = si[e0 + 1];
-                cx(d0, i0, d1, i1, up);
-                sd[e0] = d0, sd[e0 + 1] = d1;
-                si[e0] = i0, si[e0 + 1] = i1;
-            }
-            wsync();
-        }
     };
-    // bitonic sort of the n entries at (sd, si), ascending or descending by (distance, index)
-    auto bitonic = [&](double *sd, uint32_t *si, const uint32_t n, const bool descending) {
-#pragma unroll 1
-        for (uint32_t size = 2; size <= n; size <<= 1) stages(sd, si, n, size, size >> 1, descending);
+    // the buffer's entries in order, the first min(cnt, k) of them exact (every lane of the wave)
+    auto order_entries = [&]() {
+        if (kRank) {
+            rank_sort(k);
+        } else {
+            uint32_t mx = group_reduce<64>(cnt, [](uint32_t x, uint32_t y) { return x > y ? x : y; });
+            uint32_t n = 64;
+            mx = uniform_u32(mx);
+            while (n < mx) n <<= 1;
+            bitonic(n);
+        }
+        if (cnt > k) cnt = k;
+    };
+    auto set_bound = [&](const bool part) {  // T is valid: the k-th distance lies below (T + 1) << 32
+        if (part) {
+            const double ub = __longlong_as_double((long long)(((uint64_t)T + 1ull) << 32));
+            tau = ub * (1.0 + 0x1p-40);
+            tauf = __double2float_ru(tau);
+        }
     };
 
-    // merge every query's appended entries into its kept ones, keep its k best
+    // selection, for the groups with at least k entries: T such that k .. kw entries have upper bits <= T
+    // (more where they tie); the others leave the buffer
     auto select = [&]() {
         n_select++;
         wsync();
-        if (merge) {
-            // appended half [KC, 2 KC) sorted descending (empty slots hold +inf and end up first)
-            bitonic(bd + KC, bi + KC, (uint32_t)KC, true);
-            // ascending kept half + descending appended half is bitonic: one merge sorts all 2 KC
-            stages(bd, bi, (uint32_t)CAP, 2u * CAP, (uint32_t)KC, false);
-        } else {
-            bitonic(bd, bi, (uint32_t)CAP, false);  // kept and appended entries, [0, cnt + fresh)
+        const bool part = cnt >= k && k > 0;
+        uint32_t key[ROWS];
+        uint32_t mx = 0;
+#pragma unroll
+        for (int j = 0; j < ROWS; j++) {
+            const uint32_t t = j * S + c;
+            key[j] = t < cnt ? hi32(bd[t]) : 0xffffffffu;
+            if (t < cnt && key[j] > mx) mx = key[j];
         }
-        const uint32_t tot = cnt + fresh;  // entries, now sorted at [0, tot)
-        const uint32_t keep = tot < k ? tot : k;
-        for (uint32_t t = keep + g; t < tot; t += S) bd[t] = __builtin_huge_val(), bi[t] = 0xffffffffu;
-        cnt = keep;
-        fresh = 0;
-        if (keep == k && k > 0) {
-            full = true;
-            tau = bd[k - 1];
-            tau_i = bi[k - 1];
-            tau_pr = tau * (1.0 + 0x1p-40);
-            tau32 = __double2float_ru(tau);
+        mx = group_reduce<S>(mx, [](uint32_t x, uint32_t y) { return x > y ? x : y; });
+        // count(<= hi) = ch >= k, count(<= lo) = cl < k (lo = -1: none); keys stay below 2^31 (or a NaN's)
+        uint32_t hi = mx, ch = cnt, cl = 0;
+        int64_t lo = -1;
+        double vlo = 0.0;
+        const uint32_t target = k + ((kw - k) >> 1);
+        for (uint32_t iter = 0;; iter++) {
+            const bool go = part && ch > kw && (int64_t)hi - lo > 1;
+            if (!ballot64(go)) break;
+            const double vhi = key_value(hi);
+            uint32_t mid = hi32(dbits(vlo + (vhi - vlo) * (double)((float)(target - cl) * __builtin_amdgcn_rcpf((float)(ch - cl)))));
+            if (iter >= 6 || !((int64_t)mid > lo && mid < hi)) mid = (uint32_t)(lo + ((int64_t)hi - lo) / 2);
+            uint32_t nle = 0;
+#pragma unroll
+            for (int j = 0; j < ROWS; j++) nle += key[j] <= mid ? 1u : 0u;
+            nle = group_reduce<S>(nle, [](uint32_t x, uint32_t y) { return x + y; });
+            if (go) {
+                if (nle >= k)
+                    hi = mid, ch = nle;
+                else
+                    lo = (int64_t)mid, cl = nle, vlo = key_value(mid);
+            }
         }
-        wsync();
+        if (part) T = hi;
+        // entries at or below T move to the front (towards lower slots only, row by row)
+        if (ballot64(part && ch < cnt)) {
+            uint32_t base = 0;
+#pragma unroll
+            for (int j = 0; j < ROWS; j++) {
+                const uint32_t t = j * S + c;
+                const bool keep = t < cnt && key[j] <= T;
+                const uint64_t m = ballot64(keep);
+                uint64_t d = 0;
+                uint32_t ix = 0;
+                if (keep) d = bd[t], ix = bi[t];
+                wsync();
+                if (keep) {
+                    const uint32_t pos = base + gbelow(m);
+                    bd[pos] = d, bi[pos] = ix;
+                }
+                base += gcount(m);
+                wsync();
+            }
+            cnt = base;
+        }
+        set_bound(part);
+        if (ballot64(cnt > (uint32_t)(CAP - STEP))) {  // ties fill the buffer: keep exactly the k best
+            order_entries();
+            wsync();
+        }
+        kept = cnt;
     };
 
-    // leaf [first, last) with centre c and FP32 bound amx, for the queries with need set
-    auto leaf = [&](bool need, uint32_t first, uint32_t last, double cx, double cy, double cz, float amx) {
+    // appends the accepted points of a step; accepted lanes: upper distance bits <= T
+    auto append = [&](const bool acc, const uint64_t d, const uint32_t id) {
+        const uint64_t m = ballot64(acc);
+        if (acc) {
+            const uint32_t pos = cnt + gbelow(m);
+            bd[pos] = d, bi[pos] = id;
+        }
+        cnt += gcount(m);
+    };
+
+    // tests every group's leaf (need: the group has one)
+    auto leaf = [&](const bool need, const uint32_t node) {
+        uint32_t i = 0, e = 0;
         float m2x = 0.f, m2y = 0.f, m2z = 0.f, bb = 0.f, hw = 0.f;
         bool force = false;
-        if (F32) {
-            const float bx = (float)(qx - cx), by = (float)(qy - cy), bz = (float)(qz - cz);
-            bb = bx * bx + by * by + bz * bz;
-            const float s = amx + bb;
-            force = !(s < 1e30f);
-            hw = s * 0x1p-18f;
-            m2x = -2.0f * bx, m2y = -2.0f * by, m2z = -2.0f * bz;
-        }
-        if (need && g == 0) n_nodes++;
-        for (uint32_t base = first; base < last; base += kKnnChunk) {
-            const uint32_t P = (last - base) < (uint32_t)kKnnChunk ? (last - base) : (uint32_t)kKnnChunk;
-            const uint32_t nsteps = (P + STEP - 1) / STEP;
-            const uint32_t slots = nsteps * STEP;
-            for (uint32_t t = lane; t < slots; t += 64) {
-                if (F32)
-                    s32[t] = t < P ? a.p32[base + t] : make_float4(0.f, 0.f, 0.f, 0.f);
-                else
-                    s64[t] = t < P ? a.p64[base + t] : make_double4(0.0, 0.0, 0.0, 0.0);
+        if (need) {
+            const NodeRec nr = a.nodes[node];
+            i = nr.first, e = nr.last;
+            if (F32) {
+                const float amx = a.amax[node];
+                const float bx = (float)(qx - nr.cx), by = (float)(qy - nr.cy), bz = (float)(qz - nr.cz);
+                bb = bx * bx + by * by + bz * bz;
+                const float s = amx + bb;
+                force = !(s < 1e30f);
+                hw = s * 0x1p-18f;
+                m2x = -2.0f * bx, m2y = -2.0f * by, m2z = -2.0f * bz;
             }
-            wsync();
-            for (uint32_t s = 0; s < nsteps; s++) {
-                // appended entries start at KC (merge) or right after the kept ones (full sort)
-                if (ballot64(need && fresh + STEP > (merge ? (uint32_t)KC : (uint32_t)CAP - cnt))) select();
-                n_steps++;
-                float thr = __builtin_huge_valf();
-                if (F32 && full && !force) thr = ((tau32 + hw) * (1.0f + 0x1p-20f));
-                double d[U];
-                uint32_t id[U];
-                bool c[U];
+            if (c == 0) n_nodes++;
+        }
+        float thr = 0.0f;
+        bool stale = true;
+        while (ballot64(i < e)) {
+            if (ballot64(i < e && cnt + STEP > (uint32_t)CAP)) select(), stale = true;
+            n_steps++;
+            if (F32 && stale) {
+                thr = T == 0xffffffffu || force ? __builtin_huge_valf() : (tauf + hw) * (1.0f + 0x1p-20f);
+                stale = false;
+            }
+            bool acc[U];
+            uint64_t d[U];
 #pragma unroll
-                for (int u = 0; u < U; u++) {
-                    const uint32_t t = s * STEP + u * S + g;
-                    id[u] = base + t;
-                    const bool real = need && t < P;
-                    if (F32) {
-                        const float4 p = s32[t];
-                        const float e = __builtin_fmaf(p.x, m2x, __builtin_fmaf(p.y, m2y, __builtin_fmaf(p.z, m2z, p.w + bb)));
-                        c[u] = real && !(e > thr);
-                        d[u] = 0.0;
-                    } else {
-                        const double4 p = s64[t];
-                        const double dx = qx - p.x, dy = qy - p.y, dz = qz - p.z;
-                        d[u] = dx * dx + dy * dy + dz * dz;
-                        c[u] = real && (!full || knn_less(d[u], id[u], tau, tau_i));
-                    }
-                    if (real) n_test++;
-                }
+            for (int u = 0; u < U; u++) {
+                const uint32_t id = i + (uint32_t)(u * S) + c;
+                acc[u] = id < e;
+                d[u] = 0;
                 if (F32) {
-#pragma unroll
-                    for (int u = 0; u < U; u++) {
-                        if (c[u]) {
-                            const double4 p = a.p64[id[u]];
-                            const double dx = qx - p.x, dy = qy - p.y, dz = qz - p.z;
-                            d[u] = dx * dx + dy * dy + dz * dz;
-                            c[u] = !full || knn_less(d[u], id[u], tau, tau_i);
-                            n_recheck++;
-                        }
+                    float ev = 0.0f;
+                    if (i < e) {  // reads up to 2 S - 1 points past the range: the sorted clouds are padded
+                        const float4 p = a.p32[id];
+                        ev = __builtin_fmaf(p.x, m2x, __builtin_fmaf(p.y, m2y, __builtin_fmaf(p.z, m2z, p.w + bb)));
                     }
-                }
-#pragma unroll
-                for (int u = 0; u < U; u++) {
-                    const uint64_t m = ballot64(c[u]) & segmask;
-                    if (c[u]) {
-                        const uint32_t pos = (merge ? (uint32_t)KC : cnt) + fresh + (uint32_t)__popcll(m & lanemask_lt());
-                        bd[pos] = d[u];
-                        bi[pos] = id[u];
-                    }
-                    fresh += (uint32_t)__popcll(m);
+                    acc[u] = acc[u] & !(ev > thr);
                 }
             }
-            wsync();  // the next chunk overwrites the staging area
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const uint32_t id = i + (uint32_t)(u * S) + c;
+                if (acc[u]) {
+                    const double4 p = a.p64[id];
+                    const double dx = qx - p.x, dy = qy - p.y, dz = qz - p.z;
+                    d[u] = dbits(dx * dx + dy * dy + dz * dz);
+                    acc[u] = hi32(d[u]) <= T;
+                    if (F32) n_recheck++;
+                }
+                if (id < e) n_test++;
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++) append(acc[u], d[u], i + (uint32_t)(u * S) + c);
+            i = i < e ? i + STEP : i;
         }
+        // a first bound as soon as k points are known, a new one when enough points came in
+        if (ballot64(cnt >= k && k > 0 && (T == 0xffffffffu || cnt - kept >= kFresh))) select();
     };
 
-    // reference query for the child order: the middle valid query of the wave
-    // (a forest's wave tile holds nvt valid slots: the rest are padding whose centre is not a query)
-    uint32_t nvalid = a.nq - slot0 < (uint32_t)G ? a.nq - slot0 : (uint32_t)G;
-    if (nvt < nvalid) nvalid = nvt;
-    const int refl = (int)(S * (nvalid / 2));
-
-    uint32_t sp = 0;
-    bool overflow = false;  // wave-uniform: a push found the stack full (cannot happen within 21 levels)
+    // levels with waiting children (the same in the group's lanes); levels at which this lane's child waits
+    uint32_t lvl = 0, pend = 0;
+    bool overflow = false;
+    uint32_t at = 0;      // the group's leaf
+    bool have = false;
+    wsync();
+    auto judge = [&](const bool act, const uint32_t fc, const uint32_t L) {
+        // children fc .. fc + 7 (level L) of a node of the group's query, one per lane c < 8
+        bool wait = false;
+        uint32_t ent = 0, lbits = 0;
+        if (act && c < 8) {
+            const uint32_t node = fc + c;
+            const NodeRec nr = a.nodes[node];
+            const uint32_t gc = a.child[node];
+            const double lb = (gap2(qx, nr.cx, s_rad[3 * L], dlx) + gap2(qy, nr.cy, s_rad[3 * L + 1], dly)) +
+                              gap2(qz, nr.cz, s_rad[3 * L + 2], dlz);
+            wait = nr.last > nr.first && !(lb > tau);
+            ent = gc ? gc : (node | kKnnLeafBit);
+            lbits = __float_as_uint((float)lb);  // rounded to nearest: one ulp less is a lower bound
+            lbits -= lbits ? 1u : 0u;
+        }
+        if (wait) {
+            if (L < a.levels) {
+                lev.node[(L * G + qs) * 8 + c] = ent;
+                lev.key[(L * G + qs) * 8 + c] = (uint16_t)(lbits >> 16);
+                pend |= 1u << L;
+            } else {
+                overflow = true;  // below the tree's last level: cannot happen
+            }
+        }
+        if (act && gmask(ballot64(wait))) lvl |= 1u << L;
+    };
     {
         const uint32_t c0 = uniform_u32(a.child[root]);
         if (c0 == 0) {
-            const NodeRec nr = a.nodes[root];
-            leaf(valid, uniform_u32(nr.first), uniform_u32(nr.last), nr.cx, nr.cy, nr.cz, a.amax[root]);
+            have = valid, at = root;
         } else {
-            s_node[0] = (c0 - 1) >> 3, s_lev[0] = 0;
-            sp = 1;
+            judge(valid, c0, 1);
+            if (c == 0 && valid) n_nodes += 8;
         }
     }
-    wsync();
-    while (sp > 0) {
-        sp--;
-        const uint32_t ent = uniform_u32(s_node[sp]);
-        const uint32_t lv = uniform_u32(s_lev[sp]);
-        if (lv & 0x80u) {
-            // a leaf: entry = NodeExt index * 8 + combo; re-test it against the current k-th distances
-            ConstNodeExt &E = node_ext(a.next, ent >> 3);
-            const uint32_t c = ent & 7u, L = lv & 31u;
-            const double cx = E.ax[c & 1u], cy = E.ax[2 + ((c >> 1) & 1u)], cz = E.ax[4 + (c >> 2)];
-            const double lb = (gap2(qx, cx, radp[3 * L], dlx) + gap2(qy, cy, radp[3 * L + 1], dly)) + gap2(qz, cz, radp[3 * L + 2], dlz);
-            const bool need = valid && !(lb > tau_pr);
-            if (!ballot64(need)) continue;
-            leaf(need, E.first[c], E.last[c], cx, cy, cz, E.amax[c]);
-            continue;
-        }
-        // an internal node at level lv: judge its 8 children (level lv + 1) from per-axis terms
-        ConstNodeExt &E = node_ext(a.next, ent);
-        const uint32_t d = lv + 1;
-        const double rx = radp[3 * d], ry = radp[3 * d + 1], rz = radp[3 * d + 2];
-        double gx[2], gy[2], gz[2];
-#pragma unroll
-        for (int b = 0; b < 2; b++) {
-            gx[b] = gap2(qx, E.ax[b], rx, dlx);
-            gy[b] = gap2(qy, E.ax[2 + b], ry, dly);
-            gz[b] = gap2(qz, E.ax[4 + b], rz, dlz);
-        }
-        uint32_t needbits = 0;
-#pragma unroll
-        for (int c = 0; c < 8; c++) {
-            const double lb = (gx[c & 1] + gy[(c >> 1) & 1]) + gz[c >> 2];
-            const bool nd = valid && E.last[c] > E.first[c] && !(lb > tau_pr);
-            if (ballot64(nd)) needbits |= 1u << c;
-        }
-        if (g == 0) n_nodes += 8 * (valid ? 1 : 0);
-        needbits = uniform_u32(needbits);  // built from ballots: the same in every lane
-        if (needbits == 0) continue;
-        // push the farthest octants (relative to the reference query) first
-        const uint32_t oc = (qx >= 0.5 * (E.ax[0] + E.ax[1]) ? 1u : 0u) | (qy >= 0.5 * (E.ax[2] + E.ax[3]) ? 2u : 0u) |
-                            (qz >= 0.5 * (E.ax[4] + E.ax[5]) ? 4u : 0u);
-        const uint32_t qc = readlane_u32(oc, refl);
-        constexpr uint32_t kOrder = 0x02416537u;  // nibbles, low first: 7 3 5 6 1 4 2 0
-#pragma unroll
-        for (int t = 0; t < 8; t++) {
-            const uint32_t c = ((kOrder >> (4 * t)) & 7u) ^ qc;
-            if ((needbits >> c) & 1u) {
-                if (sp < (uint32_t)kKnnStack) {
-                    const uint32_t gc = E.gc[c];
-                    s_node[sp] = gc ? (gc - 1) >> 3 : ent * 8 + c;
-                    s_lev[sp] = (uint8_t)(gc ? d : (d | 0x80u));
-                    sp++;
-                } else {
-                    overflow = true;
-                }
+    for (;;) {
+        for (;;) {  // every group without a leaf takes its nearest waiting child
+            const bool go = !have && lvl != 0;
+            if (!ballot64(go)) break;
+            wsync();
+            const uint32_t L = go ? 31u - (uint32_t)__clz(lvl) : 0u;
+            const bool mine = go && ((pend >> L) & 1u);
+            uint32_t key = mine ? ((uint32_t)lev.key[(L * G + qs) * 8 + (c & 7u)] << 16) | c : 0xffffffffu;
+            key = group_reduce<S>(key, [](uint32_t x, uint32_t y) { return x < y ? x : y; });
+            const float lb = __uint_as_float(key & 0xffff0000u);
+            const bool none = key == 0xffffffffu || lb > tauf;  // nothing waits at L, or all of it is too far
+            if (go && none) lvl &= ~(1u << L), pend &= ~(1u << L);
+            const uint32_t oct = key & 7u;
+            const bool take = go && !none;
+            const uint32_t ent = take ? lev.node[(L * G + qs) * 8 + oct] : 0u;
+            if (take && c == oct) pend &= ~(1u << L);
+            const bool lf = take && (ent & kKnnLeafBit) != 0;
+            if (lf) have = true, at = ent & ~kKnnLeafBit;
+            const bool down = take && !lf;
+            if (ballot64(down)) {
+                if (down && c == 0) n_nodes += 8;
+                judge(down, ent, L + 1);
             }
         }
-        wsync();
+        if (!ballot64(have)) break;  // every traversal is done
+        leaf(have, at);
+        have = false;
     }
-    select();
-    if (overflow && lane == 0) atomicOr(a.err, kErrStack);
+    if (ballot64(cnt > kw)) select();
+    order_entries();
+    if (ballot64(overflow) && lane == 0) atomicOr(a.err, kErrStack);
 
+    wsync();
     if (valid) {
         const uint32_t off = a.cloud_off ? a.cloud_off[cloud] : 0u;  // the tile's cloud holds every neighbour
-        for (uint32_t t = g; t < kw; t += S) {
-            const bool have = t < cnt;
-            a.idx_out[(size_t)qid * kw + t] = have ? (int32_t)(bi[t] - off) : -1;
-            if (a.d2_out) a.d2_out[(size_t)qid * kw + t] = have ? bd[t] : __builtin_nan("");
-            if (a.d2f_out) a.d2f_out[(size_t)qid * kw + t] = have ? (float)bd[t] : __builtin_nanf("");
+        for (uint32_t t = c; t < kw_out; t += S) {
+            const bool have_t = t < cnt;
+            const double d = have_t ? __longlong_as_double((long long)bd[t]) : 0.0;
+            a.idx_out[(size_t)qid * kw_out + t] = have_t ? (int32_t)(bi[t] - off) : -1;
+            if (a.d2_out) a.d2_out[(size_t)qid * kw_out + t] = have_t ? d : __builtin_nan("");
+            if (a.d2f_out) a.d2f_out[(size_t)qid * kw_out + t] = have_t ? (float)d : __builtin_nanf("");
         }
     }
     if (a.stats) {
-        uint64_t found = (valid && g == 0) ? cnt : 0;
+        uint64_t found = (valid && c == 0) ? cnt : 0, sn = n_nodes, st = n_test, sr = n_recheck;
         for (int off = 32; off > 0; off >>= 1) {
-            n_nodes += __shfl_xor(n_nodes, off);
-            n_test += __shfl_xor(n_test, off);
-            n_recheck += __shfl_xor(n_recheck, off);
+            sn += __shfl_xor(sn, off);
+            st += __shfl_xor(st, off);
+            sr += __shfl_xor(sr, off);
             found += __shfl_xor(found, off);
         }
         if (lane == 0) {
-            atomicAdd(&a.stats[0], (unsigned long long)n_nodes);
-            atomicAdd(&a.stats[1], (unsigned long long)n_test);
-            atomicAdd(&a.stats[2], (unsigned long long)n_recheck);
+            atomicAdd(&a.stats[0], (unsigned long long)sn);
+            atomicAdd(&a.stats[1], (unsigned long long)st);
+            atomicAdd(&a.stats[2], (unsigned long long)sr);
             atomicAdd(&a.stats[3], (unsigned long long)found);
             atomicAdd(&a.stats[4], (unsigned long long)n_select);  // wave-wide selections
             atomicAdd(&a.stats[5], (unsigned long long)n_steps);   // wave-wide leaf steps
@@ -443,18 +467,20 @@ __device__ __attribute__((always_inline)) inline void knn_tile(const KnnArgs &a,
     }
 }
 
-// Occupancy target (waves per SIMD): 6 for the 8-lanes, k <= 16, FP32 shape (80 VGPRs and a 20-byte
-// spill instead of 92 VGPRs at 5 waves: 75.1 vs 79.9 ms for all 20 M points of the tile at k = 10);
-// every other shape, and the work-queue form (which would spill 56 bytes at that target), keep the
-// compiler's choice.
-template <int S, int KC, int PREC>
-constexpr int knn_waves() {
-    return (S == 8 && KC == 16 && PREC == OCT_PREC_FP32_RECHECK) ? 6 : 1;
+// dynamic LDS of one wave: rows for `levels` levels
+template <int S>
+constexpr size_t knn_lds(uint32_t levels) {
+    return (size_t)levels * (64 / S) * 8 * (sizeof(uint32_t) + sizeof(uint16_t));
+}
+template <int S>
+__device__ inline KnnLevels knn_levels(const KnnArgs &a) {
+    extern __shared__ uint32_t s_lev[];
+    return KnnLevels{s_lev, reinterpret_cast<uint16_t *>(s_lev + (size_t)a.levels * (64 / S) * 8)};
 }
 
 template <int S, int KC, int PREC>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(knn_waves<S, KC, PREC>()))) void k_knn(const KnnArgs a) {
-    knn_tile<S, KC, PREC>(a, blockIdx.x);
+__global__ __launch_bounds__(64) void k_knn(const KnnArgs a) {
+    knn_tile<S, KC, PREC>(a, blockIdx.x, knn_levels<S>(a));
 }
 
 // Work-queue form (batches): a grid of resident waves; each takes the next wave tile from a device
@@ -468,7 +494,7 @@ __global__ __launch_bounds__(64) void k_knn_queue(const KnnArgs a) {
         if (lane_id() == 0) t = atomicAdd(a.queue_next, 1u);
         t = readlane_u32(t, 0);
         if (t >= ntiles) return;
-        knn_tile<S, KC, PREC>(a, t);
+        knn_tile<S, KC, PREC>(a, t, knn_levels<S>(a));
     }
 }
 
@@ -479,25 +505,26 @@ static unsigned knn_queue_grid() {
     int dev = 0, cus = 0, per = 0;
     (void)hipGetDevice(&dev);
     (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-    (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k_knn_queue<S, KC, PREC>, 64, 0);
+    (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k_knn_queue<S, KC, PREC>, 64, knn_lds<S>(kMaxDepth + 1));
     cached = (unsigned)((cus > 0 ? cus : 256) * (per > 0 ? per : 1));
     return cached;
 }
 
 template <int S, int KC>
 static void launch_sk(const KnnArgs &a, int precision, hipStream_t s) {
+    const size_t lds = knn_lds<S>(a.levels);
     if (a.queue_next) {
         if (precision == OCT_PREC_FP32_RECHECK)
-            k_knn_queue<S, KC, OCT_PREC_FP32_RECHECK><<<knn_queue_grid<S, KC, OCT_PREC_FP32_RECHECK>(), 64, 0, s>>>(a);
+            k_knn_queue<S, KC, OCT_PREC_FP32_RECHECK><<<knn_queue_grid<S, KC, OCT_PREC_FP32_RECHECK>(), 64, lds, s>>>(a);
         else
-            k_knn_queue<S, KC, OCT_PREC_FP64><<<knn_queue_grid<S, KC, OCT_PREC_FP64>(), 64, 0, s>>>(a);
+            k_knn_queue<S, KC, OCT_PREC_FP64><<<knn_queue_grid<S, KC, OCT_PREC_FP64>(), 64, lds, s>>>(a);
         return;
     }
-    const unsigned nb = (unsigned)((a.nq + (64 / S) - 1) / (64 / S));
+    const unsigned nb = (unsigned)(((size_t)a.nq + (64 / S) - 1) / (64 / S));
     if (precision == OCT_PREC_FP32_RECHECK)
-        k_knn<S, KC, OCT_PREC_FP32_RECHECK><<<nb, 64, 0, s>>>(a);
+        k_knn<S, KC, OCT_PREC_FP32_RECHECK><<<nb, 64, lds, s>>>(a);
     else
-        k_knn<S, KC, OCT_PREC_FP64><<<nb, 64, 0, s>>>(a);
+        k_knn<S, KC, OCT_PREC_FP64><<<nb, 64, lds, s>>>(a);
 }
 
 // buffer size class of k (entries per query kept between selections)
@@ -507,16 +534,26 @@ static int knn_kc(uint32_t k) {
     return kc;
 }
 
-// lanes per query offered for each size class, default first
+// lanes-per-query shapes of each size class, default first
 int knn_lane_options(uint32_t k, int out[3]) {
     switch (knn_kc(k)) {
-        case 16: out[0] = 4, out[1] = 2, out[2] = 8; return 3;
-        case 32: out[0] = 4, out[1] = 2, out[2] = 8; return 3;
-        case 64: out[0] = 8, out[1] = 4, out[2] = 16; return 3;
-        case 128: out[0] = 16, out[1] = 8, out[2] = 32; return 3;
-        case 256: out[0] = 64, out[1] = 32, out[2] = 16; return 3;
+        case 16: case 32: out[0] = 8; return 1;
+        case 64: out[0] = 16, out[1] = 8; return 2;
+        case 128: out[0] = 32, out[1] = 16; return 2;
+        case 256: out[0] = 64, out[1] = 32; return 2;
         default: out[0] = 64; return 1;
     }
+}
+// the shape that runs a requested number of lanes per query (0: not offered for this k): the smaller
+// requests a class accepts run its smallest shape
+int knn_shape_lanes(uint32_t k, int lanes) {
+    const int kc = knn_kc(k);
+    if (lanes != 2 && lanes != 4 && lanes != 8 && lanes != 16 && lanes != 32 && lanes != 64) return 0;
+    if (kc <= 32) return lanes <= 8 ? 8 : 0;
+    if (kc == 64) return lanes < 4 || lanes > 16 ? 0 : (lanes == 16 ? 16 : 8);
+    if (kc == 128) return lanes < 8 || lanes > 32 ? 0 : (lanes == 32 ? 32 : 16);
+    if (kc == 256) return lanes < 16 ? 0 : (lanes == 64 ? 64 : 32);
+    return lanes == 64 ? 64 : 0;
 }
 
 static bool launch_knn_shape(const KnnArgs &a, int kc, int precision, int lanes, hipStream_t s) {
@@ -525,11 +562,10 @@ static bool launch_knn_shape(const KnnArgs &a, int kc, int precision, int lanes,
         launch_sk<SV, KCV>(a, precision, s);      \
         return true;                              \
     }
-    OCT_KNN_CASE(16, 2) OCT_KNN_CASE(16, 4) OCT_KNN_CASE(16, 8)
-    OCT_KNN_CASE(32, 2) OCT_KNN_CASE(32, 4) OCT_KNN_CASE(32, 8)
-    OCT_KNN_CASE(64, 4) OCT_KNN_CASE(64, 8) OCT_KNN_CASE(64, 16)
-    OCT_KNN_CASE(128, 8) OCT_KNN_CASE(128, 16) OCT_KNN_CASE(128, 32)
-    OCT_KNN_CASE(256, 16) OCT_KNN_CASE(256, 32) OCT_KNN_CASE(256, 64)
+    OCT_KNN_CASE(16, 8) OCT_KNN_CASE(32, 8)
+    OCT_KNN_CASE(64, 8) OCT_KNN_CASE(64, 16)
+    OCT_KNN_CASE(128, 16) OCT_KNN_CASE(128, 32)
+    OCT_KNN_CASE(256, 32) OCT_KNN_CASE(256, 64)
     OCT_KNN_CASE(512, 64) OCT_KNN_CASE(1024, 64)
 #undef OCT_KNN_CASE
     return false;
@@ -553,7 +589,6 @@ hipError_t launch_knn(oct_ctx *ctx, const KnnLaunch &L, std::string &err) {
     a.p32 = ctx->p32.p;
     a.amax = ctx->amax.p;
     a.nodes = ctx->nodes.p;
-    a.next = ctx->next.p;
     a.child = ctx->child.p;
     a.order = L.order;
     a.qidx = L.qidx;
@@ -578,7 +613,9 @@ hipError_t launch_knn(oct_ctx *ctx, const KnnLaunch &L, std::string &err) {
     const uint32_t kcls = L.kq && L.kclass ? L.kclass : k;  // selection size class of the launch
     int opts[3];
     knn_lane_options(kcls, opts);
-    const int lanes = L.lanes > 0 ? L.lanes : opts[0];
+    const int lanes = L.lanes > 0 ? knn_shape_lanes(kcls, L.lanes) : opts[0];
+    // rows of waiting children: levels 1 .. the deepest (a forest's depth is known on the device only)
+    a.levels = L.roots ? kMaxDepth + 1 : (ctx->n_levels > 1 ? ctx->n_levels : 1u);
     stage_begin(ctx, ST_KNN);
     if (!launch_knn_shape(a, knn_kc(kcls), precision, lanes, ctx->stream)) {
         err = "knn: lanes per query not offered for this k";
