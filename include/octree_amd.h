@@ -197,8 +197,8 @@ int oct_radius_approx(oct_ctx *ctx, int kernel, int precision, const double *cen
 /* ---- H6 kNN: LinearOctree::knn (linear_octree.hpp:899-942), benchmark label KNNV2. Exact k
  * nearest under the (squared FP64 distance, sorted index) order; returns min(n, k) per query,
  * ascending; k <= 1024. idx_out: nq x k int32 (-1 pads), d2_out: nq x k FP64 squared distances
- * (NaN pads). OCT_PREC_FP32_RECHECK screens points with leaf-recentred FP32 distances and computes
- * the FP64 distance only for points that may beat the current k-th; results are identical. */
+ * (NaN pads). Both precisions compute FP64 distances (an FP32 screen in front of them measured slower
+ * at every k), so their results are identical and stats->rechecked is 0. */
 int oct_knn(oct_ctx *ctx, int precision, const double *centers, const uint32_t *center_idx, size_t nq, uint32_t k,
             int32_t *idx_out, double *d2_out, oct_search_stats *stats);
 /* Device-resident kNN for throughput runs, same neighbour sets in the compact output form: int32
@@ -234,11 +234,12 @@ int oct_knn_checksum(oct_ctx *ctx, const int32_t *idx_dev, const float *d2_dev, 
  * OCT_TUNE_RADIUS_REMAP: 1 (default, also -1) lets the count-mode vector point tests move the
  * queries of a leaf that at most half of a wave's queries want onto all 64 lanes; 0 keeps every
  * query on its own lanes.
- * OCT_TUNE_KNN_LANES: lanes per query of the kNN kernel (64 / lanes queries share one wave's
- * traversal); each k size class (k <= 16, 32, 64, ... 1024) offers up to three shapes, the
- * default first (k <= 32: 4, 2, 8; <= 64: 8, 4, 16; <= 128: 16, 8, 32; <= 256: 64, 32, 16;
- * above: 64); a value a class does not offer makes its kNN calls fail with OCT_ERR_ARG; -1
- * restores "autotuned, else the default". oct_autotune_knn times the offered shapes on sample_nq
+ * OCT_TUNE_KNN_LANES: lanes per query of the kNN kernel, each query walking its own path (64 / lanes
+ * queries per wave). Each k size class (k <= 16, 32, 64, ... 1024) accepts a few values and runs up to two
+ * shapes, the default first (k <= 32: 8; <= 64: 16, 8; <= 128: 32, 16; <= 256: 64, 32; above: 64); accepted
+ * are 2, 4, 8 (k <= 32), 4, 8, 16 (<= 64), 8, 16, 32 (<= 128), 16, 32, 64 (<= 256) and 64, a value below
+ * the smallest shape running that; other values make the class's kNN calls fail with OCT_ERR_ARG; -1
+ * restores "autotuned, else the default". oct_autotune_knn times the shapes on sample_nq
  * all-points queries (16 strided chunks, as above; 0 = 2^18), stores the fastest for (precision,
  * size class of k), returns it in *best and the best milliseconds per shape in ms_out[0..2].
  * oct_tuned_knn: the lanes per query a kNN call with this k would use now.

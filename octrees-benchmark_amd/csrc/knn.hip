@@ -18,10 +18,11 @@
 //    keeps those and drops the rest; T bounds the k-th distance from above. No entry is sorted until the
 //    end, when the k best of the remaining few are ordered exactly. More than kw entries can share T's
 //    upper bits (ties): where they would fill the buffer, an exact selection keeps the k best.
-// FP32_RECHECK filters the points with the leaf-recentred FP32 form e = w - 2 a.b + |b|^2 (the count
-// kernel's representation), whose error is below hw / 2 = 2^-19 (amax + |b|^2); only points with
-// e <= bound + hw get their exact FP64 distance.
+// Both precisions run the same FP64 distances: MI355X issues FP64 at the rate of unpacked FP32, and a
+// leaf-recentred FP32 screen in front of them (16 instead of 32 bytes per point, a second load for what
+// passes) was 6 - 17 % slower at every k from 1 to 1000.
 #include <cfloat>
+#include <type_traits>
 
 #include "device.hpp"
 #include "search_common.hpp"
@@ -30,8 +31,6 @@ namespace oct {
 
 struct KnnArgs {
     const double4 *__restrict__ p64;
-    const float4 *__restrict__ p32;
-    const float *__restrict__ amax;
     const NodeRec *__restrict__ nodes;
     const uint32_t *__restrict__ child;
     const uint32_t *__restrict__ order;
@@ -83,14 +82,13 @@ struct KnnLevels {
 };
 
 // One wave tile (64 / S queries) of a kNN search, run by one wave (a 64-thread block).
-template <int S, int KC, int PREC>
+template <int S, int KC>
 __device__ __attribute__((always_inline)) inline void knn_tile(const KnnArgs &a, const uint32_t tile, const KnnLevels lev) {
     constexpr int G = 64 / S;                // queries per wave
     constexpr int CAP = knn_cap(KC);         // buffer entries per query
     constexpr int U = S <= 16 ? 2 : 1;       // points per lane per step
     constexpr int STEP = S * U;              // points per query per step
     constexpr int ROWS = (CAP + S - 1) / S;  // buffer entries per lane
-    constexpr bool F32 = PREC == OCT_PREC_FP32_RECHECK;
     constexpr bool kRank = KC <= 32;         // final order by counting ranks, else by a bitonic sort in LDS
     static_assert(CAP - STEP >= KC, "a step must fit after a selection");
     __shared__ uint64_t s_bd[G * CAP];
@@ -149,22 +147,26 @@ __device__ __attribute__((always_inline)) inline void knn_tile(const KnnArgs &a,
     auto dbits = [](double d) -> uint64_t { return (uint64_t)__double_as_longlong(d); };
     auto key_value = [](uint32_t key) -> double { return __longlong_as_double((long long)((uint64_t)key << 32)); };
 
-    const uint32_t kw = k + (k >> 2) + 2 < (uint32_t)(CAP - STEP) ? k + (k >> 2) + 2 : (uint32_t)(CAP - STEP);
+    // a selection stops at k .. kw entries (an eighth more than k; a size class's own size where that bound
+    // lies in between, so that the final sort stays at that size). k + k / 4 was 1 - 10 % slower.
+    uint32_t kw = k + (k >> 3) + 1;
+    if (kw > (uint32_t)KC && k < (uint32_t)KC) kw = KC;
     constexpr uint32_t kFresh = KC / 2 > 8 ? KC / 2 : 8;  // appended entries that are worth a new bound
     uint32_t cnt = 0, kept = 0;   // entries in the buffer; of them, after the last selection
     uint32_t T = 0xffffffffu;     // entries have upper distance bits <= T; ~0: fewer than k seen
     double tau = __builtin_huge_val();      // FP64 upper bound of the k-th distance with the pruning margin
     float tauf = __builtin_huge_valf();     // the same rounded up to FP32
-    uint32_t n_nodes = 0, n_test = 0, n_recheck = 0, n_select = 0, n_steps = 0;
+    uint32_t n_nodes = 0, n_test = 0, n_select = 0, n_steps = 0;
 
     // rank of entry (d, i) among the group's cnt entries, for every row of the buffer; entries of rank
     // below `keep` move to their rank. Afterwards the first `keep` entries are sorted.
-    auto rank_sort = [&](const uint32_t keep) {
+    auto rank_sort = [&](auto rows, const uint32_t keep) {
+        constexpr int R = decltype(rows)::value;
         wsync();
-        uint64_t d[ROWS];
-        uint32_t ix[ROWS], rk[ROWS];
+        uint64_t d[R];
+        uint32_t ix[R], rk[R];
 #pragma unroll
-        for (int j = 0; j < ROWS; j++) {
+        for (int j = 0; j < R; j++) {
             const uint32_t t = j * S + c;
             d[j] = t < cnt ? bd[t] : ~0ull, ix[j] = t < cnt ? bi[t] : 0xffffffffu, rk[j] = 0;
         }
@@ -173,30 +175,57 @@ __device__ __attribute__((always_inline)) inline void knn_tile(const KnnArgs &a,
             const uint64_t dt = in ? bd[t] : ~0ull;
             const uint32_t it = in ? bi[t] : 0xffffffffu;
 #pragma unroll
-            for (int j = 0; j < ROWS; j++) rk[j] += knn_less(dt, it, d[j], ix[j]) ? 1u : 0u;
+            for (int j = 0; j < R; j++) rk[j] += knn_less(dt, it, d[j], ix[j]) ? 1u : 0u;
         }
         wsync();
 #pragma unroll
-        for (int j = 0; j < ROWS; j++)
+        for (int j = 0; j < R; j++)
             if ((uint32_t)(j * S) + c < cnt && rk[j] < keep) bd[rk[j]] = d[j], bi[rk[j]] = ix[j];
         wsync();
     };
-    // bitonic sort of the buffer's first n entries (n a power of two) by (distance, index)
+    // bitonic sort of the buffer's first n entries (n a power of two) by (distance, index), two stages per
+    // LDS round trip: a lane takes the 4 entries that strides s and s / 2 connect through both
+    auto cx = [](uint64_t &da, uint32_t &ia, uint64_t &db, uint32_t &ib, const bool up) {
+        const bool sw = up ? knn_less(db, ib, da, ia) : knn_less(da, ia, db, ib);
+        const uint64_t d = sw ? db : da;
+        const uint32_t i = sw ? ib : ia;
+        db = sw ? da : db, ib = sw ? ia : ib;
+        da = d, ia = i;
+    };
     auto bitonic = [&](const uint32_t n) {
         for (uint32_t t = cnt + c; t < n; t += S) bd[t] = ~0ull, bi[t] = 0xffffffffu;
         wsync();
 #pragma unroll 1
         for (uint32_t size = 2; size <= n; size <<= 1) {
+            uint32_t stride = size >> 1;
 #pragma unroll 1
-            for (uint32_t stride = size >> 1; stride > 0; stride >>= 1) {
+            for (; stride >= 2; stride >>= 2) {
+                const uint32_t h = stride >> 1;
+#pragma unroll 1
+                for (uint32_t t = c; t < n / 4; t += S) {
+                    const uint32_t e0 = ((t & ~(h - 1)) << 2) | (t & (h - 1));
+                    const uint32_t e1 = e0 + h, e2 = e0 + stride, e3 = e2 + h;
+                    const bool up = (e0 & size) == 0;
+                    uint64_t d0 = bd[e0], d1 = bd[e1], d2 = bd[e2], d3 = bd[e3];
+                    uint32_t i0 = bi[e0], i1 = bi[e1], i2 = bi[e2], i3 = bi[e3];
+                    cx(d0, i0, d2, i2, up);
+                    cx(d1, i1, d3, i3, up);
+                    cx(d0, i0, d1, i1, up);
+                    cx(d2, i2, d3, i3, up);
+                    bd[e0] = d0, bd[e1] = d1, bd[e2] = d2, bd[e3] = d3;
+                    bi[e0] = i0, bi[e1] = i1, bi[e2] = i2, bi[e3] = i3;
+                }
+                wsync();
+            }
+            if (stride == 1) {  // an odd number of stages: the last one alone
 #pragma unroll 1
                 for (uint32_t t = c; t < n / 2; t += S) {
-                    const uint32_t e0 = ((t & ~(stride - 1)) << 1) | (t & (stride - 1)), e1 = e0 + stride;
-                    const uint64_t d0 = bd[e0], d1 = bd[e1];
-                    const uint32_t i0 = bi[e0], i1 = bi[e1];
-                    const bool up = (e0 & size) == 0;
-                    if (up ? knn_less(d1, i1, d0, i0) : knn_less(d0, i0, d1, i1))
-                        bd[e0] = d1, bi[e0] = i1, bd[e1] = d0, bi[e1] = i0;
+                    const uint32_t e0 = t << 1;
+                    uint64_t d0 = bd[e0], d1 = bd[e0 + 1];
+                    uint32_t i0 = bi[e0], i1 = bi[e0 + 1];
+                    cx(d0, i0, d1, i1, (e0 & size) == 0);
+                    bd[e0] = d0, bd[e0 + 1] = d1;
+                    bi[e0] = i0, bi[e0 + 1] = i1;
                 }
                 wsync();
             }
@@ -205,7 +234,11 @@ __device__ __attribute__((always_inline)) inline void knn_tile(const KnnArgs &a,
     // the buffer's entries in order, the first min(cnt, k) of them exact (every lane of the wave)
     auto order_entries = [&]() {
         if (kRank) {
-            rank_sort(k);
+            constexpr int kFew = (KC + KC / 8 + 1 + S - 1) / S;  // rows that hold kw entries
+            if (ballot64(cnt > (uint32_t)(kFew * S)))
+                rank_sort(std::integral_constant<int, ROWS>(), k);
+            else
+                rank_sort(std::integral_constant<int, kFew>(), k);
         } else {
             uint32_t mx = group_reduce<64>(cnt, [](uint32_t x, uint32_t y) { return x > y ? x : y; });
             uint32_t n = 64;
@@ -300,75 +333,10 @@ __device__ __attribute__((always_inline)) inline void knn_tile(const KnnArgs &a,
         cnt += gcount(m);
     };
 
-    // tests every group's leaf (need: the group has one)
-    auto leaf = [&](const bool need, const uint32_t node) {
-        uint32_t i = 0, e = 0;
-        float m2x = 0.f, m2y = 0.f, m2z = 0.f, bb = 0.f, hw = 0.f;
-        bool force = false;
-        if (need) {
-            const NodeRec nr = a.nodes[node];
-            i = nr.first, e = nr.last;
-            if (F32) {
-                const float amx = a.amax[node];
-                const float bx = (float)(qx - nr.cx), by = (float)(qy - nr.cy), bz = (float)(qz - nr.cz);
-                bb = bx * bx + by * by + bz * bz;
-                const float s = amx + bb;
-                force = !(s < 1e30f);
-                hw = s * 0x1p-18f;
-                m2x = -2.0f * bx, m2y = -2.0f * by, m2z = -2.0f * bz;
-            }
-            if (c == 0) n_nodes++;
-        }
-        float thr = 0.0f;
-        bool stale = true;
-        while (ballot64(i < e)) {
-            if (ballot64(i < e && cnt + STEP > (uint32_t)CAP)) select(), stale = true;
-            n_steps++;
-            if (F32 && stale) {
-                thr = T == 0xffffffffu || force ? __builtin_huge_valf() : (tauf + hw) * (1.0f + 0x1p-20f);
-                stale = false;
-            }
-            bool acc[U];
-            uint64_t d[U];
-#pragma unroll
-            for (int u = 0; u < U; u++) {
-                const uint32_t id = i + (uint32_t)(u * S) + c;
-                acc[u] = id < e;
-                d[u] = 0;
-                if (F32) {
-                    float ev = 0.0f;
-                    if (i < e) {  // reads up to 2 S - 1 points past the range: the sorted clouds are padded
-                        const float4 p = a.p32[id];
-                        ev = __builtin_fmaf(p.x, m2x, __builtin_fmaf(p.y, m2y, __builtin_fmaf(p.z, m2z, p.w + bb)));
-                    }
-                    acc[u] = acc[u] & !(ev > thr);
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < U; u++) {
-                const uint32_t id = i + (uint32_t)(u * S) + c;
-                if (acc[u]) {
-                    const double4 p = a.p64[id];
-                    const double dx = qx - p.x, dy = qy - p.y, dz = qz - p.z;
-                    d[u] = dbits(dx * dx + dy * dy + dz * dz);
-                    acc[u] = hi32(d[u]) <= T;
-                    if (F32) n_recheck++;
-                }
-                if (id < e) n_test++;
-            }
-#pragma unroll
-            for (int u = 0; u < U; u++) append(acc[u], d[u], i + (uint32_t)(u * S) + c);
-            i = i < e ? i + STEP : i;
-        }
-        // a first bound as soon as k points are known, a new one when enough points came in
-        if (ballot64(cnt >= k && k > 0 && (T == 0xffffffffu || cnt - kept >= kFresh))) select();
-    };
-
     // levels with waiting children (the same in the group's lanes); levels at which this lane's child waits
     uint32_t lvl = 0, pend = 0;
     bool overflow = false;
-    uint32_t at = 0;      // the group's leaf
-    bool have = false;
+    uint32_t i = 0, e = 0;  // the group's leaf: points left to test
     wsync();
     auto judge = [&](const bool act, const uint32_t fc, const uint32_t L) {
         // children fc .. fc + 7 (level L) of a node of the group's query, one per lane c < 8
@@ -399,41 +367,74 @@ __device__ __attribute__((always_inline)) inline void knn_tile(const KnnArgs &a,
     {
         const uint32_t c0 = uniform_u32(a.child[root]);
         if (c0 == 0) {
-            have = valid, at = root;
+            if (valid) i = a.nodes[root].first, e = a.nodes[root].last, n_nodes += c == 0 ? 1u : 0u;
         } else {
             judge(valid, c0, 1);
             if (c == 0 && valid) n_nodes += 8;
         }
     }
     for (;;) {
-        for (;;) {  // every group without a leaf takes its nearest waiting child
-            const bool go = !have && lvl != 0;
-            if (!ballot64(go)) break;
+        // Groups without points take their nearest waiting child until three quarters of the groups that go on
+        // have points; then those test them until more groups wait than test. (Every group until all had a leaf,
+        // and until all were done with it: 72 pops and 44 steps per wave at k = 10 on the tile.)
+        for (;;) {
+            const bool go = i >= e && lvl != 0;
+            const uint64_t wait = ballot64(go);
+            if (!wait || __popcll(ballot64(i < e)) >= 3 * __popcll(wait)) break;
             wsync();
             const uint32_t L = go ? 31u - (uint32_t)__clz(lvl) : 0u;
             const bool mine = go && ((pend >> L) & 1u);
             uint32_t key = mine ? ((uint32_t)lev.key[(L * G + qs) * 8 + (c & 7u)] << 16) | c : 0xffffffffu;
             key = group_reduce<S>(key, [](uint32_t x, uint32_t y) { return x < y ? x : y; });
-            const float lb = __uint_as_float(key & 0xffff0000u);
-            const bool none = key == 0xffffffffu || lb > tauf;  // nothing waits at L, or all of it is too far
-            if (go && none) lvl &= ~(1u << L), pend &= ~(1u << L);
+            const bool far = __uint_as_float(key & 0xffff0000u) > tauf;  // and so are the others of the level
             const uint32_t oct = key & 7u;
-            const bool take = go && !none;
+            const bool take = go && !far;
             const uint32_t ent = take ? lev.node[(L * G + qs) * 8 + oct] : 0u;
-            if (take && c == oct) pend &= ~(1u << L);
+            if (mine && (far || c == oct)) pend &= ~(1u << L);
+            if (go && !gmask(ballot64(mine && !far && c != oct))) lvl &= ~(1u << L);  // nothing waits at L any more
             const bool lf = take && (ent & kKnnLeafBit) != 0;
-            if (lf) have = true, at = ent & ~kKnnLeafBit;
+            if (lf) {
+                const NodeRec &nr = a.nodes[ent & ~kKnnLeafBit];
+                i = nr.first, e = nr.last;
+                n_nodes += c == 0 ? 1u : 0u;
+            }
             const bool down = take && !lf;
             if (ballot64(down)) {
-                if (down && c == 0) n_nodes += 8;
+                n_nodes += down && c == 0 ? 8u : 0u;
                 judge(down, ent, L + 1);
             }
         }
-        if (!ballot64(have)) break;  // every traversal is done
-        leaf(have, at);
-        have = false;
+        // leaf points, STEP at a time; selections in between: a first bound as soon as k points are known, a
+        // new one when enough points came in or no step's points fit, and one at the end
+        const bool last = ballot64(i < e) == 0;  // every traversal is done
+        for (;;) {
+            const bool full = i < e ? cnt + STEP > (uint32_t)CAP
+                                    : (last ? cnt > kw : cnt >= k && (T == 0xffffffffu || cnt - kept >= kFresh));
+            if (ballot64(full)) select();
+            const uint64_t test = ballot64(i < e);
+            if (!test || __popcll(ballot64(i >= e && lvl != 0)) > __popcll(test)) break;
+            n_steps++;
+            bool acc[U];
+            uint64_t d[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const uint32_t id = i + (uint32_t)(u * S) + c;
+                acc[u] = id < e;
+                d[u] = 0;
+                if (i < e) {  // reads up to 2 S - 1 points past the range: the sorted clouds are padded
+                    const double4 p = a.p64[id];
+                    const double dx = qx - p.x, dy = qy - p.y, dz = qz - p.z;
+                    d[u] = dbits(dx * dx + dy * dy + dz * dz);
+                    n_test += acc[u] ? 1u : 0u;
+                    acc[u] = acc[u] & (hi32(d[u]) <= T);
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++) append(acc[u], d[u], i + (uint32_t)(u * S) + c);
+            i = i < e ? i + STEP : i;
+        }
+        if (last) break;
     }
-    if (ballot64(cnt > kw)) select();
     order_entries();
     if (ballot64(overflow) && lane == 0) atomicOr(a.err, kErrStack);
 
@@ -449,17 +450,15 @@ __device__ __attribute__((always_inline)) inline void knn_tile(const KnnArgs &a,
         }
     }
     if (a.stats) {
-        uint64_t found = (valid && c == 0) ? cnt : 0, sn = n_nodes, st = n_test, sr = n_recheck;
+        uint64_t found = (valid && c == 0) ? cnt : 0, sn = n_nodes, st = n_test;
         for (int off = 32; off > 0; off >>= 1) {
             sn += __shfl_xor(sn, off);
             st += __shfl_xor(st, off);
-            sr += __shfl_xor(sr, off);
             found += __shfl_xor(found, off);
         }
         if (lane == 0) {
             atomicAdd(&a.stats[0], (unsigned long long)sn);
             atomicAdd(&a.stats[1], (unsigned long long)st);
-            atomicAdd(&a.stats[2], (unsigned long long)sr);
             atomicAdd(&a.stats[3], (unsigned long long)found);
             atomicAdd(&a.stats[4], (unsigned long long)n_select);  // wave-wide selections
             atomicAdd(&a.stats[5], (unsigned long long)n_steps);   // wave-wide leaf steps
@@ -478,15 +477,15 @@ __device__ inline KnnLevels knn_levels(const KnnArgs &a) {
     return KnnLevels{s_lev, reinterpret_cast<uint16_t *>(s_lev + (size_t)a.levels * (64 / S) * 8)};
 }
 
-template <int S, int KC, int PREC>
+template <int S, int KC>
 __global__ __launch_bounds__(64) void k_knn(const KnnArgs a) {
-    knn_tile<S, KC, PREC>(a, blockIdx.x, knn_levels<S>(a));
+    knn_tile<S, KC>(a, blockIdx.x, knn_levels<S>(a));
 }
 
 // Work-queue form (batches): a grid of resident waves; each takes the next wave tile from a device
 // counter (queue_next) until the device-resident tile count (queue_tiles) is reached. Every wave
 // leaves once the counter has passed the count.
-template <int S, int KC, int PREC>
+template <int S, int KC>
 __global__ __launch_bounds__(64) void k_knn_queue(const KnnArgs a) {
     const uint32_t ntiles = uniform_u32(*a.queue_tiles);
     for (;;) {
@@ -494,37 +493,31 @@ __global__ __launch_bounds__(64) void k_knn_queue(const KnnArgs a) {
         if (lane_id() == 0) t = atomicAdd(a.queue_next, 1u);
         t = readlane_u32(t, 0);
         if (t >= ntiles) return;
-        knn_tile<S, KC, PREC>(a, t, knn_levels<S>(a));
+        knn_tile<S, KC>(a, t, knn_levels<S>(a));
     }
 }
 
-template <int S, int KC, int PREC>
+template <int S, int KC>
 static unsigned knn_queue_grid() {
     static unsigned cached = 0;
     if (cached) return cached;
     int dev = 0, cus = 0, per = 0;
     (void)hipGetDevice(&dev);
     (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-    (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k_knn_queue<S, KC, PREC>, 64, knn_lds<S>(kMaxDepth + 1));
+    (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k_knn_queue<S, KC>, 64, knn_lds<S>(kMaxDepth + 1));
     cached = (unsigned)((cus > 0 ? cus : 256) * (per > 0 ? per : 1));
     return cached;
 }
 
 template <int S, int KC>
-static void launch_sk(const KnnArgs &a, int precision, hipStream_t s) {
+static void launch_sk(const KnnArgs &a, hipStream_t s) {
     const size_t lds = knn_lds<S>(a.levels);
     if (a.queue_next) {
-        if (precision == OCT_PREC_FP32_RECHECK)
-            k_knn_queue<S, KC, OCT_PREC_FP32_RECHECK><<<knn_queue_grid<S, KC, OCT_PREC_FP32_RECHECK>(), 64, lds, s>>>(a);
-        else
-            k_knn_queue<S, KC, OCT_PREC_FP64><<<knn_queue_grid<S, KC, OCT_PREC_FP64>(), 64, lds, s>>>(a);
+        k_knn_queue<S, KC><<<knn_queue_grid<S, KC>(), 64, lds, s>>>(a);
         return;
     }
     const unsigned nb = (unsigned)(((size_t)a.nq + (64 / S) - 1) / (64 / S));
-    if (precision == OCT_PREC_FP32_RECHECK)
-        k_knn<S, KC, OCT_PREC_FP32_RECHECK><<<nb, 64, lds, s>>>(a);
-    else
-        k_knn<S, KC, OCT_PREC_FP64><<<nb, 64, lds, s>>>(a);
+    k_knn<S, KC><<<nb, 64, lds, s>>>(a);
 }
 
 // buffer size class of k (entries per query kept between selections)
@@ -556,10 +549,10 @@ int knn_shape_lanes(uint32_t k, int lanes) {
     return lanes == 64 ? 64 : 0;
 }
 
-static bool launch_knn_shape(const KnnArgs &a, int kc, int precision, int lanes, hipStream_t s) {
+static bool launch_knn_shape(const KnnArgs &a, int kc, int lanes, hipStream_t s) {
 #define OCT_KNN_CASE(KCV, SV)                     \
     if (kc == KCV && lanes == SV) {               \
-        launch_sk<SV, KCV>(a, precision, s);      \
+        launch_sk<SV, KCV>(a, s);                 \
         return true;                              \
     }
     OCT_KNN_CASE(16, 8) OCT_KNN_CASE(32, 8)
@@ -574,7 +567,6 @@ static bool launch_knn_shape(const KnnArgs &a, int kc, int precision, int lanes,
 hipError_t launch_knn(oct_ctx *ctx, const KnnLaunch &L, std::string &err) {
     const size_t nq = L.nq;
     const uint32_t k = L.k;
-    const int precision = L.precision;
     if (k > 1024) {
         err = "knn: k above 1024 is not supported";
         return hipErrorInvalidValue;
@@ -586,8 +578,6 @@ hipError_t launch_knn(oct_ctx *ctx, const KnnLaunch &L, std::string &err) {
     if (nq == 0 || k == 0) return hipSuccess;
     KnnArgs a;
     a.p64 = ctx->p64.p;
-    a.p32 = ctx->p32.p;
-    a.amax = ctx->amax.p;
     a.nodes = ctx->nodes.p;
     a.child = ctx->child.p;
     a.order = L.order;
@@ -617,7 +607,7 @@ hipError_t launch_knn(oct_ctx *ctx, const KnnLaunch &L, std::string &err) {
     // rows of waiting children: levels 1 .. the deepest (a forest's depth is known on the device only)
     a.levels = L.roots ? kMaxDepth + 1 : (ctx->n_levels > 1 ? ctx->n_levels : 1u);
     stage_begin(ctx, ST_KNN);
-    if (!launch_knn_shape(a, knn_kc(kcls), precision, lanes, ctx->stream)) {
+    if (!launch_knn_shape(a, knn_kc(kcls), lanes, ctx->stream)) {
         err = "knn: lanes per query not offered for this k";
         return hipErrorInvalidValue;
     }
