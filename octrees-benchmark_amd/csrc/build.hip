@@ -102,34 +102,24 @@ __global__ __launch_bounds__(256) void k_node_ext(const NodeRec *__restrict__ no
 
 // ---- device-driven level loop: no host round trip between levels
 //
-// Each level is two launches that take the level's node range [ls, le) from ctl[l] (written by the
-// level above): k_level_scan ranks the split flags of 2048-node tiles with a chained scan (dynamic
-// tile ids, decoupled look-back in which one wave reads 64 predecessor tiles per step, bounded spins),
-// points every node at its first child (0 = leaf) and, in its last tile, writes ctl[l + 1];
-// k_level_children then builds the children of the split nodes, 8 lanes per node over a grid-stride
-// loop that fills the device (as k_children). Levels past the last one find an empty range and
-// return, so the host enqueues a batch of levels and reads the level table back once. The node
-// arrays are sized up front; a level that would outgrow them raises an error bit, and the host then
-// runs the level loop with growing arrays instead.
-constexpr uint32_t kLvlPer = 8, kLvlTile = 256 * kLvlPer;
+// Each level is one launch that takes the level's node range [ls, le) from ctl[l] (written by the level
+// above). k_level_step walks the level in tiles of 256 nodes (dynamic tile ids): it ranks a tile's split
+// flags with ballots, takes the tile's offset from a chained scan over the tiles (decoupled look-back in
+// which one wave reads 64 predecessor tiles per step, bounded spins), points every node at its first
+// child (0 = leaf) and builds the children of the split nodes, 8 lanes per node; the last tile writes
+// ctl[l + 1]. Levels past the last one find an empty range and return (about 2.5 us each), so the host
+// enqueues all of them and reads the level table back once. The node arrays are sized up front; a level
+// that would outgrow them raises an error bit, and the host then runs the level loop with growing arrays
+// instead. Two launches per level for the first 13 levels, and the host loop for anything deeper, took
+// 0.9 ms of a 120 k-point frame whose duplicates reach below level 12.
+constexpr uint32_t kLvlTile = 256;
 constexpr uint32_t kLvlAgg = 1u << 30, kLvlInc = 2u << 30, kLvlMask = (1u << 30) - 1u, kLvlSpin = 1u << 24;
 constexpr uint32_t kLvlErrSpin = 1u, kLvlErrCap = 2u;
 constexpr int kLvlCount = kMaxDepth + 1;  // levels 0 .. 21 (level 21 nodes never split)
-constexpr int kLvlFirstBatch = 13;        // levels enqueued before the first read-back (depth <= 12)
 
 struct LevelCtl {
     uint32_t ls, le;
 };
-
-__device__ inline uint32_t lvl_wave_incl_scan(uint32_t v) {
-    const uint32_t l = lane_id();
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        const uint32_t o = __shfl_up(v, off);
-        if (l >= (uint32_t)off) v += o;
-    }
-    return v;
-}
 
 // root, level table (level 0 = the root, every other level empty until its parent level fills it),
 // zero look-back words, tile counters and error word
@@ -150,37 +140,37 @@ __global__ __launch_bounds__(256) void k_level_init(NodeRec *nodes, uint64_t *nk
     }
 }
 
-__global__ __launch_bounds__(256) void k_level_scan(const uint32_t *__restrict__ flags, uint32_t *__restrict__ child,
-                                                    LevelCtl *__restrict__ ctl, uint32_t level, uint32_t *__restrict__ lookback,
-                                                    uint32_t *__restrict__ tile_counter, uint32_t cap, uint32_t *__restrict__ err,
+__global__ __launch_bounds__(256) void k_level_step(const uint64_t *__restrict__ keys, NodeRec *__restrict__ nodes,
+                                                    uint64_t *__restrict__ nkey, uint32_t *__restrict__ child,
+                                                    uint32_t *__restrict__ flags, LevelCtl *__restrict__ ctl, uint32_t level,
+                                                    uint32_t *__restrict__ lookback, uint32_t *__restrict__ tile_counter,
+                                                    uint32_t cap, uint32_t max_leaf, BuildGeom g, uint32_t *__restrict__ err,
                                                     uint32_t *__restrict__ total) {
-    __shared__ uint32_t s_wsum[4], s_tile, s_prefix;
+    __shared__ uint32_t s_w[4], s_tile, s_prefix, s_u[kLvlTile];
     const LevelCtl L = ctl[level];
     if (L.le <= L.ls) return;
     const uint32_t ntiles = (L.le - L.ls + kLvlTile - 1) / kLvlTile;
     const uint32_t tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const uint32_t cl = level + 1, k = tid & 7u;
+    const uint64_t step = node_range(cl);
     for (;;) {
         if (tid == 0) s_tile = atomicAdd(tile_counter, 1u);
         __syncthreads();
         const uint32_t tile = s_tile;
         if (tile >= ntiles) break;
-        const uint32_t b0 = L.ls + tile * kLvlTile + tid * kLvlPer;  // this thread's nodes b0 .. b0 + 7
-        uint32_t f[kLvlPer], sum = 0;
-#pragma unroll
-        for (uint32_t i = 0; i < kLvlPer; i++) {
-            f[i] = b0 + i < L.le ? flags[b0 + i] : 0u;
-            sum += f[i];
-        }
-        const uint32_t incl = lvl_wave_incl_scan(sum);
-        if (lane == 63) s_wsum[w] = incl;
+        const uint32_t u = L.ls + tile * kLvlTile + tid;
+        const bool f = u < L.le && flags[u] != 0;
+        const uint64_t m = ballot64(f);
+        if (lane == 0) s_w[w] = (uint32_t)__popcll(m);
         __syncthreads();
-        uint32_t pre = 0, tot = 0;
+        uint32_t j = (uint32_t)__popcll(m & lanemask_lt()), tot = 0;  // rank of the node in the tile; split nodes
 #pragma unroll
         for (uint32_t ww = 0; ww < 4; ww++) {
-            const uint32_t x = s_wsum[ww];
-            pre += ww < w ? x : 0u;
+            const uint32_t x = s_w[ww];
+            j += ww < w ? x : 0u;
             tot += x;
         }
+        if (f) s_u[j] = u;
         if (w == 0) {  // chained scan over the tiles: wave 0 looks back 64 tiles per step
             uint32_t excl = 0;
             if (tile == 0) {
@@ -217,51 +207,38 @@ __global__ __launch_bounds__(256) void k_level_scan(const uint32_t *__restrict__
                 if (tile == ntiles - 1) {  // the level's split count: the next level's range
                     const uint64_t nle = (uint64_t)L.le + 8ull * (excl + tot);
                     if (nle <= cap) {
-                        ctl[level + 1] = LevelCtl{L.le, (uint32_t)nle};
+                        ctl[cl] = LevelCtl{L.le, (uint32_t)nle};
+                        // no node splits, or the children are the deepest level's: the tree is complete
+                        if (excl + tot == 0 || cl == kMaxDepth) *total = (uint32_t)nle;
                     } else {
-                        ctl[level + 1] = LevelCtl{L.le, L.le};
+                        ctl[cl] = LevelCtl{L.le, L.le};
                         atomicOr(err, kLvlErrCap);
                     }
-                    if (excl + tot == 0) *total = L.le;  // no node splits: the tree is complete
                 }
             }
         }
         __syncthreads();
-        uint32_t r = s_prefix + pre + incl - sum;  // rank of this thread's first split node in the level
-#pragma unroll
-        for (uint32_t i = 0; i < kLvlPer; i++) {
-            if (b0 + i < L.le) child[b0 + i] = f[i] ? L.le + 8u * r : 0u;
-            r += f[i];
+        const uint32_t prefix = s_prefix;
+        if (u < L.le) child[u] = f ? L.le + 8u * (prefix + j) : 0u;
+        // the tile's split nodes, 8 lanes each: lane k finds child k's end and takes its start from lane k - 1
+        // (a search over the whole parent range finds the same index as one from the child's start)
+        for (uint32_t q = tid >> 3; q < tot; q += kLvlTile / 8) {
+            const uint32_t pu = s_u[q];
+            const uint64_t cb = (uint64_t)L.le + 8ull * (prefix + q);
+            if (cb + 8u > cap) {  // the node's 8 lanes move together
+                if (k == 0) atomicOr(err, kLvlErrCap);
+                continue;
+            }
+            const NodeRec pr = nodes[pu];
+            const uint64_t pkey = nkey[pu];
+            const uint32_t hi = (k == 7) ? pr.last : lower_bound_keys(keys, pr.first, pr.last, pkey + (uint64_t)(k + 1) * step);
+            const uint32_t prev = __shfl_up(hi, 1, 8);
+            const uint32_t lo = (k == 0) ? pr.first : prev;
+            write_node(nodes, nkey, (uint32_t)cb + k, pkey + (uint64_t)k * step, cl, lo, hi, g);
+            flags[cb + k] = (hi - lo > max_leaf && cl < kMaxDepth) ? 1u : 0u;
+            if (cl == kMaxDepth) child[cb + k] = 0u;  // no step visits the deepest level
         }
-        __syncthreads();
-    }
-}
-
-__global__ __launch_bounds__(256) void k_level_children(const uint64_t *__restrict__ keys, NodeRec *__restrict__ nodes,
-                                                        uint64_t *__restrict__ nkey, const uint32_t *__restrict__ child,
-                                                        uint32_t *__restrict__ flags, const LevelCtl *__restrict__ ctl,
-                                                        uint32_t level, uint32_t cap, uint32_t max_leaf, BuildGeom g,
-                                                        uint32_t *__restrict__ err) {
-    const LevelCtl L = ctl[level];
-    if (L.le <= L.ls || ctl[level + 1].le <= ctl[level + 1].ls) return;  // no node of this level splits
-    const size_t lanes = (size_t)(L.le - L.ls) * 8, stride = (size_t)gridDim.x * blockDim.x;  // stride: a multiple of 8
-    const uint32_t k = threadIdx.x & 7u, cl = level + 1;
-    const uint64_t step = node_range(cl);
-    for (size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x; t < lanes; t += stride) {
-        const uint32_t u = L.ls + (uint32_t)(t >> 3);  // a node's 8 lanes move together
-        const uint32_t cb = child[u];
-        if (cb == 0) continue;
-        if ((uint64_t)cb + 8u > cap) {
-            if (k == 0) atomicOr(err, kLvlErrCap);
-            continue;
-        }
-        const NodeRec pr = nodes[u];
-        const uint64_t pkey = nkey[u];
-        const uint32_t hi = (k == 7) ? pr.last : lower_bound_keys(keys, pr.first, pr.last, pkey + (uint64_t)(k + 1) * step);
-        const uint32_t prev = __shfl_up(hi, 1, 8);
-        const uint32_t lo = (k == 0) ? pr.first : prev;
-        write_node(nodes, nkey, cb + k, pkey + (uint64_t)k * step, cl, lo, hi, g);
-        flags[cb + k] = (hi - lo > max_leaf && cl < kMaxDepth) ? 1u : 0u;
+        __syncthreads();  // the next tile rewrites the shared lists
     }
 }
 
@@ -369,16 +346,14 @@ hipError_t launch_build(oct_ctx *ctx, uint32_t M, std::string &err) {
                                                   counters, errw, totw);
         int cus = 0;
         (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device);
-        const size_t sgrid = (size_t)std::max(1, cus) * 4, cgrid = (size_t)std::max(1, cus) * 8;
-        for (int l = 0; l < kLvlFirstBatch; l++) {
+        const size_t sgrid = (size_t)std::max(1, cus) * 8;
+        for (int l = 0; l < (int)kMaxDepth; l++) {
             // level l holds at most min(8^l, cap) nodes: small grids for the top levels
             const size_t nmax = l < 10 ? std::min<size_t>(cap, 1ull << (3 * l)) : cap;
             const unsigned gs = (unsigned)std::min(sgrid, (nmax + kLvlTile - 1) / kLvlTile);
-            const unsigned gc = (unsigned)std::min(cgrid, (nmax * 8 + 255) / 256);
-            k_level_scan<<<gs, 256, 0, ctx->stream>>>(ctx->flags.p, ctx->child.p, ctl, (uint32_t)l,
-                                                      ctx->lookback.p + (size_t)l * maxtiles, counters + l, (uint32_t)cap, errw, totw);
-            k_level_children<<<gc, 256, 0, ctx->stream>>>(ctx->sorted_keys, ctx->nodes.p, ctx->nkey.p, ctx->child.p, ctx->flags.p,
-                                                          ctl, (uint32_t)l, (uint32_t)cap, M, g, errw);
+            k_level_step<<<gs, 256, 0, ctx->stream>>>(ctx->sorted_keys, ctx->nodes.p, ctx->nkey.p, ctx->child.p, ctx->flags.p, ctl,
+                                                      (uint32_t)l, ctx->lookback.p + (size_t)l * maxtiles, counters + l,
+                                                      (uint32_t)cap, M, g, errw, totw);
         }
         k_recentre_dev<<<(unsigned)((cap * kRecentreLanes + 255) / 256), 256, 0, ctx->stream>>>(
             ctx->p64.p, ctx->nodes.p, ctx->child.p, totw, ctx->p32.p, ctx->amax.p);
@@ -395,10 +370,10 @@ hipError_t launch_build(oct_ctx *ctx, uint32_t M, std::string &err) {
             err = "build: look-back wait exceeded its bound";
             return hipErrorUnknown;
         }
-        // complete within the first levels and the capacity: done (else the host loop below redoes it)
-        if (!(hw[0] & kLvlErrCap) && hc[kLvlFirstBatch].le <= hc[kLvlFirstBatch].ls && hw[1] > 0) {
+        // complete within the capacity: done (else the host loop below redoes it)
+        if (!(hw[0] & kLvlErrCap) && hw[1] > 0) {
             uint32_t D = 0;  // the deepest non-empty level
-            for (int l = 0; l < kLvlFirstBatch; l++)
+            for (int l = 0; l < kLvlCount; l++)
                 if (hc[l].le > hc[l].ls) D = (uint32_t)l;
             const uint32_t n_total = hc[D].le;
             if (n_total != hw[1]) {

@@ -155,6 +155,40 @@ hipError_t resolve_scratch(int device) {
     return e;
 }
 
+// Pinned pages for the contexts' mail: one slab of kMailSlots for the whole process, allocated with the
+// first context (a pinned allocation costs about 0.3 ms, too much for every context) and reused as
+// contexts come and go; contexts beyond it get an allocation of their own.
+constexpr int kMailSlots = 64;
+std::mutex g_mail_mu;
+oct_ctx::Mail *g_mail = nullptr;
+uint64_t g_mail_used = 0;  // one bit per slot
+
+hipError_t mail_acquire(oct_ctx::Mail **out) {
+    std::lock_guard<std::mutex> g(g_mail_mu);
+    if (!g_mail) {
+        const hipError_t e = hipHostMalloc((void **)&g_mail, kMailSlots * sizeof(oct_ctx::Mail), hipHostMallocPortable);
+        if (e != hipSuccess) {
+            g_mail = nullptr;
+            return e;
+        }
+    }
+    if (~g_mail_used) {
+        const int s = __builtin_ctzll(~g_mail_used);
+        g_mail_used |= 1ull << s;
+        *out = g_mail + s;
+        return hipSuccess;
+    }
+    return hipHostMalloc((void **)out, sizeof(oct_ctx::Mail), hipHostMallocPortable);
+}
+void mail_release(oct_ctx::Mail *m) {
+    if (!m) return;
+    std::lock_guard<std::mutex> g(g_mail_mu);
+    if (g_mail && m >= g_mail && m < g_mail + kMailSlots)
+        g_mail_used &= ~(1ull << (m - g_mail));
+    else
+        (void)hipHostFree(m);
+}
+
 __device__ __forceinline__ uint64_t wave_incl_scan(uint64_t x, int lane) {
     for (int d = 1; d < 64; d <<= 1) {
         const uint64_t y = __shfl_up(x, d);
@@ -380,13 +414,13 @@ int oct_create(oct_ctx **out, int device) {
         delete ctx;
         return OCT_ERR_HIP;
     }
-    if (hipHostMalloc((void **)&ctx->mail, sizeof(*ctx->mail), hipHostMallocDefault) != hipSuccess) {
+    if (mail_acquire(&ctx->mail) != hipSuccess) {
         delete ctx;
         return OCT_ERR_HIP;
     }
     if (ctx->derr.reserve(4) != hipSuccess || hipMemset(ctx->derr.p, 0, 4 * sizeof(uint32_t)) != hipSuccess) {
         ctx->derr.release();
-        (void)hipHostFree(ctx->mail);
+        mail_release(ctx->mail);
         delete ctx;
         return OCT_ERR_HIP;
     }
@@ -414,7 +448,7 @@ int oct_destroy(oct_ctx *ctx) {
         if (ctx->ev0[s]) (void)hipEventDestroy(ctx->ev0[s]);
         if (ctx->ev1[s]) (void)hipEventDestroy(ctx->ev1[s]);
     }
-    (void)hipHostFree(ctx->mail);
+    mail_release(ctx->mail);
     (void)hipStreamDestroy(ctx->stream);
     delete ctx;
     return OCT_OK;

@@ -173,7 +173,7 @@ struct oct_ctx {
     int knn_lanes_tuned[2][8];      // autotuned lanes per query per (precision, size class), -1 = not tuned
 
     // small results on their way to the host: a pinned page, written by copies on the stream
-    struct Mail {
+    struct alignas(128) Mail {
         unsigned long long stats[8];
         uint64_t total;
         uint32_t err;
