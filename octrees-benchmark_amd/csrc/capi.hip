@@ -683,9 +683,10 @@ static int check_search_args(oct_ctx *ctx, int kernel, int algo, int precision, 
 // 524 k 3.8 / 3.2; one in 32: 524 k 4.8 / 4.8; 40 M box, one in 8: 2.8 / 2.6, one in 32: 3.2 / 4.7.
 constexpr size_t kUnionMinQueries = 1u << 17;
 constexpr double kUnionMinDensity = 1.0 / 16;
+static bool shared_traversal(size_t nq, double density) { return nq > kUnionMinQueries && density >= kUnionMinDensity; }
 static int radius_group(const oct_ctx *ctx, int kernel, int algo, int precision, size_t nq, double density) {
     if (ctx->group_override >= 0) return ctx->group_override;
-    if (nq <= kUnionMinQueries || density < kUnionMinDensity) return 0;
+    if (!shared_traversal(nq, density)) return 0;
     const int t = ctx->group_tuned[kernel & 3][algo & 3][precision & 1];
     return t >= 0 ? t : 64;
 }
@@ -717,7 +718,9 @@ static int radius_impl(oct_ctx *ctx, int kernel, int algo, int precision, const 
         for (size_t i = 0; i < nq; i++)
             if (center_idx[i] >= ctx->n) return fail(ctx, OCT_ERR_ARG, "center index out of range");
     HCHK(hipSetDevice(ctx->device), "set device");
-    const int group = want_lists ? 0 : radius_group(ctx, kernel, algo, precision, nq, query_density(ctx, centers, center_idx, nq));
+    const double density = query_density(ctx, centers, center_idx, nq);
+    const int group = !want_lists ? radius_group(ctx, kernel, algo, precision, nq, density)
+                                  : (algo != OCT_ALGO_APPROX && shared_traversal(nq, density) ? 64 : 0);
     // the group kernel takes queries in any order: sorting them costs the host more than their locality gives
     std::vector<uint32_t> order;
     if (group) query_order(ctx, centers, center_idx, nq, order);
@@ -817,6 +820,7 @@ int oct_radius_lists_noalloc(oct_ctx *ctx, int kernel, int algo, int precision, 
     // sizes: per-query neighbour counts and entry counts (indices, or ranges for Struct)
     RadiusLaunch L;
     L.kernel = kernel, L.algo = algo, L.precision = precision, L.mode = 1;
+    L.group = shared_traversal(nq, 1.0) ? 64 : 0;  // the indices' spread is not known here
     L.qidx = center_idx_dev;
     L.radius = radius;
     L.nq = nq;

@@ -33,7 +33,8 @@ struct alignas(64) NodeExt {
     uint32_t first[8];  // combo c: point range [first, last)
     uint32_t last[8];
     uint32_t gc[8];     // combo c: its first child, 0 = leaf
-    uint32_t pad[4];
+    uint32_t order[2];  // byte o: the combo of octant o (the o-th child in key order)
+    uint32_t pad[2];
 };
 static_assert(sizeof(NodeExt) == 192, "NodeExt is three 64-byte lines");
 
@@ -202,7 +203,7 @@ hipError_t launch_build(oct_ctx *ctx, uint32_t max_points_leaf, std::string &err
 // centre is qxyz[id] if given, else the sorted point qidx[id] (or id); outputs are indexed by id.
 struct RadiusLaunch {
     int kernel = 1, algo = 3, precision = 0, mode = 0;
-    int group = 16;  // count mode: queries per wave (16, 32, 64), or 0 for the group kernel (8 lanes per query)
+    int group = 16;  // queries per wave (16, 32, 64; lists: 64), or 0 for the group kernel (8 lanes per query)
     bool remap = true;  // count mode, vector point tests: compact the queries of sparsely wanted leaves
     uint32_t approx_level = ~0u;  // OCT_ALGO_APPROX: neighborsApprox depth cutoff and bound mode
     bool approx_upper = false;

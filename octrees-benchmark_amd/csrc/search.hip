@@ -381,10 +381,13 @@ constexpr int count_waves() {
     if (ALGO == OCT_ALGO_NEIGHBORS || !(KERNEL == OCT_KERNEL_SPHERE || KERNEL == OCT_KERNEL_CIRCLE)) return 2;
     return PREC == OCT_PREC_FP32_RECHECK ? 7 : 6;
 }
-// One wave tile (G queries) of a count-mode search, run by one wave.
-template <int KERNEL, int ALGO, int PREC, int G, bool STATS>
+// One wave tile (G queries) of a search, run by one wave. MODE 0: neighbour counts. MODE 1 (range lists,
+// G = 64): counts and list-entry counts. MODE 2 (G = 64): the lists, in the reference's emission order.
+template <int KERNEL, int ALGO, int PREC, int G, bool STATS, int MODE = 0>
 __device__ __attribute__((always_inline)) inline void count_tile(const SearchArgs &a, const uint32_t tile) {
     constexpr int S = 64 / G;
+    static_assert(MODE == 0 || G == 64, "lists: one lane per query");
+    constexpr bool kRanges = ALGO == OCT_ALGO_STRUCT || ALGO == OCT_ALGO_APPROX;  // lists of [first, last) ranges
     constexpr bool kFp32 = PREC == OCT_PREC_FP32_RECHECK && (KERNEL == OCT_KERNEL_SPHERE || KERNEL == OCT_KERNEL_CIRCLE);
     // real points per staging chunk: 64 FP32 or 48 FP64 points (leaves average ~30 points; a small
     // chunk keeps the LDS per block low enough for 7 (FP32) or 6 (FP64) waves per SIMD: 19.0 / 26.0 KB
@@ -399,6 +402,8 @@ __device__ __attribute__((always_inline)) inline void count_tile(const SearchArg
     __shared__ uint64_t s_leafm[kWaves][8];  // OVERLAP leaf children of the popped node (query masks)
     __shared__ uint8_t s_rmap[kWaves][64];   // remapped leaf: home slot of compacted query r
     __shared__ uint32_t s_rtot[kWaves][64];  // remapped leaf: count of compacted query r
+    __shared__ uint64_t s_hits[MODE ? kWaves : 1][MODE ? 64 : 1];     // its hits (lists)
+    __shared__ uint64_t s_inm[MODE == 2 ? kWaves : 1][8];             // INSIDE children of the popped node (query masks)
     __shared__ __attribute__((aligned(16))) unsigned char s_stage[kWaves][(CAP + PAD) * (kFp32 ? 16 : 32)];
 
     const uint32_t w = threadIdx.x >> 6;
@@ -440,7 +445,9 @@ __device__ __attribute__((always_inline)) inline void count_tile(const SearchArg
     if (KERNEL == OCT_KERNEL_CUBE || KERNEL == OCT_KERNEL_SQUARE) box_radii(a, valid, qid, q);
     const float qRf = (float)q.R;
 
-    uint32_t cnt = 0;
+    uint32_t cnt = 0, ecnt = 0;
+    uint32_t *out = nullptr;  // MODE 2: the next word of the lane's list
+    if (MODE == 2 && valid) out = a.entries + a.offsets[qid] * (kRanges ? 2u : 1u);
     uint64_t n_class = 0, n_test = 0, n_recheck = 0, n_cslots = 0, n_tslots = 0;
 
     // a value of another lane (ds_bpermute)
@@ -659,6 +666,187 @@ __device__ __attribute__((always_inline)) inline void count_tile(const SearchArg
         if (STATS) n_tslots += 64ull * ((last - first + Sp - 1) / Sp);
     };
 
+    // Lists: a leaf's points are tested as for counts, but each lane collects its hits as a bit mask, 64 points
+    // (48 in FP64) at a time: one shift per test instead of a popcount per four. A remapped leaf's lanes take
+    // contiguous points (a power of two per lane), so their masks are shifted into place and OR-ed over the
+    // lanes of a query. Counts and runs are then popcounts, and a list's words are the set bits of the mask
+    // (indices), or of the mask XOR its neighbour (a run's first point and the one after its last).
+    auto leaf_lists = [&](uint64_t m, float am, const NodeRec &nr) {
+        const uint32_t first = nr.first, last = nr.last;
+        if (STATS) n_test += (uint64_t)__popcll(m) * (last - first);
+        const uint32_t mc = (uint32_t)__popcll(m);
+        const bool rm = a.remap && 2 * mc <= 64;  // wave-uniform
+        const bool act = ((m >> lane) & 1ull) != 0 && valid;  // this lane's query wants the leaf
+        uint32_t lg = 0, lgs = 0, gp = 0, src = lane, rank = 0;
+        bool ract = act;
+        if (rm) {
+            lg = mc <= 4 ? 2u : 32u - (uint32_t)__builtin_clz(mc - 1);
+            lgs = 6u - lg;
+            gp = lane >> lg;
+            const uint32_t r = lane & ((1u << lg) - 1u);
+            rank = (uint32_t)__popcll(m & (qbit - 1ull));
+            if (act) s_rmap[w][rank] = (uint8_t)lane;
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            ract = r < mc;
+            src = ract ? (uint32_t)s_rmap[w][r] : lane;
+        }
+        auto qf = [&](float v) -> float { return rm ? bperm_f32(src, v) : v; };
+        auto qd = [&](double v) -> double { return rm ? bperm_f64(src, v) : v; };
+        auto fetch_query = [&]() {
+            Query qr = q;
+            if (KERNEL == OCT_KERNEL_SPHERE || KERNEL == OCT_KERNEL_CIRCLE) {
+                qr.x = qd(q.x), qr.y = qd(q.y), qr.R = qd(q.R);
+                if (KERNEL == OCT_KERNEL_SPHERE) qr.z = qd(q.z);
+            } else {
+                qr.lox = qd(q.lox), qr.hix = qd(q.hix), qr.loy = qd(q.loy), qr.hiy = qd(q.hiy);
+                if (KERNEL == OCT_KERNEL_CUBE) qr.loz = qd(q.loz), qr.hiz = qd(q.hiz);
+            }
+            return qr;
+        };
+        float C = 0.f, ux = 0.f, uy = 0.f, uz = 0.f;
+        uint32_t lim = 0;
+        Query qr = q;
+        if (kFp32) {  // the count leaf's terms and bound
+            const float bx = (float)(q.x - nr.cx), by = (float)(q.y - nr.cy), bz = (float)(q.z - nr.cz);
+            const float b2 = KERNEL == OCT_KERNEL_SPHERE ? __builtin_fmaf(bx, bx, __builtin_fmaf(by, by, bz * bz))
+                                                         : __builtin_fmaf(bx, bx, by * by);
+            const float sum = (am + b2) + qRf;
+            const float hw = 3.814697265625e-06f * sum;  // 2^-18
+            C = qf((hw - qRf) + b2);
+            lim = __float_as_uint(qf(__uint_as_float(sum < 1e30f ? __float_as_uint(2.0f * hw) : 0xffffffffu)));
+            ux = qf(-2.0f * bx), uy = qf(-2.0f * by);
+            uz = KERNEL == OCT_KERNEL_SPHERE ? qf(-2.0f * bz) : 0.0f;
+        } else {
+            qr = fetch_query();
+        }
+        bool open = false;  // range lists: the lane's current run reaches the chunk's first point
+        for (uint32_t base = first; base < last; base += CAP) {
+            const uint32_t P = (last - base) < (uint32_t)CAP ? (last - base) : (uint32_t)CAP;
+            const uint32_t per = (P + (1u << lgs) - 1) >> lgs;  // points per lane, then a multiple of 4 or a power of two
+            const uint32_t iters = lgs == 0 ? (P + 3u) & ~3u : (per <= 4 ? 4u : per <= 8 ? 8u : per <= 16 ? 16u : 32u);
+            const uint32_t li = 31u - (uint32_t)__builtin_clz(iters);  // lgs > 0: log2(iters)
+            const uint32_t rs = lgs ? iters + 1 : 0u;                  // rows of lane groups, one slot apart in the banks
+            const uint32_t slots = iters << lgs;
+            constexpr int NI = 1;
+            {
+                const uint32_t t = lane;
+                const bool real = t < P;
+                const uint32_t at = lgs ? (t >> li) * rs + (t & (iters - 1)) : t;
+                if (kFp32) {
+                    const float4 v = a.p32[base + min(t, P - 1)];
+                    if (t < slots)
+                        sp32[at] = real ? v
+                                        : (KERNEL == OCT_KERNEL_CIRCLE ? make_float4(1e30f, 1e30f, 0.0f, 0.0f)
+                                                                       : make_float4(0.0f, 0.0f, 0.0f, 1e30f));
+                } else {
+                    const double4 v = a.p64[base + min(t, P - 1)];
+                    if (t < slots) sp64[at] = make_double4(real ? v.x : 1e300, real ? v.y : 1e300, real ? v.z : 1e300, 0.0);
+                }
+            }
+            static_assert(NI == 1 && CAP <= 64, "one load per lane and chunk");
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            uint32_t mnb = 0xffffffffu;
+            // hits of points [k0, k1) of the lane's row, first point in the highest of the k1 - k0 low bits
+            auto hits = [&](const uint32_t k0, const uint32_t k1) -> uint32_t {
+                uint32_t hm = 0;
+                if (kFp32) {
+                    const float4 *pl = sp32 + gp * rs + k0;
+                    for (uint32_t k = k0; k < k1; k += 4, pl += 4) {
+                        const float4 p0 = pl[0], p1 = pl[1], p2 = pl[2], p3 = pl[3];
+                        float t0, t1, t2, t3;
+                        if (KERNEL == OCT_KERNEL_SPHERE) {
+                            t0 = __builtin_fmaf(p0.x, ux, __builtin_fmaf(p0.y, uy, __builtin_fmaf(p0.z, uz, p0.w + C)));
+                            t1 = __builtin_fmaf(p1.x, ux, __builtin_fmaf(p1.y, uy, __builtin_fmaf(p1.z, uz, p1.w + C)));
+                            t2 = __builtin_fmaf(p2.x, ux, __builtin_fmaf(p2.y, uy, __builtin_fmaf(p2.z, uz, p2.w + C)));
+                            t3 = __builtin_fmaf(p3.x, ux, __builtin_fmaf(p3.y, uy, __builtin_fmaf(p3.z, uz, p3.w + C)));
+                        } else {
+                            t0 = __builtin_fmaf(p0.x, p0.x + ux, __builtin_fmaf(p0.y, p0.y + uy, C));
+                            t1 = __builtin_fmaf(p1.x, p1.x + ux, __builtin_fmaf(p1.y, p1.y + uy, C));
+                            t2 = __builtin_fmaf(p2.x, p2.x + ux, __builtin_fmaf(p2.y, p2.y + uy, C));
+                            t3 = __builtin_fmaf(p3.x, p3.x + ux, __builtin_fmaf(p3.y, p3.y + uy, C));
+                        }
+                        const uint32_t d0 = __float_as_uint(t0), d1 = __float_as_uint(t1);
+                        const uint32_t d2 = __float_as_uint(t2), d3 = __float_as_uint(t3);
+                        hm = __builtin_amdgcn_alignbit(hm, d0, 31);  // hm << 1 | sign
+                        hm = __builtin_amdgcn_alignbit(hm, d1, 31);
+                        hm = __builtin_amdgcn_alignbit(hm, d2, 31);
+                        hm = __builtin_amdgcn_alignbit(hm, d3, 31);
+                        mnb = min(min(mnb, d0), d1);
+                        mnb = min(min(mnb, d2), d3);
+                    }
+                } else {
+                    const double4 *pl = sp64 + gp * rs + k0;
+                    for (uint32_t k = k0; k < k1; k += 4, pl += 4) {
+                        const double4 p0 = pl[0], p1 = pl[1], p2 = pl[2], p3 = pl[3];
+                        hm = hm + hm + (inside64<KERNEL>(qr, p0.x, p0.y, p0.z) ? 1u : 0u);
+                        hm = hm + hm + (inside64<KERNEL>(qr, p1.x, p1.y, p1.z) ? 1u : 0u);
+                        hm = hm + hm + (inside64<KERNEL>(qr, p2.x, p2.y, p2.z) ? 1u : 0u);
+                        hm = hm + hm + (inside64<KERNEL>(qr, p3.x, p3.y, p3.z) ? 1u : 0u);
+                    }
+                }
+                return __builtin_bitreverse32(hm) >> ((32u - (k1 - k0)) & 31u);
+            };
+            const uint32_t n0 = iters < 32u ? iters : 32u;
+            uint64_t hm = hits(0, n0);
+            if (iters > 32u) hm |= (uint64_t)hits(32, iters) << 32;
+            if (STATS) n_tslots += 64ull * iters;
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            if (kFp32) {
+                const bool band = ract && mnb <= lim;
+                if (ballot64(band)) {  // rare: exact FP64 decisions for this lane's share of the chunk
+                    const Query qe = fetch_query();
+                    if (band) {
+                        hm = 0;
+                        for (uint32_t k = 0; k < iters && gp * iters + k < P; k++) {
+                            const double4 pd = a.p64[base + gp * iters + k];
+                            hm |= (uint64_t)(inside64<KERNEL>(qe, pd.x, pd.y, pd.z) ? 1u : 0u) << k;
+                            if (STATS) n_recheck++;
+                        }
+                    }
+                }
+            }
+            if (!ract) hm = 0;
+            if (rm) {
+                hm <<= gp * iters;
+                uint32_t hl = (uint32_t)hm, hh = (uint32_t)(hm >> 32);
+                if (lg <= 2) hl |= lane_xor<4>(hl), hh |= lane_xor<4>(hh);
+                if (lg <= 3) hl |= lane_xor<8>(hl), hh |= lane_xor<8>(hh);
+                if (lg <= 4) hl |= lane_xor<16>(hl), hh |= lane_xor<16>(hh);
+                hl |= lane_xor32(hl), hh |= lane_xor32(hh);
+                if (ract && gp == 0) s_hits[w][lane] = ((uint64_t)hh << 32) | hl;
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                hm = act ? s_hits[w][rank] : 0ull;
+            }
+            const uint64_t pm = P == 64 ? ~0ull : (1ull << P) - 1ull;
+            hm &= pm;
+            const uint64_t pr = (hm << 1) | (open ? 1ull : 0ull);
+            if (MODE == 1) {
+                cnt += (uint32_t)__popcll(hm);
+                ecnt += (uint32_t)__popcll(hm & ~pr);
+            } else {
+                const uint64_t words = kRanges ? (hm ^ pr) & pm : hm;
+                uint32_t wl = (uint32_t)words, wh = (uint32_t)(words >> 32);
+                while (wl) {
+                    *out++ = base + (uint32_t)__builtin_ctz(wl);
+                    wl &= wl - 1u;
+                }
+                while (wh) {
+                    *out++ = base + 32u + (uint32_t)__builtin_ctz(wh);
+                    wh &= wh - 1u;
+                }
+            }
+            if (kRanges) open = ((hm >> (P - 1u)) & 1ull) != 0;
+        }
+        if (MODE == 2 && kRanges && open) *out++ = last;  // a run ends with its leaf
+    };
+
     // The 8 children of a popped node are judged from per-axis terms: they take two centre values
     // per axis (NodeExt), so |q - c|, the kernel-box bounds and the squared extents are computed
     // once per axis value and combined per child, in the reference's operation order, e.g. for the
@@ -757,7 +945,15 @@ __device__ __attribute__((always_inline)) inline void count_tile(const SearchArg
         const NodeRec nr = a.nodes[root];
         const int jr = judge(valid, nr, 0);
         if (STATS) n_class += __popcll(ballot64(valid) & gmask), n_cslots += 64;
-        if (g == 0 && jr == J_INSIDE) cnt += nr.last - nr.first;
+        if (g == 0 && jr == J_INSIDE) {
+            cnt += nr.last - nr.first, ecnt++;
+            if (MODE == 2) {
+                if (kRanges)
+                    *out++ = nr.first, *out++ = nr.last;
+                else
+                    for (uint32_t i = nr.first; i < nr.last; i++) *out++ = i;
+            }
+        }
         const uint64_t ov = ballot64(jr == J_OVERLAP) & gmask;
         if (ov) {
             const uint32_t c0 = uniform_u32(a.child[root]);
@@ -765,7 +961,12 @@ __device__ __attribute__((always_inline)) inline void count_tile(const SearchArg
                 NodeRec ur;
                 ur.cx = nr.cx, ur.cy = nr.cy, ur.cz = nr.cz;
                 ur.first = uniform_u32(nr.first), ur.last = uniform_u32(nr.last);
-                if (ur.last > ur.first) leaf(ov, a.amax[root], ur);
+                if (ur.last > ur.first) {
+                    if constexpr (MODE == 0)
+                        leaf(ov, a.amax[root], ur);
+                    else
+                        leaf_lists(ov, a.amax[root], ur);
+                }
             } else {
                 s_node[w][0] = c0, s_mask[w][0] = ov, s_depth[w][0] = 0;
                 sp = 1;
@@ -783,52 +984,112 @@ __device__ __attribute__((always_inline)) inline void count_tile(const SearchArg
         uint64_t inl[8], ovl[8];
         judge8(E, d, actm, inl, ovl);
         if (STATS) n_class += 8ull * __popcll(m), n_cslots += 64ull * 8;
-        // INSIDE children first: group 0's lanes (0 .. G - 1) hold the counts
+        if constexpr (MODE == 2) {
+            // lists: the children in octant order - INSIDE ranges and leaves are emitted, internal nodes wait (popped
+            // last pushed first, as the reference does). ev: combos with an INSIDE or OVERLAP query; an empty
+            // child changes nothing but a range list, which keeps empty INSIDE ranges (neighbor_set.hpp:84-89)
+            uint32_t ev = 0;
 #pragma unroll
-        for (int c = 0; c < 8; c++)
-            if (__builtin_amdgcn_inverse_ballot_w64(inl[c] & gmask)) cnt += E.last[c] - E.first[c];
-        uint32_t leaves = 0;  // combos of the OVERLAP non-empty leaf children (bit c)
-#pragma unroll
-        for (int c = 0; c < 8; c++) {
-            const uint32_t f = E.first[c], l = E.last[c];
-            const uint64_t ov = ovl[c] & gmask;  // ballots: uniform already
-            if (ov) {
-                const uint32_t gc = E.gc[c];
-                if (gc == 0) {
-                    if (l > f) {  // an empty leaf adds nothing to a count
-                        if (lane == 0) s_leafm[w][c] = ov;
-                        leaves |= 1u << c;
-                    }
-                } else if (sp < kStack) {
-                    s_node[w][sp] = gc, s_mask[w][sp] = ov, s_depth[w][sp] = (uint8_t)d;
-                    sp++;
-                } else {
-                    overflow = true;
+            for (int c = 0; c < 8; c++) {
+                const bool some = E.last[c] > E.first[c];
+                const uint64_t im = kRanges || some ? inl[c] : 0ull, om = some ? ovl[c] : 0ull;
+                if (im | om) {
+                    if (lane == 0) s_inm[w][c] = im, s_leafm[w][c] = om;
+                    ev |= 1u << c;
                 }
             }
-        }
-        // the leaves, one code copy: their records are scalar loads from E at a uniform index
-        leaves = uniform_u32(leaves);  // built from ballots: the same in every lane
-        if (leaves) {
+            ev = uniform_u32(ev);
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
             __builtin_amdgcn_wave_barrier();
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        }
-        while (leaves) {
-            const uint32_t c = (uint32_t)__builtin_ctz(leaves);
-            leaves &= leaves - 1;
-            const uint64_t ov = uniform_u64(s_leafm[w][c]);
-            NodeRec ur;
-            ur.cx = E.ax[c & 1], ur.cy = E.ax[2 + ((c >> 1) & 1)], ur.cz = E.ax[4 + ((c >> 2) & 1)];
-            ur.first = E.first[c], ur.last = E.last[c];
-            leaf(ov, E.amax[c], ur);
+#pragma unroll 1
+            for (uint32_t o = 0; o < 8; o++) {
+                const uint32_t c = (E.order[o >> 2] >> (8u * (o & 3u))) & 7u;
+                if (!((ev >> c) & 1u)) continue;
+                const uint64_t im = uniform_u64(s_inm[w][c]), om = uniform_u64(s_leafm[w][c]);
+                const uint32_t f = E.first[c], l = E.last[c];
+                if (__builtin_amdgcn_inverse_ballot_w64(im)) {
+                    if (kRanges) {
+                        out[0] = f, out[1] = l;
+                        out += 2;
+                    } else {
+                        for (uint32_t i = f; i < l; i++) *out++ = i;
+                    }
+                }
+                if (om) {
+                    const uint32_t gc = E.gc[c];
+                    if (gc == 0) {
+                        NodeRec ur;
+                        ur.cx = E.ax[c & 1], ur.cy = E.ax[2 + ((c >> 1) & 1)], ur.cz = E.ax[4 + ((c >> 2) & 1)];
+                        ur.first = f, ur.last = l;
+                        leaf_lists(om, E.amax[c], ur);
+                    } else if (sp < kStack) {
+                        s_node[w][sp] = gc, s_mask[w][sp] = om, s_depth[w][sp] = (uint8_t)d;
+                        sp++;
+                    } else {
+                        overflow = true;
+                    }
+                }
+            }
+        } else {
+            // INSIDE children first: group 0's lanes (0 .. G - 1) hold the counts
+    #pragma unroll
+            for (int c = 0; c < 8; c++)
+                if (__builtin_amdgcn_inverse_ballot_w64(inl[c] & gmask)) {
+                    cnt += E.last[c] - E.first[c];
+                    if (MODE == 1) ecnt++;  // NeighborSet::addRange keeps empty ranges (neighbor_set.hpp:84-89)
+                }
+            uint32_t leaves = 0;  // combos of the OVERLAP non-empty leaf children (bit c)
+    #pragma unroll
+            for (int c = 0; c < 8; c++) {
+                const uint32_t f = E.first[c], l = E.last[c];
+                const uint64_t ov = ovl[c] & gmask;  // ballots: uniform already
+                if (ov) {
+                    const uint32_t gc = E.gc[c];
+                    if (gc == 0) {
+                        if (l > f) {  // an empty leaf adds nothing to a count
+                            if (lane == 0) s_leafm[w][c] = ov;
+                            leaves |= 1u << c;
+                        }
+                    } else if (sp < kStack) {
+                        s_node[w][sp] = gc, s_mask[w][sp] = ov, s_depth[w][sp] = (uint8_t)d;
+                        sp++;
+                    } else {
+                        overflow = true;
+                    }
+                }
+            }
+            // the leaves, one code copy: their records are scalar loads from E at a uniform index
+            leaves = uniform_u32(leaves);  // built from ballots: the same in every lane
+            if (leaves) {
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            }
+            while (leaves) {
+                const uint32_t c = (uint32_t)__builtin_ctz(leaves);
+                leaves &= leaves - 1;
+                const uint64_t ov = uniform_u64(s_leafm[w][c]);
+                NodeRec ur;
+                ur.cx = E.ax[c & 1], ur.cy = E.ax[2 + ((c >> 1) & 1)], ur.cz = E.ax[4 + ((c >> 2) & 1)];
+                ur.first = E.first[c], ur.last = E.last[c];
+                if constexpr (MODE == 0)
+                    leaf(ov, E.amax[c], ur);
+                else
+                    leaf_lists(ov, E.amax[c], ur);
+            }
         }
     }
     // the S lanes of a query hold parts of its count: lanes j, j + G, ... (G >= 16)
     if constexpr (G <= 16) cnt += lane_xor<16>(cnt);
     if constexpr (G <= 32) cnt += lane_xor32(cnt);
     if (overflow && lane == 0) atomicOr(a.err, kErrStack);
-    if (valid && g == 0 && a.counts) a.counts[qid] = cnt;
+    if (MODE != 2 && valid && g == 0) {
+        if (a.counts) a.counts[qid] = cnt;
+        const uint32_t ec = MODE == 1 ? ecnt : cnt;  // index lists: one entry per neighbour
+        if (a.ecounts) a.ecounts[qid] = ec;
+        if (a.ecounts64) a.ecounts64[qid] = ec;
+    }
     if (STATS) {
         if (lane == 0) {
             atomicAdd(&a.stats[0], (unsigned long long)n_class);
@@ -848,6 +1109,12 @@ __device__ __attribute__((always_inline)) inline void count_tile(const SearchArg
 template <int KERNEL, int ALGO, int PREC, int G, bool STATS>
 __global__ __launch_bounds__(kSearchBlock) __attribute__((amdgpu_waves_per_eu(count_waves<KERNEL, ALGO, PREC>()))) void k_count(const SearchArgs a) {
     count_tile<KERNEL, ALGO, PREC, G, STATS>(a, blockIdx.x * kWaves + (threadIdx.x >> 6));
+}
+
+// Sizes (MODE 1, range lists) and fill (MODE 2) of result lists, 64 consecutive queries per wave.
+template <int KERNEL, int ALGO, int PREC, bool STATS, int MODE>
+__global__ __launch_bounds__(kSearchBlock) void k_lists(const SearchArgs a) {
+    count_tile<KERNEL, ALGO, PREC, 64, STATS, MODE>(a, blockIdx.x * kWaves + (threadIdx.x >> 6));
 }
 
 // Work-queue form (batches): a grid of resident waves; each wave takes the next wave tile from a
@@ -918,6 +1185,20 @@ static void launch_k(const SearchArgs &a, int mode, int G, hipStream_t s) {
     if (mode == 0 && G > 0) {
         launch_count<KERNEL, ALGO, PREC>(a, G, s);
         return;
+    }
+    if constexpr (ALGO != OCT_ALGO_APPROX) {
+        if (G > 0) {  // lists of many queries that lie together
+            const unsigned nb = (unsigned)(((size_t)a.nq + 64 * kWaves - 1) / (64 * kWaves));
+            if (mode == 2)
+                k_lists<KERNEL, ALGO, PREC, false, 2><<<nb, kSearchBlock, 0, s>>>(a);
+            else if constexpr (ALGO != OCT_ALGO_STRUCT)
+                launch_count<KERNEL, ALGO, PREC>(a, 64, s);  // an index list is as long as its count
+            else if (a.stats)
+                k_lists<KERNEL, ALGO, PREC, true, 1><<<nb, kSearchBlock, 0, s>>>(a);
+            else
+                k_lists<KERNEL, ALGO, PREC, false, 1><<<nb, kSearchBlock, 0, s>>>(a);
+            return;
+        }
     }
     const unsigned nb = (unsigned)(((size_t)a.nq + kGroupsPerWave * kWaves - 1) / (kGroupsPerWave * kWaves));
     const size_t lds = (size_t)kWaves * a.levels * 64 * sizeof(uint32_t);

@@ -86,7 +86,8 @@ __device__ inline void node_ext_child(const NodeRec *__restrict__ nodes, const u
     e->first[c] = r.first, e->last[c] = r.last;
     e->gc[c] = gc;
     e->amax[c] = gc == 0 ? amax[v] : 0.0f;
-    if (k < 4) e->pad[k] = 0;
+    reinterpret_cast<uint8_t *>(e->order)[k] = (uint8_t)c;
+    if (k < 2) e->pad[k] = 0;
 }
 
 }  // namespace oct

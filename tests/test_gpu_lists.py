@@ -61,3 +61,42 @@ def test_lists_equal_the_oracle(ctx, name, leaf):
                         counts, _ = ctx.radius(kernel, algo, prec, idx=idx, radius=radius)
                         ctx.set_group(-1)
                         assert np.array_equal(counts, sizes), tag
+
+
+def dense_clouds():
+    rng = np.random.default_rng(3)
+    flat = rng.uniform(0, 60, (140_003, 3)) * [1.0, 1.0, 0.02]
+    clump = np.concatenate([rng.normal(0, 0.02, (9_000, 3)) + [3, 3, 3], rng.uniform(0, 12, (131_001, 3))])
+    return {"flat": flat, "clump": clump}
+
+
+@pytest.mark.parametrize("name,leaf,radius", [("flat", 16, 0.4), ("flat", 130, 0.9), ("clump", 5, 0.3), ("clump", 64, 0.7)])
+def test_shared_traversal_lists(ctx, name, leaf, radius):
+    """More than 2^17 queries take the lists of 64 queries per wave (leaves tested in 64- or 48-point chunks, on
+    the queries' own lanes or moved onto lane groups): equal to the same queries in calls small enough for the
+    group kernel, and to the oracle on a sample."""
+    xyz = dense_clouds()[name]
+    ctx.set_points(xyz)
+    ctx.sort_points(A.ENC_MORTON)
+    ctx.build(leaf)
+    sx, okeys, operm, oc, orad = O.sort_points(O.ENC_MORTON, xyz)
+    tree = O.Tree(okeys, leaf, O.ENC_MORTON, oc, orad)
+    n = len(sx)
+    idx = np.arange(n, dtype=np.uint32)
+    some = np.arange(7, n, 211)
+    for kernel in KERNELS:
+        for algo in ALGOS:
+            ref, sizes = O.radius(tree, sx, kernel, algo, sx[some], radius)
+            for prec in (A.PREC_FP64, A.PREC_FP32):
+                tag = (name, leaf, radius, kernel, algo, prec)
+                w = 2 if algo == A.A_STRUCT else 1
+                counts, offs, ent, st = ctx.radius_csr(kernel, algo, prec, idx, radius)
+                parts = [ctx.radius_csr(kernel, algo, prec, h, radius) for h in np.array_split(idx, 2)]
+                assert np.array_equal(counts, np.concatenate([p[0] for p in parts])), tag
+                assert np.array_equal(np.diff(offs), np.concatenate([np.diff(p[1]) for p in parts])), tag
+                assert np.array_equal(ent, np.concatenate([p[2] for p in parts])), tag
+                assert st["points_tested"] == sum(p[3]["points_tested"] for p in parts), tag
+                assert st["nodes_classified"] == sum(p[3]["nodes_classified"] for p in parts), tag
+                assert np.array_equal(counts[some], sizes), tag
+                for q, r in zip(some, ref):
+                    assert np.array_equal(ent[w * int(offs[q]):w * int(offs[q + 1])], np.asarray(r).reshape(-1)), tag
