@@ -103,16 +103,24 @@ __global__ __launch_bounds__(256) void k_node_ext(const NodeRec *__restrict__ no
 // ---- device-driven level loop: no host round trip between levels
 //
 // Each level is one launch that takes the level's node range [ls, le) from ctl[l] (written by the level
-// above). k_level_step walks the level in tiles of 256 nodes (dynamic tile ids): it ranks a tile's split
-// flags with ballots, takes the tile's offset from a chained scan over the tiles (decoupled look-back in
-// which one wave reads 64 predecessor tiles per step, bounded spins), points every node at its first
-// child (0 = leaf) and builds the children of the split nodes, 8 lanes per node; the last tile writes
-// ctl[l + 1]. Levels past the last one find an empty range and return (about 2.5 us each), so the host
+// above). k_level_step walks the level in tiles of 32 to 256 nodes (dynamic tile ids; 32 nodes are one
+// round of 8 lanes each, so the top levels' long searches run side by side, 256 keep the tile count of
+// large levels low): it ranks a tile's split flags with ballots, takes the tile's offset from a chained
+// scan over the tiles (decoupled look-back in which one wave reads 64 predecessor tiles per step, bounded
+// spins), points every node at its first child (0 = leaf) and builds the children of the split nodes, 8
+// lanes per node; the last tile writes ctl[l + 1]. Levels past the last one find an empty range and return (about 2.5 us each), so the host
 // enqueues all of them and reads the level table back once. The node arrays are sized up front; a level
 // that would outgrow them raises an error bit, and the host then runs the level loop with growing arrays
 // instead. Two launches per level for the first 13 levels, and the host loop for anything deeper, took
 // 0.9 ms of a 120 k-point frame whose duplicates reach below level 12.
-constexpr uint32_t kLvlTile = 256;
+constexpr uint32_t kLvlTileMax = 256, kLvlTileMin = 32;
+constexpr size_t kLvlTiles = 2048;  // tiles of a level beyond which they grow
+// nodes per tile of a level of at most nmax nodes
+static uint32_t level_tile(size_t nmax) {
+    uint32_t t = kLvlTileMin;
+    while (t < kLvlTileMax && nmax > kLvlTiles * t) t *= 2;
+    return t;
+}
 constexpr uint32_t kLvlAgg = 1u << 30, kLvlInc = 2u << 30, kLvlMask = (1u << 30) - 1u, kLvlSpin = 1u << 24;
 constexpr uint32_t kLvlErrSpin = 1u, kLvlErrCap = 2u;
 constexpr int kLvlCount = kMaxDepth + 1;  // levels 0 .. 21 (level 21 nodes never split)
@@ -144,12 +152,13 @@ __global__ __launch_bounds__(256) void k_level_step(const uint64_t *__restrict__
                                                     uint64_t *__restrict__ nkey, uint32_t *__restrict__ child,
                                                     uint32_t *__restrict__ flags, LevelCtl *__restrict__ ctl, uint32_t level,
                                                     uint32_t *__restrict__ lookback, uint32_t *__restrict__ tile_counter,
-                                                    uint32_t cap, uint32_t max_leaf, BuildGeom g, uint32_t *__restrict__ err,
-                                                    uint32_t *__restrict__ total) {
-    __shared__ uint32_t s_w[4], s_tile, s_prefix, s_u[kLvlTile];
+                                                    uint32_t tile_nodes, uint32_t cap, uint32_t max_leaf, BuildGeom g,
+                                                    uint32_t *__restrict__ err, uint32_t *__restrict__ total) {
+    __shared__ uint32_t s_w[4], s_tile, s_prefix, s_u[kLvlTileMax];
     const LevelCtl L = ctl[level];
     if (L.le <= L.ls) return;
-    const uint32_t ntiles = (L.le - L.ls + kLvlTile - 1) / kLvlTile;
+    const uint32_t ntiles = (L.le - L.ls + tile_nodes - 1) / tile_nodes;
+    if (blockIdx.x >= ntiles) return;  // the others claim every tile (a claim is a serialised atomic, ~12 ns)
     const uint32_t tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const uint32_t cl = level + 1, k = tid & 7u;
     const uint64_t step = node_range(cl);
@@ -158,8 +167,9 @@ __global__ __launch_bounds__(256) void k_level_step(const uint64_t *__restrict__
         __syncthreads();
         const uint32_t tile = s_tile;
         if (tile >= ntiles) break;
-        const uint32_t u = L.ls + tile * kLvlTile + tid;
-        const bool f = u < L.le && flags[u] != 0;
+        const uint32_t u = L.ls + tile * tile_nodes + tid;
+        const bool mine = tid < tile_nodes && u < L.le;
+        const bool f = mine && flags[u] != 0;
         const uint64_t m = ballot64(f);
         if (lane == 0) s_w[w] = (uint32_t)__popcll(m);
         __syncthreads();
@@ -219,10 +229,10 @@ __global__ __launch_bounds__(256) void k_level_step(const uint64_t *__restrict__
         }
         __syncthreads();
         const uint32_t prefix = s_prefix;
-        if (u < L.le) child[u] = f ? L.le + 8u * (prefix + j) : 0u;
+        if (mine) child[u] = f ? L.le + 8u * (prefix + j) : 0u;
         // the tile's split nodes, 8 lanes each: lane k finds child k's end and takes its start from lane k - 1
         // (a search over the whole parent range finds the same index as one from the child's start)
-        for (uint32_t q = tid >> 3; q < tot; q += kLvlTile / 8) {
+        for (uint32_t q = tid >> 3; q < tot; q += 32) {
             const uint32_t pu = s_u[q];
             const uint64_t cb = (uint64_t)L.le + 8ull * (prefix + q);
             if (cb + 8u > cap) {  // the node's 8 lanes move together
@@ -238,6 +248,7 @@ __global__ __launch_bounds__(256) void k_level_step(const uint64_t *__restrict__
             flags[cb + k] = (hi - lo > max_leaf && cl < kMaxDepth) ? 1u : 0u;
             if (cl == kMaxDepth) child[cb + k] = 0u;  // no step visits the deepest level
         }
+        if (gridDim.x >= ntiles) break;  // one tile per workgroup
         __syncthreads();  // the next tile rewrites the shared lists
     }
 }
@@ -339,21 +350,22 @@ hipError_t launch_build(oct_ctx *ctx, uint32_t M, std::string &err) {
         if ((e = ctx->next.reserve((cap + 6) / 8 + 1)) != hipSuccess) return e;
         LevelCtl *ctl = reinterpret_cast<LevelCtl *>(ctx->misc.p + 4096);
         uint32_t *counters = ctx->misc.p + 4096 + 2 * (kLvlCount + 1), *errw = counters + kLvlCount, *totw = errw + 1;
-        const size_t maxtiles = (cap + kLvlTile - 1) / kLvlTile, nlook = (size_t)kLvlCount * maxtiles;
+        const size_t maxtiles = std::max<size_t>(kLvlTiles, (cap + kLvlTileMax - 1) / kLvlTileMax), nlook = (size_t)kLvlCount * maxtiles;
         if ((e = ctx->lookback.reserve(nlook + 1)) != hipSuccess) return e;
         const unsigned ig = (unsigned)std::max<size_t>(1, std::min<size_t>((nlook + 255) / 256, 1024));
         k_level_init<<<ig, 256, 0, ctx->stream>>>(ctx->nodes.p, ctx->nkey.p, ctx->flags.p, n, M, g, ctl, ctx->lookback.p, nlook,
                                                   counters, errw, totw);
         int cus = 0;
         (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device);
-        const size_t sgrid = (size_t)std::max(1, cus) * 8;
+        const size_t sgrid = (size_t)std::max(1, cus) * 8;  // resident workgroups
         for (int l = 0; l < (int)kMaxDepth; l++) {
             // level l holds at most min(8^l, cap) nodes: small grids for the top levels
             const size_t nmax = l < 10 ? std::min<size_t>(cap, 1ull << (3 * l)) : cap;
-            const unsigned gs = (unsigned)std::min(sgrid, (nmax + kLvlTile - 1) / kLvlTile);
+            const uint32_t tn = level_tile(nmax);
+            const unsigned gs = (unsigned)std::min(sgrid, (nmax + tn - 1) / tn);
             k_level_step<<<gs, 256, 0, ctx->stream>>>(ctx->sorted_keys, ctx->nodes.p, ctx->nkey.p, ctx->child.p, ctx->flags.p, ctl,
                                                       (uint32_t)l, ctx->lookback.p + (size_t)l * maxtiles, counters + l,
-                                                      (uint32_t)cap, M, g, errw, totw);
+                                                      tn, (uint32_t)cap, M, g, errw, totw);
         }
         k_recentre_dev<<<(unsigned)((cap * kRecentreLanes + 255) / 256), 256, 0, ctx->stream>>>(
             ctx->p64.p, ctx->nodes.p, ctx->child.p, totw, ctx->p32.p, ctx->amax.p);
