@@ -42,6 +42,9 @@ static_assert(sizeof(NodeExt) == 192, "NodeExt is three 64-byte lines");
 // in steps of up to 64 and ignore what lies past it.
 constexpr size_t kPointPad = 64;
 
+// Outputs above this size are written past the caches (non-temporal): half of the 256 MB memory-side cache.
+constexpr size_t kCacheBytes = 128u << 20;
+
 // Device buffer that only grows.
 template <class T>
 struct DevBuf {
