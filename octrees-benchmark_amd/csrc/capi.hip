@@ -251,6 +251,7 @@ __global__ void k_na_zero(uint64_t *p) { *p = 0; }
 static int upload_xyz_soa(oct_ctx *ctx, const double *x, const double *y, const double *z, size_t n) {
     if (n >= (1ull << 30)) return fail(ctx, OCT_ERR_ARG, "at most 2^30 - 1 points");
     ctx->las_loaded = false;
+    ctx->bbox_blocks = 0;
     HCHK(ctx->xyz.reserve(3 * n), "alloc points");
     if (n) {
         if (!x || !y || !z) return fail(ctx, OCT_ERR_ARG, "null coordinate array");
@@ -273,10 +274,13 @@ int upload_xyz(oct_ctx *ctx, const double *src, size_t n, size_t stride, hipMemc
     if (stride < 24 || stride % 8) return fail(ctx, OCT_ERR_ARG, "stride_bytes must be >= 24 and a multiple of 8");
     if (n >= (1ull << 30)) return fail(ctx, OCT_ERR_ARG, "at most 2^30 - 1 points");
     ctx->las_loaded = false;  // the cloud no longer comes from a LAS file
+    ctx->bbox_blocks = 0;
     HCHK(ctx->xyz.reserve(3 * n), "alloc points");
     if (n) {
         if (!src) return fail(ctx, OCT_ERR_ARG, "null point buffer");
-        if (stride == 24) {
+        if (stride == 24 && kind == hipMemcpyDeviceToDevice && (uintptr_t)src % 16 == 0) {
+            HCHK(launch_copy_points(ctx, src, n), "copy points");
+        } else if (stride == 24) {
             HCHK(hipMemcpyAsync(ctx->xyz.p, src, n * 24, kind, ctx->stream), "copy points");
         } else {
             const size_t words = n * (stride / 8);
@@ -443,7 +447,8 @@ int oct_destroy(oct_ctx *ctx) {
     ctx->entries.release(), ctx->stats.release(), ctx->kidx.release(), ctx->kd2.release();
     ctx->next.release(), ctx->qrad3.release(), ctx->kc_xyz.release(), ctx->kc_keys.release();
     ctx->kd2f.release(), ctx->radtab.release(), ctx->las_rec.release(), ctx->las_meta.release();
-    ctx->rec_in.release(), ctx->rec_out.release(), ctx->derr.release();
+    ctx->rec_in.release(), ctx->rec_out.release(), ctx->derr.release(), ctx->bbox_part.release();
+    ctx->box.release(), ctx->msd.release(), ctx->keys_p.release(), ctx->vals_p.release();
     for (int s = 0; s < ST_N; s++) {
         if (ctx->ev0[s]) (void)hipEventDestroy(ctx->ev0[s]);
         if (ctx->ev1[s]) (void)hipEventDestroy(ctx->ev1[s]);

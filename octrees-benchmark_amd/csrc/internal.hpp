@@ -112,6 +112,8 @@ struct oct_ctx {
     oct::DevBuf<uint64_t> keys[2];
     oct::DevBuf<uint32_t> vals[2];
     oct::DevBuf<uint32_t> hist;      // 8 x 256 digit histograms, then bits 55..62 and 47..54
+    oct::DevBuf<double> bbox_part;   // min and max per axis of the blocks of the copy that brought the points
+    int bbox_blocks = 0;             // how many, 0: not taken (the points came another way)
     oct::DevBuf<double> box;         // oct_sort_points: min, max, centre and radii per axis, on the device
     oct::DevBuf<uint32_t> lookback;  // per pass, per tile, per bin
     oct::DevBuf<uint32_t> misc;      // tile counters, flags, scan partials
@@ -193,6 +195,9 @@ namespace oct {
 
 // ---- launchers implemented in the .hip files (all enqueue on ctx->stream) ----
 hipError_t launch_bbox(oct_ctx *ctx, double mn[3], double mx[3]);
+// Copies n packed device points into ctx->xyz and leaves the blocks' minima and maxima for the bounding box.
+// src: 16-byte aligned.
+hipError_t launch_copy_points(oct_ctx *ctx, const double *src, size_t n);
 // The same reduction left on the device: ctx->box receives min, max, centre and radii (12 doubles),
 // nothing is read back (n >= 1).
 hipError_t launch_bbox_dev(oct_ctx *ctx);

@@ -206,6 +206,7 @@ int oct_las_load(oct_ctx *ctx, const char *path, oct_las_header *h_out) {
     hipError_t e;
     if ((e = hipSetDevice(ctx->device)) != hipSuccess) return las_fail(ctx, OCT_ERR_HIP, hipGetErrorString(e));
     if ((e = ctx->las_rec.reserve(bytes + 8)) != hipSuccess) return las_fail(ctx, OCT_ERR_NOMEM, "alloc point records");
+    ctx->bbox_blocks = 0;
     if ((e = ctx->xyz.reserve(3 * n + 3)) != hipSuccess) return las_fail(ctx, OCT_ERR_NOMEM, "alloc points");
     if ((e = ctx->las_meta.reserve(n + 1)) != hipSuccess) return las_fail(ctx, OCT_ERR_NOMEM, "alloc point attributes");
     // file -> pinned staging (two halves, alternating) -> device
