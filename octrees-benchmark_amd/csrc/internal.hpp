@@ -181,8 +181,9 @@ struct oct_ctx {
     // small results on their way to the host: a pinned page, written by copies on the stream
     struct alignas(128) Mail {
         unsigned long long stats[8];
+        double box[12];
         uint64_t total;
-        uint32_t err;
+        uint32_t err, sort[2];
     } *mail = nullptr;
     oct::DevBuf<uint32_t> derr;     // device error word (kErr* bits), zero when no kernel failed
 

@@ -37,13 +37,16 @@ __device__ inline uint32_t wave_incl_scan(uint32_t v) {
 // second partition pass below): tiles come from a table, each inside one segment's range; the
 // look-back stops at the segment's first tile and bin offsets are the segment's own
 // (bin_base + segment * base_stride), so every segment is sorted on its own, stably, in one launch.
-template <bool SEG>
+// DYN = true: the table's length is on the device (ntiles_dev), and a grid of any size takes the tiles in
+// turn; an empty table costs one small launch.
+template <bool SEG, bool DYN = false>
 __global__ __launch_bounds__(kSortBlock) void k_onesweep(const uint64_t *__restrict__ kin, const uint32_t *__restrict__ vin,
                                                          uint64_t *__restrict__ kout, uint32_t *__restrict__ vout, size_t n,
                                                          uint32_t shift, const uint32_t *__restrict__ bin_base,
                                                          uint32_t *__restrict__ lookback, uint32_t *__restrict__ tile_counter,
                                                          uint32_t *__restrict__ err, const SortTile *__restrict__ tiles,
-                                                         uint32_t base_stride, uint32_t *__restrict__ hist16) {
+                                                         uint32_t base_stride, uint32_t *__restrict__ hist16,
+                                                         const uint32_t *__restrict__ ntiles_dev = nullptr) {
     __shared__ uint64_t s_keys[kSortTile];
     __shared__ uint32_t s_vals[kSortTile];
     __shared__ uint32_t s_wave[kSortBlock / 64][256];
@@ -53,136 +56,140 @@ __global__ __launch_bounds__(kSortBlock) void k_onesweep(const uint64_t *__restr
     __shared__ uint32_t s_tile;
 
     const uint32_t tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
-    if (tid == 0) s_tile = atomicAdd(tile_counter, 1u);
-    for (uint32_t i = tid; i < (kSortBlock / 64) * 256; i += kSortBlock) (&s_wave[0][0])[i] = 0;
-    __syncthreads();
-    const uint32_t tile = s_tile;
-    size_t tile_base, limit;
-    uint32_t first_tile = 0, cloud = 0;
-    if constexpr (SEG) {
-        const SortTile T = tiles[tile];
-        tile_base = T.start, limit = (size_t)T.start + T.len, first_tile = T.first, cloud = T.cloud;
-    } else {
-        tile_base = (size_t)tile * kSortTile, limit = n;
-    }
-    const size_t wave_base = tile_base + (size_t)w * 64 * kSortItems;
-
-    uint64_t k[kSortItems];
-    uint32_t v[kSortItems];
-#pragma unroll
-    for (int r = 0; r < kSortItems; r++) {
-        size_t p = wave_base + (size_t)r * 64 + lane;
-        bool valid = p < limit;
-        k[r] = valid ? kin[p] : 0ull;
-        v[r] = valid ? (vin ? vin[p] : (uint32_t)p) : 0u;
-    }
-    uint32_t rank[kSortItems];
-#pragma unroll
-    for (int r = 0; r < kSortItems; r++) {
-        size_t p = wave_base + (size_t)r * 64 + lane;
-        bool valid = p < limit;
-        uint32_t d = (uint32_t)(k[r] >> shift) & 255u;
-        uint64_t peers = ballot64(valid);
-#pragma unroll
-        for (int b = 0; b < 8; b++) {
-            bool bit = (d >> b) & 1u;
-            uint64_t m = ballot64(bit);
-            peers &= bit ? m : ~m;
+    do {
+        if (tid == 0) s_tile = atomicAdd(tile_counter, 1u);
+        for (uint32_t i = tid; i < (kSortBlock / 64) * 256; i += kSortBlock) (&s_wave[0][0])[i] = 0;
+        __syncthreads();
+        const uint32_t tile = s_tile;
+        if constexpr (DYN)
+            if (tile >= *ntiles_dev) return;
+        size_t tile_base, limit;
+        uint32_t first_tile = 0, cloud = 0;
+        if constexpr (SEG) {
+            const SortTile T = tiles[tile];
+            tile_base = T.start, limit = (size_t)T.start + T.len, first_tile = T.first, cloud = T.cloud;
+        } else {
+            tile_base = (size_t)tile * kSortTile, limit = n;
         }
-        // the lowest lane of each digit group adds the group to the wave's digit count and hands the
-        // count before it to its group; a wave's LDS atomics run in program order, so rows rank in order
-        const uint32_t below = (uint32_t)__popcll(peers & lanemask_lt());
-        uint32_t prev = 0;
-        if (valid && below == 0) prev = atomicAdd(&s_wave[w][d], (uint32_t)__popcll(peers));
-        const uint32_t leader = peers ? (uint32_t)__builtin_ctzll(peers) : 0u;
-        rank[r] = (uint32_t)__builtin_amdgcn_ds_bpermute((int)(leader << 2), (int)prev) + below;
-    }
-    __syncthreads();
+        const size_t wave_base = tile_base + (size_t)w * 64 * kSortItems;
 
-    // per-bin tile count and per-wave exclusive offsets (thread b < 256 owns bin b; with more than
-    // 256 threads the other waves wait at the barriers)
-    const uint32_t b = tid;
-    const bool owner = kSortBlock == 256 || tid < 256;
-    uint32_t tile_count = 0;
-    uint32_t *lb = lookback + (size_t)tile * 256;
-    if (owner) {
-#pragma unroll
-        for (int ww = 0; ww < kSortBlock / 64; ww++) {
-            uint32_t c = s_wave[ww][b];
-            s_wave[ww][b] = tile_count;
-            tile_count += c;
+        uint64_t k[kSortItems];
+        uint32_t v[kSortItems];
+    #pragma unroll
+        for (int r = 0; r < kSortItems; r++) {
+            size_t p = wave_base + (size_t)r * 64 + lane;
+            bool valid = p < limit;
+            k[r] = valid ? kin[p] : 0ull;
+            v[r] = valid ? (vin ? vin[p] : (uint32_t)p) : 0u;
         }
-        if (tile == first_tile)
-            store_flag(&lb[b], kFlagInc | tile_count);
-        else
-            store_flag(&lb[b], kFlagAgg | tile_count);
-    }
-
-    // local exclusive scan of the tile counts over bins
-    uint32_t incl = 0;
-    if (owner) {
-        incl = wave_incl_scan(tile_count);
-        if (lane == 63) s_wsum[w] = incl;
-    }
-    __syncthreads();
-    if (owner) {
-        uint32_t wpre = 0;
-        for (uint32_t ww = 0; ww < w; ww++) wpre += s_wsum[ww];
-        s_tile_start[b] = wpre + incl - tile_count;
-
-        // decoupled look-back over preceding tiles for bin b
-        uint32_t excl = 0;
-        if (tile > first_tile) {
-            int64_t t = (int64_t)tile - 1;
-            uint32_t spins = 0;
-            while (t >= (int64_t)first_tile) {
-                uint32_t x = load_flag(&lookback[(size_t)t * 256 + b]);
-                if ((x >> 30) == 0) {
-                    if (++spins > kSpinLimit) {
-                        atomicOr(err, 1u);
-                        break;
-                    }
-                    __builtin_amdgcn_s_sleep(1);
-                    continue;
-                }
-                excl += x & kValMask;
-                if ((x >> 30) == 2) break;
-                t--;
-            }
-            store_flag(&lb[b], kFlagInc | ((excl + tile_count) & kValMask));
-        }
-        s_global[b] = bin_base[(size_t)cloud * base_stride + b] + excl;
-    }  // owner
-    __syncthreads();
-
-    // stage the tile in LDS in (bin, original order) order
-#pragma unroll
-    for (int r = 0; r < kSortItems; r++) {
-        size_t p = wave_base + (size_t)r * 64 + lane;
-        if (p < limit) {
+        uint32_t rank[kSortItems];
+    #pragma unroll
+        for (int r = 0; r < kSortItems; r++) {
+            size_t p = wave_base + (size_t)r * 64 + lane;
+            bool valid = p < limit;
             uint32_t d = (uint32_t)(k[r] >> shift) & 255u;
-            uint32_t pos = s_tile_start[d] + s_wave[w][d] + rank[r];
-            s_keys[pos] = k[r];
-            s_vals[pos] = v[r];
+            uint64_t peers = ballot64(valid);
+    #pragma unroll
+            for (int b = 0; b < 8; b++) {
+                bool bit = (d >> b) & 1u;
+                uint64_t m = ballot64(bit);
+                peers &= bit ? m : ~m;
+            }
+            // the lowest lane of each digit group adds the group to the wave's digit count and hands the
+            // count before it to its group; a wave's LDS atomics run in program order, so rows rank in order
+            const uint32_t below = (uint32_t)__popcll(peers & lanemask_lt());
+            uint32_t prev = 0;
+            if (valid && below == 0) prev = atomicAdd(&s_wave[w][d], (uint32_t)__popcll(peers));
+            const uint32_t leader = peers ? (uint32_t)__builtin_ctzll(peers) : 0u;
+            rank[r] = (uint32_t)__builtin_amdgcn_ds_bpermute((int)(leader << 2), (int)prev) + below;
         }
-    }
-    __syncthreads();
-    const uint32_t tile_n = (uint32_t)((limit - tile_base) < (size_t)kSortTile ? (limit - tile_base) : (size_t)kSortTile);
-    for (uint32_t j = tid; j < tile_n; j += kSortBlock) {
-        uint64_t key = s_keys[j];
-        uint32_t d = (uint32_t)(key >> shift) & 255u;
-        uint32_t dst = s_global[d] + (j - s_tile_start[d]);
-        kout[dst] = key;
-        vout[dst] = s_vals[j];
-        if (hist16) {
-            // the keys' top 16 bits (47..62) per prefix: when this pass orders bits 55..62 after a pass
-            // on 47..54, the staged tile is ordered by them, so each run of one prefix adds its length
-            // (its first key subtracts its index, its last adds index + 1)
-            const uint32_t pre = (uint32_t)(key >> kMsdShift2);
-            if (j == 0 || (uint32_t)(s_keys[j - 1] >> kMsdShift2) != pre) atomicAdd(&hist16[pre], 0u - j);
-            if (j + 1 == tile_n || (uint32_t)(s_keys[j + 1] >> kMsdShift2) != pre) atomicAdd(&hist16[pre], j + 1u);
+        __syncthreads();
+
+        // per-bin tile count and per-wave exclusive offsets (thread b < 256 owns bin b; with more than
+        // 256 threads the other waves wait at the barriers)
+        const uint32_t b = tid;
+        const bool owner = kSortBlock == 256 || tid < 256;
+        uint32_t tile_count = 0;
+        uint32_t *lb = lookback + (size_t)tile * 256;
+        if (owner) {
+    #pragma unroll
+            for (int ww = 0; ww < kSortBlock / 64; ww++) {
+                uint32_t c = s_wave[ww][b];
+                s_wave[ww][b] = tile_count;
+                tile_count += c;
+            }
+            if (tile == first_tile)
+                store_flag(&lb[b], kFlagInc | tile_count);
+            else
+                store_flag(&lb[b], kFlagAgg | tile_count);
         }
-    }
+
+        // local exclusive scan of the tile counts over bins
+        uint32_t incl = 0;
+        if (owner) {
+            incl = wave_incl_scan(tile_count);
+            if (lane == 63) s_wsum[w] = incl;
+        }
+        __syncthreads();
+        if (owner) {
+            uint32_t wpre = 0;
+            for (uint32_t ww = 0; ww < w; ww++) wpre += s_wsum[ww];
+            s_tile_start[b] = wpre + incl - tile_count;
+
+            // decoupled look-back over preceding tiles for bin b
+            uint32_t excl = 0;
+            if (tile > first_tile) {
+                int64_t t = (int64_t)tile - 1;
+                uint32_t spins = 0;
+                while (t >= (int64_t)first_tile) {
+                    uint32_t x = load_flag(&lookback[(size_t)t * 256 + b]);
+                    if ((x >> 30) == 0) {
+                        if (++spins > kSpinLimit) {
+                            atomicOr(err, 1u);
+                            break;
+                        }
+                        __builtin_amdgcn_s_sleep(1);
+                        continue;
+                    }
+                    excl += x & kValMask;
+                    if ((x >> 30) == 2) break;
+                    t--;
+                }
+                store_flag(&lb[b], kFlagInc | ((excl + tile_count) & kValMask));
+            }
+            s_global[b] = bin_base[(size_t)cloud * base_stride + b] + excl;
+        }  // owner
+        __syncthreads();
+
+        // stage the tile in LDS in (bin, original order) order
+    #pragma unroll
+        for (int r = 0; r < kSortItems; r++) {
+            size_t p = wave_base + (size_t)r * 64 + lane;
+            if (p < limit) {
+                uint32_t d = (uint32_t)(k[r] >> shift) & 255u;
+                uint32_t pos = s_tile_start[d] + s_wave[w][d] + rank[r];
+                s_keys[pos] = k[r];
+                s_vals[pos] = v[r];
+            }
+        }
+        __syncthreads();
+        const uint32_t tile_n = (uint32_t)((limit - tile_base) < (size_t)kSortTile ? (limit - tile_base) : (size_t)kSortTile);
+        for (uint32_t j = tid; j < tile_n; j += kSortBlock) {
+            uint64_t key = s_keys[j];
+            uint32_t d = (uint32_t)(key >> shift) & 255u;
+            uint32_t dst = s_global[d] + (j - s_tile_start[d]);
+            kout[dst] = key;
+            vout[dst] = s_vals[j];
+            if (hist16) {
+                // the keys' top 16 bits (47..62) per prefix: when this pass orders bits 55..62 after a pass
+                // on 47..54, the staged tile is ordered by them, so each run of one prefix adds its length
+                // (its first key subtracts its index, its last adds index + 1)
+                const uint32_t pre = (uint32_t)(key >> kMsdShift2);
+                if (j == 0 || (uint32_t)(s_keys[j - 1] >> kMsdShift2) != pre) atomicAdd(&hist16[pre], 0u - j);
+                if (j + 1 == tile_n || (uint32_t)(s_keys[j + 1] >> kMsdShift2) != pre) atomicAdd(&hist16[pre], j + 1u);
+            }
+        }        if constexpr (DYN) __syncthreads();  // the next tile reuses the LDS
+    } while (DYN);
 }
 
 __global__ void k_iota_copy(const uint64_t *__restrict__ kin, uint64_t *__restrict__ kout, uint32_t *__restrict__ vout,
@@ -209,14 +216,40 @@ __global__ void k_iota_copy(const uint64_t *__restrict__ kin, uint64_t *__restri
 //     segment, so no look-back), until every piece fits. The workgroup then reads the points of its
 //     sorted range through the permutation and writes the sorted cloud (the gather), so the random
 //     reads overlap other workgroups' LDS work.
+// A few long 16-bit segments (scans cluster along their trajectory) would keep a few workgroups busy long
+// after the others, or not fit one at all. They are split by their next 8 bits (39..46) with one more
+// device-wide pass over such segments only: k_huge_jobs counts their digits and lists the pieces, the
+// onesweep pass moves the keys. Without such segments both launches return at once. A piece still above
+// kSegMaxLen sends the whole sort to the LSD passes.
 // Every step keeps equal keys in input order, so the permutation is the stable sort by key, as with
 // the 8 LSD passes. Traffic per key: 20 B + 24 B (passes) + 24 B (LDS sort) + 56 B (gather), plus
 // 32 B for keys in segments that are split, against 188 B + 60 B for eight passes and a gather.
 
+// A job of k_seg_sort: len is its length, with kSegInB if the device-wide split has ordered it by bits
+// 39..46 already, from buffer a (the second pass's output) into b.
 struct SegJob {
     uint32_t start, len;
 };
-constexpr uint32_t kSegMaxLen = 1u << 15;  // longest 16-bit segment the workgroup sort takes
+constexpr uint32_t kSegInB = 1u << 31;
+constexpr uint32_t kSegMaxLen = 1u << 15;  // longest segment the workgroup sort takes
+// The segments the device-wide split takes, those above `min` keys: start, length, keys counted so far, bin
+// starts (256 per segment) and sort tiles; n[0] segments, n[1] tiles. n null: no split.
+struct HugeList {
+    uint32_t *start, *len, *done, *bases;
+    SortTile *tiles;
+    uint32_t *n;
+    uint32_t min;
+};
+// Shortest segment worth the split. A segment is split when it is longer than one resident workgroup's share
+// of the keys (n / 1024, four workgroups per CU: a longer one ends after all others) and than this, the
+// length below which the split inside the workgroup costs less than a third pass; above kSegMaxLen always.
+// Sort stage, sweep clouds, before and with the split: 20 M 2.40 and 1.52 ms, 5 M 0.83 and 0.47, 1.5 M 0.48
+// and 0.27; 50 M tile (segments of 24 k keys) 3.24 either way, 3.33 with every segment above 2^14 split.
+constexpr uint32_t kHugeMin = 1u << 12;
+// Fewest keys with which the split is launched: its two launches cost 8 us where no segment needs it
+// (5 M tile: 0.383 and 0.391 ms), which the LSD passes' excess over it pays from here (150 k sweep: 0.119 and
+// 0.122 ms, 500 k: 0.207 and 0.184).
+constexpr size_t kHugeMinKeys = 1u << 18;
 // pieces awaiting a split: a split of up to 2^15 keys pushes at most 15 pieces above 2048 keys and
 // pops one, over at most 6 levels (bits 39..46 down to 0..7)
 constexpr int kSegStack = 96;
@@ -395,17 +428,18 @@ __device__ void seg_local_sort(SegShared<W, IPT> &S, const uint64_t *ks, const u
     }
 }
 
-// Complete sort of one 16-bit segment longer than kCap, [start, start + len) of buffer a, into the
-// same range of buffer b (buffer a's range is scratch): stable splits by the next 8 bits until every
+// Complete sort of one segment longer than kCap, [start, start + len) of buffer a (in_b: of buffer b), into
+// the same range of buffer b (buffer a's range is scratch): stable splits by the next 8 bits until every
 // piece fits, then LDS sorts of runs of consecutive pieces. A piece whose bits are used up holds
 // equal keys, already in input order.
 template <int W, int IPT>
 __device__ void seg_split_sort(SegShared<W, IPT> &S, uint64_t *ka, uint32_t *va, uint64_t *kb, uint32_t *vb,
-                               uint32_t start, uint32_t len, uint32_t *err, const double *xyz, double4 *p64) {
+                               uint32_t start, uint32_t len, bool in_b, uint32_t *err, const double *xyz,
+                               double4 *p64) {
     constexpr uint32_t kCap = SegShared<W, IPT>::kCap;
     const uint32_t tid = threadIdx.x, w = tid >> 6, lane = tid & 63, base = w * 64 * IPT;
     if (tid == 0) {
-        S.stack[0] = make_uint4(start, len, kMsdShift3 + 1u, 0u);
+        S.stack[0] = make_uint4(start, len, in_b ? kMsdShift3 - 7u : kMsdShift3 + 1u, in_b ? 1u : 0u);
         S.sp = 1u;
     }
     __syncthreads();
@@ -562,61 +596,163 @@ __global__ __attribute__((amdgpu_flat_work_group_size(W * 64, W * 64), amdgpu_wa
         const SegJob job = S.job;
         __syncthreads();
         if (kind == 2u) break;
-        if (job.len > SegShared<W, IPT>::kCap)
-            seg_split_sort(S, ka, va, kb, vb, job.start, job.len, err, xyz, p64);
+        const uint32_t len = job.len & ~kSegInB;
+        const bool in_b = job.len & kSegInB;
+        if (len > SegShared<W, IPT>::kCap)
+            seg_split_sort(S, ka, va, kb, vb, job.start, len, in_b, err, xyz, p64);
         else
-            seg_local_sort(S, ka, va, kb, vb, job.start, job.len, xyz, p64);
+            seg_local_sort(S, in_b ? kb : ka, in_b ? vb : va, kb, vb, job.start, len, xyz, p64);
         __syncthreads();
     }
 }
 
-// One workgroup per top-8-bit bin: the start of each of its 16-bit segments (hist2[bin * 256 + digit]
-// keys each; the bin starts at base1[bin]) and its jobs - a segment above cap alone (big), runs of
-// consecutive smaller segments up to cap together (small). njobs: [0] big, [1] small, [2] longest
-// segment.
-__global__ __launch_bounds__(256) void k_msd_jobs(const uint32_t *__restrict__ hist2, const uint32_t *__restrict__ base1,
-                                                  uint32_t cap, SegJob *__restrict__ big, SegJob *__restrict__ small,
-                                                  uint32_t *__restrict__ njobs) {
-    __shared__ uint32_t s_c[256], s_st[256], s_wsum[4], s_nb, s_ns, s_ob, s_os;
-    __shared__ SegJob s_big[256], s_small[256];
-    const uint32_t bin = blockIdx.x, tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
-    const uint32_t c = hist2[bin * 256 + tid];
-    const uint32_t incl = wave_incl_scan(c);
-    if (lane == 63) s_wsum[w] = incl;
-    __syncthreads();
-    uint32_t pre = 0;
-    for (uint32_t ww = 0; ww < w; ww++) pre += s_wsum[ww];
-    const uint32_t st = base1[bin] + pre + incl - c;
+// The jobs of 256 consecutive segments (digit tid of the workgroup: c keys from st on), by one workgroup:
+// segments above H.min go on the list of the split, or without one their longest length to njobs[2]; others
+// above cap become a job each (big, njobs[0]), runs of consecutive smaller ones one up to cap (small,
+// njobs[1]). in_b: kSegInB or 0.
+__device__ inline void emit_seg_jobs(uint32_t c, uint32_t st, uint32_t cap, uint32_t in_b, SegJob *__restrict__ big,
+                                     SegJob *__restrict__ small, uint32_t *__restrict__ njobs, const HugeList &H) {
+    __shared__ uint32_t s_c[256], s_st[256], s_nb, s_ns, s_nh, s_ob, s_os;
+    __shared__ SegJob s_big[256], s_small[256], s_huge[256];
+    const uint32_t tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
     s_c[tid] = c, s_st[tid] = st;
     __syncthreads();
     if (w == 0) {
         uint32_t c4[4], s4[4];
 #pragma unroll
         for (int sl = 0; sl < 4; sl++) c4[sl] = s_c[4 * lane + sl], s4[sl] = s_st[4 * lane + sl];
-        uint32_t nb = 0, ns = 0, mx = 0;  // segments up to cap never exceed the longest big one's limit
+        uint32_t nb = 0, ns = 0, nh = 0;
         pack_digit_ranges(
             c4, s4, cap,
             [&](uint32_t a, uint32_t l) {
-                if (lane == 0) s_big[nb] = SegJob{a, l};
-                nb++;
-                mx = l > mx ? l : mx;
+                if (l > H.min) {
+                    if (lane == 0) s_huge[nh] = SegJob{a, l};
+                    nh++;
+                } else {
+                    if (lane == 0) s_big[nb] = SegJob{a, l | in_b};
+                    nb++;
+                }
             },
             [&](uint32_t a, uint32_t l) {
-                if (lane == 0) s_small[ns] = SegJob{a, l};
+                if (lane == 0) s_small[ns] = SegJob{a, l | in_b};
                 ns++;
-                mx = l > mx ? l : mx;
             });
         if (lane == 0) {
-            s_nb = nb, s_ns = ns;
+            s_nb = nb, s_ns = ns, s_nh = nh;
             s_ob = nb ? atomicAdd(&njobs[0], nb) : 0u;
             s_os = ns ? atomicAdd(&njobs[1], ns) : 0u;
-            if (mx) atomicMax(&njobs[2], mx);
         }
     }
     __syncthreads();
     if (tid < s_nb) big[s_ob + tid] = s_big[tid];
     if (tid < s_ns) small[s_os + tid] = s_small[tid];
+    for (uint32_t h = 0; h < s_nh; h++) {
+        const uint32_t a = s_huge[h].start, l = s_huge[h].len;
+        if (!H.n) {
+            if (tid == 0) atomicMax(&njobs[2], l);
+            continue;
+        }
+        __shared__ uint32_t s_id, s_tile0;
+        const uint32_t nt = (l + kSortTile - 1) / kSortTile;
+        __syncthreads();
+        if (tid == 0) s_id = atomicAdd(&H.n[0], 1u), s_tile0 = atomicAdd(&H.n[1], nt);
+        __syncthreads();
+        const uint32_t id = s_id, t0 = s_tile0;
+        if (tid == 0) H.start[id] = a, H.len[id] = l, H.done[id] = 0u;
+        H.bases[256 * (size_t)id + tid] = 0u;
+        for (uint32_t t = tid; t < nt; t += 256) {
+            const uint32_t p = t * kSortTile;
+            H.tiles[t0 + t] = SortTile{a + p, l - p < (uint32_t)kSortTile ? l - p : (uint32_t)kSortTile, id, t0};
+        }
+    }
 }
+
+// exclusive prefix sum over the 256 threads of a workgroup, and the sum
+__device__ inline uint32_t block_excl_256(uint32_t c, uint32_t &total) {
+    __shared__ uint32_t s_wsum[4];
+    const uint32_t tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
+    const uint32_t incl = wave_incl_scan(c);
+    __syncthreads();  // an earlier call's sums have been read
+    if (lane == 63) s_wsum[w] = incl;
+    __syncthreads();
+    uint32_t pre = 0;
+    for (uint32_t ww = 0; ww < w; ww++) pre += s_wsum[ww];
+    total = s_wsum[0] + s_wsum[1] + s_wsum[2] + s_wsum[3];
+    return pre + incl - c;
+}
+
+// One workgroup per top-8-bit bin: the jobs of its 16-bit segments (hist2[bin * 256 + digit] keys each; the
+// bin starts at base1[bin]).
+__global__ __launch_bounds__(256) void k_msd_jobs(const uint32_t *__restrict__ hist2, const uint32_t *__restrict__ base1,
+                                                  uint32_t cap, SegJob *__restrict__ big, SegJob *__restrict__ small,
+                                                  uint32_t *__restrict__ njobs, HugeList H) {
+    const uint32_t bin = blockIdx.x;
+    const uint32_t c = hist2[bin * 256 + threadIdx.x];
+    uint32_t total;
+    const uint32_t st = base1[bin] + block_excl_256(c, total);
+    emit_seg_jobs(c, st, cap, 0u, big, small, njobs, H);
+}
+
+// The digit counts of the huge segments, tile by tile, and the tiles' look-back words zeroed; the workgroup
+// that counts a segment's last tile turns its counts into bin starts and its pieces into jobs.
+__global__ __launch_bounds__(256) void k_huge_jobs(const uint64_t *__restrict__ keys, HugeList H,
+                                                   uint32_t *__restrict__ lookback, uint32_t cap,
+                                                   SegJob *__restrict__ big, SegJob *__restrict__ small,
+                                                   uint32_t *__restrict__ njobs, uint32_t *__restrict__ err) {
+    __shared__ uint32_t s_h[256], s_last;
+    const uint32_t nt = H.n[1], tid = threadIdx.x;
+    for (uint32_t t = blockIdx.x; t < nt; t += gridDim.x) {
+        const SortTile T = H.tiles[t];
+        s_h[tid] = 0u;
+        lookback[(size_t)t * 256 + tid] = 0u;
+        __syncthreads();
+        // one add per run of equal digits in a wave's row: neighbours in a clustered segment mostly share it
+        for (uint32_t i0 = tid; i0 - tid < T.len; i0 += 8 * 256) {
+            uint32_t d[8];
+#pragma unroll
+            for (uint32_t r = 0; r < 8; r++) {
+                const uint32_t i = i0 + 256 * r;
+                d[r] = i < T.len ? (uint32_t)(keys[T.start + i] >> kMsdShift3) & 255u : 256u;
+            }
+#pragma unroll
+            for (uint32_t r = 0; r < 8; r++) {
+                const uint32_t lane = tid & 63, left = (uint32_t)__shfl_up((int)d[r], 1);
+                const bool first = lane == 0 || left != d[r];
+                const uint64_t after = ballot64(first) & ~(lanemask_lt() | (1ull << lane));
+                const uint32_t end = after ? (uint32_t)__builtin_ctzll(after) : 64u;
+                if (first && d[r] < 256u) atomicAdd(&s_h[d[r]], end - lane);
+            }
+        }
+        __syncthreads();
+        uint32_t *base = H.bases + 256 * (size_t)T.cloud + tid;
+        if (s_h[tid]) atomicAdd(base, s_h[tid]);
+        const uint32_t len = H.len[T.cloud];
+        if (tid == 0) s_last = atomicAdd(&H.done[T.cloud], T.len) + T.len == len ? 1u : 0u;
+        __syncthreads();
+        if (!s_last) continue;
+        // every tile's adds are on their way: the counts are complete once they add up to the length (a
+        // release fence per tile instead would write the whole L2 back)
+        uint32_t c = 0, pre = 0, spins = 0;
+        for (;;) {
+            uint32_t total;
+            c = load_flag(base);
+            pre = block_excl_256(c, total);
+            if (total == len) break;
+            if (++spins > kSpinLimit / 16) {  // the same for every thread
+                if (tid == 0) atomicOr(err, 1u);
+                return;
+            }
+        }
+        const uint32_t st = H.start[T.cloud] + pre;
+        *base = st;
+        HugeList none = {};
+        none.min = kSegMaxLen;
+        emit_seg_jobs(c, st, cap, kSegInB, big, small, njobs, none);
+        __syncthreads();
+    }
+}
+
+constexpr int kNJobs = 6;  // njobs words: k_seg_sort's four, then the split's segments and tiles
 
 // Everything the partition passes start from, in one launch (no host copies or fills in between):
 // zero look-back words, prefix counts, job and tile counters and the error flag; the bin starts of
@@ -628,7 +764,7 @@ __global__ __launch_bounds__(256) void k_part_init(const uint32_t *__restrict__ 
     const size_t g = (size_t)blockIdx.x * 256 + threadIdx.x, stride = (size_t)gridDim.x * 256;
     for (size_t i = g; i < nlook; i += stride) lookback[i] = 0u;
     for (size_t i = g; i < 65536; i += stride) hist2[i] = 0u;
-    if (g < 4) njobs[g] = 0u;
+    if (g < (size_t)kNJobs) njobs[g] = 0u;
     if (g < 32) counters[g] = 0u;
     if (blockIdx.x == 0) {
         __shared__ uint32_t s_w[2][4];
@@ -688,12 +824,20 @@ hipError_t sort_partition(oct_ctx *ctx, uint32_t *counters, uint32_t *errflag, u
     const size_t n = ctx->n;
     const uint32_t *h55 = ctx->hist.p + kRadixPassCount * 256, *h47 = h55 + 256;  // the encode kernel's
     const size_t tiles = (n + kSortTile - 1) / kSortTile;
-    // msd layout (u32 words): bases [2 x 256], hist2 [65536], njobs [4], big and small jobs
-    const size_t o_bases = 0, o_hist2 = 512, o_njobs = o_hist2 + 65536, o_big = o_njobs + 4, o_small = o_big + 2 * kSegJobsMax,
-                 words = o_small + 2 * kSegJobsMax;
+    const bool split = n >= kHugeMinKeys;
+    HugeList huge = {}, none = {};
+    huge.min = (uint32_t)std::min<size_t>(std::max<size_t>(n / 1024, kHugeMin), kSegMaxLen), none.min = kSegMaxLen;
+    const size_t huge_max = split ? n / huge.min + 1 : 0, huge_tiles = split ? tiles + huge_max : 0;
+    // jobs of either kind: at most one per 16-bit segment; of the pieces of huge ones at most 2 * keys / cap + 1
+    const size_t jobs_max = kSegJobsMax + (split ? 2 * (n / cap) + huge_max : 0);
+    // msd layout (u32 words): bases [2 x 256], hist2 [65536], njobs [kNJobs], big and small jobs, huge segments'
+    // tiles, starts, lengths, key counts and bases
+    const size_t o_bases = 0, o_hist2 = 512, o_njobs = o_hist2 + 65536, o_big = o_njobs + kNJobs, o_small = o_big + 2 * jobs_max,
+                 o_tiles = (o_small + 2 * jobs_max + 3) / 4 * 4, o_huge = o_tiles + 4 * huge_tiles,
+                 words = o_huge + (3 + 256) * huge_max;
     hipError_t e;
     if ((e = ctx->msd.reserve(words)) != hipSuccess) return e;
-    if ((e = ctx->lookback.reserve(2 * tiles * 256 + 1)) != hipSuccess) return e;
+    if ((e = ctx->lookback.reserve(2 * tiles * 256 + 1 + huge_tiles * 256)) != hipSuccess) return e;
     if ((e = ctx->p64.reserve(n + kPointPad)) != hipSuccess) return e;
     if ((e = ctx->keys_p.reserve(n)) != hipSuccess) return e;
     if ((e = ctx->vals_p.reserve(n)) != hipSuccess) return e;
@@ -711,7 +855,20 @@ hipError_t sort_partition(oct_ctx *ctx, uint32_t *counters, uint32_t *errflag, u
     k_onesweep<false><<<(unsigned)tiles, kSortBlock, 0, s>>>(ctx->keys[1].p, ctx->vals[1].p, ctx->keys_p.p, ctx->vals_p.p, n,
                                                              kMsdShift1, M + o_bases + 256, ctx->lookback.p + tiles * 256,
                                                              counters + 1, errflag, nullptr, 0u, M + o_hist2);
-    k_msd_jobs<<<256, 256, 0, s>>>(M + o_hist2, M + o_bases + 256, cap, big, small, M + o_njobs);
+    if (split) {
+        huge.tiles = reinterpret_cast<SortTile *>(M + o_tiles);
+        huge.start = M + o_huge, huge.len = huge.start + huge_max, huge.done = huge.len + huge_max;
+        huge.bases = huge.done + huge_max, huge.n = M + o_njobs + 4;
+    }
+    k_msd_jobs<<<256, 256, 0, s>>>(M + o_hist2, M + o_bases + 256, cap, big, small, M + o_njobs, split ? huge : none);
+    if (split) {  // bits 39..46 of the huge segments: keys_p / vals_p -> keys[1] / vals[1]
+        uint32_t *look = ctx->lookback.p + nlook;
+        k_huge_jobs<<<(unsigned)std::min<size_t>(huge_tiles, 2048), 256, 0, s>>>(ctx->keys_p.p, huge, look, cap, big, small,
+                                                                                 M + o_njobs, errflag);
+        k_onesweep<true, true><<<(unsigned)std::min<size_t>(huge_tiles, 512), kSortBlock, 0, s>>>(
+            ctx->keys_p.p, ctx->vals_p.p, ctx->keys[1].p, ctx->vals[1].p, n, kMsdShift3, huge.bases, look, counters + 4, errflag,
+            huge.tiles, 256u, nullptr, huge.n + 1);
+    }
     // every 16-bit segment sorted by one workgroup: keys_p / vals_p -> keys[1] / vals[1], sorted cloud
     k_seg_sort<W, IPT><<<seg_grid<W, IPT>(), W * 64, 0, s>>>(ctx->keys_p.p, ctx->vals_p.p, ctx->keys[1].p, ctx->vals[1].p,
                                                              big, small, M + o_njobs, counters + 2, errflag, ctx->xyz.p,
@@ -828,7 +985,8 @@ hipError_t launch_sort(oct_ctx *ctx, std::string &err) {
     }
     stage_end(ctx, ST_SORT);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    uint32_t fb[2] = {0, 0};  // error flag, longest 16-bit segment
+    uint32_t *fb = ctx->mail->sort;  // error flag, longest segment that no workgroup sorted
+    fb[1] = 0;
     if ((e = hipMemcpyAsync(&fb[0], errflag, sizeof(uint32_t), hipMemcpyDeviceToHost, ctx->stream)) != hipSuccess) return e;
     if (njobs_dev && (e = hipMemcpyAsync(&fb[1], njobs_dev + 2, sizeof(uint32_t), hipMemcpyDeviceToHost, ctx->stream)) != hipSuccess)
         return e;
