@@ -13,6 +13,7 @@
 // range (the reference's lower_bound counting, :317-321); its FP64 centre is getCenter
 // (point_encoder.hpp:517-539) evaluated in the reference's operation order.
 // A last pass writes the leaf-recentred FP32 copy of the cloud used by the FP32 searches.
+#include <cfloat>
 #include <algorithm>
 
 #include "tree_common.hpp"
@@ -288,6 +289,114 @@ __global__ __launch_bounds__(256) void k_node_ext_dev(const NodeRec *__restrict_
     for (uint32_t l = 0; l < (uint32_t)kLvlCount; l++)
         if (s_ctl[l].ls <= u && u < s_ctl[l].le) level = l;
     node_ext_child(nodes, nkey, child, amax, fc, (uint32_t)(t & 7u), level, encoder, ext + ((fc - 1) >> 3));
+}
+
+// The box of every leaf's points relative to the leaf's centre, kRecentreLanes lanes per leaf: the FP32
+// coordinates' extremes, widened by their rounding.
+__global__ __launch_bounds__(256) void k_leaf_box(const float4 *__restrict__ p32, const NodeRec *__restrict__ nodes,
+                                                 const uint32_t *__restrict__ child, const float *__restrict__ amax,
+                                                 uint32_t n_total, PointBox *__restrict__ pbox) {
+    const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const size_t u = t / kRecentreLanes;
+    const uint32_t g = (uint32_t)(t % kRecentreLanes);
+    if (u >= n_total || child[u] != 0) return;
+    const uint32_t first = nodes[u].first, last = nodes[u].last;
+    float v[6] = {FLT_MAX, FLT_MAX, FLT_MAX, FLT_MAX, FLT_MAX, FLT_MAX};  // lo, -hi
+    for (uint32_t i = first + g; i < last; i += kRecentreLanes) {
+        const float4 p = p32[i];
+        v[0] = fminf(v[0], p.x), v[1] = fminf(v[1], p.y), v[2] = fminf(v[2], p.z);
+        v[3] = fminf(v[3], -p.x), v[4] = fminf(v[4], -p.y), v[5] = fminf(v[5], -p.z);
+    }
+    for (int off = kRecentreLanes / 2; off > 0; off >>= 1)
+        for (int a = 0; a < 6; a++) v[a] = fminf(v[a], __shfl_xor(v[a], off));
+    if (g == 0) {
+        PointBox b;
+        for (int a = 0; a < 3; a++) {
+            b.lo[a] = v[a] - fabsf(v[a]) * 2.384185791015625e-07f;  // 2^-22
+            b.hi[a] = -(v[3 + a] - fabsf(v[3 + a]) * 2.384185791015625e-07f);
+        }
+        b.bad = last > first && !(amax[u] < 1e30f) ? 1u : 0u;
+        b.pad = 0;
+        pbox[u] = b;
+    }
+}
+
+// One level of internal nodes [ls, le), 8 lanes per node, from the deepest level up: the children's boxes
+// become the node's record (around the node's centre) and their union its own box.
+__global__ __launch_bounds__(256) void k_node_box(const NodeRec *__restrict__ nodes, const uint32_t *__restrict__ child,
+                                                 const NodeExt *__restrict__ ext, uint32_t ls, uint32_t le, float scale,
+                                                 PointBox *__restrict__ pbox, NodeBox *__restrict__ nbox) {
+    const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t k = (uint32_t)(t & 7u);
+    if (t / 8 >= le - ls) return;
+    const uint32_t u = ls + (uint32_t)(t / 8);
+    const uint32_t fc = child[u];
+    if (fc == 0) return;  // the node's lanes together
+    const uint32_t rec = (fc - 1) >> 3, c = (ext[rec].order[k >> 2] >> (8u * (k & 3u))) & 7u;
+    const NodeRec nu = nodes[u], nv = nodes[fc + k];
+    const PointBox b = pbox[fc + k];
+    const bool some = nv.last > nv.first;
+    const double d[3] = {nv.cx - nu.cx, nv.cy - nu.cy, nv.cz - nu.cz}, cu[3] = {nu.cx, nu.cy, nu.cz};
+    float ch[6] = {}, lo[3], nhi[3], e2 = 0.0f;
+    uint32_t bad = some ? b.bad : 0u;
+    for (int a = 0; a < 3; a++) {
+        lo[a] = nhi[a] = FLT_MAX;
+        if (!some) continue;
+        const double l = d[a] + (double)b.lo[a], h = d[a] + (double)b.hi[a];
+        lo[a] = __double2float_rd(l), nhi[a] = -__double2float_ru(h);
+        const float m = (float)(0.5 * (l + h));
+        const double half = fmax(h - (double)m, (double)m - l);
+        ch[a] = scale * m, ch[3 + a] = scale * __double2float_ru(half * (1.0 + 4.76837158203125e-07));  // 2^-21
+        const float e = fabsf(ch[a]) + ch[3 + a];
+        e2 += e * e;
+        bad |= !(e < 1e15f) ? 1u : 0u;
+    }
+    uint32_t occ = some ? 1u << c : 0u;
+    e2 *= 1.0f + 9.5367431640625e-07f;
+    NodeBox *o = nbox + rec;
+    ChildBox cb;
+    for (int a = 0; a < 3; a++) cb.c[a] = ch[a], cb.h[a] = ch[3 + a];
+    cb.n = nv.last - nv.first, cb.gc = child[fc + k];
+    cb.ctr[0] = nv.cx, cb.ctr[1] = nv.cy, cb.ctr[2] = nv.cz;
+    cb.first = nv.first, cb.amax = ext[rec].amax[c];
+    o->ch[c] = cb;
+    for (int off = 4; off > 0; off >>= 1) {
+        occ |= __shfl_xor(occ, off), bad |= __shfl_xor(bad, off);
+        e2 = fmaxf(e2, __shfl_xor(e2, off));
+        for (int a = 0; a < 3; a++) lo[a] = fminf(lo[a], __shfl_xor(lo[a], off)), nhi[a] = fminf(nhi[a], __shfl_xor(nhi[a], off));
+    }
+    if (k < 3) o->c[k] = cu[k];
+    if (k == 0) {
+        o->ext2 = bad ? __builtin_huge_valf() : e2;
+        o->occ = occ;
+        PointBox p;
+        for (int a = 0; a < 3; a++) p.lo[a] = lo[a], p.hi[a] = -nhi[a];
+        p.bad = bad, p.pad = 0;
+        pbox[u] = p;
+    }
+}
+
+hipError_t launch_boxes(oct_ctx *ctx) {
+    if (ctx->has_boxes) return hipSuccess;
+    const uint32_t nt = ctx->n_total;
+    hipError_t e;
+    if ((e = ctx->pbox.reserve(nt)) != hipSuccess) return e;
+    if ((e = ctx->nbox.reserve(ctx->n_internal + 1)) != hipSuccess) return e;
+    double ext = 0.0;
+    for (int a = 0; a < 3; a++) ext = std::max(ext, 2.0 * fabs(ctx->radii[a]));
+    // 2^-k with 2^k in [4, 8] extents; degenerate or huge boxes keep their unit (their squares would leave FP32)
+    ctx->box_scale = ext > 1e-15 && ext < 1e15 ? (float)exp2(-ceil(log2(4.0 * ext))) : 1.0f;
+    const unsigned nb = (unsigned)(((size_t)nt * kRecentreLanes + 255) / 256);
+    k_leaf_box<<<nb, 256, 0, ctx->stream>>>(ctx->p32.p, ctx->nodes.p, ctx->child.p, ctx->amax.p, nt, ctx->pbox.p);
+    for (int l = (int)ctx->n_levels - 2; l >= 0; l--) {
+        const uint32_t ls = ctx->level_start[l], le = ctx->level_start[l + 1];
+        if (le > ls)
+            k_node_box<<<(unsigned)(((size_t)(le - ls) * 8 + 255) / 256), 256, 0, ctx->stream>>>(
+                ctx->nodes.p, ctx->child.p, ctx->next.p, ls, le, ctx->box_scale, ctx->pbox.p, ctx->nbox.p);
+    }
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+    ctx->has_boxes = true;
+    return hipSuccess;
 }
 
 template <class T>

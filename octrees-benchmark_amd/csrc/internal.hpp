@@ -38,6 +38,31 @@ struct alignas(64) NodeExt {
 };
 static_assert(sizeof(NodeExt) == 192, "NodeExt is three 64-byte lines");
 
+// Tight boxes of the children of one internal node (same index as NodeExt), for the neighbour counts: child
+// combo c's points lie within ch[c].h of ch[c].c per axis, relative to the node's centre, in units of
+// 1 / ctx->box_scale, a power of two above 4 root box extents. ext2: max |p - centre|^2 in these units, or +inf
+// when a point below is not finite in FP32 (the boxes are then not used).
+struct alignas(64) ChildBox {  // one scalar load
+    float c[3], h[3];
+    uint32_t n, gc;       // points, first child (0 = leaf)
+    double ctr[3];        // the child's centre
+    uint32_t first;       // its first point
+    float amax;           // NodeExt::amax
+};
+struct alignas(64) NodeBox {
+    double c[3];
+    float ext2;
+    uint32_t occ;  // bit c: combo c holds points
+    float pad[8];
+    ChildBox ch[8];
+};
+static_assert(sizeof(ChildBox) == 64 && sizeof(NodeBox) == 576, "one scalar load per child");
+// A node's points relative to its own centre, rounded outward; bad: not finite.
+struct alignas(32) PointBox {
+    float lo[3], hi[3];
+    uint32_t bad, pad;
+};
+
 // Points allocated past the end of the sorted clouds (p64, p32): the group kernels read a leaf's points
 // in steps of up to 64 and ignore what lies past it.
 constexpr size_t kPointPad = 64;
@@ -149,6 +174,10 @@ struct oct_ctx {
     oct::DevBuf<uint32_t> nrank;    // per-node rank among split nodes of its level (build scratch)
     oct::DevBuf<float> amax;        // per-leaf max squared norm of its recentred FP32 points
     oct::DevBuf<oct::NodeExt> next;  // per internal node: its children in combo order
+    oct::DevBuf<oct::NodeBox> nbox;  // per internal node: its children's tight boxes (launch_boxes)
+    oct::DevBuf<oct::PointBox> pbox; // per node
+    bool has_boxes = false;          // nbox belongs to the current tree
+    float box_scale = 1.0f;          // its unit
     oct::DevBuf<uint32_t> scan;     // scan scratch
 
     // searches
@@ -242,6 +271,8 @@ struct RadiusLaunch {
     unsigned long long *stats = nullptr;
 };
 hipError_t launch_radius(oct_ctx *ctx, const RadiusLaunch &L);
+// The tight boxes of the current tree (ctx->nbox), unless it has them.
+hipError_t launch_boxes(oct_ctx *ctx);
 hipError_t launch_key_codec(oct_ctx *ctx, int encoder, bool decode, uint32_t *xyz_dev, uint64_t *keys_dev, size_t n);
 // One kNN launch. Query slot s (0..nq-1) processes query id order[s] (or s); the centre is qxyz[id]
 // if given, else the sorted point qidx[id] (or qoff + id); outputs (nq x k, row id) go to idx and

@@ -381,6 +381,19 @@ constexpr int count_waves() {
     if (ALGO == OCT_ALGO_NEIGHBORS || !(KERNEL == OCT_KERNEL_SPHERE || KERNEL == OCT_KERNEL_CIRCLE)) return 2;
     return PREC == OCT_PREC_FP32_RECHECK ? 7 : 6;
 }
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+// leaf_mfma's terms of the queries that want the leaf, compacted
+struct MfmaQueries {
+    struct alignas(16) Lim {
+        uint32_t lim, home;  // band limit (float bits), lane
+        __device__ void operator=(const uint2 &v) { lim = v.x, home = v.y; }
+    };
+    float4 u[64];  // -2 b, 1
+    float4 c[64];  // C four times: the accumulator the products are added to
+    Lim lh[64];    // 1 KB after c
+    alignas(16) uint32_t acc[64];
+};
 // One wave tile (G queries) of a search, run by one wave. MODE 0: neighbour counts. MODE 1 (range lists,
 // G = 64): counts and list-entry counts. MODE 2 (G = 64): the lists, in the reference's emission order.
 template <int KERNEL, int ALGO, int PREC, int G, bool STATS, int MODE = 0>
@@ -394,6 +407,12 @@ __device__ __attribute__((always_inline)) inline void count_tile(const SearchArg
     // per 4-wave block). Both take two loads per lane; 96 FP32 points (three) ran 4 % slower, 48
     // FP64 points instead of 32 (fewer chunks for the larger leaves) 4 % faster.
     constexpr int CAP = kFp32 ? kStageBytes / 32 : 48;
+    // leaf tests on the matrix cores (leaf_mfma): FP32 sphere counts with one lane per query
+    constexpr bool kMfma = kFp32 && KERNEL == OCT_KERNEL_SPHERE && G == 64 && MODE == 0;
+    // children judged by their tight boxes; not when the search counters are asked for, which are those of the
+    // octree cells, nor for OCT_ALGO_NEIGHBORS, whose box overlaps take few comparisons (5 M tile, r = 1: 1.45
+    // against 1.67 ms with boxes)
+    constexpr bool kTight = kMfma && !STATS && (ALGO == OCT_ALGO_PRUNE || ALGO == OCT_ALGO_STRUCT);
     constexpr int SMX = S > 16 ? S : 16;                               // largest lane-group count of a leaf
     constexpr int PAD = kUnroll * SMX + SMX;                           // sentinel + row-padding slots after a chunk
     __shared__ uint32_t s_node[kWaves][kStack];
@@ -404,7 +423,8 @@ __device__ __attribute__((always_inline)) inline void count_tile(const SearchArg
     __shared__ uint32_t s_rtot[kWaves][64];  // remapped leaf: count of compacted query r
     __shared__ uint64_t s_hits[MODE ? kWaves : 1][MODE ? 64 : 1];     // its hits (lists)
     __shared__ uint64_t s_inm[MODE == 2 ? kWaves : 1][8];             // INSIDE children of the popped node (query masks)
-    __shared__ __attribute__((aligned(16))) unsigned char s_stage[kWaves][(CAP + PAD) * (kFp32 ? 16 : 32)];
+    __shared__ __attribute__((aligned(16))) unsigned char s_stage[kMfma ? 1 : kWaves][kMfma ? 16 : (CAP + PAD) * (kFp32 ? 16 : 32)];
+    __shared__ MfmaQueries s_mq[kMfma ? kWaves : 1];
 
     const uint32_t w = threadIdx.x >> 6;
     const uint32_t lane = threadIdx.x & 63;
@@ -422,8 +442,9 @@ __device__ __attribute__((always_inline)) inline void count_tile(const SearchArg
     ConstDouble *radp = const_doubles(a.radtab) + 66 * cloud;  // level radii: radp[3 * level + axis]
     const bool valid = slot < a.nq && j < nvt;
     const uint64_t qbit = 1ull << j;
-    float4 *sp32 = reinterpret_cast<float4 *>(&s_stage[w][0]);
-    double4 *sp64 = reinterpret_cast<double4 *>(&s_stage[w][0]);
+    float4 *sp32 = reinterpret_cast<float4 *>(&s_stage[kMfma ? 0 : w][0]);
+    double4 *sp64 = reinterpret_cast<double4 *>(&s_stage[kMfma ? 0 : w][0]);
+    MfmaQueries &mq = s_mq[kMfma ? w : 0];
 
     Query q;
     uint32_t qid = 0;
@@ -445,6 +466,18 @@ __device__ __attribute__((always_inline)) inline void count_tile(const SearchArg
     if (KERNEL == OCT_KERNEL_CUBE || KERNEL == OCT_KERNEL_SQUARE) box_radii(a, valid, qid, q);
     const float qRf = (float)q.R;
 
+    const float qRs = kTight ? qRf * (a.box_scale * a.box_scale) : 0.0f;
+    auto clamp01 = [](float v) -> float { return __builtin_amdgcn_fmed3f(v, 0.0f, 1.0f); };  // an output modifier
+    // tight boxes: not for a wave with a query whose scale their margin does not cover
+    bool boxes = false;
+    if constexpr (kTight) {
+        if (a.nbox) {
+            ConstNodeBox &B = node_box(a.nbox, 0);
+            const float dx = (float)(q.x - B.c[0]), dy = (float)(q.y - B.c[1]), dz = (float)(q.z - B.c[2]);
+            const float far = __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, dz * dz)) + qRf;
+            boxes = ballot64(valid && !(q.r >= 0.0 && qRf > a.tight_min && far < 1e29f)) == 0;
+        }
+    }
     uint32_t cnt = 0, ecnt = 0;
     uint32_t *out = nullptr;  // MODE 2: the next word of the lane's list
     if (MODE == 2 && valid) out = a.entries + a.offsets[qid] * (kRanges ? 2u : 1u);
@@ -664,6 +697,169 @@ __device__ __attribute__((always_inline)) inline void count_tile(const SearchArg
         }
         cnt += lc;
         if (STATS) n_tslots += 64ull * ((last - first + Sp - 1) / Sp);
+    };
+
+    // Tight boxes (kTight): a child whose points' box lies inside a query's sphere, or outside it, by a margin of
+    // 2^-18 (ext2 + |b|^2 + R) needs no further look, whatever the octree cells say: every point then passes, or
+    // fails, its own test, and no cell that holds it can have been judged otherwise up to rounding. The margin
+    // is 64 u (u = 2^-24) of that sum; the FP32 distances to the box are within 45 u. Between, a child is
+    // descended into or its points are tested. The FP64 judgement of the cells (the reference's answer) can
+    // differ from the points' own tests only where a point lies on the sphere to the last FP64 bits: such a point
+    // is in the band of its leaf's test, and its lane's points are then decided by path_class, the reference's
+    // walk itself. tie_scale sqrt(S) + 2^-46 S bounds the cells' and points' rounding (S as above, coordinates
+    // up to 2^46 tie_scale), and S > tight_min keeps it below the margin's slack.
+    //
+    // 50 M tile, r = 2.5 (all points): 1418 point tests per query instead of 1684, 38.2 -> 29.9 ms with leaf_mfma;
+    // leaf_mfma alone, the cells judged in FP64, 36.8 ms.
+
+    // How the reference's walk from the root decides the leaf that starts at point `first` for query qr:
+    // INSIDE or OUTSIDE at a node on the way, or OVERLAP down to the leaf. The whole wave calls it.
+    auto path_class = [&](const Query &qr, uint32_t first) -> int {
+        int cls = J_OVERLAP;
+        uint32_t node = root;
+        for (uint32_t d = 0; d <= kMaxDepth; d++) {
+            const NodeRec nr = a.nodes[node];
+            if (cls == J_OVERLAP) {
+                const double rx = radp[3 * d], ry = radp[3 * d + 1], rz = radp[3 * d + 2];
+                if (ALGO == OCT_ALGO_NEIGHBORS)
+                    cls = overlap64<KERNEL>(qr, nr.cx, nr.cy, nr.cz, rx, ry, rz) ? J_OVERLAP : J_OUTSIDE;
+                else
+                    cls = classify64<KERNEL>(qr, nr.cx, nr.cy, nr.cz, rx, ry, rz);
+            }
+            const uint32_t c0 = uniform_u32(a.child[node]);
+            if (c0 == 0) break;
+            const NodeRec cr = a.nodes[c0 + (lane & 7u)];
+            const uint64_t at = ballot64(cr.first <= first && first < cr.last) & 0xffull;
+            if (!at) break;
+            node = c0 + (uint32_t)__builtin_ctzll(at);
+        }
+        return cls;
+    };
+
+    // The leaf tests on the matrix cores. t of leaf() is the product of a point's (x, y, z, w) with a query's
+    // (-2 b, 1) plus its C: v_mfma_f32_16x16x4 makes it for 16 points and 16 queries. The queries that want the
+    // leaf (m) are compacted into columns, their terms go through LDS once; a leaf's 64 points are one load,
+    // turned into four row operands by lane swaps. Lane 16 g + c of a result holds points 4 g .. 4 g + 3 and
+    // query c; hits and the band are counted per lane as in leaf(), whose error bound holds for any order of the
+    // sum and either rounding. Vector FMAs run at the matrix rate (2 cycles per wave here), so the gain is
+    // what surrounds them: 4 LDS reads and a staging pass fewer per 4 tests. Here 2-operand FP32 and integer
+    // instructions on VGPRs take 2.5 cycles, all others (3 operands, scalar operands, compares, min, FP64) 4.3.
+    auto leaf_mfma = [&](const uint64_t m, const float am, const NodeRec &nr) {
+        const uint32_t first = nr.first, last = nr.last;
+        if (STATS) n_test += (uint64_t)__popcll(m) * (last - first);
+        const uint32_t mc = (uint32_t)__popcll(m);
+        const bool act = __builtin_amdgcn_inverse_ballot_w64(m);
+        const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+        const float4 sent = make_float4(0.0f, 0.0f, 0.0f, 1e30f);  // outside every query, above the band
+        float4 v = sent;
+        if (lane < last - first) v = (a.p32 + first)[lane];
+        if (act) {
+            const float bx = (float)(q.x - nr.cx), by = (float)(q.y - nr.cy), bz = (float)(q.z - nr.cz);
+            const float b2 = __builtin_fmaf(bx, bx, __builtin_fmaf(by, by, bz * bz));
+            const float sum = (am + b2) + qRf;
+            const float hw = 3.814697265625e-06f * sum;  // 2^-18
+            const float C = (hw - qRf) + b2;
+            float lim = 2.0f * hw;
+            if (!boxes && !(sum < 1e30f && sum > 1e-30f)) lim = __uint_as_float(0xffffffffu);
+            mq.u[rank] = make_float4(-2.0f * bx, -2.0f * by, -2.0f * bz, 1.0f);
+            mq.c[rank] = make_float4(C, C, C, C);
+            mq.lh[rank] = make_uint2(__float_as_uint(lim), lane);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        const uint32_t nt = (mc + 15) >> 4, col = lane & 15;
+        for (uint32_t base = first; base < last; base += 64) {
+            const uint32_t P = (last - base) < 64u ? (last - base) : 64u;
+            if (base != first) {
+                v = sent;
+                if (lane < P) v = (a.p32 + base)[lane];
+            }
+            // the four terms of points 16 i .. 16 i + 15 into one register
+            const u32x2 s02 = __builtin_amdgcn_permlane32_swap(__float_as_uint(v.x), __float_as_uint(v.z), false, false);
+            const u32x2 s13 = __builtin_amdgcn_permlane32_swap(__float_as_uint(v.y), __float_as_uint(v.w), false, false);
+            const u32x2 a01 = __builtin_amdgcn_permlane16_swap(s02[0], s13[0], false, false);
+            const u32x2 a23 = __builtin_amdgcn_permlane16_swap(s02[1], s13[1], false, false);
+            const float A[4] = {__uint_as_float(a01[0]), __uint_as_float(a01[1]), __uint_as_float(a23[0]), __uint_as_float(a23[1])};
+            uint32_t band = 0;  // bit t: a point of this lane's is in the band of its query of tile t
+            uint32_t acc = 0;   // byte t: 8 x the hits of this lane's points and its query of tile t (at most 16)
+            auto rows = [&](auto rt_c) {
+                constexpr int RT = decltype(rt_c)::value;
+                const float *pu = reinterpret_cast<const float *>(mq.u) + col * 4 + (lane >> 4);
+                const float4 *pc = mq.c + col;
+                for (uint32_t t = 0; t < nt; t++, pu += 64, pc += 16) {
+                    const float B = *pu;
+                    const float4 c4 = *pc;
+                    const uint32_t lim = reinterpret_cast<const MfmaQueries::Lim *>(pc + 64)->lim;  // mq.lh
+                    const f32x4 cq = {c4.x, c4.y, c4.z, c4.w};
+                    f32x4 d[RT];
+#pragma unroll
+                    for (int i = 0; i < RT; i++) d[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(A[i], B, cq, 0, 0, 0);
+                    uint32_t c8 = 0, mnb = 0xffffffffu;
+#pragma unroll
+                    for (int i = 0; i < RT; i++) {
+                        const uint32_t d0 = __float_as_uint(d[i][0]), d1 = __float_as_uint(d[i][1]);
+                        const uint32_t d2 = __float_as_uint(d[i][2]), d3 = __float_as_uint(d[i][3]);
+                        c8 = __builtin_popcount(__builtin_amdgcn_perm(d0, d1, 0x0c0c0b09u)) + c8;
+                        c8 = __builtin_popcount(__builtin_amdgcn_perm(d2, d3, 0x0c0c0b09u)) + c8;
+                        mnb = min(min(mnb, d0), d1);
+                        mnb = min(min(mnb, d2), d3);
+                    }
+                    const uint64_t bm = ballot64(mnb <= lim);
+                    if (bm) band |= __builtin_amdgcn_inverse_ballot_w64(bm) ? 1u << t : 0u;
+                    acc += c8 << (8 * t);
+                }
+                if (STATS) n_tslots += 256ull * RT * nt;
+            };
+            if (P > 48)
+                rows(std::integral_constant<int, 4>{});
+            else if (P > 32)
+                rows(std::integral_constant<int, 3>{});
+            else if (P > 16)
+                rows(std::integral_constant<int, 2>{});
+            else
+                rows(std::integral_constant<int, 1>{});
+            for (uint32_t t = 0; ballot64(band >> t); t++) {  // rare: exact FP64 counts of a lane's points
+                const bool redo = ((band >> t) & 1u) && col + 16 * t < mc;
+                if (!ballot64(redo)) continue;
+                const uint32_t src = mq.lh[col + 16 * t].home & 63u;
+                Query qr = q;
+                qr.x = bperm_f64(src, q.x), qr.y = bperm_f64(src, q.y), qr.z = bperm_f64(src, q.z);
+                qr.r = bperm_f64(src, q.r), qr.R = qr.r * qr.r;
+                bool tie = false;
+                uint32_t np = 0, c8 = 0;
+                if (redo) {
+                    const double bx = qr.x - nr.cx, by = qr.y - nr.cy, bz = qr.z - nr.cz;
+                    const double sc = ((double)am + (bx * bx + by * by + bz * bz)) + qr.R;
+                    const double thr = a.tie_scale * (double)sqrtf((float)sc) + 1.4210854715202004e-14 * sc;  // 2^-46
+                    for (uint32_t i = 4 * (lane >> 4); i < P; i = (i & 3u) == 3u ? i + 13u : i + 1u, np++) {
+                        const double4 pd = a.p64[base + i];
+                        c8 += inside64<KERNEL>(qr, pd.x, pd.y, pd.z) ? 8u : 0u;
+                        const double dx = pd.x - qr.x, dy = pd.y - qr.y, dz = pd.z - qr.z;
+                        tie |= !(fabs(((dx * dx + dy * dy) + dz * dz) - qr.R) > thr);
+                        if (STATS) n_recheck++;
+                    }
+                }
+                if (boxes && ballot64(tie)) {
+                    qr.lox = qr.x - qr.r, qr.loy = qr.y - qr.r, qr.loz = qr.z - qr.r;
+                    qr.hix = qr.x + qr.r, qr.hiy = qr.y + qr.r, qr.hiz = qr.z + qr.r;
+                    const int cls = path_class(qr, first);
+                    if (tie && cls != J_OVERLAP) c8 = cls == J_INSIDE ? 8u * np : 0u;
+                }
+                if (redo) acc = (acc & ~(0xffu << (8 * t))) | (c8 << (8 * t));
+            }
+            // word (column, row group) of the hits: a query's four words hold its count in byte rank / 16
+            mq.acc[4 * col + (lane >> 4)] = acc >> 3;
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            if (act) {
+                const uint4 h = *reinterpret_cast<const uint4 *>(mq.acc + 4 * (rank & 15u));
+                cnt += ((h.x + h.y + h.z + h.w) >> (8 * (rank >> 4))) & 0xffu;
+            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+        }
     };
 
     // Lists: a leaf's points are tested as for counts, but each lane collects its hits as a bit mask, 64 points
@@ -940,7 +1136,7 @@ __device__ __attribute__((always_inline)) inline void count_tile(const SearchArg
     // Stack entries hold the FIRST CHILD of an OVERLAP internal node; its NodeExt record is one
     // uniform load.
     uint32_t sp = 0;
-    bool overflow = false;  // wave-uniform: a push found the stack full (cannot happen within 21 levels)
+    uint32_t overflow = 0;  // wave-uniform: a push found the stack full (cannot happen within 21 levels)
     {
         const NodeRec nr = a.nodes[root];
         const int jr = judge(valid, nr, 0);
@@ -962,7 +1158,9 @@ __device__ __attribute__((always_inline)) inline void count_tile(const SearchArg
                 ur.cx = nr.cx, ur.cy = nr.cy, ur.cz = nr.cz;
                 ur.first = uniform_u32(nr.first), ur.last = uniform_u32(nr.last);
                 if (ur.last > ur.first) {
-                    if constexpr (MODE == 0)
+                    if constexpr (kMfma)
+                        leaf_mfma(ov, a.amax[root], ur);
+                    else if constexpr (MODE == 0)
                         leaf(ov, a.amax[root], ur);
                     else
                         leaf_lists(ov, a.amax[root], ur);
@@ -981,6 +1179,49 @@ __device__ __attribute__((always_inline)) inline void count_tile(const SearchArg
         ConstNodeExt &E = node_ext(a.next, (fc - 1) >> 3);
         // lanes whose query wants the node: bit j of m for lane g * G + j
         const uint64_t actm = G == 64 ? m : ballot64((m & qbit) != 0);
+        if constexpr (kTight) {
+            ConstNodeBox &B = node_box(a.nbox, (fc - 1) >> 3);
+            if (boxes && B.ext2 < 1e29f) {
+                const float bx = a.box_scale * (float)(q.x - B.c[0]), by = a.box_scale * (float)(q.y - B.c[1]);
+                const float bz = a.box_scale * (float)(q.z - B.c[2]);
+                const float b2 = __builtin_fmaf(bx, bx, __builtin_fmaf(by, by, bz * bz));
+                const float hw = 3.814697265625e-06f * ((B.ext2 + b2) + qRs);  // 2^-18
+                const float rin = qRs - hw, rout = qRs + hw;
+                const uint32_t occ = B.occ;
+                // each child's record is loaded while the one before it is judged
+                uint32_t todo = occ, c = (uint32_t)__builtin_ctz(occ | 256u);
+                u32x16 nx = child_box(B, c & 7u);
+                while (todo) {
+                    const u32x16 x = nx;
+                    todo &= todo - 1u;
+                    c = (uint32_t)__builtin_ctz(todo | 256u);
+                    nx = child_box(B, c & 7u);
+                    const float hx = __uint_as_float(x[3]), hy = __uint_as_float(x[4]), hz = __uint_as_float(x[5]);
+                    const float ex = fabsf(bx - __uint_as_float(x[0])), ey = fabsf(by - __uint_as_float(x[1]));
+                    const float ez = fabsf(bz - __uint_as_float(x[2]));
+                    const float mx = ex + hx, my = ey + hy, mz = ez + hz;
+                    const float fx = clamp01(ex - hx), fy = clamp01(ey - hy), fz = clamp01(ez - hz);
+                    const uint64_t in = m & ballot64(__builtin_fmaf(mx, mx, __builtin_fmaf(my, my, mz * mz)) <= rin);
+                    const uint64_t ov = m & ~in & ~ballot64(__builtin_fmaf(fx, fx, __builtin_fmaf(fy, fy, fz * fz)) > rout);
+                    if (__builtin_amdgcn_inverse_ballot_w64(in)) cnt += x[6];
+                    if (ov) {
+                        if (x[7] == 0) {
+                            NodeRec ur;
+                            auto f64 = [](uint32_t lo, uint32_t hi) { return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo)); };
+                            ur.cx = f64(x[8], x[9]), ur.cy = f64(x[10], x[11]), ur.cz = f64(x[12], x[13]);
+                            ur.first = x[14], ur.last = x[14] + x[6];
+                            leaf_mfma(ov, __uint_as_float(x[15]), ur);
+                        } else if (sp < kStack) {
+                            s_node[w][sp] = x[7], s_mask[w][sp] = ov, s_depth[w][sp] = (uint8_t)d;
+                            sp++;
+                        } else {
+                            overflow = 1;
+                        }
+                    }
+                }
+                continue;
+            }
+        }
         uint64_t inl[8], ovl[8];
         judge8(E, d, actm, inl, ovl);
         if (STATS) n_class += 8ull * __popcll(m), n_cslots += 64ull * 8;
@@ -1027,20 +1268,20 @@ __device__ __attribute__((always_inline)) inline void count_tile(const SearchArg
                         s_node[w][sp] = gc, s_mask[w][sp] = om, s_depth[w][sp] = (uint8_t)d;
                         sp++;
                     } else {
-                        overflow = true;
+                        overflow = 1;
                     }
                 }
             }
         } else {
             // INSIDE children first: group 0's lanes (0 .. G - 1) hold the counts
-    #pragma unroll
+#pragma unroll
             for (int c = 0; c < 8; c++)
                 if (__builtin_amdgcn_inverse_ballot_w64(inl[c] & gmask)) {
                     cnt += E.last[c] - E.first[c];
                     if (MODE == 1) ecnt++;  // NeighborSet::addRange keeps empty ranges (neighbor_set.hpp:84-89)
                 }
             uint32_t leaves = 0;  // combos of the OVERLAP non-empty leaf children (bit c)
-    #pragma unroll
+#pragma unroll
             for (int c = 0; c < 8; c++) {
                 const uint32_t f = E.first[c], l = E.last[c];
                 const uint64_t ov = ovl[c] & gmask;  // ballots: uniform already
@@ -1055,7 +1296,7 @@ __device__ __attribute__((always_inline)) inline void count_tile(const SearchArg
                         s_node[w][sp] = gc, s_mask[w][sp] = ov, s_depth[w][sp] = (uint8_t)d;
                         sp++;
                     } else {
-                        overflow = true;
+                        overflow = 1;
                     }
                 }
             }
@@ -1073,7 +1314,9 @@ __device__ __attribute__((always_inline)) inline void count_tile(const SearchArg
                 NodeRec ur;
                 ur.cx = E.ax[c & 1], ur.cy = E.ax[2 + ((c >> 1) & 1)], ur.cz = E.ax[4 + ((c >> 2) & 1)];
                 ur.first = E.first[c], ur.last = E.last[c];
-                if constexpr (MODE == 0)
+                if constexpr (kMfma)
+                    leaf_mfma(ov, E.amax[c], ur);
+                else if constexpr (MODE == 0)
                     leaf(ov, E.amax[c], ur);
                 else
                     leaf_lists(ov, E.amax[c], ur);
@@ -1238,6 +1481,21 @@ hipError_t launch_radius(oct_ctx *ctx, const RadiusLaunch &L) {
     a.amax = ctx->amax.p;
     a.nodes = ctx->nodes.p;
     a.next = ctx->next.p;
+    a.nbox = nullptr, a.tie_scale = 0.0, a.tight_min = a.box_scale = 0.0f;
+    if (L.mode == 0 && L.group == 64 && L.kernel == OCT_KERNEL_SPHERE && L.precision == OCT_PREC_FP32_RECHECK &&
+        (L.algo == OCT_ALGO_PRUNE || L.algo == OCT_ALGO_STRUCT) && !L.tile_info && !L.stats && ctx->n_total > 1) {
+        const hipError_t e = launch_boxes(ctx);
+        if (e != hipSuccess && e != hipErrorOutOfMemory) return e;
+        double mc = 0.0;
+        for (int k = 0; k < 3; k++) mc = std::max(mc, ctx->geo[66 + k]);
+        if (e == hipSuccess)
+            a.nbox = ctx->nbox.p;
+        else
+            (void)hipGetLastError();  // no room for the boxes: the cells are judged
+        a.box_scale = ctx->box_scale;
+        a.tie_scale = mc * 1.4210854715202004e-14;                                // 2^-46
+        a.tight_min = (float)std::max(1e-30, mc * mc * 8.881784197001252e-16);  // (2^-25 mc)^2
+    }
     a.child = ctx->child.p;
     a.order = L.order;
     a.qidx = L.qidx;

@@ -18,6 +18,10 @@ struct SearchArgs {
     const float *__restrict__ amax;
     const NodeRec *__restrict__ nodes;
     const NodeExt *__restrict__ next;
+    const NodeBox *__restrict__ nbox;  // tight boxes (one cloud, FP32 sphere counts), or null
+    double tie_scale;  // 2^-46 x the largest coordinate of the root box: see leaf_exact
+    float box_scale;   // unit of the boxes
+    float tight_min;   // smallest squared distance scale at which the boxes' margin covers the FP64 rounding
     const uint32_t *__restrict__ child;
     const uint32_t *__restrict__ order;
     const uint32_t *__restrict__ qidx;
@@ -63,6 +67,12 @@ struct Query {
 typedef const __attribute__((address_space(4))) NodeExt ConstNodeExt;
 typedef const __attribute__((address_space(4))) double ConstDouble;
 __device__ inline ConstDouble *const_doubles(const double *p) { return (ConstDouble *)(uintptr_t)p; }
+typedef const __attribute__((address_space(4))) NodeBox ConstNodeBox;
+__device__ inline ConstNodeBox &node_box(const NodeBox *p, uint32_t i) { return ((ConstNodeBox *)(uintptr_t)p)[i]; }
+typedef uint32_t u32x16 __attribute__((ext_vector_type(16)));
+__device__ inline u32x16 child_box(ConstNodeBox &b, uint32_t c) {  // the words of b.ch[c]
+    return ((const __attribute__((address_space(4))) u32x16 *)b.ch)[c];
+}
 __device__ inline ConstNodeExt &node_ext(const NodeExt *p, uint32_t i) {
     return ((ConstNodeExt *)(uintptr_t)p)[i];
 }
