@@ -21,6 +21,16 @@ void stage_end(oct_ctx *ctx, Stage s) {
     (void)hipEventRecord(ctx->ev1[s], ctx->stream);
     ctx->ev_used[s] = true;
 }
+// Queries per wave for a count-mode search of nq queries, about one every 1 / density points of the sorted
+// cloud: an explicit override; 0 (the group kernel, 8 lanes per query) for few or scattered queries; else
+// the autotuned number, else 64. A wave of 64 queries shares the judgements and staged points of one
+// traversal, but 2^17 queries are only two such waves per SIMD, and far-apart queries share little.
+// Sphere counts, ns per query, group kernel / 64 per wave: 5 M tile, every point of a run, r = 1: 131 k
+// queries 0.96 / 1.61, 2 M 0.90 / 0.35; one point in 64, r = 2.5: 78 k queries 4.1 / 15; 40 M tile, one in 8:
+// 524 k 3.8 / 3.2; one in 32: 524 k 4.8 / 4.8; 40 M box, one in 8: 2.8 / 2.6, one in 32: 3.2 / 4.7.
+constexpr size_t kUnionMinQueries = 1u << 17;
+constexpr double kUnionMinDensity = 1.0 / 16;
+bool shared_traversal(size_t nq, double density) { return nq > kUnionMinQueries && density >= kUnionMinDensity; }
 }  // namespace oct
 
 namespace {
@@ -679,16 +689,6 @@ static int check_search_args(oct_ctx *ctx, int kernel, int algo, int precision, 
     return OCT_OK;
 }
 
-// Queries per wave for a count-mode search of nq queries, about one every 1 / density points of the sorted
-// cloud: an explicit override; 0 (the group kernel, 8 lanes per query) for few or scattered queries; else
-// the autotuned number, else 64. A wave of 64 queries shares the judgements and staged points of one
-// traversal, but 2^17 queries are only two such waves per SIMD, and far-apart queries share little.
-// Sphere counts, ns per query, group kernel / 64 per wave: 5 M tile, every point of a run, r = 1: 131 k
-// queries 0.96 / 1.61, 2 M 0.90 / 0.35; one point in 64, r = 2.5: 78 k queries 4.1 / 15; 40 M tile, one in 8:
-// 524 k 3.8 / 3.2; one in 32: 524 k 4.8 / 4.8; 40 M box, one in 8: 2.8 / 2.6, one in 32: 3.2 / 4.7.
-constexpr size_t kUnionMinQueries = 1u << 17;
-constexpr double kUnionMinDensity = 1.0 / 16;
-static bool shared_traversal(size_t nq, double density) { return nq > kUnionMinQueries && density >= kUnionMinDensity; }
 static int radius_group(const oct_ctx *ctx, int kernel, int algo, int precision, size_t nq, double density) {
     if (ctx->group_override >= 0) return ctx->group_override;
     if (!shared_traversal(nq, density)) return 0;

@@ -271,6 +271,9 @@ struct RadiusLaunch {
     unsigned long long *stats = nullptr;
 };
 hipError_t launch_radius(oct_ctx *ctx, const RadiusLaunch &L);
+// Whether nq queries, `density` of the points they lie among, are counted 64 per wave with one traversal (else
+// each by its own).
+bool shared_traversal(size_t nq, double density);
 // The tight boxes of the current tree (ctx->nbox), unless it has them.
 hipError_t launch_boxes(oct_ctx *ctx);
 hipError_t launch_key_codec(oct_ctx *ctx, int encoder, bool decode, uint32_t *xyz_dev, uint64_t *keys_dev, size_t n);

@@ -96,28 +96,22 @@ __device__ inline void judge_node(const Query &q, const NodeRec &n, double rx, d
     }
 }
 
-// MODE 0: neighbour counts; 1: counts and list-entry counts; 2: fill the lists at their offsets.
-template <int KERNEL, int ALGO, int PREC, int MODE>
-__global__ __launch_bounds__(kSearchBlock) void k_group(const SearchArgs a) {
+// One wave's queries (tile: 8 slots). MODE 0: neighbour counts; 1: counts and list-entry counts; 2: fill the
+// lists at their offsets. root and s_rad (level radii): the slots' cloud; limit: the first slot past its
+// valid ones.
+template <int KERNEL, int ALGO, int PREC, int MODE, class Items>
+__device__ __attribute__((always_inline)) inline void group_tile(const SearchArgs &a, const uint32_t tile, const uint32_t root,
+                                                                 const uint32_t limit, Items &Q, const double *s_rad,
+                                                                 uint32_t *s_gc) {
     constexpr bool kFp32 = PREC == OCT_PREC_FP32_RECHECK && (KERNEL == OCT_KERNEL_SPHERE || KERNEL == OCT_KERNEL_CIRCLE);
     constexpr bool kRanges = ALGO == OCT_ALGO_STRUCT || ALGO == OCT_ALGO_APPROX;  // lists of [first, last) ranges
     constexpr uint32_t kInside = 0x80000000u;
     constexpr uint64_t kBit0 = 0x0101010101010101ull;  // the first lane of every group
-    __shared__ GroupItems<kFp32> s_items[kWaves];
-    __shared__ double s_rad[3 * (kMaxDepth + 1)];
-    extern __shared__ uint32_t s_gc_all[];  // per wave, per level: each lane's child's first child
-    for (uint32_t i = threadIdx.x; i < 3 * (kMaxDepth + 1); i += kSearchBlock) s_rad[i] = a.radtab[i];
-    __syncthreads();
-
-    const uint32_t w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const uint32_t lane = threadIdx.x & 63;
     const uint32_t grp = lane >> 3, c = lane & 7u, gshift = lane & 56u;
     const uint32_t below = (1u << c) - 1u;
-    uint32_t *s_gc = s_gc_all + (size_t)w * a.levels * 64;
-    GroupItems<kFp32> &Q = s_items[w];
-    const uint32_t tile = blockIdx.x * kWaves + w;
-    if (uniform_u32(tile * kGroupsPerWave) >= a.nq) return;
     const uint32_t slot = tile * kGroupsPerWave + grp;
-    const bool valid = slot < a.nq;
+    const bool valid = slot < limit;
     auto wsync = [&]() {
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
@@ -304,7 +298,7 @@ __global__ __launch_bounds__(kSearchBlock) void k_group(const SearchArgs a) {
     };
 
     // root (singleTraversal, linear_octree.hpp:655-662): judged by the group's first lane
-    take(valid && c == 0, a.nodes[0], a.child[0], a.amax[0], 0);
+    take(valid && c == 0, a.nodes[root], a.child[root], a.amax[root], 0);
     for (;;) {
         for (;;) {
             const bool go = lvl != 0 && qn <= (uint32_t)(kGroupQueue - 8);
@@ -356,6 +350,52 @@ __global__ __launch_bounds__(kSearchBlock) void k_group(const SearchArgs a) {
             atomicAdd(&a.stats[4], 64ull * n_csteps);
             atomicAdd(&a.stats[5], 128ull * n_tsteps);
         }
+    }
+}
+
+template <int PREC, int KERNEL>
+constexpr bool group_fp32() {
+    return PREC == OCT_PREC_FP32_RECHECK && (KERNEL == OCT_KERNEL_SPHERE || KERNEL == OCT_KERNEL_CIRCLE);
+}
+
+template <int KERNEL, int ALGO, int PREC, int MODE>
+__global__ __launch_bounds__(kSearchBlock) void k_group(const SearchArgs a) {
+    __shared__ GroupItems<group_fp32<PREC, KERNEL>()> s_items[kWaves];
+    __shared__ double s_rad[3 * (kMaxDepth + 1)];
+    extern __shared__ uint32_t s_gc_all[];  // per wave, per level: each lane's child's first child
+    for (uint32_t i = threadIdx.x; i < 3 * (kMaxDepth + 1); i += kSearchBlock) s_rad[i] = a.radtab[i];
+    __syncthreads();
+    const uint32_t w = threadIdx.x >> 6, tile = blockIdx.x * kWaves + w;
+    if (uniform_u32(tile * kGroupsPerWave) >= a.nq) return;
+    group_tile<KERNEL, ALGO, PREC, MODE>(a, tile, 0u, a.nq, s_items[w], s_rad, s_gc_all + (size_t)w * a.levels * 64);
+}
+
+// Counts over a forest (batches): resident waves take eighths of the 64-slot wave tiles, each of one cloud,
+// from a counter until the device-resident number of tiles has been served.
+// Forms chosen as for one cloud (shared_traversal). 48 clouds of 12 M points together, sparse queries:
+// k_count_queue 2.65 ms, this one 0.55.
+template <int KERNEL, int ALGO, int PREC>
+__global__ __launch_bounds__(kSearchBlock) void k_group_queue(const SearchArgs a) {
+    __shared__ GroupItems<group_fp32<PREC, KERNEL>()> s_items[kWaves];
+    __shared__ double s_rad[kWaves][3 * (kMaxDepth + 1)];
+    extern __shared__ uint32_t s_gc_all[];
+    constexpr uint32_t kParts = 64 / kGroupsPerWave;
+    const uint32_t w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const uint32_t nparts = uniform_u32(*a.queue_tiles) * kParts;
+    for (;;) {
+        uint32_t t = 0;
+        if (lane == 0) t = atomicAdd(a.queue_next, 1u);
+        t = readlane_u32(t, 0);
+        if (t >= nparts) return;
+        const uint32_t ti = uniform_u32(a.tile_info[t / kParts]);
+        const uint32_t cloud = ti & 0xfffffu, limit = (t / kParts) * 64 + (ti >> 20);
+        if (t * kGroupsPerWave >= limit) continue;
+        for (uint32_t i = lane; i < 3 * (kMaxDepth + 1); i += 64) s_rad[w][i] = a.radtab[66 * (size_t)cloud + i];
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        group_tile<KERNEL, ALGO, PREC, 0>(a, t, uniform_u32(a.roots[cloud]), min(limit, a.nq), s_items[w], s_rad[w],
+                                          s_gc_all + (size_t)w * a.levels * 64);
     }
 }
 
@@ -1390,6 +1430,17 @@ static void launch_count_s(const SearchArgs &a, int G, hipStream_t s) {
 
 // resident waves of the work-queue kernel: blocks per CU at its occupancy, times the CUs
 template <int KERNEL, int ALGO, int PREC>
+static unsigned group_queue_grid(size_t lds) {  // lds: always that of kGroupMaxLevels
+    static unsigned cached = 0;
+    if (cached) return cached;
+    int dev = 0, cus = 0, per = 0;
+    (void)hipGetDevice(&dev);
+    (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+    (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k_group_queue<KERNEL, ALGO, PREC>, kSearchBlock, lds);
+    cached = (unsigned)((cus > 0 ? cus : 256) * (per > 0 ? per : 1));
+    return cached;
+}
+template <int KERNEL, int ALGO, int PREC>
 static unsigned queue_grid() {
     static unsigned cached = 0;
     if (cached) return cached;
@@ -1445,6 +1496,12 @@ static void launch_k(const SearchArgs &a, int mode, int G, hipStream_t s) {
     }
     const unsigned nb = (unsigned)(((size_t)a.nq + kGroupsPerWave * kWaves - 1) / (kGroupsPerWave * kWaves));
     const size_t lds = (size_t)kWaves * a.levels * 64 * sizeof(uint32_t);
+    if constexpr (ALGO != OCT_ALGO_APPROX) {
+        if (a.queue_next) {
+            k_group_queue<KERNEL, ALGO, PREC><<<group_queue_grid<KERNEL, ALGO, PREC>(lds), kSearchBlock, lds, s>>>(a);
+            return;
+        }
+    }
     if (mode == 0)
         k_group<KERNEL, ALGO, PREC, 0><<<nb, kSearchBlock, lds, s>>>(a);
     else if (mode == 1)
@@ -1522,7 +1579,9 @@ hipError_t launch_radius(oct_ctx *ctx, const RadiusLaunch &L) {
     a.stats = L.stats;
     a.err = ctx->derr.p;
     // levels that hold internal nodes: every level but the deepest
-    a.levels = ctx->n_levels > 1 ? std::min<uint32_t>(ctx->n_levels - 1, (uint32_t)kGroupMaxLevels) : 1u;
+    a.levels = L.tile_info ? (uint32_t)kGroupMaxLevels  // a forest's depth is not known here
+               : ctx->n_levels > 1 ? std::min<uint32_t>(ctx->n_levels - 1, (uint32_t)kGroupMaxLevels)
+                                   : 1u;
     stage_begin(ctx, ST_SEARCH);
     const int G = L.group;
     switch (L.kernel) {
