@@ -606,7 +606,7 @@ def main():
     # Roofline of the dominant kernel (the FP32 search): 9 flops (3 sub + 3 mul + 2 add + 1 compare) per
     # point test of the reference traversal (T, identical for both precisions), over the kernel's
     # device time (HIP events on the context's stream), against MI355X's FP32 compute roof; the kernel
-    # runs on the vector ALUs. traffic: the kernel's HBM bytes per launch from the committed rocprofv3
+    # is bound by vector-instruction issue. traffic: the kernel's HBM bytes per launch from the committed rocprofv3
     # FETCH_SIZE / WRITE_SIZE summary of this workload (calibrated on a copy kernel), used only when the
     # summary was taken from this kernel's current sources and tile shape.
     T = fp32["stats"]["points_tested"]

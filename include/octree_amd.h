@@ -223,9 +223,9 @@ int oct_knn_checksum(oct_ctx *ctx, const int32_t *idx_dev, const float *d2_dev, 
  * OCT_TUNE_RADIUS_GROUP: queries per wave of the count-mode radius kernel (16, 32 or 64 queries
  * share one wave's traversal, 64 / G lanes serve each query), or 0 for the kernel in which 8 lanes
  * walk each query's own traversal; -1 restores the library's choice (0 for few or scattered
- * queries, else the autotuned number, else 64). OCT_TUNE_RADIUS_MFMA: the point tests run on the vector
- * ALUs (a matrix-core form measured slower on every workload and is not built): 0 and -1 are
- * accepted, 1 fails with OCT_ERR_UNSUPPORTED.
+ * queries, else the autotuned number, else 64). OCT_TUNE_RADIUS_MFMA selects nothing: where
+ * the point tests run on the matrix cores (FP32 sphere counts, 64 queries per wave) they are faster
+ * there; 0 and -1 are accepted, 1 fails with OCT_ERR_UNSUPPORTED.
  * oct_autotune_radius: times each candidate (G = 0, 16, 32, 64) on sample_nq queries taken from the
  * sorted cloud (16 equal strided chunks of consecutive SFC points; sample_nq >= n uses every point),
  * stores the fastest for (kernel, algo, precision), returns its G in *best and the milliseconds per G
@@ -246,8 +246,8 @@ int oct_knn_checksum(oct_ctx *ctx, const int32_t *idx_dev, const float *d2_dev, 
  * OCT_TUNE_SORT: how oct_sort sorts more than 2048 (4096) keys: 1 orders them by their top 16 bits
  * in two device-wide passes, then sorts each 16-bit segment inside one workgroup (2048 keys per LDS
  * sort), which also writes the sorted cloud; 2 the same with 4096-key LDS sorts; 0 runs the
- * device-wide LSD pass per 8-bit digit and a separate gather. A 16-bit segment above 32768 keys
- * selects the LSD passes. -1 (the default) is 1, except that once a sort of the current points has
+ * device-wide LSD pass per 8-bit digit and a separate gather. Long segments of clouds of 2^18 keys and more
+ * are split by 8 further bits device-wide; a segment still above 32768 keys selects the LSD passes. -1 (the default) is 1, except that once a sort of the current points has
  * fallen back to the LSD passes, later sorts of the same points run them directly (new points reset
  * this). Results never depend on the tuning. */
 enum oct_tune_knob {

@@ -469,7 +469,7 @@ static hipError_t enqueue_search(oct_batch *b, int kernel, int algo, int precisi
         if ((e = enqueue_query_groups(s, b->rpass.Q, C, b->cloud_off.p)) != hipSuccess) return e;
         RadiusLaunch L;
         L.kernel = kernel, L.algo = algo, L.precision = precision, L.mode = 0;
-        L.group = shared_traversal(b->rpass.n, (double)b->rpass.n / (double)std::max<size_t>(b->n_all, 1)) ? 64 : 0;
+        L.group = shared_counts(b->rpass.n, (double)b->rpass.n / (double)std::max<size_t>(b->n_all, 1)) ? 64 : 0;
         L.remap = true;
         L.order = b->rpass.Q.order[0], L.qidx = b->rpass.Q.gidx, L.qrad = b->p_rad.p, L.nq = b->rpass.Q.slots[0];
         L.counts = b->p_counts.p, L.tile_info = b->rpass.Q.tile_info[0], L.roots = b->roots.p, L.radtab = b->radtab.p;

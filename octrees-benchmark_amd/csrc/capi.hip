@@ -31,6 +31,15 @@ void stage_end(oct_ctx *ctx, Stage s) {
 constexpr size_t kUnionMinQueries = 1u << 17;
 constexpr double kUnionMinDensity = 1.0 / 16;
 bool shared_traversal(size_t nq, double density) { return nq > kUnionMinQueries && density >= kUnionMinDensity; }
+// Counts of very many queries share a traversal at lower densities as well, whatever the radius. 100 M clouds, r = 0.5
+// to 5, group kernel's time over that of 64 per wave: one point in 24 (4.2 M queries) tile 2.7 to 3.3, box 1.3 to
+// 2.9; one in 64 (1.6 M) tile 1.7 to 2.1, box 0.9 to 2.3; one in 256 (0.4 M) tile 0.7 to 0.95, box 0.5 to 1.15. A
+// batch of 256 clouds, 10 M queries, one point in 20: 62 against 15 ms.
+constexpr size_t kUnionManyQueries = 1u << 20;
+constexpr double kUnionManyDensity = 1.0 / 64;
+bool shared_counts(size_t nq, double density) {
+    return shared_traversal(nq, density) || (nq > kUnionManyQueries && density >= kUnionManyDensity);
+}
 }  // namespace oct
 
 namespace {
@@ -691,7 +700,7 @@ static int check_search_args(oct_ctx *ctx, int kernel, int algo, int precision, 
 
 static int radius_group(const oct_ctx *ctx, int kernel, int algo, int precision, size_t nq, double density) {
     if (ctx->group_override >= 0) return ctx->group_override;
-    if (!shared_traversal(nq, density)) return 0;
+    if (!shared_counts(nq, density)) return 0;
     const int t = ctx->group_tuned[kernel & 3][algo & 3][precision & 1];
     return t >= 0 ? t : 64;
 }
@@ -965,9 +974,9 @@ int oct_radius_dev(oct_ctx *ctx, int kernel, int algo, int precision, const uint
 
 int oct_set_tuning(oct_ctx *ctx, int knob, int value) {
     if (!ctx) return OCT_ERR_ARG;
-    if (knob == OCT_TUNE_RADIUS_MFMA) {  // the point tests run on the vector ALUs only
+    if (knob == OCT_TUNE_RADIUS_MFMA) {  // selects nothing: the point tests run where they are faster
         if (value == 1)
-            return fail(ctx, OCT_ERR_UNSUPPORTED, "no matrix-core point tests: the vector ALUs measured faster on every workload");
+            return fail(ctx, OCT_ERR_UNSUPPORTED, "the point tests choose their unit themselves");
         if (value != -1 && value != 0) return fail(ctx, OCT_ERR_ARG, "radius mfma switch must be -1 or 0");
         return OCT_OK;
     }
@@ -1053,7 +1062,7 @@ int oct_tuned_radius(oct_ctx *ctx, int kernel, int algo, int precision, int *gro
     if (kernel < 0 || kernel > 3 || algo < 1 || algo > 3 || (precision != 0 && precision != 1))
         return fail(ctx, OCT_ERR_ARG, "unknown kernel, algorithm or precision");
     if (group) *group = radius_group(ctx, kernel, algo, precision, std::max(ctx->n, kUnionMinQueries + 1), 1.0);
-    if (mfma) *mfma = 0;  // point tests on the vector ALUs
+    if (mfma) *mfma = 0;  // selects nothing
     return OCT_OK;
 }
 

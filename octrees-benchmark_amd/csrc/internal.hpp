@@ -250,7 +250,7 @@ struct RadiusLaunch {
     const uint32_t *tile_info = nullptr;
     const uint32_t *roots = nullptr;
     const double *radtab = nullptr;
-    // work-queue form (count mode over a forest, 64-slot tiles, vector ALUs, no stats): device-resident
+    // work-queue form (count mode over a forest, 64-slot tiles, no stats): device-resident
     // tile count and a zeroed tile counter; the grid is the resident waves, not the tiles
     const uint32_t *queue_tiles = nullptr;
     uint32_t *queue_next = nullptr;
@@ -271,9 +271,10 @@ struct RadiusLaunch {
     unsigned long long *stats = nullptr;
 };
 hipError_t launch_radius(oct_ctx *ctx, const RadiusLaunch &L);
-// Whether nq queries, `density` of the points they lie among, are counted 64 per wave with one traversal (else
-// each by its own).
+// Whether nq queries, `density` of the points they lie among, get their lists (their counts) 64 per wave with one
+// traversal, else each by its own.
 bool shared_traversal(size_t nq, double density);
+bool shared_counts(size_t nq, double density);
 // The tight boxes of the current tree (ctx->nbox), unless it has them.
 hipError_t launch_boxes(oct_ctx *ctx);
 hipError_t launch_key_codec(oct_ctx *ctx, int encoder, bool decode, uint32_t *xyz_dev, uint64_t *keys_dev, size_t n);

@@ -1,11 +1,12 @@
 // H5: radius searches (neighbors / neighborsPrune / neighborsStruct x sphere / circle / cube /
 // square) on gfx950.
 //
-// Two kernels, both making exactly the reference's decisions for every query:
+// Two kernels, both giving exactly the reference's results for every query:
 //  - k_group: a group of 8 lanes per query, each group with its own traversal (result lists, and counts
 //    of queries that are far apart or few);
 //  - k_count: 16 - 64 consecutive queries per wave that share one traversal (counts of many queries that
-//    lie together, the all-points searches).
+//    lie together, the all-points searches; k_lists: their result lists). FP32 sphere counts test leaves on
+//    the matrix cores and judge children by tight boxes.
 //
 // Per-point tests:
 //  - FP64: the reference's isInside expression (kernel_3d.hpp:127-138, 232-242; kernel_2d.hpp:53-63,
@@ -372,7 +373,7 @@ __global__ __launch_bounds__(kSearchBlock) void k_group(const SearchArgs a) {
 
 // Counts over a forest (batches): resident waves take eighths of the 64-slot wave tiles, each of one cloud,
 // from a counter until the device-resident number of tiles has been served.
-// Forms chosen as for one cloud (shared_traversal). 48 clouds of 12 M points together, sparse queries:
+// Forms chosen as for one cloud (shared_counts). 48 clouds of 12 M points together, sparse queries:
 // k_count_queue 2.65 ms, this one 0.55.
 template <int KERNEL, int ALGO, int PREC>
 __global__ __launch_bounds__(kSearchBlock) void k_group_queue(const SearchArgs a) {
@@ -413,9 +414,9 @@ __global__ __launch_bounds__(kSearchBlock) void k_group_queue(const SearchArgs a
 // depend on the order of the traversal, which is therefore free.
 
 // Occupancy targets (waves per SIMD), measured on the 50 M-point tile for the sphere kernel with the
-// Struct / Prune algorithms: 7 for the FP32 vector path (71 VGPRs, no scratch; at 8 the 64-VGPR and
-// 72-SGPR budget spills the children's judgement masks and the search runs 3 % slower), 6 for FP64
-// (80 VGPRs). The other variants keep the compiler's choice (forcing them spills registers).
+// Struct / Prune algorithms: 7 for FP32 (72 VGPRs, 12 bytes of scratch touched at a wave's start and end; at 8
+// the 64-VGPR and 72-SGPR budget spilled the children's judgement masks and the search ran 3 % slower), 6 for
+// FP64 (80 VGPRs). The other variants keep the compiler's choice (forcing them spills registers).
 template <int KERNEL, int ALGO, int PREC>
 constexpr int count_waves() {
     if (ALGO == OCT_ALGO_NEIGHBORS || !(KERNEL == OCT_KERNEL_SPHERE || KERNEL == OCT_KERNEL_CIRCLE)) return 2;
@@ -1455,12 +1456,12 @@ static unsigned queue_grid() {
 template <int KERNEL, int ALGO, int PREC>
 static void launch_count(const SearchArgs &a, int G, hipStream_t s) {
     if constexpr (ALGO != OCT_ALGO_APPROX) {
-        if (a.queue_next) {  // work-queue form: 64 queries per wave tile, vector ALUs, no counters
+        if (a.queue_next) {  // work-queue form: 64 queries per wave tile, no counters
             k_count_queue<KERNEL, ALGO, PREC><<<queue_grid<KERNEL, ALGO, PREC>(), kSearchBlock, 0, s>>>(a);
             return;
         }
     }
-    if constexpr (ALGO == OCT_ALGO_APPROX) {  // one shape: 64 queries per wave, vector ALUs
+    if constexpr (ALGO == OCT_ALGO_APPROX) {  // one shape: 64 queries per wave
         const unsigned nb = (unsigned)(((size_t)a.nq + 64 * kWaves - 1) / (64 * kWaves));
         if (a.stats)
             k_count<KERNEL, ALGO, PREC, 64, true><<<nb, kSearchBlock, 0, s>>>(a);

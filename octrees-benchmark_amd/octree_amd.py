@@ -747,8 +747,8 @@ class Octree:
         self._chk(self.L.oct_set_tuning(self.h, 1, g), "oct_set_tuning")
 
     def set_mfma(self, on):
-        """The OCT_TUNE_RADIUS_MFMA knob: the point tests run on the vector ALUs, so None and False are
-        accepted and True raises OctError (no matrix-core form is built)."""
+        """The OCT_TUNE_RADIUS_MFMA knob, which selects nothing (the point tests run where they are faster):
+        None and False are accepted and True raises OctError."""
         self._chk(self.L.oct_set_tuning(self.h, 2, -1 if on is None else (1 if on else 0)), "oct_set_tuning")
 
     def tuned_radius(self, kernel, algo, precision):
