@@ -630,7 +630,7 @@ def main():
     roofline = {"bound": "valu", "achieved": achieved, "peak": PEAK_FP32_TFLOPS, "unit": "TFLOP/s",
                 "frac": achieved / PEAK_FP32_TFLOPS, "traffic": traffic, "traffic_source": traffic_note,
                 "kernel": "radius count (FP32 + FP64 re-check)",
-                "compute_unit": "vector ALUs",
+                "compute_unit": "vector ALUs; leaf tests on the matrix cores",
                 "work": f"9 flops x {T} point tests of the reference traversal"}
 
     es_ms = med(bbox_ms) + med(enc_ms) + med(sort_ms) + med(gather_ms)
