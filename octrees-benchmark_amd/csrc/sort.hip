@@ -219,18 +219,19 @@ __global__ void k_iota_copy(const uint64_t *__restrict__ kin, uint64_t *__restri
 // A few long 16-bit segments (scans cluster along their trajectory) would keep a few workgroups busy long
 // after the others, or not fit one at all. They are split by their next 8 bits (39..46) with one more
 // device-wide pass over such segments only: k_huge_jobs counts their digits and lists the pieces, the
-// onesweep pass moves the keys. Without such segments both launches return at once. A piece still above
-// kSegMaxLen sends the whole sort to the LSD passes.
+// onesweep pass moves the keys; very large clouds repeat this on the next 8 bits, twice. Without such segments
+// the launches return at once. A piece still above kSegMaxLen sends the whole sort to the LSD passes.
 // Every step keeps equal keys in input order, so the permutation is the stable sort by key, as with
 // the 8 LSD passes. Traffic per key: 20 B + 24 B (passes) + 24 B (LDS sort) + 56 B (gather), plus
 // 32 B for keys in segments that are split, against 188 B + 60 B for eight passes and a gather.
 
-// A job of k_seg_sort: len is its length, with kSegInB if the device-wide split has ordered it by bits
-// 39..46 already, from buffer a (the second pass's output) into b.
+// A job of k_seg_sort: len is its length, with seg_splits(s) if s device-wide splits have ordered it by 8 s bits
+// below the top 16 (an odd number of them from buffer a, the second pass's output, into b).
 struct SegJob {
     uint32_t start, len;
 };
-constexpr uint32_t kSegInB = 1u << 31;
+constexpr int kMaxSplits = 3;
+__host__ __device__ inline uint32_t seg_splits(uint32_t s) { return s << 28; }
 constexpr uint32_t kSegMaxLen = 1u << 15;  // longest segment the workgroup sort takes
 // The segments the device-wide split takes, those above `min` keys: start, length, keys counted so far, bin
 // starts (256 per segment) and sort tiles; n[0] segments, n[1] tiles. n null: no split.
@@ -250,6 +251,9 @@ constexpr uint32_t kHugeMin = 1u << 12;
 // (5 M tile: 0.383 and 0.391 ms), which the LSD passes' excess over it pays from here (150 k sweep: 0.119 and
 // 0.122 ms, 500 k: 0.207 and 0.184).
 constexpr size_t kHugeMinKeys = 1u << 18;
+// Clouds of this many keys get kMaxSplits splits (the others' pieces fit a workgroup after one; 8 us each): sort and
+// gather of a new 400 M sweep, which fell back to the LSD passes: 46.3 -> 34.9 ms; 100 M sweep 11.5 -> 8.2 ms.
+constexpr size_t kManySplitsKeys = 1u << 26;
 // pieces awaiting a split: a split of up to 2^15 keys pushes at most 15 pieces above 2048 keys and
 // pops one, over at most 6 levels (bits 39..46 down to 0..7)
 constexpr int kSegStack = 96;
@@ -428,18 +432,18 @@ __device__ void seg_local_sort(SegShared<W, IPT> &S, const uint64_t *ks, const u
     }
 }
 
-// Complete sort of one segment longer than kCap, [start, start + len) of buffer a (in_b: of buffer b), into
+// Complete sort of one segment longer than kCap, [start, start + len) of buffer a (splits odd: b), into
 // the same range of buffer b (buffer a's range is scratch): stable splits by the next 8 bits until every
 // piece fits, then LDS sorts of runs of consecutive pieces. A piece whose bits are used up holds
 // equal keys, already in input order.
 template <int W, int IPT>
 __device__ void seg_split_sort(SegShared<W, IPT> &S, uint64_t *ka, uint32_t *va, uint64_t *kb, uint32_t *vb,
-                               uint32_t start, uint32_t len, bool in_b, uint32_t *err, const double *xyz,
-                               double4 *p64) {
+                               uint32_t start, uint32_t len, uint32_t splits, uint32_t *err,
+                               const double *xyz, double4 *p64) {
     constexpr uint32_t kCap = SegShared<W, IPT>::kCap;
     const uint32_t tid = threadIdx.x, w = tid >> 6, lane = tid & 63, base = w * 64 * IPT;
     if (tid == 0) {
-        S.stack[0] = make_uint4(start, len, in_b ? kMsdShift3 - 7u : kMsdShift3 + 1u, in_b ? 1u : 0u);
+        S.stack[0] = make_uint4(start, len, kMsdShift3 + 1u - 8u * splits, splits & 1u);
         S.sp = 1u;
     }
     __syncthreads();
@@ -596,10 +600,10 @@ __global__ __attribute__((amdgpu_flat_work_group_size(W * 64, W * 64), amdgpu_wa
         const SegJob job = S.job;
         __syncthreads();
         if (kind == 2u) break;
-        const uint32_t len = job.len & ~kSegInB;
-        const bool in_b = job.len & kSegInB;
+        const uint32_t splits = job.len >> 28, len = job.len & 0xfffffffu;
+        const bool in_b = splits & 1u;
         if (len > SegShared<W, IPT>::kCap)
-            seg_split_sort(S, ka, va, kb, vb, job.start, len, in_b, err, xyz, p64);
+            seg_split_sort(S, ka, va, kb, vb, job.start, len, splits, err, xyz, p64);
         else
             seg_local_sort(S, in_b ? kb : ka, in_b ? vb : va, kb, vb, job.start, len, xyz, p64);
         __syncthreads();
@@ -609,8 +613,8 @@ __global__ __attribute__((amdgpu_flat_work_group_size(W * 64, W * 64), amdgpu_wa
 // The jobs of 256 consecutive segments (digit tid of the workgroup: c keys from st on), by one workgroup:
 // segments above H.min go on the list of the split, or without one their longest length to njobs[2]; others
 // above cap become a job each (big, njobs[0]), runs of consecutive smaller ones one up to cap (small,
-// njobs[1]). in_b: kSegInB or 0.
-__device__ inline void emit_seg_jobs(uint32_t c, uint32_t st, uint32_t cap, uint32_t in_b, SegJob *__restrict__ big,
+// njobs[1]). tag: their seg_splits.
+__device__ inline void emit_seg_jobs(uint32_t c, uint32_t st, uint32_t cap, uint32_t tag, SegJob *__restrict__ big,
                                      SegJob *__restrict__ small, uint32_t *__restrict__ njobs, const HugeList &H) {
     __shared__ uint32_t s_c[256], s_st[256], s_nb, s_ns, s_nh, s_ob, s_os;
     __shared__ SegJob s_big[256], s_small[256], s_huge[256];
@@ -629,12 +633,12 @@ __device__ inline void emit_seg_jobs(uint32_t c, uint32_t st, uint32_t cap, uint
                     if (lane == 0) s_huge[nh] = SegJob{a, l};
                     nh++;
                 } else {
-                    if (lane == 0) s_big[nb] = SegJob{a, l | in_b};
+                    if (lane == 0) s_big[nb] = SegJob{a, l | tag};
                     nb++;
                 }
             },
             [&](uint32_t a, uint32_t l) {
-                if (lane == 0) s_small[ns] = SegJob{a, l | in_b};
+                if (lane == 0) s_small[ns] = SegJob{a, l | tag};
                 ns++;
             });
         if (lane == 0) {
@@ -694,13 +698,14 @@ __global__ __launch_bounds__(256) void k_msd_jobs(const uint32_t *__restrict__ h
 }
 
 // The digit counts of the huge segments, tile by tile, and the tiles' look-back words zeroed; the workgroup
-// that counts a segment's last tile turns its counts into bin starts and its pieces into jobs.
-__global__ __launch_bounds__(256) void k_huge_jobs(const uint64_t *__restrict__ keys, HugeList H,
-                                                   uint32_t *__restrict__ lookback, uint32_t cap,
+// that counts a segment's last tile turns its counts into bin starts and its pieces into jobs or the segments of the
+// next split. splits: device-wide splits up to this one.
+__global__ __launch_bounds__(256) void k_huge_jobs(const uint64_t *__restrict__ keys, HugeList H, HugeList next,
+                                                   uint32_t splits, uint32_t *__restrict__ lookback, uint32_t cap,
                                                    SegJob *__restrict__ big, SegJob *__restrict__ small,
                                                    uint32_t *__restrict__ njobs, uint32_t *__restrict__ err) {
     __shared__ uint32_t s_h[256], s_last;
-    const uint32_t nt = H.n[1], tid = threadIdx.x;
+    const uint32_t nt = H.n[1], tid = threadIdx.x, shift = kMsdShift3 + 8u - 8u * splits;
     for (uint32_t t = blockIdx.x; t < nt; t += gridDim.x) {
         const SortTile T = H.tiles[t];
         s_h[tid] = 0u;
@@ -712,7 +717,7 @@ __global__ __launch_bounds__(256) void k_huge_jobs(const uint64_t *__restrict__ 
 #pragma unroll
             for (uint32_t r = 0; r < 8; r++) {
                 const uint32_t i = i0 + 256 * r;
-                d[r] = i < T.len ? (uint32_t)(keys[T.start + i] >> kMsdShift3) & 255u : 256u;
+                d[r] = i < T.len ? (uint32_t)(keys[T.start + i] >> shift) & 255u : 256u;
             }
 #pragma unroll
             for (uint32_t r = 0; r < 8; r++) {
@@ -745,14 +750,12 @@ __global__ __launch_bounds__(256) void k_huge_jobs(const uint64_t *__restrict__ 
         }
         const uint32_t st = H.start[T.cloud] + pre;
         *base = st;
-        HugeList none = {};
-        none.min = kSegMaxLen;
-        emit_seg_jobs(c, st, cap, kSegInB, big, small, njobs, none);
+        emit_seg_jobs(c, st, cap, seg_splits(splits), big, small, njobs, next);
         __syncthreads();
     }
 }
 
-constexpr int kNJobs = 6;  // njobs words: k_seg_sort's four, then the split's segments and tiles
+constexpr int kNJobs = 4 + 2 * kMaxSplits;  // njobs words: k_seg_sort's four, then each split's segments and tiles
 
 // Everything the partition passes start from, in one launch (no host copies or fills in between):
 // zero look-back words, prefix counts, job and tile counters and the error flag; the bin starts of
@@ -824,17 +827,18 @@ hipError_t sort_partition(oct_ctx *ctx, uint32_t *counters, uint32_t *errflag, u
     const size_t n = ctx->n;
     const uint32_t *h55 = ctx->hist.p + kRadixPassCount * 256, *h47 = h55 + 256;  // the encode kernel's
     const size_t tiles = (n + kSortTile - 1) / kSortTile;
-    const bool split = n >= kHugeMinKeys;
-    HugeList huge = {}, none = {};
-    huge.min = (uint32_t)std::min<size_t>(std::max<size_t>(n / 1024, kHugeMin), kSegMaxLen), none.min = kSegMaxLen;
-    const size_t huge_max = split ? n / huge.min + 1 : 0, huge_tiles = split ? tiles + huge_max : 0;
-    // jobs of either kind: at most one per 16-bit segment; of the pieces of huge ones at most 2 * keys / cap + 1
-    const size_t jobs_max = kSegJobsMax + (split ? 2 * (n / cap) + huge_max : 0);
-    // msd layout (u32 words): bases [2 x 256], hist2 [65536], njobs [kNJobs], big and small jobs, huge segments'
-    // tiles, starts, lengths, key counts and bases
+    const int nsplit = n < kHugeMinKeys ? 0 : n < kManySplitsKeys ? 1 : kMaxSplits;
+    HugeList huge[kMaxSplits + 1] = {};  // [nsplit]: no further split
+    const uint32_t huge_min = (uint32_t)std::min<size_t>(std::max<size_t>(n / 1024, kHugeMin), kSegMaxLen);
+    const size_t huge_max = nsplit ? n / huge_min + 1 : 0, huge_tiles = nsplit ? tiles + huge_max : 0;
+    // jobs of either kind: at most one per 16-bit segment; of the pieces of huge ones, between two that are split
+    // again, at most 2 * keys / cap + 1
+    const size_t jobs_max = kSegJobsMax + (nsplit ? 2 * (n / cap) + 2 * (size_t)nsplit * huge_max : 0);
+    // msd layout (u32 words): bases [2 x 256], hist2 [65536], njobs [kNJobs], big and small jobs, per split the huge
+    // segments' tiles, starts, lengths, key counts and bases
     const size_t o_bases = 0, o_hist2 = 512, o_njobs = o_hist2 + 65536, o_big = o_njobs + kNJobs, o_small = o_big + 2 * jobs_max,
-                 o_tiles = (o_small + 2 * jobs_max + 3) / 4 * 4, o_huge = o_tiles + 4 * huge_tiles,
-                 words = o_huge + (3 + 256) * huge_max;
+                 o_huge = (o_small + 2 * jobs_max + 3) / 4 * 4,
+                 huge_words = (4 * huge_tiles + (3 + 256) * huge_max + 3) / 4 * 4, words = o_huge + (size_t)nsplit * huge_words;
     hipError_t e;
     if ((e = ctx->msd.reserve(words)) != hipSuccess) return e;
     if ((e = ctx->lookback.reserve(2 * tiles * 256 + 1 + huge_tiles * 256)) != hipSuccess) return e;
@@ -855,19 +859,24 @@ hipError_t sort_partition(oct_ctx *ctx, uint32_t *counters, uint32_t *errflag, u
     k_onesweep<false><<<(unsigned)tiles, kSortBlock, 0, s>>>(ctx->keys[1].p, ctx->vals[1].p, ctx->keys_p.p, ctx->vals_p.p, n,
                                                              kMsdShift1, M + o_bases + 256, ctx->lookback.p + tiles * 256,
                                                              counters + 1, errflag, nullptr, 0u, M + o_hist2);
-    if (split) {
-        huge.tiles = reinterpret_cast<SortTile *>(M + o_tiles);
-        huge.start = M + o_huge, huge.len = huge.start + huge_max, huge.done = huge.len + huge_max;
-        huge.bases = huge.done + huge_max, huge.n = M + o_njobs + 4;
+    for (int l = 0; l < nsplit; l++) {
+        uint32_t *w = M + o_huge + (size_t)l * huge_words;
+        huge[l].tiles = reinterpret_cast<SortTile *>(w);
+        huge[l].start = w + 4 * huge_tiles, huge[l].len = huge[l].start + huge_max, huge[l].done = huge[l].len + huge_max;
+        huge[l].bases = huge[l].done + huge_max, huge[l].n = M + o_njobs + 4 + 2 * l, huge[l].min = huge_min;
     }
-    k_msd_jobs<<<256, 256, 0, s>>>(M + o_hist2, M + o_bases + 256, cap, big, small, M + o_njobs, split ? huge : none);
-    if (split) {  // bits 39..46 of the huge segments: keys_p / vals_p -> keys[1] / vals[1]
-        uint32_t *look = ctx->lookback.p + nlook;
-        k_huge_jobs<<<(unsigned)std::min<size_t>(huge_tiles, 2048), 256, 0, s>>>(ctx->keys_p.p, huge, look, cap, big, small,
-                                                                                 M + o_njobs, errflag);
+    huge[nsplit].min = kSegMaxLen;
+    k_msd_jobs<<<256, 256, 0, s>>>(M + o_hist2, M + o_bases + 256, cap, big, small, M + o_njobs, huge[0]);
+    uint64_t *kb[2] = {ctx->keys_p.p, ctx->keys[1].p};
+    uint32_t *vb[2] = {ctx->vals_p.p, ctx->vals[1].p};
+    uint32_t *look = ctx->lookback.p + nlook;
+    for (int l = 0; l < nsplit; l++) {  // bits 39..46, then 31..38 and 23..30, of the huge segments, between the buffers
+        const int f = l & 1;
+        k_huge_jobs<<<(unsigned)std::min<size_t>(huge_tiles, 2048), 256, 0, s>>>(
+            kb[f], huge[l], huge[l + 1], (uint32_t)l + 1u, look, cap, big, small, M + o_njobs, errflag);
         k_onesweep<true, true><<<(unsigned)std::min<size_t>(huge_tiles, 512), kSortBlock, 0, s>>>(
-            ctx->keys_p.p, ctx->vals_p.p, ctx->keys[1].p, ctx->vals[1].p, n, kMsdShift3, huge.bases, look, counters + 4, errflag,
-            huge.tiles, 256u, nullptr, huge.n + 1);
+            kb[f], vb[f], kb[f ^ 1], vb[f ^ 1], n, kMsdShift3 - 8u * (uint32_t)l, huge[l].bases, look, counters + 4 + l, errflag,
+            huge[l].tiles, 256u, nullptr, huge[l].n + 1);
     }
     // every 16-bit segment sorted by one workgroup: keys_p / vals_p -> keys[1] / vals[1], sorted cloud
     k_seg_sort<W, IPT><<<seg_grid<W, IPT>(), W * 64, 0, s>>>(ctx->keys_p.p, ctx->vals_p.p, ctx->keys[1].p, ctx->vals[1].p,

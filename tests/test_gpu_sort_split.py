@@ -61,3 +61,29 @@ def test_split_sort_matches_oracle(ctx, name, enc, mode):
     np.testing.assert_array_equal(gkeys, keys)
     np.testing.assert_array_equal(gperm, perm)
     np.testing.assert_array_equal(gc, c)
+
+
+def test_repeated_splits(ctx):
+    """From 2^26 keys on the split is repeated on the next two digits: a cluster whose 24-bit pieces are too long, and
+    one that only 40 bits separate. The permutation is checked by what defines it."""
+    n, big, narrow = (1 << 26) + 5, 20_000_000, 100_000
+    rng = np.random.default_rng(12)
+    xyz = 1000.0 * rng.random((n, 3))
+    xyz[1000 : 1000 + big] = 321.0 + 5.0 * rng.random((big, 3))
+    xyz[-narrow:] = 654.3 + 0.5 * rng.random((narrow, 3))
+    print(f"[sort split] repeated n={n}", flush=True)
+    ctx.set_points(xyz)
+    ctx.current = None
+    del xyz
+    c, r = ctx.bbox()
+    keys = ctx.encode(A.ENC_MORTON, c, r)
+    perm, skeys = ctx.sort()
+    seen = np.zeros(n, np.uint8)
+    seen[perm] = 1
+    assert seen.all()
+    np.testing.assert_array_equal(skeys, keys[perm])
+    up, same = skeys[1:] > skeys[:-1], skeys[1:] == skeys[:-1]
+    assert (up | same).all()
+    assert (perm[1:][same] > perm[:-1][same]).all()
+    ctx.set_points(np.zeros((1, 3)))  # gives the memory's owner a small cloud for the tests that follow
+    ctx.current = None
