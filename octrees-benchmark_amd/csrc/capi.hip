@@ -30,15 +30,20 @@ void stage_end(oct_ctx *ctx, Stage s) {
 // 524 k 3.8 / 3.2; one in 32: 524 k 4.8 / 4.8; 40 M box, one in 8: 2.8 / 2.6, one in 32: 3.2 / 4.7.
 constexpr size_t kUnionMinQueries = 1u << 17;
 constexpr double kUnionMinDensity = 1.0 / 16;
-bool shared_traversal(size_t nq, double density) { return nq > kUnionMinQueries && density >= kUnionMinDensity; }
-// Counts of very many queries share a traversal at lower densities as well, whatever the radius. 100 M clouds, r = 0.5
+// Very many queries share a traversal at lower densities as well. Lists of 60 M clouds, whole calls, group kernel / 64
+// per wave in ms: one point in 20 (3 M queries) tile r = 2.5 41.8 / 23.2, sweep r = 0.5 99.9 / 49.3, box r = 0.5
+// 6.9 / 8.4; one in 50 (1.2 M) 18.5 / 14.7, 44.2 / 28.6, 3.0 / 4.8.
+constexpr size_t kUnionManyQueries = 1u << 20;
+constexpr double kListsManyDensity = 1.0 / 48, kCountsManyDensity = 1.0 / 64;
+bool shared_traversal(size_t nq, double density) {
+    return (nq > kUnionMinQueries && density >= kUnionMinDensity) || (nq > kUnionManyQueries && density >= kListsManyDensity);
+}
+// Counts, whatever the radius. 100 M clouds, r = 0.5
 // to 5, group kernel's time over that of 64 per wave: one point in 24 (4.2 M queries) tile 2.7 to 3.3, box 1.3 to
 // 2.9; one in 64 (1.6 M) tile 1.7 to 2.1, box 0.9 to 2.3; one in 256 (0.4 M) tile 0.7 to 0.95, box 0.5 to 1.15. A
 // batch of 256 clouds, 10 M queries, one point in 20: 62 against 15 ms.
-constexpr size_t kUnionManyQueries = 1u << 20;
-constexpr double kUnionManyDensity = 1.0 / 64;
 bool shared_counts(size_t nq, double density) {
-    return shared_traversal(nq, density) || (nq > kUnionManyQueries && density >= kUnionManyDensity);
+    return shared_traversal(nq, density) || (nq > kUnionManyQueries && density >= kCountsManyDensity);
 }
 }  // namespace oct
 

@@ -100,3 +100,26 @@ def test_shared_traversal_lists(ctx, name, leaf, radius):
                 assert np.array_equal(counts[some], sizes), tag
                 for q, r in zip(some, ref):
                     assert np.array_equal(ent[w * int(offs[q]):w * int(offs[q + 1])], np.asarray(r).reshape(-1)), tag
+
+
+@pytest.mark.parametrize("stride", [17, 18])
+def test_many_sparse_queries(ctx, stride):
+    """More than 2^20 queries at one point in 17 or 18 share traversals (counts and lists); the same queries in calls
+    of at most 2^17 go their own way. Equal counts and list sizes."""
+    nq = (1 << 20) + 3
+    rng = np.random.default_rng(stride)
+    ctx.set_points(rng.uniform(0, 100, (nq * stride, 3)) * [1.0, 1.0, 0.05])
+    ctx.sort_points(A.ENC_MORTON, fetch=False)
+    ctx.build(64)
+    idx = (np.arange(nq, dtype=np.uint64) * stride).astype(np.uint32)
+    for algo in (A.A_PRUNE, A.A_STRUCT):
+        print(f"[lists] {nq} queries, one point in {stride}, algo={algo}", flush=True)
+        counts, _ = ctx.radius(A.K_SPHERE, algo, A.PREC_FP32, idx=idx, radius=0.3)
+        listed = np.empty(nq, np.uint32)
+        rc = ctx.L.oct_radius(ctx.h, A.K_SPHERE, algo, A.PREC_FP32, None, idx.ctypes.data, None, 0.3, nq, 1, listed.ctypes.data, None)
+        assert rc == 0
+        np.testing.assert_array_equal(listed, counts)
+        for a in range(0, nq, 1 << 19):  # a part of each half million, one small call
+            part = idx[a : a + 4001]
+            few, _ = ctx.radius(A.K_SPHERE, algo, A.PREC_FP32, idx=part, radius=0.3)
+            np.testing.assert_array_equal(counts[a : a + 4001], few)
