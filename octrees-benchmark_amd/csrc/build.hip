@@ -292,10 +292,17 @@ __global__ __launch_bounds__(256) void k_node_ext_dev(const NodeRec *__restrict_
 }
 
 // The box of every leaf's points relative to the leaf's centre, kRecentreLanes lanes per leaf: the FP32
-// coordinates' extremes, widened by their rounding.
-__global__ __launch_bounds__(256) void k_leaf_box(const float4 *__restrict__ p32, const NodeRec *__restrict__ nodes,
-                                                 const uint32_t *__restrict__ child, const float *__restrict__ amax,
-                                                 uint32_t n_total, PointBox *__restrict__ pbox) {
+// coordinates' extremes, widened by their rounding. A leaf is bad where a point's FP32 form overflows, and where a
+// point lies outside the leaf's cell: keys of a box smaller than the cloud clamp the points beyond it into the edge
+// cells, and the keys of an already sorted cloud are the caller's. The reference counts an INSIDE cell's points
+// unseen and drops an OUTSIDE cell's, so such points count by their cell and not by where they are. slack: 2^-49 of
+// the largest coordinate, several times the rounding of the keys and the cells' centres and small against the ties
+// that the counts resolve by the walk from the root (tie_scale, 2^-46). The FP32 extremes settle almost every leaf;
+// one whose points reach its faces to FP32's last bit is looked at in FP64.
+__global__ __launch_bounds__(256) void k_leaf_box(const double4 *__restrict__ p64, const float4 *__restrict__ p32,
+                                                 const NodeRec *__restrict__ nodes, const uint32_t *__restrict__ child,
+                                                 const float *__restrict__ amax, const double *__restrict__ radtab,
+                                                 LevelTable lt, double slack, uint32_t n_total, PointBox *__restrict__ pbox) {
     const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     const size_t u = t / kRecentreLanes;
     const uint32_t g = (uint32_t)(t % kRecentreLanes);
@@ -309,13 +316,33 @@ __global__ __launch_bounds__(256) void k_leaf_box(const float4 *__restrict__ p32
     }
     for (int off = kRecentreLanes / 2; off > 0; off >>= 1)
         for (int a = 0; a < 6; a++) v[a] = fminf(v[a], __shfl_xor(v[a], off));
+    uint32_t level = 0, out = 0;
+    while (level + 1 < kMaxDepth + 2 && lt.start[level + 1] <= u) level++;
+    if (last > first) {
+        double room[3];
+        bool in = true;
+        for (int a = 0; a < 3; a++) {
+            room[a] = radtab[3 * level + a] + slack;
+            // |p - c| <= e (1 + 2^-24) + 2^-150, e the largest |fl32(p - c)|
+            const double e = fmax(-(double)v[a], -(double)v[3 + a]);
+            in = in && e * (1.0 + 0x1p-23) + 0x1p-149 <= room[a];
+        }
+        if (!in) {  // the leaf's lanes together
+            const NodeRec nr = nodes[u];
+            for (uint32_t i = first + g; i < last; i += kRecentreLanes) {
+                const double4 p = p64[i];
+                out |= fabs(p.x - nr.cx) <= room[0] && fabs(p.y - nr.cy) <= room[1] && fabs(p.z - nr.cz) <= room[2] ? 0u : 1u;
+            }
+            for (int off = kRecentreLanes / 2; off > 0; off >>= 1) out |= __shfl_xor(out, off);
+        }
+    }
     if (g == 0) {
         PointBox b;
         for (int a = 0; a < 3; a++) {
             b.lo[a] = v[a] - fabsf(v[a]) * 2.384185791015625e-07f;  // 2^-22
             b.hi[a] = -(v[3 + a] - fabsf(v[3 + a]) * 2.384185791015625e-07f);
         }
-        b.bad = last > first && !(amax[u] < 1e30f) ? 1u : 0u;
+        b.bad = last > first && (out || !(amax[u] < 1e30f)) ? 1u : 0u;
         b.pad = 0;
         pbox[u] = b;
     }
@@ -387,7 +414,11 @@ hipError_t launch_boxes(oct_ctx *ctx) {
     // 2^-k with 2^k in [4, 8] extents; degenerate or huge boxes keep their unit (their squares would leave FP32)
     ctx->box_scale = ext > 1e-15 && ext < 1e15 ? (float)exp2(-ceil(log2(4.0 * ext))) : 1.0f;
     const unsigned nb = (unsigned)(((size_t)nt * kRecentreLanes + 255) / 256);
-    k_leaf_box<<<nb, 256, 0, ctx->stream>>>(ctx->p32.p, ctx->nodes.p, ctx->child.p, ctx->amax.p, nt, ctx->pbox.p);
+    LevelTable lt;
+    for (uint32_t l = 0; l < kMaxDepth + 3; l++) lt.start[l] = ctx->level_start[l];
+    const double mc = std::max(ctx->geo[66], std::max(ctx->geo[67], ctx->geo[68]));
+    k_leaf_box<<<nb, 256, 0, ctx->stream>>>(ctx->p64.p, ctx->p32.p, ctx->nodes.p, ctx->child.p, ctx->amax.p, ctx->radtab.p, lt,
+                                            mc * 0x1p-49, nt, ctx->pbox.p);
     for (int l = (int)ctx->n_levels - 2; l >= 0; l--) {
         const uint32_t ls = ctx->level_start[l], le = ctx->level_start[l + 1];
         if (le > ls)

@@ -41,7 +41,7 @@ static_assert(sizeof(NodeExt) == 192, "NodeExt is three 64-byte lines");
 // Tight boxes of the children of one internal node (same index as NodeExt), for the neighbour counts: child
 // combo c's points lie within ch[c].h of ch[c].c per axis, relative to the node's centre, in units of
 // 1 / ctx->box_scale, a power of two above 4 root box extents. ext2: max |p - centre|^2 in these units, or +inf
-// when a point below is not finite in FP32 (the boxes are then not used).
+// when a point below is not finite in FP32 or lies outside its leaf's cell (the boxes are then not used).
 struct alignas(64) ChildBox {  // one scalar load
     float c[3], h[3];
     uint32_t n, gc;       // points, first child (0 = leaf)
@@ -57,7 +57,7 @@ struct alignas(64) NodeBox {
     ChildBox ch[8];
 };
 static_assert(sizeof(ChildBox) == 64 && sizeof(NodeBox) == 576, "one scalar load per child");
-// A node's points relative to its own centre, rounded outward; bad: not finite.
+// A node's points relative to its own centre, rounded outward; bad: not finite, or not in their cell.
 struct alignas(32) PointBox {
     float lo[3], hi[3];
     uint32_t bad, pad;

@@ -747,7 +747,8 @@ __device__ __attribute__((always_inline)) inline void count_tile(const SearchArg
     // descended into or its points are tested. The FP64 judgement of the cells (the reference's answer) can
     // differ from the points' own tests only where a point lies on the sphere to the last FP64 bits: such a point
     // is in the band of its leaf's test, and its lane's points are then decided by path_class, the reference's
-    // walk itself. tie_scale sqrt(S) + 2^-46 S bounds the cells' and points' rounding (S as above, coordinates
+    // walk itself. This holds for points inside their cells; a node with others below it has no boxes (ext2 is
+    // infinite) and is judged by its cells. tie_scale sqrt(S) + 2^-46 S bounds the cells' and points' rounding (S as above, coordinates
     // up to 2^46 tie_scale), and S > tight_min keeps it below the margin's slack.
     //
     // 50 M tile, r = 2.5 (all points): 1418 point tests per query instead of 1684, 38.2 -> 29.9 ms with leaf_mfma;
