@@ -411,8 +411,8 @@ hipError_t launch_boxes(oct_ctx *ctx) {
     if ((e = ctx->nbox.reserve(ctx->n_internal + 1)) != hipSuccess) return e;
     double ext = 0.0;
     for (int a = 0; a < 3; a++) ext = std::max(ext, 2.0 * fabs(ctx->radii[a]));
-    // 2^-k with 2^k in [4, 8] extents; degenerate or huge boxes keep their unit (their squares would leave FP32)
-    ctx->box_scale = ext > 1e-15 && ext < 1e15 ? (float)exp2(-ceil(log2(4.0 * ext))) : 1.0f;
+    // 2^-k with 2^k in [4, 8] extents; degenerate boxes keep their unit (their squares would leave FP32)
+    ctx->box_scale = ext > 1e-15 ? (float)exp2(-ceil(log2(4.0 * ext))) : 1.0f;
     const unsigned nb = (unsigned)(((size_t)nt * kRecentreLanes + 255) / 256);
     LevelTable lt;
     for (uint32_t l = 0; l < kMaxDepth + 3; l++) lt.start[l] = ctx->level_start[l];

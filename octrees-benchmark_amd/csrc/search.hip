@@ -786,7 +786,10 @@ __device__ __attribute__((always_inline)) inline void count_tile(const SearchArg
     // sum and either rounding. Vector FMAs run at the matrix rate (2 cycles per wave here), so the gain is
     // what surrounds them: 4 LDS reads and a staging pass fewer per 4 tests. Here 2-operand FP32 and integer
     // instructions on VGPRs take 2.5 cycles, all others (3 operands, scalar operands, compares, min, FP64) 4.3.
-    auto leaf_mfma = [&](const uint64_t m, const float am, const NodeRec &nr) {
+    // tight: the leaf was reached through its parent's tight boxes, whose conditions (a finite am below 1e30 in a box
+    // below 1e15, a query nearer than 3.2e14 to its centre, R above 1e-30) keep every term within FP32. Leaves
+    // reached by their cells can hold points beyond FP32 and NaNs, whatever the wave's queries.
+    auto leaf_mfma = [&](const uint64_t m, const float am, const NodeRec &nr, const bool tight) {
         const uint32_t first = nr.first, last = nr.last;
         if (STATS) n_test += (uint64_t)__popcll(m) * (last - first);
         const uint32_t mc = (uint32_t)__popcll(m);
@@ -802,7 +805,7 @@ __device__ __attribute__((always_inline)) inline void count_tile(const SearchArg
             const float hw = 3.814697265625e-06f * sum;  // 2^-18
             const float C = (hw - qRf) + b2;
             float lim = 2.0f * hw;
-            if (!boxes && !(sum < 1e30f && sum > 1e-30f)) lim = __uint_as_float(0xffffffffu);
+            if (!tight && !(sum < 1e30f && sum > 1e-30f)) lim = __uint_as_float(0xffffffffu);
             mq.u[rank] = make_float4(-2.0f * bx, -2.0f * by, -2.0f * bz, 1.0f);
             mq.c[rank] = make_float4(C, C, C, C);
             mq.lh[rank] = make_uint2(__float_as_uint(lim), lane);
@@ -1201,7 +1204,7 @@ __device__ __attribute__((always_inline)) inline void count_tile(const SearchArg
                 ur.first = uniform_u32(nr.first), ur.last = uniform_u32(nr.last);
                 if (ur.last > ur.first) {
                     if constexpr (kMfma)
-                        leaf_mfma(ov, a.amax[root], ur);
+                        leaf_mfma(ov, a.amax[root], ur, false);
                     else if constexpr (MODE == 0)
                         leaf(ov, a.amax[root], ur);
                     else
@@ -1252,7 +1255,7 @@ __device__ __attribute__((always_inline)) inline void count_tile(const SearchArg
                             auto f64 = [](uint32_t lo, uint32_t hi) { return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo)); };
                             ur.cx = f64(x[8], x[9]), ur.cy = f64(x[10], x[11]), ur.cz = f64(x[12], x[13]);
                             ur.first = x[14], ur.last = x[14] + x[6];
-                            leaf_mfma(ov, __uint_as_float(x[15]), ur);
+                            leaf_mfma(ov, __uint_as_float(x[15]), ur, true);
                         } else if (sp < kStack) {
                             s_node[w][sp] = x[7], s_mask[w][sp] = ov, s_depth[w][sp] = (uint8_t)d;
                             sp++;
@@ -1357,7 +1360,7 @@ __device__ __attribute__((always_inline)) inline void count_tile(const SearchArg
                 ur.cx = E.ax[c & 1], ur.cy = E.ax[2 + ((c >> 1) & 1)], ur.cz = E.ax[4 + ((c >> 2) & 1)];
                 ur.first = E.first[c], ur.last = E.last[c];
                 if constexpr (kMfma)
-                    leaf_mfma(ov, E.amax[c], ur);
+                    leaf_mfma(ov, E.amax[c], ur, false);
                 else if constexpr (MODE == 0)
                     leaf(ov, E.amax[c], ur);
                 else
@@ -1541,8 +1544,11 @@ hipError_t launch_radius(oct_ctx *ctx, const RadiusLaunch &L) {
     a.nodes = ctx->nodes.p;
     a.next = ctx->next.p;
     a.nbox = nullptr, a.tie_scale = 0.0, a.tight_min = a.box_scale = 0.0f;
+    double extent = 0.0;  // clouds of 1e15 and more have no boxes: their FP32 terms are checked leaf by leaf
+    for (int k = 0; k < 3; k++) extent = std::max(extent, 2.0 * fabs(ctx->radii[k]));
     if (L.mode == 0 && L.group == 64 && L.kernel == OCT_KERNEL_SPHERE && L.precision == OCT_PREC_FP32_RECHECK &&
-        (L.algo == OCT_ALGO_PRUNE || L.algo == OCT_ALGO_STRUCT) && !L.tile_info && !L.stats && ctx->n_total > 1) {
+        (L.algo == OCT_ALGO_PRUNE || L.algo == OCT_ALGO_STRUCT) && !L.tile_info && !L.stats && ctx->n_total > 1 &&
+        extent < 1e15) {
         const hipError_t e = launch_boxes(ctx);
         if (e != hipSuccess && e != hipErrorOutOfMemory) return e;
         double mc = 0.0;

@@ -1,6 +1,7 @@
 """Counts asked for without the search counters (the only calls that judge children by the tight boxes of their
 points and test leaves on the matrix cores with that judgement behind them) and lists, where the forms could
-disagree: points outside the cells their keys name. Every form returns exactly the oracle's results."""
+disagree: points outside the cells their keys name, points beyond FP32, NaNs. Every form returns exactly the
+oracle's results."""
 import numpy as np
 import pytest
 
@@ -94,3 +95,54 @@ def test_sorted_clouds_whose_codes_are_not_their_points(ctx, enc):
         ctx.set_sorted(sx, sk, enc, cc, r)
         ctx.build(24)
         check_forms(ctx, sx, O.Tree(sk, 24, enc, cc, r), centers, radii, (A.K_SPHERE, A.K_CUBE), f"{tag} enc={enc}")
+
+
+# ---- magnitudes at which the FP32 terms of a leaf overflow, or are not numbers
+def spread_cloud(extent, far, seed=33):
+    """200 points of a cluster around the box's centre, 1e-7 of the extent wide, and `far` over the whole extent: the
+    root's children are leaves whose points are mostly far from the leaf's centre."""
+    rng = np.random.default_rng(seed)
+    near = rng.normal(0.0, 1e-7 * extent, (200, 3))
+    corners = extent * np.array([[1.0, 1.0, 1.0], [-1.0, -1.0, -1.0]])
+    xyz = np.concatenate([near, rng.uniform(-extent, extent, (far, 3)), corners])
+    return xyz, np.concatenate([np.zeros((1, 3)), near[:40], near[:80] * 0.3]), xyz[-20:]
+
+
+@pytest.mark.parametrize("extent", [1e14, 4e14, 1e15, 1e18, 6e19, 1e20, 1e24, 1e30])
+@pytest.mark.parametrize("far", [3, 198])
+def test_leaves_beyond_fp32_around_the_box_centre(ctx, extent, far):
+    xyz, middle, outer = spread_cloud(extent, far)
+    for enc in (A.ENC_MORTON, A.ENC_HILBERT):
+        sx, keys, _, c, r = O.sort_points(enc, xyz)
+        ctx.set_points(xyz)
+        ctx.sort_points(enc)
+        ctx.build(128)
+        tree = O.Tree(keys, 128, enc, c, r)
+        for where, centers in (("middle", middle), ("outer", outer)):  # not in one wave
+            for rel in (1e-7, 0.3):
+                check_forms(ctx, sx, tree, centers, np.full(len(centers), rel * extent), (A.K_SPHERE, A.K_CIRCLE),
+                            f"extent={extent:g} far={far} {where} r={rel:g} enc={enc}", lists=False)
+
+
+@pytest.mark.parametrize("ml", [16, 200])
+@pytest.mark.parametrize("sign", ["positive", "negative", "both"])
+def test_points_that_are_not_numbers(ctx, sign, ml):
+    """NaN coordinates of either sign take the largest key: one deep leaf of them, and ordinary points of the box's
+    last corner in it where the leaves are large."""
+    rng = np.random.default_rng(34)
+    xyz = rng.uniform(0.0, 8.0, (3000, 3))
+    bits = {"positive": [0x7FF8000000000000], "negative": [0xFFF8000000000000],
+            "both": [0x7FF8000000000000, 0xFFF8000000000000]}[sign]
+    nan = np.array(bits, np.uint64).view(np.float64)
+    odd = np.concatenate([np.arange(40), rng.permutation(3000)[:60]])
+    xyz[odd] = rng.choice(nan, (len(odd), 1)) * np.ones((1, 3))
+    xyz[odd[::3], 0] = 7.9  # not numbers on two axes
+    good = xyz[~np.isnan(xyz).any(axis=1)]
+    centers = np.concatenate([good[rng.permutation(len(good))[:150]], rng.uniform(7.0, 8.5, (50, 3))])
+    for enc in (A.ENC_MORTON, A.ENC_HILBERT):
+        sx, keys, _, c, r = O.sort_points(enc, xyz)
+        ctx.set_points(xyz)
+        ctx.sort_points(enc)
+        ctx.build(ml)
+        check_forms(ctx, sx, O.Tree(keys, ml, enc, c, r), centers, rng.choice([0.3, 1.0, 3.0], len(centers)),
+                    (A.K_SPHERE, A.K_CIRCLE), f"NaN {sign} leaf={ml} enc={enc}", lists=False)
