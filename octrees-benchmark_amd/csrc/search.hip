@@ -17,8 +17,8 @@
 //    |b|^2 + R), amax = max |a|^2 over the leaf, that covers every rounding of this evaluation and of the
 //    reference's FP64 one (its bound: see the leaf's tests in k_count). A set sign bit is inside, t > 2 hw
 //    outside, and what lies between is decided by the FP64 expression.
-//  - A leaf/query pair whose FP32 terms could overflow, or a leaf holding a non-finite FP32 point
-//    (then amax = inf), is decided in FP64 throughout.
+//  - A leaf/query pair whose FP32 terms could overflow or become denormal (fp32_range), or a leaf holding a
+//    non-finite FP32 point (then amax = inf), is decided in FP64 throughout.
 //  - Cube/square tests are comparisons only and run on the FP64 coordinates in both modes.
 #include <algorithm>
 #include <type_traits>
@@ -175,7 +175,7 @@ __device__ __attribute__((always_inline)) inline void group_tile(const SearchArg
                 // the leaf's FP32 form with the band folded in: t = w + C - 2 a.b (circle: its two axes)
                 // approximates |p - q|^2 - R + hw; its bound stands at the count kernel's leaf tests. Sign
                 // bit set: inside; bits above lim: outside; else (or lim = ~0, where the FP32 terms could
-                // overflow) the FP64 test decides.
+                // overflow or become denormal) the FP64 test decides.
                 const float bx = (float)(q.x - nr.cx), by = (float)(q.y - nr.cy), bz = (float)(q.z - nr.cz);
                 const float b2 = KERNEL == OCT_KERNEL_SPHERE ? __builtin_fmaf(bx, bx, __builtin_fmaf(by, by, bz * bz))
                                                              : __builtin_fmaf(bx, bx, by * by);
@@ -183,7 +183,7 @@ __device__ __attribute__((always_inline)) inline void group_tile(const SearchArg
                 const float hw = 3.814697265625e-06f * sum;  // 2^-18
                 Q.range_xy[s] = make_uint4(nr.first, last, __float_as_uint(-2.0f * bx), __float_as_uint(-2.0f * by));
                 Q.z_c_lim[s] = make_uint4(__float_as_uint(-2.0f * bz), __float_as_uint((hw - qRf) + b2),
-                                          sum < 1e30f ? __float_as_uint(2.0f * hw) : 0xffffffffu, 0u);
+                                          fp32_range(sum) ? __float_as_uint(2.0f * hw) : 0xffffffffu, 0u);
             } else {
                 Q.range[s] = make_uint2(nr.first, last);
             }
@@ -651,14 +651,15 @@ __device__ __attribute__((always_inline)) inline void count_tile(const SearchArg
             // 0 <= t <= 2 hw - an unsigned compare of the bit patterns, which also sends +0 there - is
             // re-tested in FP64. Slots past the leaf are sentinels (t ~ 1e30 or +inf, above 2 hw). A
             // leaf/query pair with amax + |b|^2 + R >= 1e30 (or not finite: a non-finite point makes
-            // amax = inf) is re-tested in FP64 outright (lim = ~0), so no term can overflow.
+            // amax = inf) or <= 1e-30 is re-tested in FP64 outright (lim = ~0), so no term can overflow and
+            // what denormal products lose stays below the band.
             const float bx = (float)(q.x - nr.cx), by = (float)(q.y - nr.cy), bz = (float)(q.z - nr.cz);
             const float b2 = KERNEL == OCT_KERNEL_SPHERE ? __builtin_fmaf(bx, bx, __builtin_fmaf(by, by, bz * bz))
                                                          : __builtin_fmaf(bx, bx, by * by);
             const float sum = (am + b2) + qRf;
             const float hw = 3.814697265625e-06f * sum;  // 2^-18
             const float C = qf((hw - qRf) + b2);
-            const uint32_t lim = __float_as_uint(qf(__uint_as_float(sum < 1e30f ? __float_as_uint(2.0f * hw) : 0xffffffffu)));
+            const uint32_t lim = __float_as_uint(qf(__uint_as_float(fp32_range(sum) ? __float_as_uint(2.0f * hw) : 0xffffffffu)));
             const float ux = qf(-2.0f * bx), uy = qf(-2.0f * by);
             const float uz = KERNEL == OCT_KERNEL_SPHERE ? qf(-2.0f * bz) : 0.0f;
             uint32_t c8 = 0, c8b = 0, mnb = 0xffffffffu;
@@ -805,7 +806,7 @@ __device__ __attribute__((always_inline)) inline void count_tile(const SearchArg
             const float hw = 3.814697265625e-06f * sum;  // 2^-18
             const float C = (hw - qRf) + b2;
             float lim = 2.0f * hw;
-            if (!tight && !(sum < 1e30f && sum > 1e-30f)) lim = __uint_as_float(0xffffffffu);
+            if (!tight && !fp32_range(sum)) lim = __uint_as_float(0xffffffffu);
             mq.u[rank] = make_float4(-2.0f * bx, -2.0f * by, -2.0f * bz, 1.0f);
             mq.c[rank] = make_float4(C, C, C, C);
             mq.lh[rank] = make_uint2(__float_as_uint(lim), lane);
@@ -956,7 +957,7 @@ __device__ __attribute__((always_inline)) inline void count_tile(const SearchArg
             const float sum = (am + b2) + qRf;
             const float hw = 3.814697265625e-06f * sum;  // 2^-18
             C = qf((hw - qRf) + b2);
-            lim = __float_as_uint(qf(__uint_as_float(sum < 1e30f ? __float_as_uint(2.0f * hw) : 0xffffffffu)));
+            lim = __float_as_uint(qf(__uint_as_float(fp32_range(sum) ? __float_as_uint(2.0f * hw) : 0xffffffffu)));
             ux = qf(-2.0f * bx), uy = qf(-2.0f * by);
             uz = KERNEL == OCT_KERNEL_SPHERE ? qf(-2.0f * bz) : 0.0f;
         } else {

@@ -153,6 +153,14 @@ __device__ inline bool inside64(const Query &q, double px, double py, double pz)
     }
 }
 
+// Whether a leaf's FP32 terms and their band stay within FP32, for sum = amax + |b|^2 + R (not negative): below
+// 1e30 nothing overflows; above 1e-30 the band, 2^-18 sum, is far above the rounding of products that are denormal
+// (or flushed, on the matrix cores). A NaN fails. Two instructions: the bits of such floats order as they do.
+__device__ inline bool fp32_range(float sum) {
+    constexpr uint32_t kLow = 0x0da24260u, kHigh = 0x7149f2cau;  // 1e-30f, 1e30f
+    return __float_as_uint(sum) - kLow < kHigh - kLow;
+}
+
 constexpr int kStageBytes = 2048;  // per-wave LDS staging unit of the search kernels (bytes)
 constexpr int kUnroll = 4;
 

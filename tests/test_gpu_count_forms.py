@@ -1,7 +1,7 @@
 """Counts asked for without the search counters (the only calls that judge children by the tight boxes of their
 points and test leaves on the matrix cores with that judgement behind them) and lists, where the forms could
-disagree: points outside the cells their keys name, points beyond FP32, NaNs. Every form returns exactly the
-oracle's results."""
+disagree: points outside the cells their keys name, points beyond FP32 and below it, NaNs. Every form returns
+exactly the oracle's results."""
 import numpy as np
 import pytest
 
@@ -146,3 +146,17 @@ def test_points_that_are_not_numbers(ctx, sign, ml):
         ctx.build(ml)
         check_forms(ctx, sx, O.Tree(keys, ml, enc, c, r), centers, rng.choice([0.3, 1.0, 3.0], len(centers)),
                     (A.K_SPHERE, A.K_CIRCLE), f"NaN {sign} leaf={ml} enc={enc}", lists=False)
+
+
+# ---- magnitudes at which the FP32 terms of a leaf vanish
+@pytest.mark.parametrize("scale", [1e-15, 1e-18, 1e-20, 1e-21, 1e-22, 3e-23, 1e-24])
+def test_leaves_below_fp32(ctx, scale):
+    rng = np.random.default_rng(35)
+    xyz = rng.uniform(-1.0, 1.0, (1500, 3)) * scale
+    centers = np.concatenate([xyz[:100], rng.uniform(-1.2, 1.2, (30, 3)) * scale])
+    sx, keys, _, c, r = O.sort_points(A.ENC_HILBERT, xyz)
+    ctx.set_points(xyz)
+    ctx.sort_points(A.ENC_HILBERT)
+    ctx.build(64)
+    check_forms(ctx, sx, O.Tree(keys, 64, A.ENC_HILBERT, c, r), centers, rng.choice([0.1, 0.4, 0.8], len(centers)) * scale,
+                (A.K_SPHERE, A.K_CIRCLE), f"scale={scale:g}")
