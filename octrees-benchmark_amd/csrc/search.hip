@@ -789,7 +789,8 @@ __device__ __attribute__((always_inline)) inline void count_tile(const SearchArg
     // instructions on VGPRs take 2.5 cycles, all others (3 operands, scalar operands, compares, min, FP64) 4.3.
     // tight: the leaf was reached through its parent's tight boxes, whose conditions (a finite am below 1e30 in a box
     // below 1e15, a query nearer than 3.2e14 to its centre, R above 1e-30) keep every term within FP32. Leaves
-    // reached by their cells can hold points beyond FP32 and NaNs, whatever the wave's queries.
+    // reached by their cells can hold points beyond FP32 and NaNs, whatever the wave's queries. Their ties need no
+    // walk: a node has boxes where all below it have them, so a leaf without them had every ancestor's cell judged.
     auto leaf_mfma = [&](const uint64_t m, const float am, const NodeRec &nr, const bool tight) {
         const uint32_t first = nr.first, last = nr.last;
         if (STATS) n_test += (uint64_t)__popcll(m) * (last - first);
@@ -886,7 +887,7 @@ __device__ __attribute__((always_inline)) inline void count_tile(const SearchArg
                         if (STATS) n_recheck++;
                     }
                 }
-                if (boxes && ballot64(tie)) {
+                if (tight && ballot64(tie)) {
                     qr.lox = qr.x - qr.r, qr.loy = qr.y - qr.r, qr.loz = qr.z - qr.r;
                     qr.hix = qr.x + qr.r, qr.hiy = qr.y + qr.r, qr.hiz = qr.z + qr.r;
                     const int cls = path_class(qr, first);
