@@ -227,9 +227,11 @@ int oct_knn_checksum(oct_ctx *ctx, const int32_t *idx_dev, const float *d2_dev, 
  * the point tests run on the matrix cores (FP32 sphere counts, 64 queries per wave) they are faster
  * there; 0 and -1 are accepted, 1 fails with OCT_ERR_UNSUPPORTED.
  * oct_autotune_radius: times each candidate (G = 0, 16, 32, 64) on sample_nq queries taken from the
- * sorted cloud (16 equal strided chunks of consecutive SFC points; sample_nq >= n uses every point),
- * stores the fastest for (kernel, algo, precision), returns its G in *best and the milliseconds per G
- * in ms_out[0..3].
+ * sorted cloud (16 equal strided chunks of consecutive SFC points; sample_nq >= n uses every point; a
+ * sample that would not occupy the device twice, about 2^20 queries, is raised to that), stores the
+ * fastest for (kernel, algo, precision), returns its G in *best and the milliseconds per G
+ * in ms_out[0..3]. A sample's times are compared without the launch's idle end, so *best may be up to
+ * a fifth above the smallest of ms_out.
  * oct_tuned_radius: the G a count-mode search of many consecutive points would use now (*mfma, if given, is always 0).
  * OCT_TUNE_RADIUS_REMAP: 1 (default, also -1) lets the count-mode vector point tests move the
  * queries of a leaf that at most half of a wave's queries want onto all 64 lanes; 0 keeps every

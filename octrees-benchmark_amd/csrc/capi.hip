@@ -1009,8 +1009,6 @@ int oct_set_tuning(oct_ctx *ctx, int knob, int value) {
     return OCT_OK;
 }
 
-constexpr double kResidentWaves = 256.0 * 4 * 7;  // of the count kernel: 7 per SIMD
-
 int oct_autotune_radius(oct_ctx *ctx, int kernel, int algo, int precision, double radius, size_t sample_nq, int *best,
                         double ms_out[4]) {
     if (!ctx) return OCT_ERR_ARG;
@@ -1018,7 +1016,14 @@ int oct_autotune_radius(oct_ctx *ctx, int kernel, int algo, int precision, doubl
     if (s) return s;
     if (ctx->n == 0) return fail(ctx, OCT_ERR_STATE, "autotune on an empty cloud");
     HCHK(hipSetDevice(ctx->device), "set device");
-    size_t nq = std::min(sample_nq ? sample_nq : (size_t)1 << 20, ctx->n);
+    const int cand[4] = {0, 16, 32, 64};
+    double resident[4], least = 0.0;  // least: queries with which every candidate fills its resident waves twice
+    for (int ci = 0; ci < 4; ci++) {
+        HCHK(radius_resident_waves(ctx, kernel, algo, precision, cand[ci], resident[ci]), "occupancy");
+        resident[ci] *= cand[ci] ? cand[ci] : 8;  // in queries
+        least = std::max(least, 2.0 * resident[ci]);
+    }
+    const size_t nq = std::min(std::max(sample_nq ? sample_nq : (size_t)1 << 20, (size_t)least), ctx->n);
     // 16 chunks of consecutive SFC positions spread over the cloud
     std::vector<uint32_t> idx(nq);
     const size_t chunks = 16, per = (nq + chunks - 1) / chunks;
@@ -1030,7 +1035,6 @@ int oct_autotune_radius(oct_ctx *ctx, int kernel, int algo, int precision, doubl
     HCHK(ctx->qidx.reserve(nq + 1), "alloc queries");
     HCHK(ctx->counts.reserve(nq + 1), "alloc counts");
     HCHK(hipMemcpyAsync(ctx->qidx.p, idx.data(), nq * 4, hipMemcpyHostToDevice, ctx->stream), "copy sample");
-    const int cand[4] = {0, 16, 32, 64};
     double bestms = 1e300;
     int bestg = 32;
     for (int ci = 0; ci < 4; ci++) {
@@ -1050,9 +1054,9 @@ int oct_autotune_radius(oct_ctx *ctx, int kernel, int algo, int precision, doubl
         if (ms_out) ms_out[ci] = t;
         // half a round of resident waves idles at the end of a launch, which weighs more in a short sample
         // than in the search it stands for (2^20 queries of the 50 M tile: 32 per wave 1.70 ms, 64 per wave
-        // 1.78; all 50 M: 57 and 39.8 ms)
-        if (cand[ci] && nq < ctx->n) {
-            const double rounds = (double)nq / cand[ci] / kResidentWaves;
+        // 1.78; all 50 M: 57 and 39.8 ms). At least two rounds: the correction is a fifth at most.
+        if (nq < ctx->n) {
+            const double rounds = (double)nq / resident[ci];
             t *= rounds / (rounds + 0.5);
         }
         if (t < bestms) bestms = t, bestg = cand[ci];

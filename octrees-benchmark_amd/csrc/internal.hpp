@@ -271,6 +271,8 @@ struct RadiusLaunch {
     unsigned long long *stats = nullptr;
 };
 hipError_t launch_radius(oct_ctx *ctx, const RadiusLaunch &L);
+// Waves of a count-mode search (queries per wave as in RadiusLaunch::group) that the device holds at once.
+hipError_t radius_resident_waves(const oct_ctx *ctx, int kernel, int algo, int precision, int group, double &waves);
 // Whether nq queries, `density` of the points they lie among, get their lists (their counts) 64 per wave with one
 // traversal, else each by its own.
 bool shared_traversal(size_t nq, double density);

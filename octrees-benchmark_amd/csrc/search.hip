@@ -1517,24 +1517,58 @@ static void launch_k(const SearchArgs &a, int mode, int G, hipStream_t s) {
         k_group<KERNEL, ALGO, PREC, 2><<<nb, kSearchBlock, lds, s>>>(a);
 }
 
-template <int KERNEL, int ALGO>
-static void launch_p(const SearchArgs &a, int prec, int mode, int G, hipStream_t s) {
-    if (prec == OCT_PREC_FP32_RECHECK)
-        launch_k<KERNEL, ALGO, OCT_PREC_FP32_RECHECK>(a, mode, G, s);
-    else
-        launch_k<KERNEL, ALGO, OCT_PREC_FP64>(a, mode, G, s);
+// f(kernel, algorithm, precision), as integral constants
+template <class F>
+static void with_variant(int kernel, int algo, int prec, F &&f) {
+    auto by_prec = [&](auto K, auto A) {
+        if (prec == OCT_PREC_FP32_RECHECK)
+            f(K, A, std::integral_constant<int, OCT_PREC_FP32_RECHECK>{});
+        else
+            f(K, A, std::integral_constant<int, OCT_PREC_FP64>{});
+    };
+    auto by_algo = [&](auto K) {
+        if (algo == OCT_ALGO_NEIGHBORS)
+            by_prec(K, std::integral_constant<int, OCT_ALGO_NEIGHBORS>{});
+        else if (algo == OCT_ALGO_PRUNE)
+            by_prec(K, std::integral_constant<int, OCT_ALGO_PRUNE>{});
+        else if (algo == OCT_ALGO_STRUCT)
+            by_prec(K, std::integral_constant<int, OCT_ALGO_STRUCT>{});
+        else
+            by_prec(K, std::integral_constant<int, OCT_ALGO_APPROX>{});
+    };
+    switch (kernel) {
+    case OCT_KERNEL_SPHERE: by_algo(std::integral_constant<int, OCT_KERNEL_SPHERE>{}); break;
+    case OCT_KERNEL_CIRCLE: by_algo(std::integral_constant<int, OCT_KERNEL_CIRCLE>{}); break;
+    case OCT_KERNEL_CUBE: by_algo(std::integral_constant<int, OCT_KERNEL_CUBE>{}); break;
+    default: by_algo(std::integral_constant<int, OCT_KERNEL_SQUARE>{}); break;
+    }
 }
 
-template <int KERNEL>
-static void launch_a(const SearchArgs &a, int algo, int prec, int mode, int G, hipStream_t s) {
-    if (algo == OCT_ALGO_NEIGHBORS)
-        launch_p<KERNEL, OCT_ALGO_NEIGHBORS>(a, prec, mode, G, s);
-    else if (algo == OCT_ALGO_PRUNE)
-        launch_p<KERNEL, OCT_ALGO_PRUNE>(a, prec, mode, G, s);
-    else if (algo == OCT_ALGO_STRUCT)
-        launch_p<KERNEL, OCT_ALGO_STRUCT>(a, prec, mode, G, s);
-    else
-        launch_p<KERNEL, OCT_ALGO_APPROX>(a, prec, mode, G, s);
+// levels that hold internal nodes: every level but the deepest
+static uint32_t group_levels(const oct_ctx *ctx) {
+    return ctx->n_levels > 1 ? std::min<uint32_t>(ctx->n_levels - 1, (uint32_t)kGroupMaxLevels) : 1u;
+}
+
+hipError_t radius_resident_waves(const oct_ctx *ctx, int kernel, int algo, int precision, int group, double &waves) {
+    int cus = 0, per = 0;
+    hipError_t e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device);
+    if (e != hipSuccess) return e;
+    with_variant(kernel, algo, precision, [&](auto K, auto A, auto P) {
+        constexpr int k = decltype(K)::value, al = decltype(A)::value, p = decltype(P)::value;
+        if constexpr (al != OCT_ALGO_APPROX) {
+            if (group == 0)
+                e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k_group<k, al, p, 0>, kSearchBlock,
+                                                                 (size_t)kWaves * group_levels(ctx) * 64 * sizeof(uint32_t));
+            else if (group == 16)
+                e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k_count<k, al, p, 16, false>, kSearchBlock, 0);
+            else if (group == 32)
+                e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k_count<k, al, p, 32, false>, kSearchBlock, 0);
+            else
+                e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k_count<k, al, p, 64, false>, kSearchBlock, 0);
+        }
+    });
+    waves = (double)std::max(1, cus) * (double)std::max(1, per) * kWaves;
+    return e;
 }
 
 hipError_t launch_radius(oct_ctx *ctx, const RadiusLaunch &L) {
@@ -1588,18 +1622,11 @@ hipError_t launch_radius(oct_ctx *ctx, const RadiusLaunch &L) {
     a.entries = L.entries;
     a.stats = L.stats;
     a.err = ctx->derr.p;
-    // levels that hold internal nodes: every level but the deepest
-    a.levels = L.tile_info ? (uint32_t)kGroupMaxLevels  // a forest's depth is not known here
-               : ctx->n_levels > 1 ? std::min<uint32_t>(ctx->n_levels - 1, (uint32_t)kGroupMaxLevels)
-                                   : 1u;
+    a.levels = L.tile_info ? (uint32_t)kGroupMaxLevels : group_levels(ctx);  // a forest's depth is not known here
     stage_begin(ctx, ST_SEARCH);
-    const int G = L.group;
-    switch (L.kernel) {
-    case OCT_KERNEL_SPHERE: launch_a<OCT_KERNEL_SPHERE>(a, L.algo, L.precision, L.mode, G, ctx->stream); break;
-    case OCT_KERNEL_CIRCLE: launch_a<OCT_KERNEL_CIRCLE>(a, L.algo, L.precision, L.mode, G, ctx->stream); break;
-    case OCT_KERNEL_CUBE: launch_a<OCT_KERNEL_CUBE>(a, L.algo, L.precision, L.mode, G, ctx->stream); break;
-    default: launch_a<OCT_KERNEL_SQUARE>(a, L.algo, L.precision, L.mode, G, ctx->stream); break;
-    }
+    with_variant(L.kernel, L.algo, L.precision, [&](auto K, auto A, auto P) {
+        launch_k<decltype(K)::value, decltype(A)::value, decltype(P)::value>(a, L.mode, L.group, ctx->stream);
+    });
     stage_end(ctx, ST_SEARCH);
     return hipGetLastError();
 }
