@@ -962,13 +962,24 @@ hipError_t launch_sort(oct_ctx *ctx, std::string &err) {
     // keys come from the 3-D encoders (63 bits), so bits 47..62 are the top 16 the partition sort uses
     const int mode = sort_mode(ctx);
     const bool partition = sort_partition_planned(ctx);
-    // the LSD passes are planned on the host from the encode kernel's histograms; the partition sort
-    // takes its bin starts from them on the device, so nothing is read back before it
-    uint32_t h[kEncHists * 256];
-    if (!partition) {
-        if ((e = hipMemcpyAsync(h, ctx->hist.p, sizeof(h), hipMemcpyDeviceToHost, ctx->stream)) != hipSuccess) return e;
-        if ((e = hipStreamSynchronize(ctx->stream)) != hipSuccess) return e;
-    }
+    // the LSD passes are planned on the host from the encode kernel's digit histograms (taken here where it wrote
+    // only the partition sort's); the partition sort takes its bin starts from them on the device, so nothing is
+    // read back before it
+    uint32_t h[kRadixPassCount * 256];
+    auto lsd_histograms = [&]() -> hipError_t {
+        hipError_t r;
+        if (!ctx->hist_lsd) {
+            if ((r = hipMemsetAsync(ctx->hist.p, 0, sizeof(h), ctx->stream)) != hipSuccess) return r;
+            const unsigned nb = (unsigned)std::max<size_t>(1, std::min<size_t>((n + 255) / 256, 1024));
+            k_digit_hist<<<nb, 256, 0, ctx->stream>>>(ctx->keys[0].p, n, ctx->hist.p);
+        }
+        if ((r = hipMemcpyAsync(h, ctx->hist.p, sizeof(h), hipMemcpyDeviceToHost, ctx->stream)) != hipSuccess) return r;
+        if ((r = hipStreamSynchronize(ctx->stream)) != hipSuccess) return r;
+        ctx->hist_lsd = true;
+        return hipSuccess;
+    };
+    const bool ready = !partition && ctx->hist_lsd;  // only a copy: not part of the stage
+    if (ready && (e = lsd_histograms()) != hipSuccess) return e;
     stage_begin(ctx, ST_SORT);
     uint32_t *njobs_dev = nullptr;
     if (partition) {
@@ -980,16 +991,7 @@ hipError_t launch_sort(oct_ctx *ctx, std::string &err) {
         ctx->perm = ctx->vals[1].p;
     } else {
         if ((e = hipMemsetAsync(counters, 0, 32 * sizeof(uint32_t), ctx->stream)) != hipSuccess) return e;
-        if (!ctx->hist_lsd) {  // the encode kernel wrote only the partition histogram
-            if ((e = hipMemsetAsync(ctx->hist.p, 0, kRadixPassCount * 256 * sizeof(uint32_t), ctx->stream)) != hipSuccess) return e;
-            const unsigned nb = (unsigned)std::max<size_t>(1, std::min<size_t>((n + 255) / 256, 1024));
-            k_digit_hist<<<nb, 256, 0, ctx->stream>>>(ctx->keys[0].p, n, ctx->hist.p);
-            if ((e = hipMemcpyAsync(h, ctx->hist.p, kRadixPassCount * 256 * sizeof(uint32_t), hipMemcpyDeviceToHost,
-                                    ctx->stream)) != hipSuccess)
-                return e;
-            if ((e = hipStreamSynchronize(ctx->stream)) != hipSuccess) return e;
-            ctx->hist_lsd = true;
-        }
+        if (!ready && (e = lsd_histograms()) != hipSuccess) return e;
         if ((e = sort_lsd(ctx, h, counters, errflag, bases)) != hipSuccess) return e;
     }
     stage_end(ctx, ST_SORT);
@@ -1004,16 +1006,7 @@ hipError_t launch_sort(oct_ctx *ctx, std::string &err) {
         // a segment too long for one workgroup: the LSD passes over the untouched encoded keys, timed
         // as part of the same stage; later default-form sorts of these points go to them directly
         ctx->sort_lsd_learned = true;
-        if (!ctx->hist_lsd) {
-            if ((e = hipMemsetAsync(ctx->hist.p, 0, kRadixPassCount * 256 * sizeof(uint32_t), ctx->stream)) != hipSuccess) return e;
-            const unsigned nb = (unsigned)std::max<size_t>(1, std::min<size_t>((n + 255) / 256, 1024));
-            k_digit_hist<<<nb, 256, 0, ctx->stream>>>(ctx->keys[0].p, n, ctx->hist.p);
-            if ((e = hipMemcpyAsync(h, ctx->hist.p, kRadixPassCount * 256 * sizeof(uint32_t), hipMemcpyDeviceToHost,
-                                    ctx->stream)) != hipSuccess)
-                return e;
-            if ((e = hipStreamSynchronize(ctx->stream)) != hipSuccess) return e;
-            ctx->hist_lsd = true;
-        }
+        if ((e = lsd_histograms()) != hipSuccess) return e;
         if ((e = sort_lsd(ctx, h, counters, errflag, bases)) != hipSuccess) return e;
         stage_end(ctx, ST_SORT);
         if ((e = hipMemcpyAsync(&fb[0], errflag, sizeof(uint32_t), hipMemcpyDeviceToHost, ctx->stream)) != hipSuccess) return e;
