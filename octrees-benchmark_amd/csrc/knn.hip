@@ -25,6 +25,7 @@
 #include <type_traits>
 
 #include "device.hpp"
+#include "grid.hpp"
 #include "search_common.hpp"
 
 namespace oct {
@@ -478,8 +479,8 @@ __device__ inline KnnLevels knn_levels(const KnnArgs &a) {
 }
 
 template <int S, int KC>
-__global__ __launch_bounds__(64) void k_knn(const KnnArgs a) {
-    knn_tile<S, KC>(a, blockIdx.x, knn_levels<S>(a));
+__global__ __launch_bounds__(64) void k_knn(const KnnArgs a, const uint32_t tile0) {
+    knn_tile<S, KC>(a, tile0 + blockIdx.x, knn_levels<S>(a));
 }
 
 // Work-queue form (batches): a grid of resident waves; each takes the next wave tile from a device
@@ -516,8 +517,9 @@ static void launch_sk(const KnnArgs &a, hipStream_t s) {
         k_knn_queue<S, KC><<<knn_queue_grid<S, KC>(), 64, lds, s>>>(a);
         return;
     }
-    const unsigned nb = (unsigned)(((size_t)a.nq + (64 / S) - 1) / (64 / S));
-    k_knn<S, KC><<<nb, 64, lds, s>>>(a);
+    // one launch holds 2^29 queries of 8 lanes, 2^26 of 64
+    for_grids(((size_t)a.nq + (64 / S) - 1) / (64 / S), 64,
+              [&](uint32_t tile0, unsigned nb) { k_knn<S, KC><<<nb, 64, lds, s>>>(a, tile0); });
 }
 
 // buffer size class of k (entries per query kept between selections)

@@ -23,6 +23,7 @@
 #include <algorithm>
 #include <type_traits>
 
+#include "grid.hpp"
 #include "search_common.hpp"
 
 namespace oct {
@@ -360,13 +361,13 @@ constexpr bool group_fp32() {
 }
 
 template <int KERNEL, int ALGO, int PREC, int MODE>
-__global__ __launch_bounds__(kSearchBlock) void k_group(const SearchArgs a) {
+__global__ __launch_bounds__(kSearchBlock) void k_group(const SearchArgs a, const uint32_t block0) {
     __shared__ GroupItems<group_fp32<PREC, KERNEL>()> s_items[kWaves];
     __shared__ double s_rad[3 * (kMaxDepth + 1)];
     extern __shared__ uint32_t s_gc_all[];  // per wave, per level: each lane's child's first child
     for (uint32_t i = threadIdx.x; i < 3 * (kMaxDepth + 1); i += kSearchBlock) s_rad[i] = a.radtab[i];
     __syncthreads();
-    const uint32_t w = threadIdx.x >> 6, tile = blockIdx.x * kWaves + w;
+    const uint32_t w = threadIdx.x >> 6, tile = (block0 + blockIdx.x) * kWaves + w;
     if (uniform_u32(tile * kGroupsPerWave) >= a.nq) return;
     group_tile<KERNEL, ALGO, PREC, MODE>(a, tile, 0u, a.nq, s_items[w], s_rad, s_gc_all + (size_t)w * a.levels * 64);
 }
@@ -1501,7 +1502,6 @@ static void launch_k(const SearchArgs &a, int mode, int G, hipStream_t s) {
             return;
         }
     }
-    const unsigned nb = (unsigned)(((size_t)a.nq + kGroupsPerWave * kWaves - 1) / (kGroupsPerWave * kWaves));
     const size_t lds = (size_t)kWaves * a.levels * 64 * sizeof(uint32_t);
     if constexpr (ALGO != OCT_ALGO_APPROX) {
         if (a.queue_next) {
@@ -1509,12 +1509,16 @@ static void launch_k(const SearchArgs &a, int mode, int G, hipStream_t s) {
             return;
         }
     }
-    if (mode == 0)
-        k_group<KERNEL, ALGO, PREC, 0><<<nb, kSearchBlock, lds, s>>>(a);
-    else if (mode == 1)
-        k_group<KERNEL, ALGO, PREC, 1><<<nb, kSearchBlock, lds, s>>>(a);
-    else
-        k_group<KERNEL, ALGO, PREC, 2><<<nb, kSearchBlock, lds, s>>>(a);
+    // one launch holds 2^29 queries
+    for_grids(((size_t)a.nq + kGroupsPerWave * kWaves - 1) / (kGroupsPerWave * kWaves), kSearchBlock,
+              [&](uint32_t block0, unsigned nb) {
+                  if (mode == 0)
+                      k_group<KERNEL, ALGO, PREC, 0><<<nb, kSearchBlock, lds, s>>>(a, block0);
+                  else if (mode == 1)
+                      k_group<KERNEL, ALGO, PREC, 1><<<nb, kSearchBlock, lds, s>>>(a, block0);
+                  else
+                      k_group<KERNEL, ALGO, PREC, 2><<<nb, kSearchBlock, lds, s>>>(a, block0);
+              });
 }
 
 // f(kernel, algorithm, precision), as integral constants

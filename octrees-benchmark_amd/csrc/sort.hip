@@ -14,6 +14,7 @@
 #include <algorithm>
 
 #include "device.hpp"
+#include "grid.hpp"
 
 namespace oct {
 
@@ -1083,8 +1084,7 @@ __global__ __launch_bounds__(256) void k_gather_records(const W *__restrict__ in
 
 template <class W, int L>
 static void launch_gather_words(hipStream_t s, const void *in, const uint32_t *perm, void *out, size_t n, uint32_t words) {
-    // blocks of one launch: below 2^31 (records of many words in few-byte words: the tail goes in more launches)
-    const size_t per = ((size_t)1 << 30) * 256 / L;
+    const size_t per = grid_limit(256) * 256 / L;  // records of one launch
     for (size_t at = 0; at < n; at += per) {
         const size_t m = std::min(per, n - at);
         const unsigned nb = (unsigned)((m * L + 255) / 256);
