@@ -1,0 +1,116 @@
+"""Device allocations that fail. A copy of the library is loaded behind a stand-in for hipMalloc that fails when told
+to (the device itself is never filled): a rebuild that runs out of memory, at whichever of its allocations, leaves no
+tree that a search could walk, and the next build works."""
+import ctypes as C
+import os
+import shutil
+import subprocess
+
+import numpy as np
+import pytest
+
+import octree_amd as A
+import pyoracle as O
+
+pytestmark = pytest.mark.gpu
+
+SHIM = r"""
+#include <dlfcn.h>
+#include <stddef.h>
+long shim_calls = 0, shim_allow = -1;  /* allocations so far; how many succeed from now on (-1: all) */
+int hipMalloc(void **p, size_t n) {
+    static int (*real)(void **, size_t) = 0;
+    if (!real) real = (int (*)(void **, size_t))dlsym(dlopen("libamdhip64.so.7", RTLD_NOW), "hipMalloc");
+    shim_calls++;
+    if (shim_allow == 0) return 2; /* hipErrorOutOfMemory */
+    if (shim_allow > 0) shim_allow--;
+    return real(p, n);
+}
+"""
+
+
+class Shim:
+    def __init__(self, path):
+        self.h = C.CDLL(path, mode=C.RTLD_GLOBAL)
+        self._calls, self._allow = (C.c_long.in_dll(self.h, f"shim_{n}") for n in ("calls", "allow"))
+
+    def allow(self, n):
+        self._allow.value = n
+
+    def calls(self):
+        return self._calls.value
+
+
+@pytest.fixture(scope="module")
+def shim_and_ctx(tmp_path_factory):
+    d = tmp_path_factory.mktemp("shim")
+    (d / "shim.c").write_text(SHIM)
+    subprocess.run(["gcc", "-O1", "-shared", "-fPIC", str(d / "shim.c"), "-o", str(d / "shim.so"), "-ldl"], check=True)
+    path = str(d / "liboctree_behind_shim.so")
+    shutil.copy(A.LIB_PATH, path)
+    shim = Shim(str(d / "shim.so"))
+    keep = A.lib(), A.LIB_PATH
+    A._LIB, A.LIB_PATH = None, path
+    try:
+        ctx = A.Octree(0)
+    finally:
+        A._LIB, A.LIB_PATH = keep
+    assert shim.calls() > 0, "the copy does not allocate through the stand-in"
+    yield shim, ctx
+    shim.allow(-1)
+    ctx.close()
+
+
+def cloud():
+    return np.random.default_rng(41).uniform(0.0, 10.0, (5000, 3))
+
+
+def count(ctx, centers, radius, group=64):
+    """Sphere counts in FP32 without the search counters."""
+    counts = np.empty(len(centers), np.uint32)
+    ctx.set_group(group)
+    try:
+        rc = ctx.L.oct_radius(ctx.h, A.K_SPHERE, A.A_STRUCT, A.PREC_FP32, centers.ctypes.data, None, None, radius, len(centers),
+                              0, counts.ctypes.data, None)
+    finally:
+        ctx.set_group(-1)
+    return rc, counts
+
+
+def test_failed_rebuild_leaves_no_tree(shim_and_ctx):
+    shim, ctx = shim_and_ctx
+    xyz = cloud()
+    sx, keys, _, c, r = O.sort_points(A.ENC_MORTON, xyz)
+    centers = np.ascontiguousarray(sx[::50])
+    _, want = O.radius(O.Tree(keys, 64, A.ENC_MORTON, c, r), sx, A.K_SPHERE, A.A_STRUCT, centers, 0.8)
+    leaf, failures = 64, 0
+    for allowed in range(12):
+        ctx.set_points(xyz)
+        ctx.sort_points(A.ENC_MORTON, fetch=False)
+        ctx.build(leaf)
+        rc, counts = count(ctx, centers, 0.8)
+        assert rc == 0
+        np.testing.assert_array_equal(counts, want)
+        print(f"[gpu] rebuild with {allowed} allocations", flush=True)
+        leaf = max(1, leaf // 2)  # smaller leaves: the node arrays grow
+        shim.allow(allowed)
+        try:
+            ctx.build(leaf)
+            rc, counts = count(ctx, centers, 0.8)
+            assert rc == 0  # the rebuild had enough
+            np.testing.assert_array_equal(counts, want)
+        except A.OctError:
+            failures += 1
+            rc, _ = count(ctx, centers, 0.8)
+            assert rc != 0 and b"before oct_build" in ctx.L.oct_last_error(ctx.h)
+            with pytest.raises(A.OctError, match="before oct_build"):
+                ctx.knn(3, idx=np.arange(4))
+            with pytest.raises(A.OctError, match="before oct_build"):
+                ctx.get_tree()
+        finally:
+            shim.allow(-1)
+    assert failures > 0
+    ctx.build(32)
+    rc, counts = count(ctx, centers, 0.8)
+    assert rc == 0
+    np.testing.assert_array_equal(counts, want)
