@@ -651,7 +651,7 @@ int oct_build(oct_ctx *ctx, uint32_t max_points_leaf, oct_tree_info *info) {
     if (!ctx->has_sorted) return fail(ctx, OCT_ERR_STATE, "oct_build before the cloud is sorted");
     HCHK(hipSetDevice(ctx->device), "set device");
     setup_geometry(ctx);
-    ctx->has_tree = ctx->has_boxes = false;  // of the tree that is overwritten now
+    ctx->has_tree = ctx->has_boxes = ctx->no_boxes = false;  // of the tree that is overwritten now
     std::string err;
     hipError_t e = launch_build(ctx, max_points_leaf, err);
     if (e != hipSuccess) return err.empty() ? hfail(ctx, e, "build") : fail(ctx, OCT_ERR_STATE, err);

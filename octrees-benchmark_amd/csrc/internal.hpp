@@ -177,6 +177,7 @@ struct oct_ctx {
     oct::DevBuf<oct::NodeBox> nbox;  // per internal node: its children's tight boxes (launch_boxes)
     oct::DevBuf<oct::PointBox> pbox; // per node
     bool has_boxes = false;          // nbox belongs to the current tree
+    bool no_boxes = false;           // the device had no room for the current tree's: its cells are judged
     float box_scale = 1.0f;          // its unit
     oct::DevBuf<uint32_t> scan;     // scan scratch
 

@@ -1588,15 +1588,17 @@ hipError_t launch_radius(oct_ctx *ctx, const RadiusLaunch &L) {
     for (int k = 0; k < 3; k++) extent = std::max(extent, 2.0 * fabs(ctx->radii[k]));
     if (L.mode == 0 && L.group == 64 && L.kernel == OCT_KERNEL_SPHERE && L.precision == OCT_PREC_FP32_RECHECK &&
         (L.algo == OCT_ALGO_PRUNE || L.algo == OCT_ALGO_STRUCT) && !L.tile_info && !L.stats && ctx->n_total > 1 &&
-        extent < 1e15) {
+        extent < 1e15 && !ctx->no_boxes) {
         const hipError_t e = launch_boxes(ctx);
         if (e != hipSuccess && e != hipErrorOutOfMemory) return e;
         double mc = 0.0;
         for (int k = 0; k < 3; k++) mc = std::max(mc, ctx->geo[66 + k]);
-        if (e == hipSuccess)
+        if (e == hipSuccess) {
             a.nbox = ctx->nbox.p;
-        else
-            (void)hipGetLastError();  // no room for the boxes: the cells are judged
+        } else {  // the cells are judged, and no count of this tree asks for the memory again
+            (void)hipGetLastError();
+            ctx->no_boxes = true;
+        }
         a.box_scale = ctx->box_scale;
         a.tie_scale = mc * 1.4210854715202004e-14;                                // 2^-46
         a.tight_min = (float)std::max(1e-30, mc * mc * 8.881784197001252e-16);  // (2^-25 mc)^2

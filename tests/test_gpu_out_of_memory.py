@@ -1,6 +1,6 @@
 """Device allocations that fail. A copy of the library is loaded behind a stand-in for hipMalloc that fails when told
 to (the device itself is never filled): a rebuild that runs out of memory, at whichever of its allocations, leaves no
-tree that a search could walk, and the next build works."""
+tree that a search could walk, and the next build works; counts whose tight boxes find no room do without them."""
 import ctypes as C
 import os
 import shutil
@@ -113,4 +113,36 @@ def test_failed_rebuild_leaves_no_tree(shim_and_ctx):
     ctx.build(32)
     rc, counts = count(ctx, centers, 0.8)
     assert rc == 0
+    np.testing.assert_array_equal(counts, want)
+
+
+def test_counts_without_room_for_the_boxes(shim_and_ctx):
+    """The tight boxes of a tree are allocated by its first count that can use them. Without room the cells are judged,
+    and the counts that follow do not ask again until the next build."""
+    shim, ctx = shim_and_ctx
+    xyz = np.random.default_rng(42).uniform(0.0, 10.0, (60_000, 3))  # more nodes than the other test's trees
+    sx, keys, _, c, r = O.sort_points(A.ENC_MORTON, xyz)
+    centers = np.ascontiguousarray(sx[::500])
+    _, want = O.radius(O.Tree(keys, 4, A.ENC_MORTON, c, r), sx, A.K_SPHERE, A.A_STRUCT, centers, 0.4)
+    ctx.set_points(xyz)
+    ctx.sort_points(A.ENC_MORTON, fetch=False)
+    ctx.build(4)
+    count(ctx, centers, 0.4, group=0)  # the buffers of the queries and results
+    asked = []
+    for allowed in (0, 0, 0):
+        before = shim.calls()
+        shim.allow(allowed)
+        try:
+            rc, counts = count(ctx, centers, 0.4)
+        finally:
+            shim.allow(-1)
+        asked.append(shim.calls() - before)
+        assert rc == 0, ctx.L.oct_last_error(ctx.h)
+        np.testing.assert_array_equal(counts, want)
+    print(f"[gpu] allocations of three counts: {asked}", flush=True)
+    assert asked[0] > 0 and asked[1:] == [0, 0]
+    before = shim.calls()
+    ctx.build(4)
+    rc, counts = count(ctx, centers, 0.4)
+    assert rc == 0 and shim.calls() > before
     np.testing.assert_array_equal(counts, want)
