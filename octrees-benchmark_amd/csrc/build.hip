@@ -407,7 +407,9 @@ hipError_t launch_boxes(oct_ctx *ctx) {
     if (ctx->has_boxes) return hipSuccess;
     const uint32_t nt = ctx->n_total;
     hipError_t e;
-    if ((e = ctx->pbox.reserve(nt)) != hipSuccess) return e;
+    // the nodes' own boxes are needed here only: they lie in the sort's key buffer, which no sort is using
+    if ((e = ctx->keys_p.reserve((size_t)nt * (sizeof(PointBox) / sizeof(uint64_t)))) != hipSuccess) return e;
+    PointBox *pbox = reinterpret_cast<PointBox *>(ctx->keys_p.p);
     if ((e = ctx->nbox.reserve(ctx->n_internal + 1)) != hipSuccess) return e;
     double ext = 0.0;
     for (int a = 0; a < 3; a++) ext = std::max(ext, 2.0 * fabs(ctx->radii[a]));
@@ -418,12 +420,12 @@ hipError_t launch_boxes(oct_ctx *ctx) {
     for (uint32_t l = 0; l < kMaxDepth + 3; l++) lt.start[l] = ctx->level_start[l];
     const double mc = std::max(ctx->geo[66], std::max(ctx->geo[67], ctx->geo[68]));
     k_leaf_box<<<nb, 256, 0, ctx->stream>>>(ctx->p64.p, ctx->p32.p, ctx->nodes.p, ctx->child.p, ctx->amax.p, ctx->radtab.p, lt,
-                                            mc * 0x1p-49, nt, ctx->pbox.p);
+                                            mc * 0x1p-49, nt, pbox);
     for (int l = (int)ctx->n_levels - 2; l >= 0; l--) {
         const uint32_t ls = ctx->level_start[l], le = ctx->level_start[l + 1];
         if (le > ls)
             k_node_box<<<(unsigned)(((size_t)(le - ls) * 8 + 255) / 256), 256, 0, ctx->stream>>>(
-                ctx->nodes.p, ctx->child.p, ctx->next.p, ls, le, ctx->box_scale, ctx->pbox.p, ctx->nbox.p);
+                ctx->nodes.p, ctx->child.p, ctx->next.p, ls, le, ctx->box_scale, pbox, ctx->nbox.p);
     }
     if ((e = hipGetLastError()) != hipSuccess) return e;
     ctx->has_boxes = true;

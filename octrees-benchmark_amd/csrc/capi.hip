@@ -469,7 +469,7 @@ int oct_destroy(oct_ctx *ctx) {
     ctx->amax.release(), ctx->scan.release();
     ctx->qidx.release(), ctx->qxyz.release(), ctx->qrad.release(), ctx->counts.release(), ctx->qoff.release();
     ctx->entries.release(), ctx->stats.release(), ctx->kidx.release(), ctx->kd2.release();
-    ctx->next.release(), ctx->nbox.release(), ctx->pbox.release(), ctx->qrad3.release(), ctx->kc_xyz.release(), ctx->kc_keys.release();
+    ctx->next.release(), ctx->nbox.release(), ctx->qrad3.release(), ctx->kc_xyz.release(), ctx->kc_keys.release();
     ctx->kd2f.release(), ctx->radtab.release(), ctx->las_rec.release(), ctx->las_meta.release();
     ctx->rec_in.release(), ctx->rec_out.release(), ctx->derr.release(), ctx->bbox_part.release();
     ctx->box.release(), ctx->msd.release(), ctx->keys_p.release(), ctx->vals_p.release();

@@ -175,7 +175,6 @@ struct oct_ctx {
     oct::DevBuf<float> amax;        // per-leaf max squared norm of its recentred FP32 points
     oct::DevBuf<oct::NodeExt> next;  // per internal node: its children in combo order
     oct::DevBuf<oct::NodeBox> nbox;  // per internal node: its children's tight boxes (launch_boxes)
-    oct::DevBuf<oct::PointBox> pbox; // per node
     bool has_boxes = false;          // nbox belongs to the current tree
     bool no_boxes = false;           // the device had no room for the current tree's: its cells are judged
     float box_scale = 1.0f;          // its unit

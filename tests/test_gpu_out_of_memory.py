@@ -146,3 +146,25 @@ def test_counts_without_room_for_the_boxes(shim_and_ctx):
     rc, counts = count(ctx, centers, 0.4)
     assert rc == 0 and shim.calls() > before
     np.testing.assert_array_equal(counts, want)
+
+
+def test_memory_the_boxes_keep(shim_and_ctx):
+    """Of what the boxes are made from, only the boxes themselves stay allocated."""
+    shim, ctx = shim_and_ctx
+    xyz = np.random.default_rng(43).uniform(0.0, 20.0, (400_000, 3))
+    ctx.set_points(xyz)
+    ctx.sort_points(A.ENC_MORTON, fetch=False)
+    ctx.build(16)
+    centers = np.ascontiguousarray(xyz[:100])
+    rc, want = count(ctx, centers, 0.5, group=0)
+    assert rc == 0
+    before = shim.calls()
+    rc, counts = count(ctx, centers, 0.5)
+    print(f"[gpu] allocations of the first count: {shim.calls() - before}", flush=True)
+    assert rc == 0 and shim.calls() - before == 1
+    np.testing.assert_array_equal(counts, want)
+    perm, keys = ctx.sort_points(A.ENC_MORTON)[2:]  # the sort's buffers are its own again
+    c, r = O.mbb(xyz)
+    okeys, operm = O.sort(O.encode(A.ENC_MORTON, xyz, c, r))
+    np.testing.assert_array_equal(keys, okeys)
+    np.testing.assert_array_equal(perm, operm)
