@@ -1584,6 +1584,7 @@ hipError_t launch_radius(oct_ctx *ctx, const RadiusLaunch &L) {
     a.nodes = ctx->nodes.p;
     a.next = ctx->next.p;
     a.nbox = nullptr, a.tie_scale = 0.0, a.tight_min = a.box_scale = 0.0f;
+    stage_begin(ctx, ST_SEARCH);  // a tree's first count that uses the tight boxes makes them
     double extent = 0.0;  // clouds of 1e15 and more have no boxes: their FP32 terms are checked leaf by leaf
     for (int k = 0; k < 3; k++) extent = std::max(extent, 2.0 * fabs(ctx->radii[k]));
     if (L.mode == 0 && L.group == 64 && L.kernel == OCT_KERNEL_SPHERE && L.precision == OCT_PREC_FP32_RECHECK &&
@@ -1629,7 +1630,6 @@ hipError_t launch_radius(oct_ctx *ctx, const RadiusLaunch &L) {
     a.stats = L.stats;
     a.err = ctx->derr.p;
     a.levels = L.tile_info ? (uint32_t)kGroupMaxLevels : group_levels(ctx);  // a forest's depth is not known here
-    stage_begin(ctx, ST_SEARCH);
     with_variant(L.kernel, L.algo, L.precision, [&](auto K, auto A, auto P) {
         launch_k<decltype(K)::value, decltype(A)::value, decltype(P)::value>(a, L.mode, L.group, ctx->stream);
     });

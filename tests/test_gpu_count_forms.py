@@ -160,3 +160,27 @@ def test_leaves_below_fp32(ctx, scale):
     ctx.build(64)
     check_forms(ctx, sx, O.Tree(keys, 64, A.ENC_HILBERT, c, r), centers, rng.choice([0.1, 0.4, 0.8], len(centers)) * scale,
                 (A.K_SPHERE, A.K_CIRCLE), f"scale={scale:g}")
+
+
+def test_the_first_count_reports_the_boxes_it_makes(ctx):
+    """A tree's first count that uses the tight boxes makes them, over every node; its stage time says so."""
+    xyz = np.random.default_rng(36).uniform(0.0, 50.0, (1_000_000, 3))
+    centers = np.full((64, 3), 500.0)  # outside the root: the search itself is next to nothing
+    radii = np.full(64, 0.3)
+    ctx.set_points(xyz)
+    ctx.sort_points(A.ENC_MORTON, fetch=False)
+    times = []
+    ctx.set_group(64)
+    try:
+        for _ in range(3):  # trees; the first one's count also loads code and allocates
+            ctx.build(8)
+            tree = []
+            for _ in range(4):
+                count(ctx, A.K_SPHERE, A.A_STRUCT, A.PREC_FP32, centers, radii)
+                tree.append(ctx.stage_times()["search"])
+            times.append(tree)
+    finally:
+        ctx.set_group(-1)
+    print(f"[forms] search stage, four counts of each of three trees: {times}", flush=True)
+    for tree in times[1:]:
+        assert tree[0] > 3.0 * max(tree[1:])
