@@ -291,6 +291,17 @@ static int upload_xyz_soa(oct_ctx *ctx, const double *x, const double *y, const 
     return OCT_OK;
 }
 
+// Memory of the context's own device, which its kernels can read. What else a device-to-device copy takes (another
+// device's memory, managed or host memory) is left to the runtime's copy.
+bool on_device(const oct_ctx *ctx, const void *p) {
+    hipPointerAttribute_t a;
+    if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return a.type == hipMemoryTypeDevice && a.device == ctx->device;
+}
+
 // Copies n points (x, y, z leading doubles, stride bytes apart) into the packed device array.
 // Packed input is one flat copy; strided input (e.g. the 32-byte Point) is copied flat into a
 // staging buffer and repacked on the device.
@@ -302,7 +313,7 @@ int upload_xyz(oct_ctx *ctx, const double *src, size_t n, size_t stride, hipMemc
     HCHK(ctx->xyz.reserve(3 * n), "alloc points");
     if (n) {
         if (!src) return fail(ctx, OCT_ERR_ARG, "null point buffer");
-        if (stride == 24 && kind == hipMemcpyDeviceToDevice && (uintptr_t)src % 16 == 0) {
+        if (stride == 24 && kind == hipMemcpyDeviceToDevice && (uintptr_t)src % 16 == 0 && on_device(ctx, src)) {
             HCHK(launch_copy_points(ctx, src, n), "copy points");
         } else if (stride == 24) {
             HCHK(hipMemcpyAsync(ctx->xyz.p, src, n * 24, kind, ctx->stream), "copy points");
