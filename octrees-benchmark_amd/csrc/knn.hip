@@ -17,7 +17,10 @@
 //    below it (a few interpolated guesses: the count grows about linearly with the squared distance),
 //    keeps those and drops the rest; T bounds the k-th distance from above. No entry is sorted until the
 //    end, when the k best of the remaining few are ordered exactly. More than kw entries can share T's
-//    upper bits (ties): where they would fill the buffer, an exact selection keeps the k best.
+//    upper bits (ties): where they would fill the buffer, an exact selection keeps the k best, and from then
+//    on points are held against the k-th of them, distance and index. (Against T alone every further point of
+//    a stack of duplicates is accepted, and one step in two ends in an exact selection: 100 k queries, a sixth
+//    of them at a stack of 20 k points, k = 10: 27.8 ms, with the k-th 10.9.)
 // Both precisions run the same FP64 distances: MI355X issues FP64 at the rate of unpacked FP32, and a
 // leaf-recentred FP32 screen in front of them (16 instead of 32 bytes per point, a second load for what
 // passes) was 6 - 17 % slower at every k from 1 to 1000.
@@ -94,6 +97,8 @@ __device__ __attribute__((always_inline)) inline void knn_tile(const KnnArgs &a,
     static_assert(CAP - STEP >= KC, "a step must fit after a selection");
     __shared__ uint64_t s_bd[G * CAP];
     __shared__ uint32_t s_bi[G * CAP];
+    __shared__ uint64_t s_kd[G];  // with `ties`: the k-th entry of the group's last exact selection
+    __shared__ uint32_t s_ki[G];
     __shared__ double s_rad[66];
 
     const uint32_t lane = threadIdx.x;
@@ -155,6 +160,7 @@ __device__ __attribute__((always_inline)) inline void knn_tile(const KnnArgs &a,
     constexpr uint32_t kFresh = KC / 2 > 8 ? KC / 2 : 8;  // appended entries that are worth a new bound
     uint32_t cnt = 0, kept = 0;   // entries in the buffer; of them, after the last selection
     uint32_t T = 0xffffffffu;     // entries have upper distance bits <= T; ~0: fewer than k seen
+    bool ties = false;            // an exact selection took place (the wave's groups together)
     double tau = __builtin_huge_val();      // FP64 upper bound of the k-th distance with the pruning margin
     float tauf = __builtin_huge_valf();     // the same rounded up to FP32
     uint32_t n_nodes = 0, n_test = 0, n_select = 0, n_steps = 0;
@@ -320,6 +326,14 @@ __device__ __attribute__((always_inline)) inline void knn_tile(const KnnArgs &a,
         if (ballot64(cnt > (uint32_t)(CAP - STEP))) {  // ties fill the buffer: keep exactly the k best
             order_entries();
             wsync();
+            if (c == 0) {
+                if (part)
+                    s_kd[qs] = bd[k - 1], s_ki[qs] = bi[k - 1];
+                else if (!ties)
+                    s_kd[qs] = ~0ull, s_ki[qs] = 0xffffffffu;
+            }
+            ties = true;
+            wsync();
         }
         kept = cnt;
     };
@@ -429,6 +443,12 @@ __device__ __attribute__((always_inline)) inline void knn_tile(const KnnArgs &a,
                     n_test += acc[u] ? 1u : 0u;
                     acc[u] = acc[u] & (hi32(d[u]) <= T);
                 }
+            }
+            if (ties) {
+                const uint64_t kd = s_kd[qs];
+                const uint32_t ki = s_ki[qs];
+#pragma unroll
+                for (int u = 0; u < U; u++) acc[u] = acc[u] & knn_less(d[u], i + (uint32_t)(u * S) + c, kd, ki);
             }
 #pragma unroll
             for (int u = 0; u < U; u++) append(acc[u], d[u], i + (uint32_t)(u * S) + c);
