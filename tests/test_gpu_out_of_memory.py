@@ -1,5 +1,5 @@
-"""Device allocations that fail. A copy of the library is loaded behind a stand-in for hipMalloc that fails when told
-to (the device itself is never filled): a rebuild that runs out of memory, at whichever of its allocations, leaves no
+"""Device allocations that fail, and pinned ones that are given back. A copy of the library is loaded behind a stand-in
+for hipMalloc that fails when told to (the device itself is never filled): a rebuild that runs out of memory, at whichever of its allocations, leaves no
 tree that a search could walk, and the next build works; counts whose tight boxes find no room do without them."""
 import ctypes as C
 import os
@@ -18,9 +18,21 @@ SHIM = r"""
 #include <dlfcn.h>
 #include <stddef.h>
 long shim_calls = 0, shim_allow = -1;  /* allocations so far; how many succeed from now on (-1: all) */
+long shim_pinned = 0;                  /* pinned allocations that live */
+static void *hip(const char *name) { return dlsym(dlopen("libamdhip64.so.7", RTLD_NOW), name); }
+int hipHostMalloc(void **p, size_t n, unsigned flags) {
+    int e = ((int (*)(void **, size_t, unsigned))hip("hipHostMalloc"))(p, n, flags);
+    if (!e) shim_pinned++;
+    return e;
+}
+int hipHostFree(void *p) {
+    int e = ((int (*)(void *))hip("hipHostFree"))(p);
+    if (!e && p) shim_pinned--;
+    return e;
+}
 int hipMalloc(void **p, size_t n) {
     static int (*real)(void **, size_t) = 0;
-    if (!real) real = (int (*)(void **, size_t))dlsym(dlopen("libamdhip64.so.7", RTLD_NOW), "hipMalloc");
+    if (!real) real = (int (*)(void **, size_t))hip("hipMalloc");
     shim_calls++;
     if (shim_allow == 0) return 2; /* hipErrorOutOfMemory */
     if (shim_allow > 0) shim_allow--;
@@ -32,13 +44,26 @@ int hipMalloc(void **p, size_t n) {
 class Shim:
     def __init__(self, path):
         self.h = C.CDLL(path, mode=C.RTLD_GLOBAL)
-        self._calls, self._allow = (C.c_long.in_dll(self.h, f"shim_{n}") for n in ("calls", "allow"))
+        self._calls, self._allow, self._pinned = (C.c_long.in_dll(self.h, f"shim_{n}") for n in ("calls", "allow", "pinned"))
 
     def allow(self, n):
         self._allow.value = n
 
     def calls(self):
         return self._calls.value
+
+    def pinned(self):
+        return self._pinned.value
+
+
+def context(path):
+    """A context of the library at `path`."""
+    keep = A.lib(), A.LIB_PATH
+    A._LIB, A.LIB_PATH = None, path
+    try:
+        return A.Octree(0)
+    finally:
+        A._LIB, A.LIB_PATH = keep
 
 
 @pytest.fixture(scope="module")
@@ -49,12 +74,7 @@ def shim_and_ctx(tmp_path_factory):
     path = str(d / "liboctree_behind_shim.so")
     shutil.copy(A.LIB_PATH, path)
     shim = Shim(str(d / "shim.so"))
-    keep = A.lib(), A.LIB_PATH
-    A._LIB, A.LIB_PATH = None, path
-    try:
-        ctx = A.Octree(0)
-    finally:
-        A._LIB, A.LIB_PATH = keep
+    ctx = context(path)
     assert shim.calls() > 0, "the copy does not allocate through the stand-in"
     yield shim, ctx
     shim.allow(-1)
@@ -168,3 +188,29 @@ def test_memory_the_boxes_keep(shim_and_ctx):
     okeys, operm = O.sort(O.encode(A.ENC_MORTON, xyz, c, r))
     np.testing.assert_array_equal(keys, okeys)
     np.testing.assert_array_equal(perm, operm)
+
+
+def test_pinned_pages_are_given_back(shim_and_ctx, tmp_path):
+    """The contexts share a slab of pinned pages, 64 of them; those beyond have their own. All of it goes with the last
+    context, and contexts made after that work."""
+    shim, _ = shim_and_ctx
+    path = str(tmp_path / "liboctree_pages.so")  # a copy of its own: no context of it lives yet
+    shutil.copy(A.LIB_PATH, path)
+    before = shim.pinned()
+    xyz = cloud()
+    for n in (1, 3, 66, 1):
+        print(f"[gpu] {n} contexts", flush=True)
+        ctxs = [context(path) for _ in range(n)]
+        assert shim.pinned() - before == 1 + max(0, n - 64)
+        for c in (ctxs[0], ctxs[-1]):
+            c.set_points(xyz)
+            c.sort_points(A.ENC_MORTON, fetch=False)
+            c.build(64)
+            rc, counts = count(c, np.ascontiguousarray(xyz[:10]), 0.5)
+            assert rc == 0 and counts.min() > 0
+        for c in ctxs[: n // 2]:
+            c.close()
+        assert shim.pinned() > before
+        for c in ctxs[n // 2 :]:
+            c.close()
+        assert shim.pinned() == before
