@@ -19,7 +19,7 @@ struct SearchArgs {
     const NodeRec *__restrict__ nodes;
     const NodeExt *__restrict__ next;
     const NodeBox *__restrict__ nbox;  // tight boxes (one cloud, FP32 sphere counts), or null
-    double tie_scale;  // 2^-46 x the largest coordinate of the root box: see leaf_exact
+    double tie_scale;  // 2^-46 x the largest coordinate of the root box: see leaf_mfma and path_class
     float box_scale;   // unit of the boxes
     float tight_min;   // smallest squared distance scale at which the boxes' margin covers the FP64 rounding
     const uint32_t *__restrict__ child;

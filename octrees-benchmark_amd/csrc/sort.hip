@@ -76,7 +76,7 @@ __global__ __launch_bounds__(kSortBlock) void k_onesweep(const uint64_t *__restr
 
         uint64_t k[kSortItems];
         uint32_t v[kSortItems];
-    #pragma unroll
+#pragma unroll
         for (int r = 0; r < kSortItems; r++) {
             size_t p = wave_base + (size_t)r * 64 + lane;
             bool valid = p < limit;
@@ -84,13 +84,13 @@ __global__ __launch_bounds__(kSortBlock) void k_onesweep(const uint64_t *__restr
             v[r] = valid ? (vin ? vin[p] : (uint32_t)p) : 0u;
         }
         uint32_t rank[kSortItems];
-    #pragma unroll
+#pragma unroll
         for (int r = 0; r < kSortItems; r++) {
             size_t p = wave_base + (size_t)r * 64 + lane;
             bool valid = p < limit;
             uint32_t d = (uint32_t)(k[r] >> shift) & 255u;
             uint64_t peers = ballot64(valid);
-    #pragma unroll
+#pragma unroll
             for (int b = 0; b < 8; b++) {
                 bool bit = (d >> b) & 1u;
                 uint64_t m = ballot64(bit);
@@ -113,7 +113,7 @@ __global__ __launch_bounds__(kSortBlock) void k_onesweep(const uint64_t *__restr
         uint32_t tile_count = 0;
         uint32_t *lb = lookback + (size_t)tile * 256;
         if (owner) {
-    #pragma unroll
+#pragma unroll
             for (int ww = 0; ww < kSortBlock / 64; ww++) {
                 uint32_t c = s_wave[ww][b];
                 s_wave[ww][b] = tile_count;
@@ -163,7 +163,7 @@ __global__ __launch_bounds__(kSortBlock) void k_onesweep(const uint64_t *__restr
         __syncthreads();
 
         // stage the tile in LDS in (bin, original order) order
-    #pragma unroll
+#pragma unroll
         for (int r = 0; r < kSortItems; r++) {
             size_t p = wave_base + (size_t)r * 64 + lane;
             if (p < limit) {
@@ -189,7 +189,8 @@ __global__ __launch_bounds__(kSortBlock) void k_onesweep(const uint64_t *__restr
                 if (j == 0 || (uint32_t)(s_keys[j - 1] >> kMsdShift2) != pre) atomicAdd(&hist16[pre], 0u - j);
                 if (j + 1 == tile_n || (uint32_t)(s_keys[j + 1] >> kMsdShift2) != pre) atomicAdd(&hist16[pre], j + 1u);
             }
-        }        if constexpr (DYN) __syncthreads();  // the next tile reuses the LDS
+        }
+        if constexpr (DYN) __syncthreads();  // the next tile reuses the LDS
     } while (DYN);
 }
 
