@@ -584,7 +584,7 @@ __device__ __attribute__((always_inline)) inline void count_tile(const SearchArg
                 if (64u * i < slots && t < slots) {
                     const bool real = t < P;
                     sp64[(t & (st - 1u)) * rs + (t >> lg)] =
-                        make_double4(real ? v[i].x : 1e300, real ? v[i].y : 1e300, real ? v[i].z : 1e300, 0.0);
+                        make_double4(real ? v[i].x : __builtin_nan(""), real ? v[i].y : __builtin_nan(""), real ? v[i].z : __builtin_nan(""), 0.0);
                 }
             }
         }
@@ -986,7 +986,7 @@ __device__ __attribute__((always_inline)) inline void count_tile(const SearchArg
                                                                        : make_float4(0.0f, 0.0f, 0.0f, 1e30f));
                 } else {
                     const double4 v = a.p64[base + min(t, P - 1)];
-                    if (t < slots) sp64[at] = make_double4(real ? v.x : 1e300, real ? v.y : 1e300, real ? v.z : 1e300, 0.0);
+                    if (t < slots) sp64[at] = make_double4(real ? v.x : __builtin_nan(""), real ? v.y : __builtin_nan(""), real ? v.z : __builtin_nan(""), 0.0);
                 }
             }
             static_assert(NI == 1 && CAP <= 64, "one load per lane and chunk");

@@ -184,3 +184,20 @@ def test_the_first_count_reports_the_boxes_it_makes(ctx):
     print(f"[forms] search stage, four counts of each of three trees: {times}", flush=True)
     for tree in times[1:]:
         assert tree[0] > 3.0 * max(tree[1:])
+
+
+# ---- radii whose squares, or whose boxes, leave FP64
+@pytest.mark.parametrize("radius", [1e150, 1e155, 1e200, 9e299, 1.1e300, 1.7e308, np.inf])
+def test_radii_beyond_fp64(ctx, radius):
+    """Every point is a neighbour, none twice, and nothing but points."""
+    rng = np.random.default_rng(37)
+    xyz = rng.uniform(0.0, 10.0, (700, 3))
+    centers = np.concatenate([xyz[:70], [[-50.0, 3.0, 1e5]]])
+    radii = np.full(len(centers), radius)
+    radii[::7] = 2.0
+    sx, keys, _, c, r = O.sort_points(A.ENC_MORTON, xyz)
+    ctx.set_points(xyz)
+    ctx.sort_points(A.ENC_MORTON)
+    ctx.build(64)
+    check_forms(ctx, sx, O.Tree(keys, 64, A.ENC_MORTON, c, r), centers, radii,
+                (A.K_SPHERE, A.K_CIRCLE, A.K_CUBE, A.K_SQUARE), f"radius={radius:g}")
