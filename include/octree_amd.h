@@ -61,6 +61,9 @@ typedef struct oct_tree_info {
     double build_ms;          /* device time of the build kernels */
 } oct_tree_info;
 
+/* Counters of a search. nodes_classified and points_tested are those of the reference's traversal; FP32 sphere
+ * counts asked for them judge the octree's cells for that, where the same call without (stats NULL) judges the
+ * boxes of the points and is faster, with the same counts. */
 typedef struct oct_search_stats {
     uint64_t total_neighbors;  /* sum over queries of |N(q)| */
     uint64_t points_tested;    /* per-point predicate evaluations */
@@ -362,7 +365,8 @@ int oct_las_load(oct_ctx *ctx, const char *path, oct_las_header *header);
 int oct_las_fetch(oct_ctx *ctx, double *xyz, oct_point_meta *meta);
 
 /* ---- timing: device milliseconds of the stages of the last calls (HIP events on the context's
- * stream): [0] bbox, [1] encode, [2] sort, [3] gather, [4] build, [5] search, [6] knn. */
+ * stream): [0] bbox, [1] encode, [2] sort, [3] gather, [4] build, [5] search (the first FP32 sphere
+ * count of a tree includes the boxes it makes), [6] knn. */
 int oct_stage_times(const oct_ctx *ctx, double ms[8]);
 /* Measurement aid (no reference counterpart): the best of 5 timed device copies of `bytes` bytes
  * (16-byte words), in ms -- the practical read + write ceiling for the HBM-bound stages. */

@@ -20,7 +20,8 @@
 //    upper bits (ties): where they would fill the buffer, an exact selection keeps the k best, and from then
 //    on points are held against the k-th of them, distance and index. (Against T alone every further point of
 //    a stack of duplicates is accepted, and one step in two ends in an exact selection: 100 k queries, a sixth
-//    of them at a stack of 20 k points, k = 10: 27.8 ms, with the k-th 10.9.)
+//    of them at a stack of 20 k points, k = 10: 27.8 ms, with the k-th 10.9;
+//    without stacks 0 to 1.2 % slower for it, k = 10 to 1000.)
 // Both precisions run the same FP64 distances: MI355X issues FP64 at the rate of unpacked FP32, and a
 // leaf-recentred FP32 screen in front of them (16 instead of 32 bytes per point, a second load for what
 // passes) was 6 - 17 % slower at every k from 1 to 1000.
